@@ -169,3 +169,55 @@ def tolerance(case):
     if case["op"] == "dequantize":
         return "exact"
     return {"rel": 1.2e-3, "max": 5e-3} if case["op"] == "linears" else {"rel": 2.6e-3, "max": 1.2e-2}
+
+
+def _unpack(words):
+    shifts = torch.tensor([0, 16, 4, 20, 8, 24, 12, 28], dtype=torch.int32, device=words.device)   # AWQ nibble order
+    return ((words[..., None] >> shifts) & 15).flatten(-2)
+
+
+def _weights(qw, sc, qz, k0=0, k1=None):
+    """Rows k0 .. k1 of (w - z) * s in float64 (qw [K, N / 8], sc [K / G, N], qz [K / G, N / 8])."""
+    k1 = qw.shape[0] if k1 is None else k1
+    g = torch.arange(k0, k1, device=qw.device) // (qw.shape[0] // sc.shape[0])
+    return (_unpack(qw[k0:k1]) - _unpack(qz)[g]).double() * sc.double()[g]
+
+
+def _matmul64(x, qw, sc, qz):
+    """x (float64) times the exact weights, a few thousand weight rows at a time."""
+    step = max(128, 2 ** 27 // sc.shape[1])
+    out = torch.zeros((x.shape[0], sc.shape[1]), dtype=torch.float64, device=x.device)
+    for k0 in range(0, qw.shape[0], step):
+        k1 = min(k0 + step, qw.shape[0])
+        out += x[:, k0:k1] @ _weights(qw, sc, qz, k0, k1)
+    return out
+
+
+def exact(case, seed):
+    """The pass on exact weights with float64 sums and no rounding on the way."""
+    state = prepare(case, seed)
+    if state["op"] == "dequantize":
+        return [torch.cat([_weights(*w, k0, min(k0 + 4096, w[0].shape[0])).half() for k0 in range(0, w[0].shape[0], 4096)])
+                for w in state["weights"]]
+    if state["op"] == "linears":
+        return [_matmul64(x.double(), layer.qweight, layer.scales, layer.qzeros) + (0.0 if bias is None else bias.double())
+                for layer, x, bias in state["calls"]]
+    layer, x, logits, topk = state["layer"], state["x"].double(), state["logits"].double(), state["topk"]
+    if state["scoring"] == "sigmoid":
+        score = torch.sigmoid(logits)
+        chosen = torch.topk(score + state["bias"].double(), topk, dim=-1).indices
+    else:
+        score = torch.softmax(logits, dim=-1)
+        chosen = torch.topk(score, topk, dim=-1).indices
+    weight = score.gather(1, chosen)
+    weight = weight / weight.sum(dim=-1, keepdim=True)
+    out = torch.zeros_like(x)
+    for e in range(logits.shape[1]):
+        token, slot = torch.nonzero(chosen == e, as_tuple=True)
+        if token.numel() == 0:
+            continue
+        h = _matmul64(x[token], layer.w13_qweight[e], layer.w13_scales[e], layer.w13_qzeros[e])
+        gate, up = h.chunk(2, dim=-1)
+        o = _matmul64(torch.nn.functional.silu(gate) * up, layer.w2_qweight[e], layer.w2_scales[e], layer.w2_qzeros[e])
+        out.index_add_(0, token, o * weight[token, slot, None])
+    return out
