@@ -294,9 +294,9 @@ static int ensure_kernel_attributes() {
       reinterpret_cast<const void*>(awq_gemm_mfma_kernel<true, 2>), reinterpret_cast<const void*>(awq_gemm_mfma_kernel<false, 2>),
       reinterpret_cast<const void*>(awq_gemm_mfma_kernel<true, 3>), reinterpret_cast<const void*>(awq_gemm_mfma_kernel<false, 3>),
       reinterpret_cast<const void*>(awq_gemm_mfma_kernel<true, 4>), reinterpret_cast<const void*>(awq_gemm_mfma_kernel<false, 4>),
-      reinterpret_cast<const void*>(awq_gemm_mfma_kernel<true, 1, 8, true>), reinterpret_cast<const void*>(awq_gemm_mfma_kernel<false, 1, 8, true>),
-      reinterpret_cast<const void*>(awq_gemm_mfma_kernel<true, 2, 8, true>), reinterpret_cast<const void*>(awq_gemm_mfma_kernel<false, 2, 8, true>),
-      reinterpret_cast<const void*>(awq_gemm_mfma_kernel<true, 4, 4, true>), reinterpret_cast<const void*>(awq_gemm_mfma_kernel<false, 4, 4, true>)};
+      reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<true, 1, 8>), reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<false, 1, 8>),
+      reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<true, 2, 8>), reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<false, 2, 8>),
+      reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<true, 4, 4>), reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<false, 4, 4>)};
   for (const void* fn : mfma) {
     const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, PF_LDS_BYTES);
     if (e != hipSuccess) { t_last_hip_error = (int)e; return AWQMI_LAUNCH_FAILED; }
@@ -860,17 +860,18 @@ static int moe_gemm_impl(const void* x, const int32_t* qweight, const void* scal
     p.topk_w = topk_weights; p.n_slots = n_slots; p.a_row_div = a_row_div;
     p.w_stride = (long long)K * NW; p.s_stride = (long long)(K / G) * N; p.z_stride = (long long)(K / G) * NW;
     const int nblk = (int)(awqmi_moe_align_capacity(n_slots, E, tile_m) / tile_m);
-    const dim3 grid((unsigned)nblk * p.nt);
+    p.total = nblk * p.nt;
+    const dim3 grid(((unsigned)nblk * p.nt + 7) / 8 * 8);     // whole deals to the 8 XCDs
     hipStream_t st = (hipStream_t)stream;
     if (tile_m == 64) {
-      if (pow2g) hipLaunchKernelGGL((awq_gemm_mfma_kernel<true, 1, 8, true>), grid, dim3(512), PF_LDS_BYTES, st, p);
-      else hipLaunchKernelGGL((awq_gemm_mfma_kernel<false, 1, 8, true>), grid, dim3(512), PF_LDS_BYTES, st, p);
+      if (pow2g) hipLaunchKernelGGL((awq_gemm_mfma_grouped_kernel<true, 1, 8>), grid, dim3(512), PF_LDS_BYTES, st, p);
+      else hipLaunchKernelGGL((awq_gemm_mfma_grouped_kernel<false, 1, 8>), grid, dim3(512), PF_LDS_BYTES, st, p);
     } else if (tile_m == 128) {
-      if (pow2g) hipLaunchKernelGGL((awq_gemm_mfma_kernel<true, 2, 8, true>), grid, dim3(512), PF_LDS_BYTES, st, p);
-      else hipLaunchKernelGGL((awq_gemm_mfma_kernel<false, 2, 8, true>), grid, dim3(512), PF_LDS_BYTES, st, p);
+      if (pow2g) hipLaunchKernelGGL((awq_gemm_mfma_grouped_kernel<true, 2, 8>), grid, dim3(512), PF_LDS_BYTES, st, p);
+      else hipLaunchKernelGGL((awq_gemm_mfma_grouped_kernel<false, 2, 8>), grid, dim3(512), PF_LDS_BYTES, st, p);
     } else {
-      if (pow2g) hipLaunchKernelGGL((awq_gemm_mfma_kernel<true, 4, 4, true>), grid, dim3(256), PF_LDS_BYTES, st, p);
-      else hipLaunchKernelGGL((awq_gemm_mfma_kernel<false, 4, 4, true>), grid, dim3(256), PF_LDS_BYTES, st, p);
+      if (pow2g) hipLaunchKernelGGL((awq_gemm_mfma_grouped_kernel<true, 4, 4>), grid, dim3(256), PF_LDS_BYTES, st, p);
+      else hipLaunchKernelGGL((awq_gemm_mfma_grouped_kernel<false, 4, 4>), grid, dim3(256), PF_LDS_BYTES, st, p);
     }
     return launch_status();
   }

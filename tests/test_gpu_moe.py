@@ -221,6 +221,35 @@ def test_moe_grouped_gemm_mfma_blocks(sba, gpu, bs, T, E, topk, K, N, G):
     assert awq_ref.rel_frobenius(y2, ref2) <= TOL
 
 
+@pytest.mark.parametrize("bs", [64, 128, 256])
+def test_moe_grouped_gemm_partly_filled_blocks(sba, gpu, bs):
+    """Blocks of the grouped MFMA kernel take a tile of as many rows as they hold real slots, in steps
+    of 64: experts with row counts on both sides of every step, one expert without rows, one with
+    several blocks, against per-expert oracle products."""
+    counts = [1, 64, 65, 128, 0, 129, 192, 193, 256, 257, 3 * 256 + 66]
+    E, K, N, G = len(counts), 256, 264, 64
+    rng = np.random.default_rng(bs)
+    w = rng.integers(0, 16, (E, K, N))
+    z = rng.integers(0, 16, (E, K // G, N))
+    s = (rng.random((E, K // G, N)) * 0.019 + 0.001).astype(np.float16)
+    qw, qz = awq_ref.pack_awq(w), awq_ref.pack_awq(z)
+    ids = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int32)[:, None]
+    T = len(ids)
+    x = rng.normal(0, 1, (T, K)).astype(np.float16)
+    tw = rng.random((T, 1)).astype(np.float32)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)
+    sid, eid, npp = sba.moe_align_block_size(t(ids), bs, E)
+    out = torch.full((T, N), float("nan"), dtype=torch.float16, device=gpu)
+    y = sba.moe_awq_gemm(t(x), t(qw), t(s), t(qz), sid, eid, npp, T, 1, topk_weights=t(tw), block_size=bs,
+                         out=out).cpu().numpy()
+    assert np.all(np.isfinite(y))            # every slot row written
+    for e in range(E):
+        tok = np.nonzero(ids[:, 0] == e)[0]
+        if tok.size:
+            ref = awq_ref.gemm_wide(x[tok], qw[e], s[e], qz[e], G) * tw[tok]
+            assert awq_ref.rel_frobenius(y[tok], ref) <= TOL, e
+
+
 @pytest.mark.parametrize("T,H,E,topk,I,mfma", [(2048, 2048, 128, 8, 768, False), (1024, 1024, 8, 2, 2048, False),
                                                (4096, 512, 4, 2, 384, False),     # many rows per expert
                                                (640, 256, 4, 1, 1152, False),     # top-1
