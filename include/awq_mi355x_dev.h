@@ -33,6 +33,8 @@
  *            packed words per lane and one workgroup per CU (default for tile_m = 32 without a K
  *            split: one word per lane, two 128-column blocks per workgroup, weight ring in LDS, two
  *            workgroups per CU; with 4096 its ring stays in registers)
+ *   1 << 28  awq_gemm with 33 .. 64 rows takes the one-pass kernel on layers of any size (by default
+ *            from 40 M weights on); without room for its K split's partial tiles it runs unsplit
  * The workspace must be large enough for the form that is forced: the sizes the public queries
  * return cover every variant except a forced MFMA tile size, which silently runs without its K
  * split when the workspace is too small for it.
@@ -56,7 +58,8 @@ enum {
   AWQMI_FORM_SKINNY = 1,  /* awq_gemv_kernel: up to 32 rows per pass */
   AWQMI_FORM_FUSED = 2,   /* awq_gemm_mfma_kernel: weights dequantised per tile in LDS */
   AWQMI_FORM_DENSE = 3,   /* awq_dequant_panel_kernel + awq_gemm_dense_kernel */
-  AWQMI_FORM_GENERIC = 4  /* any-shape fallback */
+  AWQMI_FORM_GENERIC = 4, /* any-shape fallback */
+  AWQMI_FORM_MID = 5      /* awq_gemm_mid_kernel: 33 .. 64 rows in one pass */
 };
 int awqmi_dev_last_gemm_form(void);
 

@@ -59,7 +59,7 @@ SIGNATURES["awqmi_dev_stream_probe"] = (c_int, [c_void_p, c_void_p, c_int, c_int
 SIGNATURES["awqmi_dev_gemm_timeline_f16"] = (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t,
                                                       c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_size_t])
 SIGNATURES["awqmi_dev_mfma_probe"] = (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p])
-FORM_SKINNY, FORM_FUSED, FORM_DENSE, FORM_GENERIC = 1, 2, 3, 4   # awqmi_dev_last_gemm_form()
+FORM_SKINNY, FORM_FUSED, FORM_DENSE, FORM_GENERIC, FORM_MID = 1, 2, 3, 4, 5   # awqmi_dev_last_gemm_form()
 
 _lib = None
 

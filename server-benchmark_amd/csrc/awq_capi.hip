@@ -15,6 +15,7 @@
 #include "awq_dequant.hpp"
 #include "awq_gemm_dense.hpp"
 #include "awq_gemm_mfma.hpp"
+#include "awq_gemm_mid.hpp"
 #include "awq_gemv.hpp"
 #include "awq_moe.hpp"
 #include "awq_probes.hpp"
@@ -67,6 +68,7 @@ enum : int {
   VAR_NO_DENSE = 1 << 25,        // awq_gemm never takes the dequantise-once form
   VAR_DENSE = 1 << 26,           // awq_gemm takes the dequantise-once form from 257 rows on (workspace permitting)
   VAR_MOE_T32_WIDE = 1 << 27,    // 32-row MoE blocks in the two-words-per-lane form (one workgroup per CU)
+  VAR_MID = 1 << 28,             // awq_gemm with 33 .. 64 rows: the one-pass mid kernel on layers of any size
 };
 inline bool variant_on(int bit) {
   return t_variant >= 0 && (t_variant & bit);
@@ -194,8 +196,43 @@ constexpr int SKINNY_MAX_M = 64;
 
 // Up to 32 rows one skinny pass (two row blocks share every unpacked operand); from 33 rows on
 // the 64-row MFMA tile beats two skinny passes on every layer shape measured (nine shapes from
-// 2048 x 5120 to 8192 x 59136, weights read from HBM: equal at worst, up to 2 x on small layers).
+// 2048 x 5120 to 8192 x 59136, weights read from HBM: equal at worst, up to 2 x on small layers), and
+// on large layers the one-pass kernel below beats both.
 inline bool skinny_rows(int M, int /*N*/) { return M <= 32; }
+
+// From 33 to 64 rows: awq_gemm_mid_kernel on layers of 40 M weights and more, wherever the skinny
+// kernel's shapes hold with two words per lane (its operands are addressed through 32-bit buffers).
+// Against the 64-row MFMA tile at 64 rows (us, weights from HBM): 8192 x 59136 79 / 115, 3584 x 37888
+// 37 / 44, 5120 x 27648 35 / 42, 29568 x 8192 50 / 62, 18944 x 3584 29 / 35, 13824 x 5120 27 / 30, 8192 x
+// 10240 28 / 29, 8192 x 8192 25 / 26; below the line its longer start and four-way sum lose: 5120 x 7168
+// even, 5120 x 5120 21.1 / 20.9, 3584 x 4608 20.4 / 18.5, 2048 x 5120 17.3 / 16.7.  Groups of 64 and 32
+// rows cost it 1 - 4 % (8192 x 59136 at 33 rows: 80, 82, 85 us for groups of 128, 64, 32 against 107 -
+// 128); 33 and 48 rows take 0.9 - 1.0 of the time of 64.
+constexpr long long MID_MIN_WEIGHTS = 40LL << 20;
+inline bool mid_shape(int M, int K, int N) {
+  return M > 32 && M <= MID_MAX_ROWS && K % 128 == 0 && N % 16 == 0 && (long long)K * N >= MID_MIN_WEIGHTS;
+}
+inline bool mid_rows(int M, int K, int N, int G, int ldw) {
+  return (mid_shape(M, K, N) || (variant_on(VAR_MID) && M > 32 && M <= MID_MAX_ROWS && N % 16 == 0)) &&
+         gemv_tiled_ok(K, G) && (size_t)M * K * 2 < (1ull << 31) && (size_t)K * ldw * 4 < (1ull << 31) &&
+         !variant_on(VAR_MID_M_SKINNY) && !variant_on(VAR_MID_M_MFMA);
+}
+inline size_t mid_partial_bytes(int N, int split) {
+  return split <= 1 ? 0 : (size_t)split * ((N + 255) / 256) * MID_SLOT_FLOATS * sizeof(float);
+}
+// K split of the mid kernel, within one round of workgroups: a 128-row chunk takes a wave about 4 us,
+// the second launch 3 us and a partial tile 64 KiB of traffic each way (the pick is within 3 % of the
+// best split on 18 layer shapes at 64 rows).
+int mid_pick_split(int K, int N) {
+  const int nchunks = K / 128, ncb = (N + 255) / 256;
+  int best = 1;
+  double best_t = 1e300;
+  for (int s = 1; s <= AWQMI_MAX_SPLIT_K && (s == 1 || (4 * s <= nchunks && ncb * s <= 256)); ++s) {
+    const double t = 4.0 * ((nchunks + 4 * s - 1) / (4 * s)) + (s > 1 ? 3.0 + 0.033 * ncb * s : 0.0);
+    if (t < best_t) { best_t = t; best = s; }
+  }
+  return best;
+}
 
 // Work split of the MFMA kernel: whole rounds of 256 tiles run one workgroup per tile; a
 // last round of fewer than 129 tiles (and any launch that small) is split in K over
@@ -491,6 +528,8 @@ size_t awqmi_gemm_workspace_bytes(int M, int K, int N, int split_k) {
     if (s <= 0) s = (K % 128 == 0) ? std::max(pick_split_k(M, K, N, 128, 1, true), pick_split_k(M, K, N, 64, 1, true)) : 1;
     skinny = gemv_partial_bytes(N, s, 1, 32);
   }
+  if (mid_shape(M, K, N))
+    skinny = std::max(skinny, mid_partial_bytes(N, split_k > 0 ? std::min(split_k, K / 128) : mid_pick_split(K, N)));
   return AWQMI_WS_COUNTER_BYTES + (mfma > skinny ? mfma : skinny);
 }
 
@@ -525,6 +564,26 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
   const bool mfma_ok = K % PF_BK == 0 && (((G & (G - 1)) == 0 && G >= 8) || G % 64 == 0) &&
                        mfma_slab_rows(M, K) > 0 && (size_t)K * ldw * 4 < (1ull << 32) &&
                        (size_t)(K / G) * N * 2 < (1ull << 32);
+  if (mid_rows(M, K, N, G, ldw)) {
+    t_last_gemm_form = AWQMI_FORM_MID;
+    MidGemmParams p{};
+    p.x = xx; p.qw = qw; p.sc = sc; p.qz = qz; p.y = yy;
+    p.M = M; p.K = K; p.N = N; p.NW = NW; p.G = G; p.ldw = ldw;
+    p.ncb = (NW + 31) / 32;
+    p.split_k = split_k > 0 ? std::min(split_k, K / 128) : mid_pick_split(K, N);
+    // the K split needs the caller's workspace; without it a workgroup takes all of K
+    if (p.split_k > 1 && (!workspace || !aligned16(workspace) ||
+                          workspace_bytes < AWQMI_WS_COUNTER_BYTES + mid_partial_bytes(N, p.split_k)))
+      p.split_k = 1;
+    p.part = workspace ? reinterpret_cast<float*>(static_cast<char*>(workspace) + AWQMI_WS_COUNTER_BYTES) : nullptr;
+    const dim3 grid(p.ncb, p.split_k);
+    if (G == 32) hipLaunchKernelGGL(awq_gemm_mid_kernel<4>, grid, dim3(256), 0, st, p);
+    else if (G == 64) hipLaunchKernelGGL(awq_gemm_mid_kernel<2>, grid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL(awq_gemm_mid_kernel<1>, grid, dim3(256), 0, st, p);
+    if (p.split_k > 1)
+      hipLaunchKernelGGL(awq_gemm_mid_reduce_kernel, dim3(p.ncb, (M + 15) / 16), dim3(256), 0, st, p);
+    return launch_status();
+  }
   bool mid_skinny = skinny_rows(M, N);
   if (variant_on(VAR_MID_M_SKINNY)) mid_skinny = true;
   if (variant_on(VAR_MID_M_MFMA)) mid_skinny = false;

@@ -50,8 +50,8 @@ struct MfmaGemmParams {
   // tile would have to pull sk_split x 256 KiB by itself, which took longer than the GEMM).
   int dp_tiles, sk_tiles, sk_split;
   float* sk_part;   // [sk_tiles][sk_split][256 * 256] fp32
-  // Expert-grouped launch (kernel instantiation GROUPED): workgroup (blk, column tile); blk is
-  // a block of BM sorted slots of one expert (moe_align with tile_m = BM).
+  // Expert-grouped launch (awq_gemm_mfma_grouped_kernel): total = launch blocks x column tiles; a
+  // block is BM sorted slots of one expert (moe_align with tile_m = BM).
   const int* sorted_ids;
   const int* expert_ids;
   const int* n_post_pad;
@@ -472,7 +472,7 @@ __global__ __launch_bounds__(64 * NWV, NWV / 4) void awq_gemm_mfma_kernel(const 
 // A workgroup takes the tile of as many rows as its block has real slots, in steps of 64: the last
 // block of an expert's run is mostly padding (65536 slots on 128 experts: 2.5 blocks of 256 per
 // expert, 2.0 of them full), and a tile costs about (rows + 112) whatever its rows hold.  With the
-// XCD order below: 8192-token block of 128 experts of 2048 x 768, top-8, 942 -> 880 us, same bits.
+// XCD order below: 8192-token block of 128 experts of 2048 x 768, top-8, 936 -> 870 us, same bits.
 //
 // The live tiles (the padded slot count is on the device only) are dealt to the eight XCDs in
 // contiguous ranges, block-major, so that the column tiles of a block share its gathered X rows and

@@ -149,6 +149,50 @@ def test_gemm_32_row_pass_with_lds_weight_ring(sba, gpu, M, K, N, G, split):
     assert np.array_equal(y.view(np.uint16), y_reg.view(np.uint16))
 
 
+@pytest.mark.parametrize("K,N,G,split", [
+    (128, 16, 128, 0),        # one chunk: three waves of four without work
+    (640, 272, 32, 0),        # ragged last column block, five chunks on four waves, a group per step
+    (768, 528, 64, 3),        # K split with more parts than chunks a part
+    (1024, 1040, 256, 2),
+    (2048, 512, -1, 4),
+    (128 * 41, 256, 128, 8),  # uneven ranges
+])
+@pytest.mark.parametrize("M", [33, 48, 49, 64])
+def test_mid_kernel_edges(sba, gpu, M, K, N, G, split):
+    """The one-pass kernel of 33 .. 64 rows (development variant bit 1 << 28 takes it on layers of any
+    size), with and without a K split, against the oracle; the result with a K split does not depend
+    on the workspace's contents."""
+    from server_benchmark_amd import _lib
+    x, qw, s, qz = _np_case(M, K, N, G if G > 0 else K, seed=K + M)
+    sba.ops.get_workspace(gpu, 32 << 20)     # room for the partial tiles of any split here
+    y = _check_gemm(sba, gpu, x, qw, s, qz, G if G > 0 else K, split, tag="one-pass", variant=1 << 28)
+    assert _lib.load().awqmi_dev_last_gemm_form() == _lib.FORM_MID
+    sba.ops.get_workspace(gpu, 32 << 20)[65536:].fill_(255)
+    y2 = sba.awq_gemm(*_dev(gpu, x, qw, s, qz), force_split_k=split, _dev_variant=1 << 28)
+    assert np.array_equal(y2.cpu().numpy(), y)
+
+
+@pytest.mark.parametrize("M,K,N,pad", [(64, 5120, 8192, True), (33, 5120, 8192, False), (48, 16384, 2560, False)])
+def test_mid_kernel_by_default_on_large_layers(sba, gpu, M, K, N, pad):
+    """Layers of 40 M weights and more take the one-pass kernel at 33 .. 64 rows, with padded rows of
+    qweight too; without room for the partial tiles of a K split it runs unsplit."""
+    from server_benchmark_amd import _lib
+    lib = _lib.load()
+    c = sba.workloads.make_linear_case(M, K, N, 128, seed=M).to(gpu)
+    qw = sba.ops.pad_qweight_rows(c.qweight) if pad else c.qweight
+    y = sba.awq_gemm(c.x, qw, c.scales, c.qzeros, 0)
+    assert lib.awqmi_dev_last_gemm_form() == _lib.FORM_MID
+    w = sba.awq_dequantize(c.qweight, c.scales, c.qzeros, 0, 0, 0)
+    ref = c.x.float() @ w.float()
+    assert float((y.float() - ref).norm() / ref.norm()) <= TOL
+    small = torch.zeros(65536, dtype=torch.uint8, device=gpu)
+    y1 = torch.empty_like(y)
+    st = lib.awqmi_gemm_f16(c.x.data_ptr(), c.qweight.data_ptr(), c.scales.data_ptr(), c.qzeros.data_ptr(), y1.data_ptr(),
+                            small.data_ptr(), small.numel(), M, K, N, 128, 0, torch.cuda.current_stream().cuda_stream)
+    assert st == 0 and lib.awqmi_dev_last_gemm_form() == _lib.FORM_MID
+    assert float((y1.float() - ref).norm() / ref.norm()) <= TOL
+
+
 @pytest.mark.parametrize("M", [32, 33, 48, 64])
 def test_gemm_wide_layer_mid_m(sba, gpu, M):
     """More than 128 column tiles: 32 rows run as one skinny pass, 33 .. 64 rows on the 64-row
