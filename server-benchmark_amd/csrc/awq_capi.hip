@@ -1073,11 +1073,13 @@ constexpr int MOE_ALIGN_SPLIT_MIN = 16384;   // slots from which it is used (409
 // three expert shapes (2048/768 x 128 experts, 6144/2560 x 160, 4096/14336 x 8):
 //   skinny: flops / (540 TFLOP/s * avg / (avg + 26)), avg = slots per expert;
 //   MFMA:   per GEMM blocks * column tiles / 256 CUs rounds (a partial last round counts as
-//           at least half) of (K / 64 + overhead) k-tiles at 5.4 ns * (rows + 112) each, plus
-//           the separate SiLU pass at 4 TB/s; blocks is the expected block count after
-//           padding each expert's run to whole blocks (slots spread evenly over the experts).
-// Within 5 % of the best forced block size on 25 points over six expert shapes (fit) and on the
-// points of three further shapes it was then checked on.
+//           at least half) of (K / 64 + overhead) k-tiles at 5.4 / 5.65 / 5.9 ns * (rows + 112) each for
+//           64 / 128 / 256 rows, plus the separate SiLU pass at 4 TB/s; blocks is the expected block count
+//           after padding each expert's run to whole blocks (slots spread evenly over the experts),
+//           a partly filled block counted by its rows in steps of 64.
+// With every block size forced in turn on 25 points (2048/768 x 128 experts, 2048/1408 x 64, 5120/1024 x
+// 64, 4096/14336 x 8; T = 64 ... 8192) the choice is within 7 % of the best size on all of them; counting
+// partly filled blocks whole was 12 % behind at worst (5120/1024 at 2000 tokens: 128 rows 457 us, 256 405).
 // The MFMA form also needs every operand under 4 GiB (32-bit buffer offsets).
 int moe_pick_tile(int n_slots, int E, int H, int inter, int group) {
   if (variant_on(VAR_MOE_TILE16)) return 16;
@@ -1095,13 +1097,18 @@ int moe_pick_tile(int n_slots, int E, int H, int inter, int group) {
   double best = flops / (540e12 * avg / (avg + 26.0));
   int tile = 16;
   for (int bm : {64, 128, 256}) {
-    // expected blocks after padding each expert's run: E * sum_j P(count > j * bm), the count
-    // of an expert taken as Poisson(avg) (normal tail for j >= 1)
-    double per_expert = 1.0 - std::exp(-avg);
-    for (int j = 1; j * (double)bm < avg + 6.0 * std::sqrt(avg) + 1.0; ++j)
-      per_expert += 0.5 * std::erfc((j * (double)bm + 0.5 - avg) / std::sqrt(2.0 * avg));
-    const double blocks = E * per_expert;
-    const double kt_s = 5.4e-9 * (bm + 112);
+    // expected blocks of `rows` after padding each expert's run: E * sum_j P(count > j * rows), the
+    // count of an expert taken as Poisson(avg) (normal tail for j >= 1)
+    auto expected = [&](int rows) {
+      double per_expert = 1.0 - std::exp(-avg);
+      for (int j = 1; j * (double)rows < avg + 6.0 * std::sqrt(avg) + 1.0; ++j)
+        per_expert += 0.5 * std::erfc((j * (double)rows + 0.5 - avg) / std::sqrt(2.0 * avg));
+      return E * per_expert;
+    };
+    // a block runs a tile of as many rows as it holds real slots, in steps of 64: its cost counts
+    // those rows and 112 for the block
+    const double blocks = (64.0 * expected(64) + 112.0 * expected(bm)) / (bm + 112);
+    const double kt_s = (bm == 64 ? 5.4e-9 : bm == 128 ? 5.65e-9 : 5.9e-9) * (bm + 112);
     const int over = bm == 256 ? 6 : 4;
     auto gemm = [&](int K, int N) {
       const double r = blocks * ((N + PF_BN - 1) / PF_BN) / 256.0;
