@@ -14,7 +14,7 @@
  *   2        MoE launches with the dense kernel's register ring of four steps
  *   4|8|16   v = bits 2..4: runs of 1 << (v - 1) sorted-token blocks per XCD
  *   64       never two column blocks per workgroup
- *   512      64- / 128-row MFMA tiles with four waves instead of eight
+ *   512      without effect
  *   1024     the one-call MoE block always runs the separate activation kernel
  *   2048     the one-call MoE block always uses 16-row blocks
  *   4096     every launch keeps the weight ring in registers (no LDS ring)
@@ -22,7 +22,8 @@
  *   1 << 16  v = bits 16..17: the one-call MoE block uses 64 / 128 / 256-row blocks (v = 1 / 2 / 3)
  *   1 << 18  awq_gemm with 17..64 rows: skinny passes wherever they can run
  *   1 << 19  awq_gemm with 17..64 rows: the MFMA kernel wherever it can run
- *   1 << 20  v = bits 20..22: MFMA tiles of 64 v rows (v = 1..4) whatever M is
+ *   1 << 20  v = bits 20..22: fused tiles of 64 v rows (v = 1..4) or 16 v rows (v = 5..7) whatever M is
+ *   1 << 29  v = bits 29..30: fused tiles of 160 / 208 / 224 rows (v = 1 / 2 / 3) whatever M is
  *   1 << 23  dense skinny launches never share left-over chunks step by step
  *   1 << 24  the one-call MoE block always routes in a launch of its own (blocks of at most four
  *            tokens otherwise fold the routing into the first expert GEMM)
@@ -57,7 +58,7 @@ int awqmi_dev_gemm_f16(const void* x_f16, const int32_t* qweight, const void* sc
 enum {
   AWQMI_FORM_NONE = 0,
   AWQMI_FORM_SKINNY = 1,  /* awq_gemv_kernel: up to 32 rows per pass */
-  AWQMI_FORM_FUSED = 2,   /* awq_gemm_mfma_kernel: weights dequantised per tile in LDS */
+  AWQMI_FORM_FUSED = 2,   /* awq_gemm_tile_kernel: weights unpacked per tile in registers */
   AWQMI_FORM_DENSE = 3,   /* awq_dequant_panel_kernel + awq_gemm_dense_kernel */
   AWQMI_FORM_GENERIC = 4, /* any-shape fallback */
   AWQMI_FORM_MID = 5      /* awq_gemm_mid_kernel: 33 .. 64 rows in one pass */

@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <cstdint>
 #include <type_traits>
 
 #include "../../include/awq_mi355x.h"
@@ -16,6 +17,7 @@
 #include "awq_gemm_dense.hpp"
 #include "awq_gemm_mfma.hpp"
 #include "awq_gemm_mid.hpp"
+#include "awq_gemm_tile.hpp"
 #include "awq_gemv.hpp"
 #include "awq_moe.hpp"
 #include "awq_probes.hpp"
@@ -54,7 +56,6 @@ enum : int {
   VAR_MOE_RING4 = 2,          // MoE launches with the dense kernel's register ring of four steps
   VAR_XCD_RUN_SHIFT = 2,      // bits 2..4 = v: force runs of 1 << (v - 1) blocks per XCD
   VAR_NO_PAIR_COLS = 64,      // never two column blocks per workgroup
-  VAR_MFMA_FOUR_WAVES = 512,  // 64- / 128-row MFMA tiles with four waves instead of eight
   VAR_NO_FUSED_ACT = 1024,    // the one-call MoE block always runs the separate activation kernel
   VAR_MOE_TILE16 = 2048,      // the one-call MoE block always uses 16-row blocks
   VAR_NO_LDS_RING = 4096,     // every launch keeps the weight ring in registers
@@ -62,16 +63,25 @@ enum : int {
   VAR_MOE_TILE_SHIFT = 16,    // bits 16..17 = v: the one-call MoE block uses 64 / 128 / 256-row blocks (v = 1 / 2 / 3)
   VAR_MID_M_SKINNY = 1 << 18, // awq_gemm with 17..64 rows: skinny passes wherever they can run
   VAR_MID_M_MFMA = 1 << 19,   // awq_gemm with 17..64 rows: the MFMA kernel wherever it can run
-  VAR_MFMA_ROWS_SHIFT = 20,   // bits 20..22 = v: MFMA tiles of 64 v rows (v = 1..4) whatever M is
+  VAR_MFMA_ROWS_SHIFT = 20,   // bits 20..22 = v: fused tiles of 64 v rows (v = 1..4) or 16 v rows (v = 5..7) whatever M is
   VAR_NO_TAIL_STEP = 1 << 23, // dense skinny launches never share left-over chunks step by step
   VAR_NO_FOLDED_ROUTE = 1 << 24, // the one-call MoE block always routes in a launch of its own
   VAR_NO_DENSE = 1 << 25,        // awq_gemm never takes the dequantise-once form
   VAR_DENSE = 1 << 26,           // awq_gemm takes the dequantise-once form from 257 rows on (workspace permitting)
   VAR_MOE_T32_WIDE = 1 << 27,    // 32-row MoE blocks in the two-words-per-lane form (one workgroup per CU)
+  VAR_TILE_ROWS_SHIFT = 29,      // bits 29..30 = v: fused tiles of 160 / 208 / 224 rows (v = 1 / 2 / 3) whatever M is
   VAR_MID = 1 << 28,             // awq_gemm with 33 .. 64 rows: the one-pass mid kernel on layers of any size
 };
 inline bool variant_on(int bit) {
   return t_variant >= 0 && (t_variant & bit);
+}
+
+// height of the fused kernel's tile that the variant forces, in 16-row steps (0: none)
+inline int forced_tile() {
+  if (t_variant < 0) return 0;
+  constexpr int hi[4] = {0, 10, 13, 14};
+  const int v = (t_variant >> VAR_MFMA_ROWS_SHIFT) & 7, h = (t_variant >> VAR_TILE_ROWS_SHIFT) & 3;
+  return h ? hi[h] : v <= 4 ? 4 * v : v;
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -318,28 +328,77 @@ inline size_t dense_panel_offset(size_t part_bytes) {
   return (AWQMI_WS_COUNTER_BYTES + part_bytes + 1023) / 1024 * 1024;
 }
 
-// Rows of the MFMA tile (64, 128, 192 or 256) for one launch.  Smaller tiles pad less and give
-// more workgroups; larger ones unpack each weight for more rows.  Cost of a choice, in units of
-// one k-tile of one row: rounds of 256 workgroups (a partial last round without a K split counts
-// as at least 0.8) x (k-tiles + 12) x (rows + 64), plus the K-split round if there is one.
-// Fitted on 96 points (six layer shapes, M = 65 ... 2048, every tile size forced in turn, two
-// runs): the choice is within 4 % of the best size on every point (0.04 % behind on average),
-// where "256 rows from 193 rows on" was 9 % behind on average.
-int mfma_pick_rows(int M, int K, int N) {
-  if (M <= 64) return 64;
-  const int KT = K / PF_BK;
-  double best = 1e300;
-  int rows = 256;
-  for (int bm = 64; bm <= 256; bm += 64) {
-    const MfmaPlan pl = plan_mfma(M, K, N, bm);
-    const double tk = bm + 64.0;
-    const int whole = pl.dp_tiles / 256;
-    const double part = (pl.dp_tiles % 256) / 256.0;
-    double t = (whole + (part > 0 ? std::max(part, 0.8) : 0.0)) * (KT + 12) * tk;
-    if (pl.sk_tiles > 0) t += ((double)KT / pl.sk_split + 12) * tk;
-    if (t < best) { best = t; rows = bm; }
+// Fused kernel: height of its tile in 16-row steps and the K split of one launch.  Whole rounds of 256
+// tiles run one workgroup per tile; a last round that leaves CUs idle (and any launch that small) may be split
+// in K over `split` workgroups per tile, at least four stages of 64 k each.
+constexpr int TILE_RT[] = {4, 5, 6, 7, 8, 10, 12, 13, 14, 16};
+struct TilePlan { int rt, dp_tiles, sk_tiles, sk_split; size_t part_bytes; };
+TilePlan tile_plan(int M, int K, int N, int rt, int split) {
+  const int tiles = ((M + 16 * rt - 1) / (16 * rt)) * ((N + TG_COLS - 1) / TG_COLS), rem = tiles % 256;
+  if (rem == 0 || split < 2) return TilePlan{rt, tiles, 0, 1, 0};
+  return TilePlan{rt, tiles - rem, rem, split, (size_t)rem * split * tg_part_floats(rt) * sizeof(float)};
+}
+// The cheapest plan whose partial tiles fit into `room` bytes, by price (us): a stage of 64 k costs 0.28 + 0.0746 rt
+// on a full chip and down to 0.79 of it on a nearly idle one (the clock), a tile 3.8 stages beside its own, a partial
+// last round counts as at least 0.88 of one, a K split 4.3 + 0.22 per part for its sum launch and 0.003 rt per
+// partial tile.  Fitted on 7800 timed launches (16 layer shapes from 1024 x 12288 to 8192 x 59136, 33 ... 2047 rows,
+// every height and up to five splits each): 0.6 % behind the best of them on average, 15 % at worst.
+TilePlan pick_tile(int M, int K, int N, size_t room) {
+  const int KT = K / 64;
+  TilePlan best{};
+  double best_t = 1e300;
+  for (const int rt : TILE_RT) {
+    const TilePlan one = tile_plan(M, K, N, rt, 1);
+    const int tiles = one.dp_tiles, rem = tiles % 256;
+    const double stage = 0.28 + 0.0746 * rt;
+    auto price = [&](const TilePlan& pl) {
+      double t = 0.0;
+      if (pl.dp_tiles > 0) {
+        const double part = (pl.dp_tiles % 256) / 256.0;
+        const double rounds = pl.dp_tiles < 256 ? 0.79 + 0.21 * part : pl.dp_tiles / 256 + (part > 0 ? std::max(part, 0.88) : 0.0);
+        t += rounds * (KT + 3.8) * stage;
+      }
+      if (pl.sk_tiles > 0) {
+        const int wgs = pl.sk_tiles * pl.sk_split;
+        t += ((KT + pl.sk_split - 1) / pl.sk_split + 3.8) * stage * (0.79 + 0.21 * wgs / 256.0) + 4.3 +
+             0.22 * pl.sk_split + 0.003 * wgs * rt;
+      }
+      return t;
+    };
+    auto take = [&](const TilePlan& pl) {
+      const double t = price(pl);
+      if (t < best_t) { best_t = t; best = pl; }
+    };
+    take(one);
+    for (int c = 2; rem > 0 && c <= 16 && c * rem <= 256 && KT / c >= 4; ++c) {
+      const TilePlan pl = tile_plan(M, K, N, rt, c);
+      if (pl.part_bytes <= room) take(pl);
+    }
+    if (16 * rt >= M) break;        // one tile holds every row: a higher one multiplies more padding
   }
-  return rows;
+  return best;
+}
+// Launch of a tile height with the larger of two kernels where the layer needs it (see awq_tile).
+template <int RT>
+void launch_tile(const MfmaGemmParams& p, hipStream_t st) {
+  const dim3 grid(p.per_xcd * 8 + p.sk_tiles * p.sk_split);
+  if (p.G % 64 == 0 && p.N % 32 == 0) hipLaunchKernelGGL((awq_gemm_tile_kernel<RT, false>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((awq_gemm_tile_kernel<RT, true>), grid, dim3(256), 0, st, p);
+  if (p.sk_tiles > 0) hipLaunchKernelGGL((awq_gemm_tile_reduce_kernel<RT>), dim3(p.sk_tiles * RT), dim3(256), 0, st, p);
+}
+void launch_tile(int rt, const MfmaGemmParams& p, hipStream_t st) {
+  switch (rt) {
+    case 4: return launch_tile<4>(p, st);
+    case 5: return launch_tile<5>(p, st);
+    case 6: return launch_tile<6>(p, st);
+    case 7: return launch_tile<7>(p, st);
+    case 8: return launch_tile<8>(p, st);
+    case 10: return launch_tile<10>(p, st);
+    case 12: return launch_tile<12>(p, st);
+    case 13: return launch_tile<13>(p, st);
+    case 14: return launch_tile<14>(p, st);
+    default: return launch_tile<16>(p, st);
+  }
 }
 
 }  // namespace
@@ -355,12 +414,6 @@ static int ensure_kernel_attributes() {
   if (dev < 0 || dev >= MAX_DEVICES) return AWQMI_BAD_ARGUMENT;
   if (done[dev].load(std::memory_order_acquire)) return AWQMI_OK;
   const void* mfma[] = {
-      reinterpret_cast<const void*>(awq_gemm_mfma_kernel<true, 1, 8>), reinterpret_cast<const void*>(awq_gemm_mfma_kernel<false, 1, 8>),
-      reinterpret_cast<const void*>(awq_gemm_mfma_kernel<true, 2, 8>), reinterpret_cast<const void*>(awq_gemm_mfma_kernel<false, 2, 8>),
-      reinterpret_cast<const void*>(awq_gemm_mfma_kernel<true, 1>), reinterpret_cast<const void*>(awq_gemm_mfma_kernel<false, 1>),
-      reinterpret_cast<const void*>(awq_gemm_mfma_kernel<true, 2>), reinterpret_cast<const void*>(awq_gemm_mfma_kernel<false, 2>),
-      reinterpret_cast<const void*>(awq_gemm_mfma_kernel<true, 3>), reinterpret_cast<const void*>(awq_gemm_mfma_kernel<false, 3>),
-      reinterpret_cast<const void*>(awq_gemm_mfma_kernel<true, 4>), reinterpret_cast<const void*>(awq_gemm_mfma_kernel<false, 4>),
       reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<true, 1, 8>), reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<false, 1, 8>),
       reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<true, 2, 8>), reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<false, 2, 8>),
       reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<true, 4, 4>), reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<false, 4, 4>)};
@@ -539,9 +592,11 @@ size_t awqmi_gemm_workspace_bytes(int M, int K, int N, int split_k) {
   if (M > 16 && K % PF_BK == 0) {
     const int slab = mfma_slab_rows(M, K);
     if (slab > 0) {
-      // the tile rows the call will pick (a forced size that needs more falls back to no K split)
-      mfma = plan_mfma(slab, K, N, mfma_pick_rows(slab, K, N)).part_bytes;
-      if (M % slab) mfma = std::max(mfma, plan_mfma(M % slab, K, N, mfma_pick_rows(M % slab, K, N)).part_bytes);
+      // the plan the call will pick, and room for the K split of 256-row tiles at least (any forced size
+      // that needs more runs unsplit)
+      for (const int m : {slab, M % slab})
+        if (m > 0)
+          mfma = std::max({mfma, pick_tile(m, K, N, SIZE_MAX).part_bytes, plan_mfma(m, K, N, 256).part_bytes});
       // the dequantise-once form of many-row calls: 256-row tiles, and the fp16 panel behind the
       // partial tiles (a call with a smaller workspace runs the fused kernel instead)
       if (dense_default(M, N)) {
@@ -660,11 +715,9 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
     return launch_status();
   }
 
-  // MFMA kernel: K % 64 == 0, G a power of two >= 8 or a multiple of 64; buffer offsets are
+  // MFMA kernels: K % 64 == 0, G a power of two >= 8 or a multiple of 64; buffer offsets are
   // 32-bit, so every operand must stay below 4 GiB
-  const bool pow2g = (G & (G - 1)) == 0 && G >= 8;
   if (mfma_ok) {
-    if (const int rc = ensure_kernel_attributes()) return rc;
     const int slab = mfma_slab_rows(M, K);
     // many rows: dequantise once into the workspace, then the dense kernel (same bits as the fused
     // kernel with 256-row tiles); needs the workspace to hold the panel
@@ -696,49 +749,29 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
       }
     }
     t_last_gemm_form = AWQMI_FORM_FUSED;
+    // room for the partial tiles of a K split; without a workspace every tile runs on one workgroup
+    const size_t room = workspace && aligned16(workspace) && workspace_bytes > AWQMI_WS_COUNTER_BYTES
+                            ? workspace_bytes - AWQMI_WS_COUNTER_BYTES : 0;
+    const int forced = forced_tile();
     for (int r0 = 0; r0 < M; r0 += slab) {
       const int Ms = M - r0 < slab ? M - r0 : slab;
+      TilePlan pl;
+      if (forced) {
+        // a forced height takes the dense kernel's split rule
+        pl = tile_plan(Ms, K, N, forced, plan_mfma(Ms, K, N, 16 * forced).sk_split);
+        if (pl.part_bytes > room) pl = tile_plan(Ms, K, N, forced, 1);
+      } else {
+        pl = pick_tile(Ms, K, N, room);
+      }
       MfmaGemmParams p{};
       p.x = xx + (size_t)r0 * K; p.qw = qw; p.sc = sc; p.qz = qz; p.y = yy + (size_t)r0 * N;
       p.M = Ms; p.K = K; p.N = N; p.NW = NW; p.ldw = ldw; p.G = G;
-      p.gshift = 0;
-      if (pow2g) while ((1 << p.gshift) < G) ++p.gshift;
-      int mi = mfma_pick_rows(Ms, K, N) / 64;
-      const int vrows = t_variant;
-      if (vrows >= 0 && ((vrows >> VAR_MFMA_ROWS_SHIFT) & 7) >= 1 && ((vrows >> VAR_MFMA_ROWS_SHIFT) & 7) <= 4)
-        mi = (vrows >> VAR_MFMA_ROWS_SHIFT) & 7;
-      const int bm = 64 * mi;
-      p.mt = (Ms + bm - 1) / bm; p.nt = (N + PF_BN - 1) / PF_BN;
-      p.total = p.mt * p.nt;
-      MfmaPlan pl = plan_mfma(Ms, K, N, bm);
-      // the K split needs the caller's workspace (counters + partial tiles); without it every
-      // tile runs on one workgroup
-      if (pl.sk_tiles > 0 && (!workspace || !aligned16(workspace) ||
-                              workspace_bytes < AWQMI_WS_COUNTER_BYTES + pl.part_bytes))
-        pl = MfmaPlan{p.total, 0, 1, 0};
+      while ((2 << p.gshift) <= G) ++p.gshift;
+      p.mt = (Ms + 16 * pl.rt - 1) / (16 * pl.rt); p.nt = (N + TG_COLS - 1) / TG_COLS;
       p.dp_tiles = pl.dp_tiles; p.sk_tiles = pl.sk_tiles; p.sk_split = pl.sk_split;
       p.per_xcd = (pl.dp_tiles + 7) / 8;
-      p.sk_part = workspace ? reinterpret_cast<float*>(static_cast<char*>(workspace) + AWQMI_WS_COUNTER_BYTES)
-                            : nullptr;
-      const dim3 grid(p.per_xcd * 8 + p.sk_tiles * p.sk_split);
-#define AWQMI_MFMA(MIV, NWVV)                                                                      \
-  do {                                                                                           \
-    if (pow2g)                                                                                   \
-      hipLaunchKernelGGL((awq_gemm_mfma_kernel<true, MIV, NWVV>), grid, dim3(64 * NWVV), PF_LDS_BYTES, st, p);  \
-    else                                                                                         \
-      hipLaunchKernelGGL((awq_gemm_mfma_kernel<false, MIV, NWVV>), grid, dim3(64 * NWVV), PF_LDS_BYTES, st, p); \
-    if (p.sk_tiles > 0)                                                                          \
-      hipLaunchKernelGGL((awq_gemm_mfma_reduce_kernel<MIV, NWVV>), dim3(p.sk_tiles * MIV * (16 / NWVV)),       \
-                         dim3(64 * NWVV), 0, st, p);                                              \
-  } while (0)
-      const bool eight = !variant_on(VAR_MFMA_FOUR_WAVES);
-      if (mi == 1 && eight) AWQMI_MFMA(1, 8);
-      else if (mi == 2 && eight) AWQMI_MFMA(2, 8);
-      else if (mi == 1) AWQMI_MFMA(1, 4);
-      else if (mi == 2) AWQMI_MFMA(2, 4);
-      else if (mi == 3) AWQMI_MFMA(3, 4);
-      else AWQMI_MFMA(4, 4);
-#undef AWQMI_MFMA
+      p.sk_part = room ? reinterpret_cast<float*>(static_cast<char*>(workspace) + AWQMI_WS_COUNTER_BYTES) : nullptr;
+      launch_tile(pl.rt, p, st);
     }
     return launch_status();
   }

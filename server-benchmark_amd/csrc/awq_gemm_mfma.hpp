@@ -462,11 +462,6 @@ __device__ __forceinline__ void awq_mfma_tile(const MfmaGemmParams& p, const int
   }
 }
 
-template <bool POW2G, int MI = 4, int NWV = 4>
-__global__ __launch_bounds__(64 * NWV, NWV / 4) void awq_gemm_mfma_kernel(const MfmaGemmParams p) {
-  awq_mfma_tile<POW2G, MI, NWV, false>(p, 0, 0, 0, nullptr, nullptr);
-}
-
 // Expert-grouped launch, blocks of 64 MI sorted slots.
 //
 // A workgroup takes the tile of as many rows as its block has real slots, in steps of 64: a tile costs
@@ -518,71 +513,6 @@ __global__ __launch_bounds__(64 * NWV, NWV / 4) void awq_gemm_mfma_grouped_kerne
   else if (MI >= 3 && rows > 128) awq_mfma_tile<POW2G, MI < 3 ? MI : 3, NWV, true>(p, m0, n0, e, s_sid, s_tw);
   else if (MI >= 2 && rows > 64) awq_mfma_tile<POW2G, MI < 2 ? MI : 2, NWV, true>(p, m0, n0, e, s_sid, s_tw);
   else if (rows > 0) awq_mfma_tile<POW2G, 1, NWV, true>(p, m0, n0, e, s_sid, s_tw);
-}
-
-// Sum of the split-K partial tiles.  Partial layout per (tile, part): [q][thread] groups of
-// four floats, q = (i * NJ + j) * 4 + r / 4 over the MI x NJ accumulator tiles of the producing
-// thread (same thread count and wave arrangement as the producer).  One workgroup takes four
-// q of one tile; parts are added in index order.
-template <int MI, int NWV = 4>
-__global__ __launch_bounds__(64 * NWV) void awq_gemm_mfma_reduce_kernel(const MfmaGemmParams p) {
-  constexpr int QPW = 4;
-  constexpr int NJ = 16 / NWV, NTH = 64 * NWV;
-  constexpr int QT = 4 * MI * NJ;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int tl = blockIdx.x / (QT / QPW);
-  const int q0 = (blockIdx.x % (QT / QPW)) * QPW;
-  const int nid = p.dp_tiles + tl;
-  const int gsize = PF_GROUP_M * p.nt;
-  const int first_m = (nid / gsize) * PF_GROUP_M;
-  const int gm = min(p.mt - first_m, PF_GROUP_M);
-  const int mt_i = first_m + (nid % gsize) % gm;
-  const int nt_i = (nid % gsize) / gm;
-  const int m0 = mt_i * (64 * MI), n0 = nt_i * PF_BN;
-  const int wm = (wave / (NWV / 2)) * (32 * MI), wn = (wave % (NWV / 2)) * (32 * NJ);
-  const int row_l = lane & 31;
-  const float* tile_base = p.sk_part + (size_t)tl * p.sk_split * PF_SK_SLOT_FLOATS;
-  f4 v[QPW];
-#pragma unroll
-  for (int u = 0; u < QPW; ++u) v[u] = f4{0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < p.sk_split; ++s) {
-    f4 t[QPW];
-#pragma unroll
-    for (int u = 0; u < QPW; ++u)
-      t[u] = *reinterpret_cast<const f4*>(tile_base + (size_t)s * PF_SK_SLOT_FLOATS +
-                                          ((size_t)(q0 + u) * NTH + tid) * 4);
-#pragma unroll
-    for (int u = 0; u < QPW; ++u) v[u] += t[u];
-  }
-  // The four groups of a thread are columns 8 rg + 4 (lane / 32) + 0..3, rg = 0..3, of one row of one
-  // 32 x 32 accumulator tile (see the producer's output comment; q0 is a multiple of four): lane l
-  // and lane l ^ 32 hold the two interleaved halves of 32 consecutive columns.  They trade two groups
-  // each, so that the lower lane stores columns 0..15 and the upper one columns 16..31 as 32 bytes.
-  static_assert(QPW == 4, "one accumulator tile row per thread");
-  const int ij = q0 >> 2;
-  const bool upper = lane >= 32;
-  u2v hv[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const h4 o = {(half_t)v[u][0], (half_t)v[u][1], (half_t)v[u][2], (half_t)v[u][3]};
-    hv[u] = __builtin_bit_cast(u2v, o);
-  }
-  u2v got[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const u2v give = upper ? hv[k] : hv[2 + k];
-    got[k][0] = (uint32_t)__shfl_xor((int)give[0], 32, 64);
-    got[k][1] = (uint32_t)__shfl_xor((int)give[1], 32, 64);
-  }
-  // lower lane: own 0, partner's 0, own 1, partner's 1; upper lane: partner's 2, own 2, partner's 3, own 3
-  const u4v lo = upper ? u4v{got[0][0], got[0][1], hv[2][0], hv[2][1]} : u4v{hv[0][0], hv[0][1], got[0][0], got[0][1]};
-  const u4v hi = upper ? u4v{got[1][0], got[1][1], hv[3][0], hv[3][1]} : u4v{hv[1][0], hv[1][1], got[1][0], got[1][1]};
-  const int col = n0 + wn + 32 * (ij % NJ) + (upper ? 16 : 0);
-  const int row = m0 + wm + 32 * (ij / NJ) + row_l;
-  if (row < p.M) {        // N % 8 == 0: eight columns are all inside or all outside
-    if (col < p.N) *reinterpret_cast<u4v*>(p.y + (size_t)row * p.N + col) = lo;
-    if (col + 8 < p.N) *reinterpret_cast<u4v*>(p.y + (size_t)row * p.N + col + 8) = hi;
-  }
 }
 
 }  // namespace awqmi

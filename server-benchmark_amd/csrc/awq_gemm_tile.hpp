@@ -1,0 +1,468 @@
+// Fused AWQ GEMM of more rows than the skinny kernel takes: Y[M,N] = X[M,K] @ dequant(W) on fp16
+// MFMA with fp32 accumulation, every weight unpacked in the registers of the wave that multiplies it.
+//
+// Workgroup tile 16 RT x 256, four waves side by side: each has all rows and 64 columns, 4 x RT
+// v_mfma_f32_16x16x32_f16 accumulators (the shape that gives the most flops under the power limit, see
+// awq_gemm_dense.hpp).  A weight is therefore unpacked once per tile, by the wave that needs it, and goes
+// through LDS packed: X and packed W both travel from global memory straight into an LDS ring of D stages of 64 k.
+//
+// Unpacking.  Lane (n, q) of a 16 x 16 x 32 A operand holds k = 8 q .. 8 q + 7 of one column.  The 16 n of a tile are the two
+// halves of eight packed words: lane n takes half n & 1 of word n >> 1, and the four nibbles of its half are its
+// columns of the wave's four tiles.  Eight words (eight k) are 32 weights: per pair of words one v_perm that puts the two
+// halves side by side, one shift, then and-or, subtract and multiply per nibble: 14 instructions for 8 weights, exact fp16
+// (w - z) * s as awq_dequantize rounds it.  An output lane ends up with 16 consecutive columns of a row, which it
+// stores as 32 bytes without a trip through LDS.
+//
+// LDS: X [row][128 B], 16-byte slot l of row r at l ^ ((r >> 1) & 7); W [k][128 B], the 32 bytes of wave w at chunk
+// w ^ ((k >> 3) & 3), so that the four k groups of a read touch different banks (no conflicts measured).
+//
+// The k-step loop is written out: every MFMA is followed by its share of the next k-step's unpacking, the fragment read eight
+// tiles ahead and the loads of the stage D - 1 ahead.  The waits are explicit.
+//
+// What bounds it: high tiles the power limit (8192 x 59136 at 2048 rows: matrix pipe busy 77 % of the cycles at 1.83 GHz), low
+// ones the issue port, where a 16-cycle MFMA leaves room for two vector instructions: a stage takes a wave 32 MFMAs per 64
+// rows and 133 vector instructions whatever the rows (at 64 rows 38 % MFMA, 21 % waiting for LDS or the barrier; with the unpacking
+// taken out 59 of 90 us).  Against the kernel before it (weights dequantised into LDS by all waves, 32 x 32 x 16 MFMAs,
+// tiles of 64 rows' steps), us: 8192 x 59136 at 80 / 128 / 400 / 1000 / 2047 rows 145 / 149 / 430 / 889 / 1701 -> 95 / 125 / 325 /
+// 757 / 1500; 29568 x 8192 at 96 / 400 / 1000 81 / 226 / 433 -> 58 / 171 / 383; 3584 x 4608 at 64 / 1000 18.1 / 51 -> 15.7 / 42.
+// Measured and dropped: eight waves on two K halves of a tile, two per SIMD (8192 x 59136 at 64 rows 80 against 84 us, split
+// layers slower); a ring of distinct LDS objects with the compiler's own waits (even, four times the code).
+#pragma once
+#include <type_traits>
+
+#include "awq_common.hpp"
+#include "awq_gemm_dense.hpp"
+
+namespace awqmi {
+
+constexpr int TG_COLS = 256;             // columns of a workgroup tile
+constexpr int TG_W_BYTES = 64 * 128;     // packed weights of a stage: 64 k x 256 columns
+
+// LDS of one stage: X rows, packed weights, then each wave's group parameters
+__host__ __device__ constexpr int tg_x_bytes(int rt) { return rt * 16 * 128; }
+__host__ __device__ constexpr int tg_param_bytes(bool any) { return any ? 1280 : 256; }
+__host__ __device__ constexpr int tg_slot_bytes(int rt, bool any) { return tg_x_bytes(rt) + TG_W_BYTES + 4 * tg_param_bytes(any); }
+// workgroups of a CU, and stages of the LDS ring
+__host__ __device__ constexpr int tg_occupancy(int rt) { return rt <= 5 ? 2 : 1; }
+__host__ __device__ constexpr int tg_depth(int rt, bool any) {
+  const int fit = 160 * 1024 / tg_occupancy(rt) / tg_slot_bytes(rt, any);
+  return fit < 7 ? fit : 7;
+}
+// floats of a K split's partial tile
+__host__ __device__ constexpr size_t tg_part_floats(int rt) { return (size_t)rt * 16 * 256; }
+// X fragments in flight: a divisor of the 2 RT fragments of a stage
+__host__ __device__ constexpr int tg_ring(int rt) {
+  return 2 * rt % 8 == 0 ? 8 : 2 * rt % 7 == 0 ? 7 : 2 * rt % 6 == 0 ? 6 : 2 * rt % 5 == 0 ? 5 : rt;
+}
+
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(3))) unsigned char lds_byte;
+template <class T>
+__device__ __forceinline__ T lds_read(uint32_t a) {
+  return *reinterpret_cast<const __attribute__((address_space(3))) T*>(a);
+}
+
+// The direct-to-LDS loads are asm statements: the compiler would put a wait for every one of them
+// that may write what an LDS read reads, and with the stage's slot computed at run time it cannot tell
+// them apart.  The waits are the kernel's own (tg_wait_and_barrier).
+// acc += a * b, then 16 bytes a lane from rsrc into LDS at lds + 16 * lane; the MFMA is the wait state between
+// the write of m0 and the load that reads it.
+__device__ __forceinline__ void tg_mfma(f4& c, u4v a, h8 b) {
+  asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void tg_mfma_load(f4& c, u4v a, h8 b, uint32_t lds, u4v rsrc, uint32_t voff, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\tbuffer_load_dwordx4 %4, %5, %6 offen lds"
+               : "+a"(c) : "v"(a), "v"(b), "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+}
+// ... of the lanes in `mask` only (every lane is active around it)
+__device__ __forceinline__ void tg_mfma_load_some(f4& c, u4v a, h8 b, uint32_t lds, u4v rsrc, uint32_t voff, uint64_t mask) {
+  asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\ts_mov_b64 exec, %6\n\t"
+               "buffer_load_dwordx4 %4, %5, 0 offen lds\n\ts_mov_b64 exec, -1"
+               : "+a"(c) : "v"(a), "v"(b), "s"(lds), "v"(voff), "s"(rsrc), "s"(mask) : "memory");
+}
+__device__ __forceinline__ void tg_load(uint32_t lds, u4v rsrc, uint32_t voff, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+}
+__device__ __forceinline__ void tg_load_some(uint32_t lds, u4v rsrc, uint32_t voff, uint64_t mask) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n\ts_mov_b64 exec, -1"
+               :: "s"(lds), "v"(voff), "s"(rsrc), "s"(mask) : "memory");
+}
+// ... from one address per lane
+__device__ __forceinline__ void tg_mfma_load_at(f4& c, u4v a, h8 b, uint32_t lds, uint64_t addr, uint64_t mask) {
+  asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\ts_mov_b64 exec, %5\n\t"
+               "global_load_lds_dwordx4 %4, off\n\ts_mov_b64 exec, -1"
+               : "+a"(c) : "v"(a), "v"(b), "s"(lds), "v"(addr), "s"(mask) : "memory");
+}
+__device__ __forceinline__ void tg_load_at(uint32_t lds, uint64_t addr, uint64_t mask) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b64 exec, -1"
+               :: "s"(lds), "v"(addr), "s"(mask) : "memory");
+}
+__device__ __forceinline__ u4v tg_rsrc(const void* base, size_t bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  return u4v{(uint32_t)a, (uint32_t)(a >> 32) & 0xFFFFu, bytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)bytes, 0x00020000u};
+}
+// At most VM of this wave's loads outstanding, then the workgroup barrier: one statement, no LDS access
+// moves across it.
+template <int VM>
+__device__ __forceinline__ void tg_wait_and_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(VM) : "memory");
+}
+
+// RT: 16-row tiles of the workgroup tile.  ANY = false: G a multiple of 64 (a stage lies in one group) and N of 32;
+// ANY = true: also G a power of two from 8 on, and any N.
+template <int RT, bool ANY, bool GROUPED>
+__device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, const int n0, const int kb, const int ke,
+                                         float* const part, const int e, const uint32_t smem) {
+  constexpr int D = tg_depth(RT, ANY);
+  constexpr int XB = tg_x_bytes(RT), SLOT = tg_slot_bytes(RT, ANY), PW = tg_param_bytes(ANY);
+  constexpr int ZO = ANY ? 1024 : 128;        // zero points behind the scales
+  constexpr int XL = (RT + 1) / 2;            // X loads of a wave and stage
+  constexpr int NL = XL + (ANY ? 4 : 3);      // all loads: weights (2), group parameters, X
+  constexpr int XF = tg_ring(RT);
+  constexpr int NP = 4 * RT;                  // MFMAs of a k-step
+  static_assert(D >= 3 && (D - 2) * NL < 64, "");
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fi = lane & 15, fq = lane >> 4;
+  const size_t es = GROUPED ? (size_t)e : 0;
+  const u4v rx = tg_rsrc(p.x, (size_t)p.M * p.K * 2);
+  const u4v rw = tg_rsrc(p.qw + es * p.w_stride, (size_t)p.K * p.ldw * 4);
+  const u4v rz = tg_rsrc(p.qz + es * p.z_stride, (size_t)(p.K / p.G) * p.NW * 4);
+  const u4v rs = tg_rsrc(p.sc + es * p.s_stride, (size_t)(p.K / p.G) * p.N * 2);
+
+  // ---- global -> LDS roles
+  uint32_t x_voff[XL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    int idx = 4 * i + wave;
+    if ((RT & 1) && idx >= 2 * RT) idx -= 2;
+    const int r = 8 * idx + (lane >> 3);
+    int gr;
+    if (GROUPED) {
+      const int sid = p.sorted_ids[m0 + r];
+      gr = sid < p.n_slots ? sid / p.a_row_div : 0;
+    } else {
+      gr = min(m0 + r, p.M - 1);
+    }
+    x_voff[i] = (uint32_t)(((size_t)gr * p.K + 8 * ((lane & 7) ^ dg_swz(r))) * 2);
+  }
+  auto x_lds = [&](int i) __attribute__((always_inline)) -> uint32_t {
+    int idx = 4 * i + wave;
+    if ((RT & 1) && idx >= 2 * RT) idx -= 2;
+    return (uint32_t)idx * 1024u;
+  };
+  const uint32_t row_w = (uint32_t)p.ldw * 4u;
+  const int w0 = n0 / 8;
+  // group parameters: the wave's eight packed columns are 128 bytes of scales and 32 of zero points a group
+  const int gps = ANY ? max(64 / p.G, 1) : 1;         // groups of a stage
+  const int spg = ANY ? max(p.G / 64, 1) : p.G / 64;  // stages of a group
+  int gl = __builtin_amdgcn_readfirstlane(kb / spg), gr = kb - gl * spg;    // first group of the next stage to load, its place in it
+  if (ANY) gl *= gps;
+  uint32_t w_voff, s_voff, z_voff;
+  uint64_t p_addr;
+  uint32_t p_step;
+  {
+    int wc = w0 + 4 * ((lane & 7) ^ (2 * wave));
+    if (wc >= p.NW) wc = 0;
+    w_voff = (uint32_t)((8 * wave + (lane >> 3)) * p.ldw + wc) * 4u;
+    int sw = w0 + 8 * wave + (lane & 7), zw = w0 + 8 * wave + 4 * (lane & 1);
+    if (sw >= p.NW) sw = 0;
+    if (zw >= p.NW) zw = 0;
+    s_voff = (uint32_t)((lane >> 3) * p.N + 8 * sw) * 2u;       // ANY: lane = (group, word) ...
+    z_voff = (uint32_t)((lane >> 1) * p.NW + zw) * 4u;          // ... and (group, four words)
+    const bool zl = lane >= 8;                                  // else: eight lanes of scales, two of zero points
+    p_addr = zl ? reinterpret_cast<uint64_t>(p.qz + es * p.z_stride + (size_t)gl * p.NW + zw)
+                : reinterpret_cast<uint64_t>(p.sc + es * p.s_stride + (size_t)gl * p.N + 8 * sw);
+    p_step = zl ? p.NW * 4u : p.N * 2u;
+  }
+  const uint64_t s_mask = gps == 8 ? ~0ull : (1ull << (8 * gps)) - 1, z_mask = (1ull << (2 * gps)) - 1;
+  const uint32_t w_lds = XB + (uint32_t)wave * 1024u, p_lds = XB + TG_W_BYTES + (uint32_t)wave * PW;
+
+  // ---- LDS -> register roles
+  const int c = fi >> 1;
+  uint32_t fx_off[2], ps_off[2], pz_off[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    fx_off[ks] = (uint32_t)(fi * 128 + (((4 * ks + fq) ^ dg_swz(fi)) << 4));
+    const int row = ANY && p.G < 64 ? (32 * ks + 8 * fq) >> p.gshift : 0;
+    ps_off[ks] = p_lds + (uint32_t)(row * 128 + c * 16);
+    pz_off[ks] = p_lds + (uint32_t)(ZO + row * 32 + c * 4);
+  }
+  const uint32_t fw_off = (uint32_t)(XB + 8 * fq * 128 + (((2 * wave + (c >> 2)) ^ (2 * fq)) << 4) + (c & 3) * 4);
+  const uint32_t sel_w = (fi & 1) ? 0x07060302u : 0x05040100u;
+  const uint32_t sel_s = (fi & 1) ? 0x03020302u : 0x01000100u;
+
+  f4 acc[4][RT];
+  NibbleMasks nm;
+  nm.init();
+
+  uint32_t zraw, zz[4], ss[4];
+  u4v sraw;
+  uint32_t wd[2][8];
+  u4v wf[2][4];
+  h8 xf[XF];
+  auto read_params = [&](uint32_t slot, int ks) __attribute__((always_inline)) {
+    zraw = lds_read<uint32_t>(slot + pz_off[ANY ? ks : 0]);
+    sraw = lds_read<u4v>(slot + ps_off[ANY ? ks : 0]);
+  };
+  auto expand = [&]() __attribute__((always_inline)) {
+    const uint32_t za = __builtin_amdgcn_perm(zraw, zraw, sel_s), zb = za >> 8;
+    zz[0] = (za & nm.lo) | MAGIC_LO;
+    zz[1] = (za & nm.hi) | MAGIC_HI;
+    zz[2] = (zb & nm.lo) | MAGIC_LO;
+    zz[3] = (zb & nm.hi) | MAGIC_HI;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ss[j] = __builtin_amdgcn_perm(sraw[j], sraw[j], sel_s);
+  };
+  auto read_words = [&](int set, uint32_t fw, int ks, int rp) __attribute__((always_inline)) {
+    wd[set][2 * rp] = lds_read<uint32_t>(fw + ks * 4096 + rp * 256);
+    wd[set][2 * rp + 1] = lds_read<uint32_t>(fw + ks * 4096 + rp * 256 + 128);
+  };
+  uint32_t ua = 0, ub = 0, t1[16], t2[16];
+  // step i of 18: pair the halves of item i's rows, subtract item i - 1, scale item i - 2
+  auto unpack = [&](int i, int set, int w) __attribute__((always_inline)) {
+    if (i < 16) {
+      const int rp = i >> 2, j = i & 3;
+      if (j == 0) {
+        ua = __builtin_amdgcn_perm(wd[w][2 * rp + 1], wd[w][2 * rp], sel_w);
+        ub = ua >> 8;
+      }
+      const uint32_t u = j < 2 ? ua : ub;
+      t1[i] = (j & 1) ? (u & nm.hi) | MAGIC_HI : (u & nm.lo) | MAGIC_LO;
+    }
+    if (i >= 1 && i < 17) t2[i - 1] = pk_sub(t1[i - 1], zz[(i - 1) & 3]);
+    if (i >= 2) wf[set][(i - 2) & 3][(i - 2) >> 2] = pk_mul(t2[i - 2], ss[(i - 2) & 3]);
+  };
+  // The operands of the next k-step are complete, and the first MFMA reads them two wait states later.
+  auto pin = [&](int set) __attribute__((always_inline)) {
+    asm volatile("s_nop 1" : "+v"(wf[set][0]), "+v"(wf[set][1]), "+v"(wf[set][2]), "+v"(wf[set][3]));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // ---- loads of one stage: kl the stage, slot its LDS
+  int kl = kb;
+  uint32_t fill = smem;
+  auto next_load = [&]() __attribute__((always_inline)) {
+    fill += SLOT;
+    if (fill == smem + D * SLOT) fill = smem;
+    // stages past the last one load the last one again, which nobody reads
+    if (kl + 1 < ke) {
+      ++kl;
+      if (++gr == spg) {
+        gr = 0;
+        gl += gps;
+        if (!ANY) p_addr += p_step;
+      }
+    }
+  };
+  auto s_addr = [&]() __attribute__((always_inline)) { return s_voff + (uint32_t)(gl * p.N) * 2u; };
+  auto z_addr = [&]() __attribute__((always_inline)) { return z_voff + (uint32_t)(gl * p.NW) * 4u; };
+  auto w_addr = [&](int i) __attribute__((always_inline)) { return w_voff + ((uint32_t)kl * 64u + 32u * i) * row_w; };
+
+  // One k-step, KS its number in the stage, out of operand set KS; meanwhile the other set is unpacked for the
+  // next k-step and the words after that are read.  cur / nxt: LDS of this stage and the next one.
+  auto kstep = [&](auto KS, const uint32_t (&xc)[2], const uint32_t (&xn)[2], uint32_t fwn, uint32_t nxt) __attribute__((always_inline)) {
+    constexpr int ks = decltype(KS)::value;
+#pragma unroll
+    for (int im = 0; im < RT; ++im)
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        // one operand changes from one MFMA to the next
+        const int j = (im & 1) ? 3 - jj : jj, m = 4 * im + jj;
+        f4& a = acc[j][im];
+        const u4v& w = wf[ks][j];
+        const h8& x = xf[(ks * RT + im) % XF];
+        // loads of a stage: dealt out over it (over its first k-step with a ring of three)
+        int ld = -1;
+#pragma unroll
+        for (int i = 0; i < NL; ++i)
+          if ((D == 3 ? 1 + i * (NP - 2) / NL : 1 + i * (2 * NP - 4) / NL) == ks * NP + m) ld = i;
+        if (ld < 0) tg_mfma(a, w, x);
+        else if (ld < 2) tg_mfma_load(a, w, x, fill + w_lds + ld * 4096, rw, w_addr(ld), 0);
+        else if (!ANY && ld == 2) tg_mfma_load_at(a, w, x, fill + p_lds, p_addr, 0x3ffull);
+        else if (ANY && ld == 2) tg_mfma_load_some(a, w, x, fill + p_lds, rs, s_addr(), s_mask);
+        else if (ANY && ld == 3) tg_mfma_load_some(a, w, x, fill + p_lds + ZO, rz, z_addr(), z_mask);
+        else tg_mfma_load(a, w, x, fill + x_lds(ld - (NL - XL)), rx, x_voff[ld < NL - XL ? 0 : ld - (NL - XL)], (uint32_t)kl * 128u);
+        __builtin_amdgcn_sched_barrier(0);
+        if (m == 0 && (ANY || ks == 1)) expand();
+        if (m == 1 && (ANY || ks == 0)) read_params(nxt, ks);
+#pragma unroll
+        for (int i = 18 * m / NP; i < 18 * (m + 1) / NP; ++i) unpack(i, ks ^ 1, ks ^ 1);
+        if (m < 4) read_words(ks, fwn, ks, m);
+        if (jj == 3) {
+          const int f = ks * RT + im + XF;
+          if (f < 2 * RT) xf[f % XF] = lds_read<h8>(xc[f / RT] + (f % RT) * 2048);
+          else xf[f % XF] = lds_read<h8>(xn[(f - 2 * RT) / RT] + ((f - 2 * RT) % RT) * 2048);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    pin(ks ^ 1);
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+
+  // ---- prologue: D - 1 stages on their way, the first one unpacked
+#pragma unroll
+  for (int d = 0; d < D - 1; ++d) {
+    tg_load(fill + w_lds, rw, w_addr(0), 0);
+    tg_load(fill + w_lds + 4096, rw, w_addr(1), 0);
+    if constexpr (ANY) {
+      tg_load_some(fill + p_lds, rs, s_addr(), s_mask);
+      tg_load_some(fill + p_lds + ZO, rz, z_addr(), z_mask);
+    } else {
+      tg_load_at(fill + p_lds, p_addr, 0x3ffull);
+    }
+#pragma unroll
+    for (int i = 0; i < XL; ++i) tg_load(fill + x_lds(i), rx, x_voff[i], (uint32_t)kl * 128u);
+    next_load();
+  }
+  // The accumulators start as products of zeros, while the first loads are on their way (as constants the
+  // compiler would make them anew on every path into the loop and move them around at its edges).
+  u4v zero = {0u, 0u, 0u, 0u};
+  asm volatile("s_nop 1" : "+v"(zero));
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %1, 0" : "=a"(acc[j][i]) : "v"(zero));
+  uint32_t cur = smem;
+  uint32_t xc[2] = {cur + fx_off[0], cur + fx_off[1]};
+  tg_wait_and_barrier<(D - 2) * NL>();
+#pragma unroll
+  for (int rp = 0; rp < 4; ++rp) {
+    read_words(0, cur + fw_off, 0, rp);
+    read_words(1, cur + fw_off, 1, rp);
+  }
+#pragma unroll
+  for (int f = 0; f < XF; ++f) xf[f] = lds_read<h8>(xc[f / RT] + (f % RT) * 2048);
+  read_params(cur, 0);
+  expand();
+  if (ANY) read_params(cur, 1);
+#pragma unroll
+  for (int i = 0; i < 18; ++i) unpack(i, 0, 0);
+  pin(0);
+
+  auto stage = [&]() __attribute__((always_inline)) {
+    // the next stage has landed (own loads; the barrier extends that to every wave's) and every wave has read
+    // the last one, whose slot takes the stage D - 1 ahead
+    tg_wait_and_barrier<(D - 3) * NL>();
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t nxt = cur + SLOT;
+    if (nxt == smem + D * SLOT) nxt = smem;
+    uint32_t xn[2] = {nxt + fx_off[0], nxt + fx_off[1]};
+    uint32_t fwn = nxt + fw_off;
+    // (opaque: the reads' offsets stay in their offset fields)
+    asm volatile("" : "+v"(xn[0]), "+v"(xn[1]), "+v"(fwn));
+    kstep(I0{}, xc, xn, fwn, nxt);
+    kstep(I1{}, xc, xn, fwn, nxt);
+    next_load();
+    cur = nxt;
+    xc[0] = xn[0];
+    xc[1] = xn[1];
+  };
+  int n = ke - kb;
+  for (; n > 1; n -= 2) {
+    stage();
+    stage();
+  }
+  if (n) stage();
+  // no load may still be writing this workgroup's LDS when it ends; the last MFMAs' results are in their registers
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+
+  // The accumulators of one row of tiles at a time leave their registers behind this statement (moved all at once, ahead
+  // of the wait above, some of them would be read too early or spilled).
+  auto settle = [&](int im) __attribute__((always_inline)) {
+    asm volatile("" : "+a"(acc[0][im]), "+a"(acc[1][im]), "+a"(acc[2][im]), "+a"(acc[3][im]));
+  };
+  if (part) {
+#pragma unroll
+    for (int im = 0; im < RT; ++im) {
+      settle(im);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) *reinterpret_cast<f4*>(part + ((size_t)(im * 4 + j) * 256 + tid) * 4) = acc[j][im];
+    }
+    return;
+  }
+  const int col = n0 + 64 * wave + 16 * fq;
+#pragma unroll
+  for (int im = 0; im < RT; ++im) {
+    settle(im);
+    int row = m0 + 16 * im + fi;
+    float tw = 1.f;
+    bool ok;
+    if (GROUPED) {
+      row = p.sorted_ids[row];
+      ok = row < p.n_slots;
+      tw = ok && p.topk_w ? p.topk_w[row] : 1.f;
+    } else {
+      ok = row < p.M;
+    }
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      h8 o;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) o[t] = (half_t)(acc[t >> 1][im][2 * hf + (t & 1)] * tw);
+      if (ok && col + 8 * hf < p.N) *reinterpret_cast<h8*>(p.y + (size_t)row * p.N + col + 8 * hf) = o;
+    }
+  }
+}
+#endif  // __HIP_DEVICE_COMPILE__
+
+template <int RT, bool ANY>
+__global__ __launch_bounds__(256, tg_occupancy(RT)) void awq_gemm_tile_kernel(const MfmaGemmParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ __align__(1024) unsigned char smem[tg_depth(RT, ANY) * tg_slot_bytes(RT, ANY)];
+  const int id = blockIdx.x;
+  const int KT = p.K / 64;
+  int nid = 0, kb = 0, ke = KT;
+  float* part = nullptr;
+  if (id < 8 * p.per_xcd) {
+    nid = (id & 7) * p.per_xcd + (id >> 3);
+    if (nid >= p.dp_tiles) return;
+  } else {
+    const int j = id - 8 * p.per_xcd;
+    const int tl = j % p.sk_tiles, pt = j / p.sk_tiles;
+    nid = p.dp_tiles + tl;
+    kb = (int)((long long)KT * pt / p.sk_split);
+    ke = (int)((long long)KT * (pt + 1) / p.sk_split);
+    part = p.sk_part + (size_t)(tl * p.sk_split + pt) * tg_part_floats(RT);
+  }
+  const int gsize = PF_GROUP_M * p.nt;
+  const int first_m = (nid / gsize) * PF_GROUP_M;
+  const int gm = min(p.mt - first_m, PF_GROUP_M);
+  const int mt_i = first_m + (nid % gsize) % gm;
+  const int nt_i = (nid % gsize) / gm;
+  awq_tile<RT, ANY, false>(p, mt_i * (16 * RT), nt_i * 256, kb, ke, part, 0, (uint32_t)(uintptr_t)(lds_byte*)smem);
+#endif
+}
+
+template <int RT>
+__global__ __launch_bounds__(256) void awq_gemm_tile_reduce_kernel(const MfmaGemmParams p) {
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, fi = lane & 15, fq = lane >> 4;
+  const int tl = blockIdx.x / RT, im = blockIdx.x % RT;
+  const int nid = p.dp_tiles + tl;
+  const int gsize = PF_GROUP_M * p.nt;
+  const int first_m = (nid / gsize) * PF_GROUP_M;
+  const int gm = min(p.mt - first_m, PF_GROUP_M);
+  const int row = (first_m + (nid % gsize) % gm) * (16 * RT) + 16 * im + fi;
+  const int col = (nid % gsize) / gm * 256 + 64 * wave + 16 * fq;
+  const float* base = p.sk_part + (size_t)tl * p.sk_split * tg_part_floats(RT) + ((size_t)im * 4 * 256 + tid) * 4;
+  f4 v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = 0; s < p.sk_split; ++s)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] += *reinterpret_cast<const f4*>(base + (size_t)s * tg_part_floats(RT) + j * 1024);
+  if (row >= p.M) return;
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    h8 o;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) o[t] = (half_t)v[t >> 1][2 * hf + (t & 1)];
+    if (col + 8 * hf < p.N) *reinterpret_cast<h8*>(p.y + (size_t)row * p.N + col + 8 * hf) = o;
+  }
+}
+
+}  // namespace awqmi

@@ -455,6 +455,41 @@ def test_gemm_several_row_tiles_of_every_size(sba, gpu, M, K, N, G, rows):
     assert np.array_equal(y1.view(np.uint16), y2.view(np.uint16))
 
 
+# fused tiles of every height: variant -> rows
+TILE_HEIGHTS = {1 << 20: 64, 5 << 20: 80, 6 << 20: 96, 7 << 20: 112, 2 << 20: 128, 1 << 29: 160, 3 << 20: 192,
+                2 << 29: 208, 3 << 29: 224, 4 << 20: 256}
+
+
+@pytest.mark.parametrize("K,N,G", [
+    (64, 256, 64),            # one stage
+    (128, 8, 8),              # one word, eight groups a stage
+    (192, 264, 32),           # an odd number of stages, a ragged column tile, two groups a stage
+    (320, 288, 16),           # four groups a stage
+    (448, 544, 64),           # whole 32 columns, seven stages
+    (1152, 1000, 128),        # K split, ragged columns
+    (1600, 512, -1),          # one group over an odd number of stages
+    (2304, 256, 192),         # three stages a group
+])
+@pytest.mark.parametrize("variant", TILE_HEIGHTS)
+def test_fused_tile_heights(sba, gpu, variant, K, N, G):
+    """Every height of the fused kernel's tile, full and with a ragged last tile, against the oracle; without room
+    for the partial tiles of a K split it runs unsplit."""
+    from server_benchmark_amd import _lib
+    lib = _lib.load()
+    rows, g = TILE_HEIGHTS[variant], K if G <= 0 else G
+    # two workspaces: room for every split, and none
+    sba.ops.get_workspace(gpu, 80 << 20)[65536:].fill_(255)
+    for M in (rows, rows + 17 if rows > 64 else 81):
+        x, qw, s, qz = _np_case(M, K, N, g, seed=K + M)
+        y = _check_gemm(sba, gpu, x, qw, s, qz, g, 0, tag=f"tile {rows}", variant=variant | (1 << 25))
+        assert lib.awqmi_dev_last_gemm_form() == _lib.FORM_FUSED
+        xd, qwd, sd, qzd = _dev(gpu, x, qw, s, qz)
+        y1 = torch.full((M, N), float("nan"), dtype=torch.float16, device=gpu)
+        assert lib.awqmi_dev_gemm_f16(xd.data_ptr(), qwd.data_ptr(), sd.data_ptr(), qzd.data_ptr(), y1.data_ptr(), 0, 0, M, K, N, g,
+                                      0, torch.cuda.current_stream().cuda_stream, variant | (1 << 25)) == 0
+        assert awq_ref.rel_frobenius(y1.cpu().numpy(), y) <= TOL
+
+
 @pytest.mark.parametrize("M,K,N", [(512, 1024, 1280), (300, 2048, 520), (2048, 512, 5120), (768, 1536, 8192 + 256)])
 def test_gemm_prefill_partial_rounds(sba, gpu, M, K, N):
     """Tile counts that are not a multiple of the CU count, ragged last row / column tiles;
