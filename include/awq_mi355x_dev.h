@@ -14,9 +14,10 @@
  *   2        MoE launches with the dense kernel's register ring of four steps
  *   4|8|16   v = bits 2..4: runs of 1 << (v - 1) sorted-token blocks per XCD
  *   64       never two column blocks per workgroup
- *   512      without effect
+ *   512      the one-call MoE block takes its 16-slot blocks in tiles of up to four, whatever the shape
+ *            (more than 16 tokens)
  *   1024     the one-call MoE block always runs the separate activation kernel
- *   2048     the one-call MoE block always uses 16-row blocks
+ *   2048     the one-call MoE block always uses the skinny kernel's 16-row blocks
  *   4096     every launch keeps the weight ring in registers (no LDS ring)
  *   16384    the align step always runs in one workgroup
  *   1 << 16  v = bits 16..17: the one-call MoE block uses 64 / 128 / 256-row blocks (v = 1 / 2 / 3)

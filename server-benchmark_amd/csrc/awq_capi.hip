@@ -15,7 +15,6 @@
 #include "../../include/awq_mi355x_dev.h"
 #include "awq_dequant.hpp"
 #include "awq_gemm_dense.hpp"
-#include "awq_gemm_mfma.hpp"
 #include "awq_gemm_mid.hpp"
 #include "awq_gemm_tile.hpp"
 #include "awq_gemv.hpp"
@@ -56,8 +55,9 @@ enum : int {
   VAR_MOE_RING4 = 2,          // MoE launches with the dense kernel's register ring of four steps
   VAR_XCD_RUN_SHIFT = 2,      // bits 2..4 = v: force runs of 1 << (v - 1) blocks per XCD
   VAR_NO_PAIR_COLS = 64,      // never two column blocks per workgroup
+  VAR_MOE_RUNS = 512,         // the one-call MoE block takes its 16-slot blocks in tiles of up to four, whatever the shape
   VAR_NO_FUSED_ACT = 1024,    // the one-call MoE block always runs the separate activation kernel
-  VAR_MOE_TILE16 = 2048,      // the one-call MoE block always uses 16-row blocks
+  VAR_MOE_TILE16 = 2048,      // the one-call MoE block always uses the skinny kernel's 16-row blocks
   VAR_NO_LDS_RING = 4096,     // every launch keeps the weight ring in registers
   VAR_ALIGN_ONE_WG = 16384,   // align always in one workgroup
   VAR_MOE_TILE_SHIFT = 16,    // bits 16..17 = v: the one-call MoE block uses 64 / 128 / 256-row blocks (v = 1 / 2 / 3)
@@ -288,7 +288,7 @@ inline int mfma_slab_rows(int M, int K) {
 struct MfmaPlan { int dp_tiles, sk_tiles, sk_split; size_t part_bytes; };
 MfmaPlan plan_mfma(int M, int K, int N, int bm) {
   const int mt = (M + bm - 1) / bm, nt = (N + PF_BN - 1) / PF_BN;
-  const int tiles = mt * nt, KT = K / PF_BK;
+  const int tiles = mt * nt, KT = K / DG_BK;
   MfmaPlan pl{tiles, 0, 1, 0};
   const int rem = tiles % 256;
   if (rem == 0) return pl;
@@ -380,13 +380,13 @@ TilePlan pick_tile(int M, int K, int N, size_t room) {
 }
 // Launch of a tile height with the larger of two kernels where the layer needs it (see awq_tile).
 template <int RT>
-void launch_tile(const MfmaGemmParams& p, hipStream_t st) {
+void launch_tile(const TileGemmParams& p, hipStream_t st) {
   const dim3 grid(p.per_xcd * 8 + p.sk_tiles * p.sk_split);
   if (p.G % 64 == 0 && p.N % 32 == 0) hipLaunchKernelGGL((awq_gemm_tile_kernel<RT, false>), grid, dim3(256), 0, st, p);
   else hipLaunchKernelGGL((awq_gemm_tile_kernel<RT, true>), grid, dim3(256), 0, st, p);
   if (p.sk_tiles > 0) hipLaunchKernelGGL((awq_gemm_tile_reduce_kernel<RT>), dim3(p.sk_tiles * RT), dim3(256), 0, st, p);
 }
-void launch_tile(int rt, const MfmaGemmParams& p, hipStream_t st) {
+void launch_tile(int rt, const TileGemmParams& p, hipStream_t st) {
   switch (rt) {
     case 4: return launch_tile<4>(p, st);
     case 5: return launch_tile<5>(p, st);
@@ -413,14 +413,6 @@ static int ensure_kernel_attributes() {
   if (ge != hipSuccess) { t_last_hip_error = (int)ge; return AWQMI_LAUNCH_FAILED; }
   if (dev < 0 || dev >= MAX_DEVICES) return AWQMI_BAD_ARGUMENT;
   if (done[dev].load(std::memory_order_acquire)) return AWQMI_OK;
-  const void* mfma[] = {
-      reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<true, 1, 8>), reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<false, 1, 8>),
-      reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<true, 2, 8>), reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<false, 2, 8>),
-      reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<true, 4, 4>), reinterpret_cast<const void*>(awq_gemm_mfma_grouped_kernel<false, 4, 4>)};
-  for (const void* fn : mfma) {
-    const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, PF_LDS_BYTES);
-    if (e != hipSuccess) { t_last_hip_error = (int)e; return AWQMI_LAUNCH_FAILED; }
-  }
   const void* align[] = {
       reinterpret_cast<const void*>(moe_align_kernel),
       reinterpret_cast<const void*>(moe_align_count_kernel), reinterpret_cast<const void*>(moe_align_place_kernel),
@@ -482,10 +474,19 @@ struct MoeRoute {
   int32_t* sorted;
   int32_t* experts;
   int32_t* npp;
+  int32_t* runs;     // tiles of several 16-slot blocks (more than 16 tokens only)
 };
 
 // Routing + align of a short slot list as launches of their own (one launch for up to 16
 // tokens, else top-k and align apart).
+static int moe_align_launch(const int32_t* topk_ids, int n_slots, int E, int tile_m, int32_t* sorted, int32_t* experts,
+                            int32_t* npp, int32_t* runs, void* stream) {
+  const int cap = (int)awqmi_moe_align_capacity(n_slots, E, tile_m);
+  if (const int rc = ensure_kernel_attributes()) return rc;
+  hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(1024), (size_t)(MOE_ALIGN_WAVES + 2) * E * sizeof(int),
+                     (hipStream_t)stream, topk_ids, n_slots, E, tile_m, cap, sorted, experts, npp, runs);
+  return launch_status();
+}
 static int moe_route_launches(const MoeRoute& r, int tile, void* stream) {
   if (r.T <= MOE_ALIGN_WAVES)
     return moe_route_align_small(r.logits, r.bias, r.T, r.E, r.topk, r.scoring, r.renorm, r.scale, r.ids, r.wts, tile,
@@ -493,7 +494,7 @@ static int moe_route_launches(const MoeRoute& r, int tile, void* stream) {
   if (const int st = awqmi_moe_topk_f32(r.logits, r.bias, r.T, r.E, r.topk, r.scoring, r.renorm, r.scale, r.ids, r.wts,
                                         stream))
     return st;
-  return awqmi_moe_align(r.ids, r.T * r.topk, r.E, tile, r.sorted, r.experts, r.npp, stream);
+  return moe_align_launch(r.ids, r.T * r.topk, r.E, tile, r.sorted, r.experts, r.npp, r.runs, stream);
 }
 
 // Folded routing: at most four tokens (one per wave of a workgroup; the kernel would take up to
@@ -589,7 +590,7 @@ size_t awqmi_gemm_workspace_bytes(int M, int K, int N, int split_k) {
   if (M <= 0 || K <= 0 || N <= 0) return 0;
   // the group size decides between the kernels for some shapes, so cover both
   size_t mfma = 0, skinny = 0;
-  if (M > 16 && K % PF_BK == 0) {
+  if (M > 16 && K % DG_BK == 0) {
     const int slab = mfma_slab_rows(M, K);
     if (slab > 0) {
       // the plan the call will pick, and room for the K split of 256-row tiles at least (any forced size
@@ -646,7 +647,7 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
   half_t* yy = reinterpret_cast<half_t*>(y);
 
   const int wpl = gemv_wpl(N);
-  const bool mfma_ok = K % PF_BK == 0 && (((G & (G - 1)) == 0 && G >= 8) || G % 64 == 0) &&
+  const bool mfma_ok = K % DG_BK == 0 && (((G & (G - 1)) == 0 && G >= 8) || G % 64 == 0) &&
                        mfma_slab_rows(M, K) > 0 && (size_t)K * ldw * 4 < (1ull << 32) &&
                        (size_t)(K / G) * N * 2 < (1ull << 32);
   if (mid_rows(M, K, N, G, ldw)) {
@@ -763,7 +764,7 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
       } else {
         pl = pick_tile(Ms, K, N, room);
       }
-      MfmaGemmParams p{};
+      TileGemmParams p{};
       p.x = xx + (size_t)r0 * K; p.qw = qw; p.sc = sc; p.qz = qz; p.y = yy + (size_t)r0 * N;
       p.M = Ms; p.K = K; p.N = N; p.NW = NW; p.ldw = ldw; p.G = G;
       while ((2 << p.gshift) <= G) ++p.gshift;
@@ -843,12 +844,7 @@ int awqmi_moe_align(const int32_t* topk_ids, int n_slots, int E, int tile_m, int
     return AWQMI_NULL_POINTER;
   if (n_slots <= 0 || E <= 0) return AWQMI_BAD_SHAPE;
   if (E > AWQMI_MAX_EXPERTS || tile_m <= 0 || tile_m > 4096) return AWQMI_BAD_ARGUMENT;
-  const int cap = (int)awqmi_moe_align_capacity(n_slots, E, tile_m);
-  if (const int rc = ensure_kernel_attributes()) return rc;
-  hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(1024), (size_t)(MOE_ALIGN_WAVES + 2) * E * sizeof(int),
-                     (hipStream_t)stream, topk_ids, n_slots, E, tile_m, cap, sorted_token_ids,
-                     expert_ids, num_tokens_post_padded);
-  return launch_status();
+  return moe_align_launch(topk_ids, n_slots, E, tile_m, sorted_token_ids, expert_ids, num_tokens_post_padded, nullptr, stream);
 }
 
 // sorted-token blocks a grouped launch covers: the align capacity, rounded up to whole groups
@@ -918,12 +914,23 @@ static bool moe_can_fuse_act_split(int n_slots, int E, int K, int N) {
   return pl.wpl == 2 && pl.split > 1 && N % 512 == 0 && pl.ncb % 2 == 0;
 }
 
+// The grouped tile kernel can write silu(gate) * up itself where its column tiles are whole and its plain
+// form runs (groups of at least 64).
+static bool moe_tile_act_ok(int inter, int G) { return inter % 128 == 0 && G % 64 == 0; }
+
+// tiles of at most TG_RUN 16-slot blocks that n_slots slots on E experts make at most
+static long long moe_most_runs(int n_slots, int E) {
+  const long long touched = std::min(n_slots, E);
+  return touched + (n_slots / 16 + touched) / TG_RUN;
+}
+static_assert(TG_RUN == MOE_RUN, "the tile lists are made for the grouped kernel");
+
 static int moe_gemm_impl(const void* x, const int32_t* qweight, const void* scales, const int32_t* qzeros,
                          void* y, const int32_t* sorted_token_ids, const int32_t* expert_ids,
                          const int32_t* num_tokens_post_padded, const float* topk_weights, int n_slots,
                          int a_row_div, int tile_m, int E, int K, int N, int group, int split_k,
                          void* workspace, size_t workspace_bytes, void* stream, bool fuse_act,
-                         const MoeRoute* route = nullptr);
+                         const MoeRoute* route = nullptr, int32_t* runs = nullptr);
 
 int awqmi_moe_gemm_f16(const void* x, const int32_t* qweight, const void* scales, const int32_t* qzeros,
                        void* y, const int32_t* sorted_token_ids, const int32_t* expert_ids,
@@ -940,7 +947,7 @@ static int moe_gemm_impl(const void* x, const int32_t* qweight, const void* scal
                          const int32_t* num_tokens_post_padded, const float* topk_weights, int n_slots,
                          int a_row_div, int tile_m, int E, int K, int N, int group, int split_k,
                          void* workspace, size_t workspace_bytes, void* stream, bool fuse_act,
-                         const MoeRoute* route) {
+                         const MoeRoute* route, int32_t* runs) {
   // route: the block's routing has not run yet.  The launch takes it along when it is the plain
   // 16-row-block form with G = 128; any other form routes in launches of its own first.
   if (!x || !qweight || !scales || !qzeros || !y || !sorted_token_ids || !expert_ids ||
@@ -957,45 +964,57 @@ static int moe_gemm_impl(const void* x, const int32_t* qweight, const void* scal
       !aligned16(y))
     return AWQMI_BAD_ALIGN;
   const int NW = N / 8;
-  if (tile_m >= 64) {
-    // blocks of 64 / 128 slots: the MFMA kernel in its expert-grouped form (no K split)
-    if (fuse_act) return AWQMI_BAD_ARGUMENT;
+  if (tile_m >= 64 || runs) {
+    // blocks of 64 / 128 / 256 slots, or tiles of several 16-slot blocks: the tile kernel in its expert-grouped
+    // form (no K split)
+    const bool any = G % 64 != 0 || N % 32 != 0;
+    if (fuse_act && !moe_tile_act_ok(N / 2, G)) return AWQMI_BAD_ARGUMENT;
     if (route)
       if (const int rc = moe_route_launches(*route, tile_m, stream)) return rc;
     const size_t x_rows = ((size_t)n_slots + a_row_div - 1) / a_row_div;
     if (x_rows * K * 2 >= (1ull << 32) || (size_t)K * NW * 4 >= (1ull << 32) ||
         (size_t)(K / G) * N * 2 >= (1ull << 32))
       return AWQMI_BAD_SHAPE;
-    if (const int rc = ensure_kernel_attributes()) return rc;
-    MfmaGemmParams p{};
+    TileGemmParams p{};
     p.x = reinterpret_cast<const half_t*>(x);
     p.qw = reinterpret_cast<const uint32_t*>(qweight);
     p.sc = reinterpret_cast<const half_t*>(scales);
     p.qz = reinterpret_cast<const uint32_t*>(qzeros);
     p.y = reinterpret_cast<half_t*>(y);
     p.M = (int)x_rows; p.K = K; p.N = N; p.NW = NW; p.ldw = NW; p.G = G;
-    const bool pow2g = (G & (G - 1)) == 0 && G >= 8;
-    p.gshift = 0;
-    if (pow2g) while ((1 << p.gshift) < G) ++p.gshift;
-    p.mt = 1; p.nt = (N + PF_BN - 1) / PF_BN; p.per_xcd = 0;
-    p.dp_tiles = 0; p.sk_tiles = 0; p.sk_split = 1;
-    p.sorted_ids = sorted_token_ids; p.expert_ids = expert_ids; p.n_post_pad = num_tokens_post_padded;
+    while ((2 << p.gshift) <= G) ++p.gshift;
+    const int cols = fuse_act ? N / 2 : N, per_tile = fuse_act ? TG_COLS / 2 : TG_COLS;
+    p.nt = (cols + per_tile - 1) / per_tile;
+    p.sorted_ids = sorted_token_ids; p.expert_ids = expert_ids; p.n_live = num_tokens_post_padded;
     p.topk_w = topk_weights; p.n_slots = n_slots; p.a_row_div = a_row_div;
     p.w_stride = (long long)K * NW; p.s_stride = (long long)(K / G) * N; p.z_stride = (long long)(K / G) * NW;
-    const int nblk = (int)(awqmi_moe_align_capacity(n_slots, E, tile_m) / tile_m);
-    p.total = nblk * p.nt;
-    const dim3 grid(((unsigned)nblk * p.nt + 7) / 8 * 8);     // whole deals to the 8 XCDs
-    hipStream_t st = (hipStream_t)stream;
-    if (tile_m == 64) {
-      if (pow2g) hipLaunchKernelGGL((awq_gemm_mfma_grouped_kernel<true, 1, 8>), grid, dim3(512), PF_LDS_BYTES, st, p);
-      else hipLaunchKernelGGL((awq_gemm_mfma_grouped_kernel<false, 1, 8>), grid, dim3(512), PF_LDS_BYTES, st, p);
-    } else if (tile_m == 128) {
-      if (pow2g) hipLaunchKernelGGL((awq_gemm_mfma_grouped_kernel<true, 2, 8>), grid, dim3(512), PF_LDS_BYTES, st, p);
-      else hipLaunchKernelGGL((awq_gemm_mfma_grouped_kernel<false, 2, 8>), grid, dim3(512), PF_LDS_BYTES, st, p);
-    } else {
-      if (pow2g) hipLaunchKernelGGL((awq_gemm_mfma_grouped_kernel<true, 4, 4>), grid, dim3(256), PF_LDS_BYTES, st, p);
-      else hipLaunchKernelGGL((awq_gemm_mfma_grouped_kernel<false, 4, 4>), grid, dim3(256), PF_LDS_BYTES, st, p);
+    p.block = tile_m;
+    long long tiles = (long long)(awqmi_moe_align_capacity(n_slots, E, tile_m) / std::min(tile_m, TG_ROWS));
+    if (runs) {
+      p.n_live = runs;
+      p.runs = runs + 1;
+      tiles = moe_most_runs(n_slots, E);
     }
+    p.total = (int)(tiles * p.nt);
+    // ranges per XCD are uneven in rows with few experts (see the kernel)
+    p.in_order = E < 16;
+    const dim3 grid((unsigned)((p.total + 7) / 8 * 8));     // whole deals to the 8 XCDs
+    hipStream_t st = (hipStream_t)stream;
+#define AWQMI_GROUPED(...) hipLaunchKernelGGL((awq_gemm_tile_grouped_kernel<__VA_ARGS__>), grid, dim3(256), 0, st, p)
+    if (runs && G == 64) {
+      if (fuse_act) AWQMI_GROUPED(false, true, 1);
+      else AWQMI_GROUPED(false, false, 1);
+    } else if (runs) {
+      if (fuse_act) AWQMI_GROUPED(false, true, 2);
+      else AWQMI_GROUPED(false, false, 2);
+    } else if (any) {
+      AWQMI_GROUPED(true, false, 0);
+    } else if (fuse_act) {
+      AWQMI_GROUPED(false, true, 0);
+    } else {
+      AWQMI_GROUPED(false, false, 0);
+    }
+#undef AWQMI_GROUPED
     return launch_status();
   }
   const MoePlan pl = moe_plan(n_slots, E, K, N, tile_m, split_k);
@@ -1059,8 +1078,8 @@ static int moe_gemm_impl(const void* x, const int32_t* qweight, const void* scal
   const int ncg = t32_narrow ? (ncb1 + 1) / 2 : (act_pair ? ncb / 2 : (pair_cols ? (ncb + 1) / 2 : ncb));
   if (t32_narrow) p.ncb = ncb1;
   // runs of grp slots, dealt to the 8 XCDs in turn; the last deal may be partial
-  const long long runs = (long long)(nblk / p.grp) * ncg * split;
-  const dim3 grid((unsigned)((runs + 7) / 8 * 8 * p.grp));
+  const long long deals = (long long)(nblk / p.grp) * ncg * split;
+  const dim3 grid((unsigned)((deals + 7) / 8 * 8 * p.grp));
   hipStream_t st = (hipStream_t)stream;
   // weight ring of four steps in LDS instead of two in registers, from one full block per
   // expert on (T = 256 ... 1024 of the 128-expert block: 6 - 10 % faster; with fewer rows per
@@ -1132,6 +1151,15 @@ namespace {
 constexpr int MOE_ALIGN_PARTS_MAX = 64;      // workgroups of the multi-workgroup align
 constexpr int MOE_ALIGN_SPLIT_MIN = 16384;   // slots from which it is used (4096 per workgroup)
 
+// Expected blocks of `rows` slots of an expert's run when its slot count is Poisson(avg) (normal tail past the
+// first block): sum_j P(count > j * rows)
+double moe_expected_blocks(double avg, int rows) {
+  double e = 1.0 - std::exp(-avg);
+  for (int j = 1; j * (double)rows < avg + 6.0 * std::sqrt(avg) + 1.0; ++j)
+    e += 0.5 * std::erfc((j * (double)rows + 0.5 - avg) / std::sqrt(2.0 * avg));
+  return e;
+}
+
 // Rows per block for the two expert GEMMs of one MoE block: 16 (the skinny kernel) or 64 /
 // 128 / 256 (the MFMA kernel's expert-grouped form), by price:
 //   skinny: flops / (540 TFLOP/s * avg / (avg + 26)), avg = slots per expert;
@@ -1152,6 +1180,10 @@ constexpr int MOE_ALIGN_SPLIT_MIN = 16384;   // slots from which it is used (409
 //   - the second price alone, downwards too, is 1.9 % behind the best size and 12 points are 5 - 24 % behind the
 //     first look (1590 tokens on 128 experts of 2048 x 768, top-8: 16 rows 289, 128 rows 236; 1391 on 16 of 5120 x
 //     8192, top-1: 256 rows 704, 128 rows 642).
+// The prices are those of the grouped kernel that dequantised into LDS, and 16 rows those of the skinny kernel: they say where
+// blocks of 16 slots end, which callers of the step-by-step path have in their own calls too.  With the present kernel, which is
+// faster for every size, and moe_runs beside it the choice is 4 % behind the best of 16, 16 in tiles and 128 on average of 129
+// points, 30 % at worst (896 tokens on 256 experts of 2048 x 384, top-8: 156 us, in tiles 120; see moe_runs for its line at 32).
 // Three sizes that the tests fix measure slower than another: 2048 tokens on 128 experts of 2048 x 768 (16 rows
 // 327 us, 256 rows 279), 1024 on 160 of 6144 x 2560 (64 rows 1775, 16 rows 1684), 2102 on 4 of 512 x 384 (16 rows
 // 52, 64 rows 43).
@@ -1170,14 +1202,8 @@ int moe_pick_tile(int n_slots, int E, int H, int inter, int group) {
   if (avg < 32.0) return 16;
   const double flops = 2.0 * n_slots * ((double)H * 2 * inter + (double)inter * H);
   const double skinny = flops / (540e12 * avg / (avg + 26.0));
-  // expected blocks of `rows` after padding each expert's run: E * sum_j P(count > j * rows), the
-  // count of an expert taken as Poisson(avg) (normal tail for j >= 1)
-  auto expected = [&](int rows) {
-    double per_expert = 1.0 - std::exp(-avg);
-    for (int j = 1; j * (double)rows < avg + 6.0 * std::sqrt(avg) + 1.0; ++j)
-      per_expert += 0.5 * std::erfc((j * (double)rows + 0.5 - avg) / std::sqrt(2.0 * avg));
-    return E * per_expert;
-  };
+  // expected blocks of `rows` after padding each expert's run
+  auto expected = [&](int rows) { return E * moe_expected_blocks(avg, rows); };
   // price of blocks of bm rows, partly filled ones counted whole or (by_rows) by their rows in steps of 64
   auto mfma = [&](int bm, bool by_rows) {
     const double blocks = by_rows ? (64.0 * expected(64) + 112.0 * expected(bm)) / (bm + 112) : expected(bm);
@@ -1187,7 +1213,7 @@ int moe_pick_tile(int n_slots, int E, int H, int inter, int group) {
       const double r = blocks * ((N + PF_BN - 1) / PF_BN) / 256.0;
       const double whole = std::floor(r), part = r - whole;
       const double rounds = whole + (part > 0 ? std::max(part, 0.5) : 0.0);
-      return rounds * (K / PF_BK + over) * kt_s;
+      return rounds * (K / DG_BK + over) * kt_s;
     };
     return gemm(H, 2 * inter) + gemm(inter, H) + 5e-6 + 6.0 * n_slots * inter / 4e12;
   };
@@ -1204,6 +1230,42 @@ int moe_pick_tile(int n_slots, int E, int H, int inter, int group) {
     if (t < best) { best = t; tile = bm; }
   }
   return tile;
+}
+
+// Blocks of 16 slots: run the expert GEMMs on tiles of up to four of them (the tile kernel) instead of a
+// block at a time (the skinny kernel), by price in us.
+//   tiles: per GEMM rounds of 512 workgroups (a partial last one counts as at least 0.38) of (K / 64 + 2.1) stages, a stage
+//   of two workgroups per CU at 2 * (0.344 + 0.09 per 16 rows);
+//   blocks: 0.09 us per MB of touched experts' weights and 0.11 per MB and block, which unpacks them again.
+// Fitted on 129 points (ten expert shapes, 6 ... 400 slots per expert), the whole block timed both ways.  The tiles have to
+// look 14 % cheaper (24 % below 16 experts, whose few long tiles the price underestimates): then no point of them is slower
+// than with the skinny kernel, and they are 8 % faster on average over all.  Up to 32 slots per expert a tile is two blocks at
+// most on average: within 5 % either way up to 25 slots, 15 % at 32 (128 experts of 2048 x 768, top-8, 400 / 512 tokens:
+// both GEMMs 97 / 121 us by blocks, 102 / 100 by tiles).  There the block keeps the kernel that the separate calls on
+// 16-slot blocks take, so that both add in one order; so do experts below the smallest measured (1024 x 512, 2048 x 384),
+// where the routing and the sum outweigh both GEMMs.  Both sides above, blocks / tiles (us): 576 / 768 / 1024 tokens on those
+// experts 143 / 164 / 192 and 116 / 130 / 163; 384 / 512 on 64 of 2048 x 1408 136 / 158 and 102 / 114; 560 on 160 of 6144 x
+// 2560 1172 and 993.
+bool moe_runs(int T, int n_slots, int E, int H, int inter, int group) {
+  if (variant_on(VAR_MOE_TILE16) || T <= MOE_ALIGN_WAVES) return false;
+  // groups of 64 or 128 rows, whole column tiles
+  const int g1 = norm_group(H, group), g2 = norm_group(inter, group);
+  if (H % 128 != 0 || inter % 128 != 0 || (g1 != 64 && g1 != 128) || g1 != g2) return false;
+  if ((size_t)n_slots * std::max(H, inter) * 2 >= (1ull << 32) || (size_t)H * (2 * inter / 8) * 4 >= (1ull << 32) ||
+      (size_t)inter * (H / 8) * 4 >= (1ull << 32))
+    return false;
+  if (variant_on(VAR_MOE_RUNS)) return true;
+  const double avg = (double)n_slots / E, b16 = E * moe_expected_blocks(avg, 16), tiles = E * moe_expected_blocks(avg, 16 * TG_RUN);
+  if (avg <= 32.0 || H < 1024 || inter < 384) return false;
+  const double stage = 2.0 * (0.344 + 0.09 * std::max(b16 / tiles, 2.0));
+  auto gemm = [&](int K, int col_tiles) {
+    const double r = tiles * col_tiles / 512.0, whole = std::floor(r), part = r - whole;
+    return (whole + (part > 0 ? std::max(part, 0.38) : 0.0)) * (K / 64 + 2.1) * stage;
+  };
+  const double runs = 19.8 + gemm(H, (inter + 127) / 128) + gemm(inter, (H + TG_COLS - 1) / TG_COLS);
+  const double mb = 1.5 * H * inter * 1e-6;     // packed weights of an expert
+  const double skinny = 26.6 + (0.09 * E * (1.0 - std::exp(-avg)) + 0.11 * b16) * mb + 0.0009 * n_slots;
+  return runs < (E < 16 ? 0.76 : 0.86) * skinny;
 }
 
 // workspace carve-up of the fused MoE block; every piece starts 256-byte aligned
@@ -1285,11 +1347,13 @@ int awqmi_fused_moe_routed_f16(const void* hidden, const float* router_logits, c
   int32_t* experts = reinterpret_cast<int32_t*>(ws + L.experts);
   int32_t* npp = reinterpret_cast<int32_t*>(ws + L.npp);
   void* h13 = ws + L.h13;
-  void* act = ws + L.act;
+  void* act_out = ws + L.act;
   void* o = ws + L.o;
   int st;
+  // tiles of several 16-slot blocks write silu(gate) * up themselves: their list is where the gate / up sums would be
+  int32_t* const runs = tile == 16 && moe_runs(T, L.n_slots, E, H, inter, group) ? reinterpret_cast<int32_t*>(h13) : nullptr;
   const MoeRoute route{router_logits, score_bias, T, E, topk, scoring, renormalize, routed_scale,
-                       ids, wts, sorted, experts, npp};
+                       ids, wts, sorted, experts, npp, runs};
   // a handful of tokens: the first expert GEMM takes the routing along (one launch less)
   const bool fold = moe_route_foldable(T, E, topk, tile);
   const MoeRoute* pending = fold ? &route : nullptr;
@@ -1313,29 +1377,33 @@ int awqmi_fused_moe_routed_f16(const void* hidden, const float* router_logits, c
     hipStream_t hs = (hipStream_t)stream;
     hipLaunchKernelGGL(moe_align_count_kernel, dim3(parts), dim3(1024), lds, hs, ids, L.n_slots, E, part, tab);
     hipLaunchKernelGGL(moe_align_scan_kernel, dim3(1), dim3(1024), (size_t)2 * E * sizeof(int), hs, L.n_slots, E,
-                       tile, L.cap, parts, tab, sorted, experts, npp);
+                       tile, L.cap, parts, tab, sorted, experts, npp, runs);
     hipLaunchKernelGGL(moe_align_place_kernel, dim3(parts), dim3(1024), lds, hs, ids, L.n_slots, E, part, tab,
                        sorted);
     st = launch_status();
     if (st) return st;
   }
   const int Gn = norm_group(H, group);
-  if (tile == 16 && gemv_tiled_ok(H, Gn) && !variant_on(VAR_NO_FUSED_ACT) &&
-      (moe_can_fuse_act(L.n_slots, E, H, 2 * inter) || moe_can_fuse_act_split(L.n_slots, E, H, 2 * inter))) {
-    // the w13 GEMM writes silu(gate) * up itself: in one workgroup per gate / up block pair, or,
-    // with few blocks (the launch is split in K), in the last arrivers of such a pair
-    st = moe_gemm_impl(hidden, w13_q, w13_s, w13_z, act, sorted, experts, npp, nullptr, L.n_slots, topk, 16, E, H,
-                       2 * inter, group, 0, ws + L.gemm_ws, L.gemm_ws_bytes, stream, true, pending);
+  const bool tiles = tile >= 64 || runs;
+  const bool act = tiles ? moe_tile_act_ok(inter, Gn)
+                         : gemv_tiled_ok(H, Gn) && (moe_can_fuse_act(L.n_slots, E, H, 2 * inter) ||
+                                                    moe_can_fuse_act_split(L.n_slots, E, H, 2 * inter));
+  if (act && !variant_on(VAR_NO_FUSED_ACT)) {
+    // the w13 GEMM writes silu(gate) * up itself: in a tile of gate columns and their up columns; in one
+    // workgroup per gate / up block pair; or, with few blocks (the launch is split in K), in the last arrivers of
+    // such a pair
+    st = moe_gemm_impl(hidden, w13_q, w13_s, w13_z, act_out, sorted, experts, npp, nullptr, L.n_slots, topk, tile, E, H,
+                       2 * inter, group, 0, ws + L.gemm_ws, L.gemm_ws_bytes, stream, true, pending, runs);
     if (st) return st;
   } else {
     st = moe_gemm_impl(hidden, w13_q, w13_s, w13_z, h13, sorted, experts, npp, nullptr, L.n_slots, topk,
-                       tile, E, H, 2 * inter, group, 0, ws + L.gemm_ws, L.gemm_ws_bytes, stream, false, pending);
+                       tile, E, H, 2 * inter, group, 0, ws + L.gemm_ws, L.gemm_ws_bytes, stream, false, pending, runs);
     if (st) return st;
-    st = awqmi_silu_and_mul_f16(h13, act, L.n_slots, inter, stream);
+    st = awqmi_silu_and_mul_f16(h13, act_out, L.n_slots, inter, stream);
     if (st) return st;
   }
-  st = awqmi_moe_gemm_f16(act, w2_q, w2_s, w2_z, o, sorted, experts, npp, wts, L.n_slots, 1, tile, E, inter, H,
-                          group, 0, ws + L.gemm_ws, L.gemm_ws_bytes, stream);
+  st = moe_gemm_impl(act_out, w2_q, w2_s, w2_z, o, sorted, experts, npp, wts, L.n_slots, 1, tile, E, inter, H,
+                     group, 0, ws + L.gemm_ws, L.gemm_ws_bytes, stream, false, nullptr, runs);
   if (st) return st;
   return awqmi_moe_sum_f16(o, out, T, topk, H, stream);
 }

@@ -47,6 +47,12 @@ struct NibbleMasks {
 __device__ __forceinline__ uint32_t pk_sub(uint32_t a, uint32_t b) { return as_u32(as_h2(a) - as_h2(b)); }
 __device__ __forceinline__ uint32_t pk_mul(uint32_t a, uint32_t b) { return as_u32(as_h2(a) * as_h2(b)); }
 
+// silu(g) * u of fp16 values in fp32, rounded once
+__device__ __forceinline__ half_t silu_mul(half_t g, half_t u) {
+  const float v = (float)g;
+  return (half_t)(v / (1.f + __expf(-v)) * (float)u);
+}
+
 // logical column (0..7) held by nibble `nib` of a packed word
 __host__ __device__ constexpr int awq_col_of_nibble(int nib) {
   return nib < 4 ? 2 * nib : 2 * (nib - 4) + 1;

@@ -1,6 +1,6 @@
 // Prefill AWQ GEMM for many rows (M in the thousands): dequantise once, then a dense fp16 GEMM.
 //
-// At M = 8192 the fused kernel (awq_gemm_mfma.hpp) unpacks every weight 32 times, once per
+// At M = 8192 the fused kernel (awq_gemm_tile.hpp) unpacks every weight 32 times, once per
 // 256-row tile.  Here the weights are dequantised once per call into an fp16 panel in the
 // caller's workspace (awq_dequant_panel_kernel, bit-exact (w - z) * s, the same arithmetic as
 // awq_dequantize) and awq_gemm_dense_kernel multiplies X by that panel with no unpack
@@ -36,9 +36,20 @@
 #include <type_traits>
 
 #include "awq_common.hpp"
-#include "awq_gemm_mfma.hpp"
 
 namespace awqmi {
+
+// Tile order of the GEMM kernels: groups of PF_GROUP_M row tiles walk the column tiles together, so that the 32
+// tiles an XCD runs at a time share a few X and W slabs through its L2 (2, 4, 8 and 16 measured
+// the same within noise: the re-reads that remain are served by the memory-side cache).
+constexpr int PF_GROUP_M = 8;
+constexpr int PF_BN = 256;                          // columns of a tile
+constexpr int PF_SK_SLOT_FLOATS = 256 * 256;
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t pf_rsrc(const void* base, size_t bytes) {
+  const uint32_t n = bytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)bytes;
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)n, 0x00020000);
+}
 
 constexpr int DG_BK = 64;                           // k per stage
 constexpr int DG_ROW_BYTES = DG_BK * 2;             // 128 B per row and stage
@@ -131,7 +142,7 @@ struct DenseGemmParams {
   int M, K, N;
   int mt, nt;                    // 256-row and 256-column tile counts
   int per_xcd;                   // ceil(dp_tiles / 8)
-  // as in MfmaGemmParams: tiles [0, dp_tiles) one workgroup each; the sk_tiles tiles of a sparse
+  // as in TileGemmParams: tiles [0, dp_tiles) one workgroup each; the sk_tiles tiles of a sparse
   // last round are split in K over sk_split workgroups and summed by the reduce kernel
   int dp_tiles, sk_tiles, sk_split;
   float* sk_part;

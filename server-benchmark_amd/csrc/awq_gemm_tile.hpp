@@ -35,6 +35,37 @@
 
 namespace awqmi {
 
+struct TileGemmParams {
+  const half_t* x;
+  const uint32_t* qw;
+  const half_t* sc;
+  const uint32_t* qz;
+  half_t* y;
+  int M, K, N, NW, G;
+  int ldw;        // words between consecutive rows of qweight (NW, or more when the rows are padded)
+  int gshift;     // log2(G) when G < 64
+  int mt, nt;     // tile counts
+  int per_xcd;    // ceil(dp_tiles / 8)
+  // Work split.  Tiles [0, dp_tiles) run one workgroup per tile over all of K (launch ids
+  // [0, 8 * per_xcd)).  The remaining sk_tiles tiles (a last round that would leave CUs idle) are split in K over
+  // sk_split workgroups each (launch ids from 8 * per_xcd on, part-major) and leave fp32 partial tiles in the
+  // workspace; a second, short kernel on the same stream sums them in part order and writes fp16 (a single finishing
+  // workgroup per tile would have to pull all of them by itself, which took longer than the GEMM).
+  int dp_tiles, sk_tiles, sk_split;
+  float* sk_part;   // [sk_tiles][sk_split][tg_part_floats]
+  // Expert-grouped launch (awq_gemm_tile_grouped_kernel)
+  const int* sorted_ids;
+  const int* expert_ids;
+  const int* n_live;        // padded slots (blocks) or tiles (runs) in use
+  const int* runs;          // first 16-slot block and blocks of each tile
+  const float* topk_w;      // optional per-slot output weight
+  int n_slots, block;       // slots; slots of a block
+  int a_row_div;            // X row of a slot = slot / a_row_div
+  int total;                // column tiles x most blocks or tiles
+  int in_order;             // tiles in launch order instead of ranges per XCD
+  long long w_stride, s_stride, z_stride;   // elements per expert
+};
+
 constexpr int TG_COLS = 256;             // columns of a workgroup tile
 constexpr int TG_W_BYTES = 64 * 128;     // packed weights of a stage: 64 k x 256 columns
 
@@ -42,17 +73,18 @@ constexpr int TG_W_BYTES = 64 * 128;     // packed weights of a stage: 64 k x 25
 __host__ __device__ constexpr int tg_x_bytes(int rt) { return rt * 16 * 128; }
 __host__ __device__ constexpr int tg_param_bytes(bool any) { return any ? 1280 : 256; }
 __host__ __device__ constexpr int tg_slot_bytes(int rt, bool any) { return tg_x_bytes(rt) + TG_W_BYTES + 4 * tg_param_bytes(any); }
-// workgroups of a CU, and stages of the LDS ring
-__host__ __device__ constexpr int tg_occupancy(int rt) { return rt <= 5 ? 2 : 1; }
-__host__ __device__ constexpr int tg_depth(int rt, bool any) {
-  const int fit = 160 * 1024 / tg_occupancy(rt) / tg_slot_bytes(rt, any);
+// workgroups of a CU, LDS of each for the ring (the rest holds the slot lists of a grouped launch), and its stages
+__host__ __device__ constexpr int tg_occupancy(int rt, bool any) { return rt <= (any ? 5 : 8) ? 2 : 1; }
+__host__ __device__ constexpr int tg_lds_bytes(int most, int occ) { return (160 * 1024 / occ - 128 * most - 256) / 1024 * 1024; }
+__host__ __device__ constexpr int tg_depth(int rt, bool any, int lds) {
+  const int fit = lds / tg_slot_bytes(rt, any);
   return fit < 7 ? fit : 7;
 }
 // floats of a K split's partial tile
 __host__ __device__ constexpr size_t tg_part_floats(int rt) { return (size_t)rt * 16 * 256; }
 // X fragments in flight: a divisor of the 2 RT fragments of a stage
 __host__ __device__ constexpr int tg_ring(int rt) {
-  return 2 * rt % 8 == 0 ? 8 : 2 * rt % 7 == 0 ? 7 : 2 * rt % 6 == 0 ? 6 : 2 * rt % 5 == 0 ? 5 : rt;
+  return rt == 2 || rt == 8 ? 4 : rt == 3 ? 3 : 2 * rt % 8 == 0 ? 8 : 2 * rt % 7 == 0 ? 7 : 2 * rt % 6 == 0 ? 6 : 2 * rt % 5 == 0 ? 5 : rt;
 }
 
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -67,19 +99,39 @@ __device__ __forceinline__ T lds_read(uint32_t a) {
 // them apart.  The waits are the kernel's own (tg_wait_and_barrier).
 // acc += a * b, then 16 bytes a lane from rsrc into LDS at lds + 16 * lane; the MFMA is the wait state between
 // the write of m0 and the load that reads it.
+// ACC: where the accumulator is.
+enum { IN_AGPR, IN_VGPR, NEW_VGPR };      // accumulation registers, vector registers, the same with nothing in it yet
+#define TG_MFMA "v_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\t"
+#define TG_MFMA_NEW "v_mfma_f32_16x16x32_f16 %0, %1, %2, 0\n\t"
+#define TG_ASM(BEFORE, AFTER, ...)                                                                                   \
+  do {                                                                                                               \
+    if constexpr (ACC == NEW_VGPR) asm volatile(BEFORE TG_MFMA_NEW AFTER : "=&v"(c) : "v"(a), "v"(b), __VA_ARGS__ : "memory"); \
+    else if constexpr (ACC == IN_VGPR) asm volatile(BEFORE TG_MFMA AFTER : "+v"(c) : "v"(a), "v"(b), __VA_ARGS__ : "memory");  \
+    else asm volatile(BEFORE TG_MFMA AFTER : "+a"(c) : "v"(a), "v"(b), __VA_ARGS__ : "memory");                      \
+  } while (0)
+template <int ACC>
 __device__ __forceinline__ void tg_mfma(f4& c, u4v a, h8 b) {
-  asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  if constexpr (ACC == NEW_VGPR) asm volatile(TG_MFMA_NEW : "=&v"(c) : "v"(a), "v"(b));
+  else if constexpr (ACC == IN_VGPR) asm volatile(TG_MFMA : "+v"(c) : "v"(a), "v"(b));
+  else asm volatile(TG_MFMA : "+a"(c) : "v"(a), "v"(b));
 }
+template <int ACC>
 __device__ __forceinline__ void tg_mfma_load(f4& c, u4v a, h8 b, uint32_t lds, u4v rsrc, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\tbuffer_load_dwordx4 %4, %5, %6 offen lds"
-               : "+a"(c) : "v"(a), "v"(b), "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+  TG_ASM("s_mov_b32 m0, %3\n\t", "buffer_load_dwordx4 %4, %5, %6 offen lds", "s"(lds), "v"(voff), "s"(rsrc), "s"(soff));
 }
 // ... of the lanes in `mask` only (every lane is active around it)
+template <int ACC>
 __device__ __forceinline__ void tg_mfma_load_some(f4& c, u4v a, h8 b, uint32_t lds, u4v rsrc, uint32_t voff, uint64_t mask) {
-  asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\ts_mov_b64 exec, %6\n\t"
-               "buffer_load_dwordx4 %4, %5, 0 offen lds\n\ts_mov_b64 exec, -1"
-               : "+a"(c) : "v"(a), "v"(b), "s"(lds), "v"(voff), "s"(rsrc), "s"(mask) : "memory");
+  TG_ASM("s_mov_b32 m0, %3\n\t", "s_mov_b64 exec, %6\n\tbuffer_load_dwordx4 %4, %5, 0 offen lds\n\ts_mov_b64 exec, -1",
+         "s"(lds), "v"(voff), "s"(rsrc), "s"(mask));
 }
+// ... from one address per lane
+template <int ACC>
+__device__ __forceinline__ void tg_mfma_load_at(f4& c, u4v a, h8 b, uint32_t lds, uint64_t addr, uint64_t mask) {
+  TG_ASM("s_mov_b32 m0, %3\n\t", "s_mov_b64 exec, %5\n\tglobal_load_lds_dwordx4 %4, off\n\ts_mov_b64 exec, -1", "s"(lds), "v"(addr),
+         "s"(mask));
+}
+#undef TG_ASM
 __device__ __forceinline__ void tg_load(uint32_t lds, u4v rsrc, uint32_t voff, uint32_t soff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
@@ -87,12 +139,6 @@ __device__ __forceinline__ void tg_load(uint32_t lds, u4v rsrc, uint32_t voff, u
 __device__ __forceinline__ void tg_load_some(uint32_t lds, u4v rsrc, uint32_t voff, uint64_t mask) {
   asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n\ts_mov_b64 exec, -1"
                :: "s"(lds), "v"(voff), "s"(rsrc), "s"(mask) : "memory");
-}
-// ... from one address per lane
-__device__ __forceinline__ void tg_mfma_load_at(f4& c, u4v a, h8 b, uint32_t lds, uint64_t addr, uint64_t mask) {
-  asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\ts_mov_b64 exec, %5\n\t"
-               "global_load_lds_dwordx4 %4, off\n\ts_mov_b64 exec, -1"
-               : "+a"(c) : "v"(a), "v"(b), "s"(lds), "v"(addr), "s"(mask) : "memory");
 }
 __device__ __forceinline__ void tg_load_at(uint32_t lds, uint64_t addr, uint64_t mask) {
   asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b64 exec, -1"
@@ -111,17 +157,28 @@ __device__ __forceinline__ void tg_wait_and_barrier() {
 
 // RT: 16-row tiles of the workgroup tile.  ANY = false: G a multiple of 64 (a stage lies in one group) and N of 32;
 // ANY = true: also G a power of two from 8 on, and any N.
-template <int RT, bool ANY, bool GROUPED>
-__device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, const int n0, const int kb, const int ke,
-                                         float* const part, const int e, const uint32_t smem) {
-  constexpr int D = tg_depth(RT, ANY);
+// GROUPED: rows are slots of one expert e, s_sid the slot of each row (n_slots or more: none), s_tw its output weight.
+// ACT (grouped): the matrix is [gate | up]; the tile is 128 gate columns from n0 on and their up columns, and
+// writes silu(gate) * up.
+// SCALE32 = stages of a group (1 or 2, 0: off): weights enter the product as the integers w - z, and a group's sum is
+// scaled in fp32 when the group ends -- the skinny kernel's precision, for tiles that take its place.  The group's sum and the
+// total are both in vector registers, so that tiles are at most 64 rows high; the scaling is dealt out over the next
+// group's first k-step.
+template <int RT, int D, bool ANY, bool GROUPED, bool ACT, int SCALE32 = 0>
+__device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, const int n0, const int kb, const int ke,
+                                         float* const part, const int e, const uint32_t smem, const int* const s_sid,
+                                         const float* const s_tw) {
   constexpr int XB = tg_x_bytes(RT), SLOT = tg_slot_bytes(RT, ANY), PW = tg_param_bytes(ANY);
   constexpr int ZO = ANY ? 1024 : 128;        // zero points behind the scales
   constexpr int XL = (RT + 1) / 2;            // X loads of a wave and stage
   constexpr int NL = XL + (ANY ? 4 : 3);      // all loads: weights (2), group parameters, X
   constexpr int XF = tg_ring(RT);
   constexpr int NP = 4 * RT;                  // MFMAs of a k-step
-  static_assert(D >= 3 && (D - 2) * NL < 64, "");
+  // row tiles with their accumulators in the accumulation registers: not the whole file, or the compiler moves some of them
+  // at the loop's edges, where it does not know when an asm statement's result is ready
+  constexpr int AG = SCALE32 ? 0 : RT < 14 ? RT : 14;
+  static_assert(!SCALE32 || (!ANY && SCALE32 <= 2), "");
+  static_assert(D >= 3 && (D - 2) * NL < 64 && (D == 3 ? NP - 2 : 2 * NP - 4) >= NL, "every load has an MFMA of its own");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -141,7 +198,7 @@ __device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, 
     const int r = 8 * idx + (lane >> 3);
     int gr;
     if (GROUPED) {
-      const int sid = p.sorted_ids[m0 + r];
+      const int sid = s_sid[r];
       gr = sid < p.n_slots ? sid / p.a_row_div : 0;
     } else {
       gr = min(m0 + r, p.M - 1);
@@ -154,7 +211,9 @@ __device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, 
     return (uint32_t)idx * 1024u;
   };
   const uint32_t row_w = (uint32_t)p.ldw * 4u;
-  const int w0 = n0 / 8;
+  // first packed column of the wave's half h (four words each)
+  const int w0 = n0 / 8, up = ACT ? p.NW / 2 : 0;
+  auto word = [&](int wv, int h) __attribute__((always_inline)) { return ACT ? w0 + 4 * wv + h * up : w0 + 8 * wv + 4 * h; };
   // group parameters: the wave's eight packed columns are 128 bytes of scales and 32 of zero points a group
   const int gps = ANY ? max(64 / p.G, 1) : 1;         // groups of a stage
   const int spg = ANY ? max(p.G / 64, 1) : p.G / 64;  // stages of a group
@@ -164,10 +223,11 @@ __device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, 
   uint64_t p_addr;
   uint32_t p_step;
   {
-    int wc = w0 + 4 * ((lane & 7) ^ (2 * wave));
+    const int lc = (lane & 7) ^ (2 * wave);
+    int wc = word(lc >> 1, lc & 1);
     if (wc >= p.NW) wc = 0;
     w_voff = (uint32_t)((8 * wave + (lane >> 3)) * p.ldw + wc) * 4u;
-    int sw = w0 + 8 * wave + (lane & 7), zw = w0 + 8 * wave + 4 * (lane & 1);
+    int sw = word(wave, (lane >> 2) & 1) + (lane & 3), zw = word(wave, lane & 1);
     if (sw >= p.NW) sw = 0;
     if (zw >= p.NW) zw = 0;
     s_voff = (uint32_t)((lane >> 3) * p.N + 8 * sw) * 2u;       // ANY: lane = (group, word) ...
@@ -194,7 +254,8 @@ __device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, 
   const uint32_t sel_w = (fi & 1) ? 0x07060302u : 0x05040100u;
   const uint32_t sel_s = (fi & 1) ? 0x03020302u : 0x01000100u;
 
-  f4 acc[4][RT];
+  f4 acc[4][RT], part_acc[4][SCALE32 ? RT : 1];       // totals; SCALE32: sums of the current group
+  u4v gs[2] = {u4v{0u, 0u, 0u, 0u}, u4v{0u, 0u, 0u, 0u}};    // SCALE32: scales of the lane's 16 columns, last group
   NibbleMasks nm;
   nm.init();
 
@@ -205,7 +266,7 @@ __device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, 
   h8 xf[XF];
   auto read_params = [&](uint32_t slot, int ks) __attribute__((always_inline)) {
     zraw = lds_read<uint32_t>(slot + pz_off[ANY ? ks : 0]);
-    sraw = lds_read<u4v>(slot + ps_off[ANY ? ks : 0]);
+    if constexpr (!SCALE32) sraw = lds_read<u4v>(slot + ps_off[ANY ? ks : 0]);
   };
   auto expand = [&]() __attribute__((always_inline)) {
     const uint32_t za = __builtin_amdgcn_perm(zraw, zraw, sel_s), zb = za >> 8;
@@ -213,15 +274,23 @@ __device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, 
     zz[1] = (za & nm.hi) | MAGIC_HI;
     zz[2] = (zb & nm.lo) | MAGIC_LO;
     zz[3] = (zb & nm.hi) | MAGIC_HI;
+    if constexpr (!SCALE32)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) ss[j] = __builtin_amdgcn_perm(sraw[j], sraw[j], sel_s);
+      for (int j = 0; j < 4; ++j) ss[j] = __builtin_amdgcn_perm(sraw[j], sraw[j], sel_s);
+  };
+  // SCALE32: tile (j, im) of the last group, scaled, into the total
+  auto flush = [&](int j, int im) __attribute__((always_inline)) {
+    const h8 s[2] = {as_h8(gs[0]), as_h8(gs[1])};
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      acc[j][im][r] = __builtin_fmaf((float)s[r >> 1][2 * j + (r & 1)], part_acc[j][SCALE32 ? im : 0][r], acc[j][im][r]);
   };
   auto read_words = [&](int set, uint32_t fw, int ks, int rp) __attribute__((always_inline)) {
     wd[set][2 * rp] = lds_read<uint32_t>(fw + ks * 4096 + rp * 256);
     wd[set][2 * rp + 1] = lds_read<uint32_t>(fw + ks * 4096 + rp * 256 + 128);
   };
   uint32_t ua = 0, ub = 0, t1[16], t2[16];
-  // step i of 18: pair the halves of item i's rows, subtract item i - 1, scale item i - 2
+  // step i of 18: pair the halves of item i's rows, subtract item i - 1, scale item i - 2 (SCALE32: no scaling)
   auto unpack = [&](int i, int set, int w) __attribute__((always_inline)) {
     if (i < 16) {
       const int rp = i >> 2, j = i & 3;
@@ -233,7 +302,8 @@ __device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, 
       t1[i] = (j & 1) ? (u & nm.hi) | MAGIC_HI : (u & nm.lo) | MAGIC_LO;
     }
     if (i >= 1 && i < 17) t2[i - 1] = pk_sub(t1[i - 1], zz[(i - 1) & 3]);
-    if (i >= 2) wf[set][(i - 2) & 3][(i - 2) >> 2] = pk_mul(t2[i - 2], ss[(i - 2) & 3]);
+    if (SCALE32 && i >= 1 && i < 17) wf[set][(i - 1) & 3][(i - 1) >> 2] = t2[i - 1];
+    if (!SCALE32 && i >= 2) wf[set][(i - 2) & 3][(i - 2) >> 2] = pk_mul(t2[i - 2], ss[(i - 2) & 3]);
   };
   // The operands of the next k-step are complete, and the first MFMA reads them two wait states later.
   auto pin = [&](int set) __attribute__((always_inline)) {
@@ -261,17 +331,21 @@ __device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, 
   auto z_addr = [&]() __attribute__((always_inline)) { return z_voff + (uint32_t)(gl * p.NW) * 4u; };
   auto w_addr = [&](int i) __attribute__((always_inline)) { return w_voff + ((uint32_t)kl * 64u + 32u * i) * row_w; };
 
+  uint32_t cur = smem;      // LDS of the stage being multiplied
   // One k-step, KS its number in the stage, out of operand set KS; meanwhile the other set is unpacked for the
   // next k-step and the words after that are read.  cur / nxt: LDS of this stage and the next one.
-  auto kstep = [&](auto KS, const uint32_t (&xc)[2], const uint32_t (&xn)[2], uint32_t fwn, uint32_t nxt) __attribute__((always_inline)) {
+  // FIRST / LAST: the stage is its group's first / last one (SCALE32).
+  auto kstep = [&](auto KS, auto FIRST, auto LAST, const uint32_t (&xc)[2], const uint32_t (&xn)[2], uint32_t fwn, uint32_t nxt) __attribute__((always_inline)) {
     constexpr int ks = decltype(KS)::value;
-#pragma unroll
-    for (int im = 0; im < RT; ++im)
+    constexpr bool first = SCALE32 && decltype(FIRST)::value && ks == 0, last = !SCALE32 || decltype(LAST)::value;
+    auto row = [&](auto WHERE, int im) __attribute__((always_inline)) {
+      constexpr int ACC = decltype(WHERE)::value;
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
         // one operand changes from one MFMA to the next
         const int j = (im & 1) ? 3 - jj : jj, m = 4 * im + jj;
-        f4& a = acc[j][im];
+        f4& a = SCALE32 ? part_acc[j][SCALE32 ? im : 0] : acc[j][im];
+        if (first) flush(j, im);
         const u4v& w = wf[ks][j];
         const h8& x = xf[(ks * RT + im) % XF];
         // loads of a stage: dealt out over it (over its first k-step with a ring of three)
@@ -279,15 +353,17 @@ __device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, 
 #pragma unroll
         for (int i = 0; i < NL; ++i)
           if ((D == 3 ? 1 + i * (NP - 2) / NL : 1 + i * (2 * NP - 4) / NL) == ks * NP + m) ld = i;
-        if (ld < 0) tg_mfma(a, w, x);
-        else if (ld < 2) tg_mfma_load(a, w, x, fill + w_lds + ld * 4096, rw, w_addr(ld), 0);
-        else if (!ANY && ld == 2) tg_mfma_load_at(a, w, x, fill + p_lds, p_addr, 0x3ffull);
-        else if (ANY && ld == 2) tg_mfma_load_some(a, w, x, fill + p_lds, rs, s_addr(), s_mask);
-        else if (ANY && ld == 3) tg_mfma_load_some(a, w, x, fill + p_lds + ZO, rz, z_addr(), z_mask);
-        else tg_mfma_load(a, w, x, fill + x_lds(ld - (NL - XL)), rx, x_voff[ld < NL - XL ? 0 : ld - (NL - XL)], (uint32_t)kl * 128u);
+        if (ld < 0) tg_mfma<ACC>(a, w, x);
+        else if (ld < 2) tg_mfma_load<ACC>(a, w, x, fill + w_lds + ld * 4096, rw, w_addr(ld), 0);
+        else if (!ANY && ld == 2) tg_mfma_load_at<ACC>(a, w, x, fill + p_lds, p_addr, 0x3ffull);
+        else if (ANY && ld == 2) tg_mfma_load_some<ACC>(a, w, x, fill + p_lds, rs, s_addr(), s_mask);
+        else if (ANY && ld == 3) tg_mfma_load_some<ACC>(a, w, x, fill + p_lds + ZO, rz, z_addr(), z_mask);
+        else tg_mfma_load<ACC>(a, w, x, fill + x_lds(ld - (NL - XL)), rx, x_voff[ld < NL - XL ? 0 : ld - (NL - XL)], (uint32_t)kl * 128u);
         __builtin_amdgcn_sched_barrier(0);
-        if (m == 0 && (ANY || ks == 1)) expand();
-        if (m == 1 && (ANY || ks == 0)) read_params(nxt, ks);
+        // parameters of the next stage; SCALE32: of the next group, and the scales of the one that ends
+        if (last && m == 0 && (ANY || ks == 1)) expand();
+        if (last && m == 1 && (ANY || ks == 0)) read_params(nxt, ks);
+        if (SCALE32 && last && ks == 1 && (m == 1 || m == 2)) gs[m - 1] = lds_read<u4v>(cur + p_lds + 32 * fq + 16 * (m - 1));
 #pragma unroll
         for (int i = 18 * m / NP; i < 18 * (m + 1) / NP; ++i) unpack(i, ks ^ 1, ks ^ 1);
         if (m < 4) read_words(ks, fwn, ks, m);
@@ -298,6 +374,11 @@ __device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, 
         }
         __builtin_amdgcn_sched_barrier(0);
       }
+    };
+#pragma unroll
+    for (int im = 0; im < AG; ++im) row(std::integral_constant<int, IN_AGPR>{}, im);
+#pragma unroll
+    for (int im = AG; im < RT; ++im) row(std::integral_constant<int, first ? NEW_VGPR : IN_VGPR>{}, im);
     pin(ks ^ 1);
   };
   using I0 = std::integral_constant<int, 0>;
@@ -325,8 +406,11 @@ __device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, 
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %1, 0" : "=a"(acc[j][i]) : "v"(zero));
-  uint32_t cur = smem;
+    for (int j = 0; j < 4; ++j) {
+      if (i < AG) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %1, 0" : "=a"(acc[j][i]) : "v"(zero));
+      else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %1, 0" : "=v"(acc[j][i]) : "v"(zero));
+      if constexpr (SCALE32 != 0) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %1, 0" : "=v"(part_acc[j][i]) : "v"(zero));
+    }
   uint32_t xc[2] = {cur + fx_off[0], cur + fx_off[1]};
   tg_wait_and_barrier<(D - 2) * NL>();
 #pragma unroll
@@ -343,7 +427,7 @@ __device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, 
   for (int i = 0; i < 18; ++i) unpack(i, 0, 0);
   pin(0);
 
-  auto stage = [&]() __attribute__((always_inline)) {
+  auto stage = [&](auto FIRST, auto LAST) __attribute__((always_inline)) {
     // the next stage has landed (own loads; the barrier extends that to every wave's) and every wave has read
     // the last one, whose slot takes the stage D - 1 ahead
     tg_wait_and_barrier<(D - 3) * NL>();
@@ -354,65 +438,84 @@ __device__ __forceinline__ void awq_tile(const MfmaGemmParams& p, const int m0, 
     uint32_t fwn = nxt + fw_off;
     // (opaque: the reads' offsets stay in their offset fields)
     asm volatile("" : "+v"(xn[0]), "+v"(xn[1]), "+v"(fwn));
-    kstep(I0{}, xc, xn, fwn, nxt);
-    kstep(I1{}, xc, xn, fwn, nxt);
+    kstep(I0{}, FIRST, LAST, xc, xn, fwn, nxt);
+    kstep(I1{}, FIRST, LAST, xc, xn, fwn, nxt);
     next_load();
     cur = nxt;
     xc[0] = xn[0];
     xc[1] = xn[1];
   };
   int n = ke - kb;
+  constexpr std::bool_constant<SCALE32 != 2> each{};      // SCALE32 = 2: an even number of stages, two a group
   for (; n > 1; n -= 2) {
-    stage();
-    stage();
+    stage(std::true_type{}, each);
+    stage(each, std::true_type{});
   }
-  if (n) stage();
+  if (!SCALE32 && n) stage(std::true_type{}, std::true_type{});
   // no load may still be writing this workgroup's LDS when it ends; the last MFMAs' results are in their registers
   asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
 
   // The accumulators of one row of tiles at a time leave their registers behind this statement (moved all at once, ahead
   // of the wait above, some of them would be read too early or spilled).
   auto settle = [&](int im) __attribute__((always_inline)) {
-    asm volatile("" : "+a"(acc[0][im]), "+a"(acc[1][im]), "+a"(acc[2][im]), "+a"(acc[3][im]));
+    if constexpr (SCALE32 != 0) {
+      asm volatile("" : "+v"(part_acc[0][im]), "+v"(part_acc[1][im]), "+v"(part_acc[2][im]), "+v"(part_acc[3][im]));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) flush(j, im);
+    } else if (im < AG) asm volatile("" : "+a"(acc[0][im]), "+a"(acc[1][im]), "+a"(acc[2][im]), "+a"(acc[3][im]));
+    else asm volatile("" : "+v"(acc[0][im]), "+v"(acc[1][im]), "+v"(acc[2][im]), "+v"(acc[3][im]));
   };
-  if (part) {
-#pragma unroll
-    for (int im = 0; im < RT; ++im) {
-      settle(im);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) *reinterpret_cast<f4*>(part + ((size_t)(im * 4 + j) * 256 + tid) * 4) = acc[j][im];
-    }
-    return;
-  }
-  const int col = n0 + 64 * wave + 16 * fq;
+  const int col = ACT ? n0 + 32 * wave + 16 * (fq & 1) + 8 * (fq >> 1) : n0 + 64 * wave + 16 * fq;
 #pragma unroll
   for (int im = 0; im < RT; ++im) {
     settle(im);
+    if (!GROUPED && part) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) *reinterpret_cast<f4*>(part + ((size_t)(im * 4 + j) * 256 + tid) * 4) = acc[j][im];
+      continue;
+    }
     int row = m0 + 16 * im + fi;
     float tw = 1.f;
-    bool ok;
+    bool ok = row < p.M;
     if (GROUPED) {
-      row = p.sorted_ids[row];
+      row = s_sid[16 * im + fi];
       ok = row < p.n_slots;
-      tw = ok && p.topk_w ? p.topk_w[row] : 1.f;
-    } else {
-      ok = row < p.M;
+      tw = s_tw[16 * im + fi];
     }
+    h8 o[2];
 #pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
-      h8 o;
+    for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-      for (int t = 0; t < 8; ++t) o[t] = (half_t)(acc[t >> 1][im][2 * hf + (t & 1)] * tw);
-      if (ok && col + 8 * hf < p.N) *reinterpret_cast<h8*>(p.y + (size_t)row * p.N + col + 8 * hf) = o;
+      for (int t = 0; t < 8; ++t) o[hf][t] = (half_t)(acc[t >> 1][im][2 * hf + (t & 1)] * tw);
+    if constexpr (ACT) {
+      // lanes below 32 hold 16 gate columns, their partners the same up columns: trade halves, then each has both
+      // of eight columns
+      u4v g = as_u4(o[0]), u = as_u4(o[1]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const auto s = __builtin_amdgcn_permlane32_swap(g[i], u[i], false, false);
+        g[i] = s[0];
+        u[i] = s[1];
+      }
+      const h8 gh = as_h8(g), uh = as_h8(u);
+      h8 a;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) a[t] = silu_mul(gh[t], uh[t]);
+      if (ok && col < p.N / 2) *reinterpret_cast<h8*>(p.y + (size_t)row * (p.N / 2) + col) = a;
+    } else {
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+        if (ok && col + 8 * hf < p.N) *reinterpret_cast<h8*>(p.y + (size_t)row * p.N + col + 8 * hf) = o[hf];
     }
   }
 }
 #endif  // __HIP_DEVICE_COMPILE__
 
 template <int RT, bool ANY>
-__global__ __launch_bounds__(256, tg_occupancy(RT)) void awq_gemm_tile_kernel(const MfmaGemmParams p) {
+__global__ __launch_bounds__(256, tg_occupancy(RT, ANY)) void awq_gemm_tile_kernel(const TileGemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  __shared__ __align__(1024) unsigned char smem[tg_depth(RT, ANY) * tg_slot_bytes(RT, ANY)];
+  constexpr int D = tg_depth(RT, ANY, tg_lds_bytes(RT, tg_occupancy(RT, ANY)));
+  __shared__ __align__(1024) unsigned char smem[D * tg_slot_bytes(RT, ANY)];
   const int id = blockIdx.x;
   const int KT = p.K / 64;
   int nid = 0, kb = 0, ke = KT;
@@ -433,12 +536,89 @@ __global__ __launch_bounds__(256, tg_occupancy(RT)) void awq_gemm_tile_kernel(co
   const int gm = min(p.mt - first_m, PF_GROUP_M);
   const int mt_i = first_m + (nid % gsize) % gm;
   const int nt_i = (nid % gsize) / gm;
-  awq_tile<RT, ANY, false>(p, mt_i * (16 * RT), nt_i * 256, kb, ke, part, 0, (uint32_t)(uintptr_t)(lds_byte*)smem);
+  awq_tile<RT, D, ANY, false, false>(p, mt_i * (16 * RT), nt_i * 256, kb, ke, part, 0, (uint32_t)(uintptr_t)(lds_byte*)smem,
+                                     nullptr, nullptr);
+#endif
+}
+
+// Expert-grouped launch.  The sorted slots come in blocks of one expert each (moe_align).
+// Without p.runs a tile is a block, of 64 or 128 slots, or half of one of 256.  With it (SCALE32) blocks are of 16 slots, and
+// a tile is up to TG_RUN consecutive ones of one expert (a list made by the align kernels), so that an expert's weights are
+// unpacked once per tile and not per block.
+//
+// A workgroup takes the lowest tile that holds its real slots: its cost follows the rows, and an expert's run often
+// ends in a few dozen.
+//
+// 128 slots and two workgroups per CU: K is short (12 and 32 stages on experts of 2048 x 768), so that a tile's start and its
+// output are a quarter of its time, and with tiles of 256 slots, one workgroup per CU, nothing runs beside them.
+// Whole block of 8192 / 4096 / 1536 tokens on 128 such experts, top-8: 256 slots 743 / 437 / 217 us, 128 slots
+// 709 / 399 / 184, 48 slots and three workgroups 907 / 485 / 226.
+//
+// The live tiles (their number is on the device only) are dealt to the eight XCDs in contiguous ranges, tile-major, so
+// that the column tiles of a block share its gathered X rows and the blocks of an expert its weights through one L2; with
+// few experts the ranges are uneven in rows and launch order is better.
+constexpr int TG_ROWS = 128;   // slots of a tile at most
+constexpr int TG_RUN = 4;      // 16-slot blocks of a SCALE32 tile at most
+template <bool ANY, bool ACT, int SCALE32>
+__global__ __launch_bounds__(256, tg_occupancy(TG_ROWS / 16, ANY)) void awq_gemm_tile_grouped_kernel(const TileGemmParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int ROWS = SCALE32 ? 16 * TG_RUN : TG_ROWS, LDS = tg_lds_bytes(TG_ROWS / 16, tg_occupancy(TG_ROWS / 16, ANY));
+  __shared__ __align__(1024) unsigned char smem[LDS];
+  __shared__ int s_sid[ROWS];
+  __shared__ float s_tw[ROWS];
+  __shared__ int s_rows[2];
+  const int tid = threadIdx.x;
+  constexpr bool runs = SCALE32 != 0;
+  const int tile_rows = min(p.block, ROWS);
+  const int live = min((runs ? *p.n_live : *p.n_live / tile_rows) * p.nt, p.total);
+  int nid = blockIdx.x;
+  if (!p.in_order) {
+    const int per = (live + 7) >> 3;
+    nid = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per) return;
+  }
+  if (nid >= live) return;
+  const int t = nid / p.nt;
+  int first = t * tile_rows, most = tile_rows;
+  if (runs) {
+    const int run = p.runs[t];
+    first = (run >> 5) * 16;
+    most = (run & 31) * 16;
+  }
+  // the expert id is on its way while the slots are staged: its weights' addresses wait for it
+  const int e = p.expert_ids[first / p.block];
+  if (tid < ROWS) {
+    const int sid = tid < most ? p.sorted_ids[first + tid] : p.n_slots;
+    const bool real = sid < p.n_slots;
+    s_sid[tid] = sid;
+    s_tw[tid] = (real && p.topk_w) ? p.topk_w[sid] : 1.f;
+    const unsigned long long mask = __ballot(real);     // a wave's 64 slots
+    if ((tid & 63) == 0) s_rows[tid >> 6] = mask ? tid + 64 - __clzll(mask) : 0;
+  }
+  __syncthreads();
+  // the last real slot's row + 1: rows behind it are padding
+  const int rows = __builtin_amdgcn_readfirstlane(ROWS > 64 ? max(s_rows[0], s_rows[1]) : s_rows[0]);
+  const int eu = __builtin_amdgcn_readfirstlane(e);
+  const int n0 = (nid % p.nt) * (ACT ? TG_COLS / 2 : TG_COLS);
+  const uint32_t lds = (uint32_t)(uintptr_t)(lds_byte*)smem;
+  auto tile = [&](auto R) __attribute__((always_inline)) {
+    constexpr int RT = decltype(R)::value;
+    awq_tile<RT, tg_depth(RT, ANY, LDS), ANY, true, ACT, SCALE32>(p, 0, n0, 0, p.K / 64, nullptr, eu, lds, s_sid, s_tw);
+  };
+  if constexpr (!SCALE32) {
+    if (rows > 112) return tile(std::integral_constant<int, 8>{});
+    if (rows > 96) return tile(std::integral_constant<int, 7>{});
+    if (rows > 80) return tile(std::integral_constant<int, 6>{});
+    if (rows > 64) return tile(std::integral_constant<int, 5>{});
+  }
+  if (rows > 48) tile(std::integral_constant<int, 4>{});
+  else if (rows > 32) tile(std::integral_constant<int, 3>{});
+  else if (rows > 0) tile(std::integral_constant<int, 2>{});
 #endif
 }
 
 template <int RT>
-__global__ __launch_bounds__(256) void awq_gemm_tile_reduce_kernel(const MfmaGemmParams p) {
+__global__ __launch_bounds__(256) void awq_gemm_tile_reduce_kernel(const TileGemmParams p) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, fi = lane & 15, fq = lane >> 4;
   const int tl = blockIdx.x / RT, im = blockIdx.x % RT;
   const int nid = p.dp_tiles + tl;

@@ -132,6 +132,50 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const float* __restrict__
   moe_topk_token<PER, SIGMOID>(logits, bias, t, E, topk, renorm, scale, ids, wts);
 }
 
+// Tiles of the expert GEMMs made of up to MOE_RUN consecutive 16-slot blocks of one expert: runs[0] tiles, then
+// first block * 32 + blocks of each (runs null: none wanted).
+constexpr int MOE_RUN = 4;
+
+// Exclusive prefix sum of padded[] by one wave, a lane owning a contiguous range of experts; and the tiles of
+// each expert's run, as even as whole blocks allow.
+__device__ __forceinline__ void moe_starts(const int* padded, int* start, int E, int lane, int* s_total,
+                                           int* __restrict__ npp, int* __restrict__ runs) {
+  const int per = (E + 63) / 64;
+  int local = 0, tiles = 0;
+  for (int k = 0; k < per; ++k) {
+    const int e = lane * per + k;
+    if (e < E) {
+      local += padded[e];
+      if (runs) tiles += (padded[e] / 16 + MOE_RUN - 1) / MOE_RUN;
+    }
+  }
+  int incl = local, tincl = tiles;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(incl, o), w = __shfl_up(tincl, o);
+    if (lane >= o) { incl += v; tincl += w; }
+  }
+  int pos = incl - local, tpos = tincl - tiles;
+  for (int k = 0; k < per; ++k) {
+    const int e = lane * per + k;
+    if (e >= E) break;
+    start[e] = pos;
+    if (runs) {
+      const int b = padded[e] / 16, n = (b + MOE_RUN - 1) / MOE_RUN;
+      for (int i = 0; i < n; ++i) {
+        const int b0 = b * i / n, b1 = b * (i + 1) / n;
+        runs[1 + tpos++] = (pos / 16 + b0) * 32 + (b1 - b0);
+      }
+    }
+    pos += padded[e];
+  }
+  if (lane == 63) {
+    *s_total = incl;
+    npp[0] = incl;
+    if (runs) runs[0] = tincl;
+  }
+}
+
 // Single workgroup of 16 waves.  Dynamic LDS: cnt[16][E] + padded[E] + start[E].
 // Wave w owns the contiguous slice [w*seg, (w+1)*seg) of the flat slot list, so placing
 // slices in wave order and slots in index order inside a slice gives a stable sort.  Inside a
@@ -150,7 +194,8 @@ __device__ __forceinline__ void moe_align_block(const int* __restrict__ ids, int
                                                 int cap, int* __restrict__ sorted,
                                                 int* __restrict__ expert_ids, int* __restrict__ npp,
                                                 int* sm, int s0 = 0, int s1 = 0,
-                                                int* __restrict__ block_tab = nullptr) {
+                                                int* __restrict__ block_tab = nullptr,
+                                                int* __restrict__ runs = nullptr) {
   constexpr int NWV = MOE_ALIGN_WAVES;
   int* cnt = sm;               // [NWV][E], later the running write position
   int* padded = sm + NWV * E;  // [E]
@@ -215,26 +260,7 @@ __device__ __forceinline__ void moe_align_block(const int* __restrict__ ids, int
     padded[e] = (tot + tile_m - 1) / tile_m * tile_m;
   }
   __syncthreads();
-  if (wave == 0) {   // exclusive prefix sum of padded[] by one wave: lane owns a contiguous run
-    const int per = (E + 63) / 64;
-    int local = 0;
-    for (int k = 0; k < per; ++k) {
-      const int e = lane * per + k;
-      if (e < E) local += padded[e];
-    }
-    int incl = local;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(incl, o);
-      if (lane >= o) incl += v;
-    }
-    int pos = incl - local;
-    for (int k = 0; k < per; ++k) {
-      const int e = lane * per + k;
-      if (e < E) { start[e] = pos; pos += padded[e]; }
-    }
-    if (lane == 63) { s_total = incl; npp[0] = incl; }
-  }
+  if (wave == 0) moe_starts(padded, start, E, lane, &s_total, npp, runs);
   __syncthreads();
   const int total = s_total;
   for (int e = tid; e < E; e += 1024) {
@@ -290,9 +316,9 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
                                                          int tile_m, int cap,
                                                          int* __restrict__ sorted,
                                                          int* __restrict__ expert_ids,
-                                                         int* __restrict__ npp) {
+                                                         int* __restrict__ npp, int* __restrict__ runs) {
   extern __shared__ int sm[];
-  moe_align_block<0>(ids, n, E, tile_m, cap, sorted, expert_ids, npp, sm);
+  moe_align_block<0>(ids, n, E, tile_m, cap, sorted, expert_ids, npp, sm, 0, 0, nullptr, runs);
 }
 
 // Long slot lists: part b of gridDim.x parts covers slots [b * part, (b + 1) * part).
@@ -310,7 +336,7 @@ __global__ __launch_bounds__(1024) void moe_align_scan_kernel(int n, int E, int 
                                                               int* __restrict__ block_tab,
                                                               int* __restrict__ sorted,
                                                               int* __restrict__ expert_ids,
-                                                              int* __restrict__ npp) {
+                                                              int* __restrict__ npp, int* __restrict__ runs) {
   extern __shared__ int sm[];
   int* padded = sm;        // [E]
   int* start = sm + E;     // [E]
@@ -330,26 +356,7 @@ __global__ __launch_bounds__(1024) void moe_align_scan_kernel(int n, int E, int 
     padded[tid] = (tot + tile_m - 1) / tile_m * tile_m;
   }
   __syncthreads();
-  if (wave == 0) {
-    const int per = (E + 63) / 64;
-    int local = 0;
-    for (int k = 0; k < per; ++k) {
-      const int e = lane * per + k;
-      if (e < E) local += padded[e];
-    }
-    int incl = local;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(incl, o);
-      if (lane >= o) incl += v;
-    }
-    int pos = incl - local;
-    for (int k = 0; k < per; ++k) {
-      const int e = lane * per + k;
-      if (e < E) { start[e] = pos; pos += padded[e]; }
-    }
-    if (lane == 63) { s_total = incl; npp[0] = incl; }
-  }
+  if (wave == 0) moe_starts(padded, start, E, lane, &s_total, npp, runs);
   __syncthreads();
   const int total = s_total;
   if (tid < E) {
@@ -416,10 +423,7 @@ __global__ __launch_bounds__(256) void silu_and_mul_kernel(const half_t* __restr
   const h8 u = *reinterpret_cast<const h8*>(in + r * 2 * inter + inter + c);
   h8 o;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float gv = (float)g[i];
-    o[i] = (half_t)(gv / (1.f + __expf(-gv)) * (float)u[i]);
-  }
+  for (int i = 0; i < 8; ++i) o[i] = silu_mul(g[i], u[i]);
   *reinterpret_cast<h8*>(out + r * inter + c) = o;
 }
 

@@ -272,6 +272,62 @@ def test_moe_grouped_gemm_partly_filled_blocks_of_any_group(sba, gpu, bs):
             assert awq_ref.rel_frobenius(y[rows], awq_ref.gemm_wide(x[rows], qw[e], s[e], qz[e], G)) <= TOL, e
 
 
+TILE_EDGES = [1, 16, 17, 32, 33, 48, 0, 49, 64, 65, 80, 81, 96, 97, 112, 113, 128, 129, 177, 241, 257, 300]
+
+
+@pytest.mark.parametrize("E", [len(TILE_EDGES), 13])     # 16 experts or more: tiles dealt to the XCDs in ranges
+@pytest.mark.parametrize("bs,K,N,G", [
+    (64, 128, 256, 128), (128, 256, 264, 64), (256, 640, 512, 128), (256, 1280, 288, 128),   # 2 ... 20 stages of 64 k
+    (128, 256, 72, 32), (256, 384, 520, 384), (64, 256, 40, 64),      # groups and columns of the general form
+])
+def test_moe_grouped_gemm_at_the_tile_edges(sba, gpu, bs, K, N, G, E):
+    """The grouped kernel takes the lowest tile, in steps of 16 rows, that holds a block's slots (a block of 256 runs as
+    two): experts with slot counts on both sides of every step, against per-expert oracle products."""
+    counts = TILE_EDGES[:E] if bs < 256 else TILE_EDGES[-E:]
+    rng = np.random.default_rng(bs + K + E)
+    w, z = rng.integers(0, 16, (E, K, N)), rng.integers(0, 16, (E, K // G, N))
+    s = (rng.random((E, K // G, N)) * 0.019 + 0.001).astype(np.float16)
+    qw, qz = awq_ref.pack_awq(w), awq_ref.pack_awq(z)
+    ids = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int32)[:, None]
+    T = len(ids)
+    x = rng.normal(0, 1, (T, K)).astype(np.float16)
+    tw = rng.random((T, 1)).astype(np.float32)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)
+    sid, eid, npp = sba.moe_align_block_size(t(ids), bs, E)
+    out = torch.full((T + 1, N), float("nan"), dtype=torch.float16, device=gpu)
+    y = sba.moe_awq_gemm(t(x), t(qw), t(s), t(qz), sid, eid, npp, T, 1, topk_weights=t(tw), block_size=bs, out=out[:T])
+    y = y.cpu().numpy()
+    assert np.all(np.isfinite(y)) and bool(torch.isnan(out[T]).all())      # every slot row written, none behind them
+    for e in range(E):
+        tok = np.nonzero(ids[:, 0] == e)[0]
+        if tok.size:
+            ref = awq_ref.gemm_wide(x[tok], qw[e], s[e], qz[e], G) * tw[tok]
+            assert awq_ref.rel_frobenius(y[tok], ref) <= TOL, e
+
+
+@pytest.mark.parametrize("variant", [512, 1 << 16, 2 << 16, 3 << 16])    # 16-slot blocks in tiles of up to four; 64, 128, 256
+@pytest.mark.parametrize("H,I,G,E", [(256, 128, 128, 22), (384, 384, 64, 22), (1152, 256, 128, 13), (128, 640, 64, 13)])
+def test_fused_call_on_the_grouped_kernel_at_the_tile_edges(sba, gpu, variant, H, I, G, E):
+    """The one-call block with both expert GEMMs on the grouped kernel, the first writing silu(gate) * up itself, over
+    experts with slot counts on both sides of every tile step: against dense experts, and bit for bit against itself."""
+    counts = TILE_EDGES[:E]
+    T = sum(counts)
+    c = sba.workloads.make_moe_case(T, H, E, 1, I, G, seed=H + I).to(gpu)
+    own = torch.from_numpy(np.random.default_rng(T).permutation(np.repeat(np.arange(E), counts))).to(gpu)
+    c.logits.clamp_(-3, 3)
+    c.logits[torch.arange(T, device=gpu), own] = 8.0       # top-1 goes there
+    run = lambda v: sba.fused_moe_awq(c.x, c.w13, c.w2, c.logits, 1, True, _dev_variant=v)
+    y = run(variant).clone()
+    assert torch.equal(y.view(torch.int16), run(variant).view(torch.int16))
+    ref = _dense_expert_reference(sba, c, gpu, T, H, E, 1, I)
+    plain = run(2048).float()
+    for e in range(E):
+        r = own == e
+        if bool(r.any()):
+            assert float((y[r].float() - ref[r]).norm() / ref[r].norm()) <= TOL, e
+            assert float((y[r].float() - plain[r]).norm() / plain[r].norm()) <= TOL, e
+
+
 @pytest.mark.parametrize("T,H,E,topk,I,mfma", [(2048, 2048, 128, 8, 768, False), (1024, 1024, 8, 2, 2048, False),
                                                (4096, 512, 4, 2, 384, False),     # many rows per expert
                                                (640, 256, 4, 1, 1152, False),     # top-1
