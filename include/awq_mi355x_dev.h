@@ -62,7 +62,8 @@ enum {
   AWQMI_FORM_FUSED = 2,   /* awq_gemm_tile_kernel: weights unpacked per tile in registers */
   AWQMI_FORM_DENSE = 3,   /* awq_dequant_panel_kernel + awq_gemm_dense_kernel */
   AWQMI_FORM_GENERIC = 4, /* any-shape fallback */
-  AWQMI_FORM_MID = 5      /* awq_gemm_mid_kernel: 33 .. 64 rows in one pass */
+  AWQMI_FORM_MID = 5      /* 33 .. 64 rows of a large layer in one pass: awq_gemm_mid_kernel on the largest, else one
+                           * row of awq_gemm_tile_kernel's tiles */
 };
 int awqmi_dev_last_gemm_form(void);
 

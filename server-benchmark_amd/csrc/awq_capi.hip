@@ -227,28 +227,16 @@ int mid_pick_split(int K, int N) {
   return best;
 }
 
-// From 33 to 64 rows: awq_gemm_mid_kernel on the layers where it measured faster than the 64-row MFMA tile,
-// wherever the skinny kernel's shapes hold with two words per lane (its operands are addressed through
-// 32-bit buffers).  Both sides at 64 rows, G = 128 (us, weights from HBM, rows as the layer method keeps
-// them): 8192 x 59136 81 / 109, 3584 x 37888 36 / 42, 5120 x 27648 35 / 40, 29568 x 8192 49 / 59, 18944 x
-// 3584 28.8 / 35.0, 13824 x 5120 27.3 / 29.5, 8192 x 10240 27.7 / 28.6, 8192 x 8192 24.8 / 25.8.
-// Where the lines lie (1700 points: 19 values of K from 512 to 40960, N from 1024 to 79000, 33 and 64
-// rows, groups of 128, 64 and 32; the rule is within 6 % of the better kernel on all but a dozen of them, and
-// within 8 % on 330 further layers of random size and row count, where "every layer of 40 Mi weights" was up
-// to 34 % behind):
-//   - at least 2048 weight rows and 40 Mi weights: a wave's start and the four-way sum outweigh its one or
-//     two chunks (768 x 58368 19.4 / 13.5, 1536 x 28672 21.7 / 21.0), and the last round of workgroups
-//     full (2048 x 65792, 257 column blocks, 52 / 41: the MFMA kernel splits its last round in K);
-//   - always from 13312 weight rows on, and from 8192 on up to 20 column blocks: the MFMA tile's K split
-//     stops at eight workgroups (29568 x 1536 30 / 50, 11008 x 3840 25.8 / 26.7);
-//   - where the column blocks are a multiple of eight (the sum kernel then finds a block's partial tiles in
-//     the L2 of the XCD that wrote them) and the K ranges are even to within 1 / 8, at any such size:
-//     5120 x 8192 22.5 / 23.6 against 3584 x 11840 25.5 / 21.3, 5120 x 9824 26.9 / 23.0 without;
-//   - else by size: from 88 Mi weights, 72 Mi above 128 column blocks, which the MFMA kernel runs unsplit
-//     on part of the chip (2560 x 40960 29.5 / 31.3; 3072 x 20480, 60 Mi, 24.9 / 24.7).
-// Rows of qweight that are no whole 128-byte lines (every row piece then touches two) move the lines by about
-// 3000 weight rows and by 24 Mi weights; more than 48 rows, and groups of 32, cost about 4 % each and move
-// the size by 8 Mi, uneven K ranges by 16 Mi.
+// From 33 to 64 rows: the layers that count as the one-pass form, and the kernel they run on.
+// The lines of mid_pays were drawn where awq_gemm_mid_kernel beat the 64-row tile of the kernel that dequantised into
+// LDS (1700 points: 19 values of K from 512 to 40960, N from 1024 to 79000; from 40 Mi weights on 2048 rows, always from 13312 weight
+// rows on, elsewhere by size, by how even its K ranges are, and later where rows of qweight are no whole 128-byte lines).
+// Against awq_gemm_tile_kernel, whose tiles of 48 and 64 rows hold all rows of the call too, the mid kernel is faster on the
+// largest of them only: mid_beats_tile.  Both, mid / tile, at 40, 48 and 64 rows (us, weights from HBM, rows as the layer
+// method keeps them): 16512 x 43904 (691 Mi weights, G = 32) 148, 149, 152 / 150, 149, 215; 8192 x 59136 (462 Mi) 81, 78, 80 / 79, 78,
+// 85; 15360 x 22848 (334 Mi) 78, 76, 77 / 75, 76, 79; 7936 x 41792 (316 Mi) 75, 74, 75 / 67, 67, 70; 29568 x 8192 49, 48, 49 / 44,
+// 44, 49; 8192 x 10240 26.4, 26.1, 27.6 / 22, 22, 23; 8320 x 5120 23, 23, 24 / 17.9, 17.8, 18.4; 13312 x 5632 28, 27, 28 / 22, 22, 23.
+// On 34 layers of mid_pays below the line the tile is 14 % faster on average and 0.3 % slower at worst.
 constexpr long long MID_MIN_WEIGHTS = 40LL << 20;
 inline bool mid_shape(int M, int K, int N) {
   const int ncb = (N + 255) / 256;
@@ -268,6 +256,8 @@ inline bool mid_pays(int M, int K, int N, int G, int ldw) {
   if (N % 2048 == 0 && K >= 3072 && even) return mi >= (heavy == 2 ? 80 : 40);
   return mi >= (ncb > 128 ? 72 : 88) + (lines ? 0 : 24) + 8 * heavy + (even ? 0 : 16);
 }
+constexpr long long MID_KERNEL_WEIGHTS = 320LL << 20;
+inline bool mid_beats_tile(int K, int N) { return (long long)K * N >= MID_KERNEL_WEIGHTS; }
 inline bool mid_rows(int M, int K, int N, int G, int ldw) {
   return (mid_pays(M, K, N, G, ldw) || (variant_on(VAR_MID) && M > 32 && M <= MID_MAX_ROWS && N % 16 == 0)) &&
          gemv_tiled_ok(K, G) && (size_t)M * K * 2 < (1ull << 31) && (size_t)K * ldw * 4 < (1ull << 31) &&
@@ -331,7 +321,7 @@ inline size_t dense_panel_offset(size_t part_bytes) {
 // Fused kernel: height of its tile in 16-row steps and the K split of one launch.  Whole rounds of 256
 // tiles run one workgroup per tile; a last round that leaves CUs idle (and any launch that small) may be split
 // in K over `split` workgroups per tile, at least four stages of 64 k each.
-constexpr int TILE_RT[] = {4, 5, 6, 7, 8, 10, 12, 13, 14, 16};
+constexpr int TILE_RT[] = {3, 4, 5, 6, 7, 8, 10, 12, 13, 14, 16};
 struct TilePlan { int rt, dp_tiles, sk_tiles, sk_split; size_t part_bytes; };
 TilePlan tile_plan(int M, int K, int N, int rt, int split) {
   const int tiles = ((M + 16 * rt - 1) / (16 * rt)) * ((N + TG_COLS - 1) / TG_COLS), rem = tiles % 256;
@@ -342,7 +332,9 @@ TilePlan tile_plan(int M, int K, int N, int rt, int split) {
 // on a full chip and down to 0.79 of it on a nearly idle one (the clock), a tile 3.8 stages beside its own, a partial
 // last round counts as at least 0.88 of one, a K split 4.3 + 0.22 per part for its sum launch and 0.003 rt per
 // partial tile.  Fitted on 7800 timed launches (16 layer shapes from 1024 x 12288 to 8192 x 59136, 33 ... 2047 rows,
-// every height and up to five splits each): 0.6 % behind the best of them on average, 15 % at worst.
+// every height of 64 rows and more, up to five splits each): 0.6 % behind the best of them on average, 15 % at worst.  The same
+// price on 56 layers at 40, 48 and 64 rows with tiles of 48 as well: 1 % behind the best split of either height.  A price with
+// terms for two workgroups on a CU (and splits over 512) is no better: 1.3 % behind on average, 11 % slower than this pick at worst.
 TilePlan pick_tile(int M, int K, int N, size_t room) {
   const int KT = K / 64;
   TilePlan best{};
@@ -388,6 +380,7 @@ void launch_tile(const TileGemmParams& p, hipStream_t st) {
 }
 void launch_tile(int rt, const TileGemmParams& p, hipStream_t st) {
   switch (rt) {
+    case 3: return launch_tile<3>(p, st);
     case 4: return launch_tile<4>(p, st);
     case 5: return launch_tile<5>(p, st);
     case 6: return launch_tile<6>(p, st);
@@ -650,7 +643,8 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
   const bool mfma_ok = K % DG_BK == 0 && (((G & (G - 1)) == 0 && G >= 8) || G % 64 == 0) &&
                        mfma_slab_rows(M, K) > 0 && (size_t)K * ldw * 4 < (1ull << 32) &&
                        (size_t)(K / G) * N * 2 < (1ull << 32);
-  if (mid_rows(M, K, N, G, ldw)) {
+  const bool mid = mid_rows(M, K, N, G, ldw);
+  if (mid && (variant_on(VAR_MID) || mid_beats_tile(K, N))) {
     t_last_gemm_form = AWQMI_FORM_MID;
     MidGemmParams p{};
     p.x = xx; p.qw = qw; p.sc = sc; p.qz = qz; p.y = yy;
@@ -749,7 +743,7 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
         return launch_status();
       }
     }
-    t_last_gemm_form = AWQMI_FORM_FUSED;
+    t_last_gemm_form = mid ? AWQMI_FORM_MID : AWQMI_FORM_FUSED;
     // room for the partial tiles of a K split; without a workspace every tile runs on one workgroup
     const size_t room = workspace && aligned16(workspace) && workspace_bytes > AWQMI_WS_COUNTER_BYTES
                             ? workspace_bytes - AWQMI_WS_COUNTER_BYTES : 0;

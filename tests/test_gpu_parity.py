@@ -490,6 +490,25 @@ def test_fused_tile_heights(sba, gpu, variant, K, N, G):
         assert awq_ref.rel_frobenius(y1.cpu().numpy(), y) <= TOL
 
 
+@pytest.mark.parametrize("M", [33, 47, 48, 49])
+@pytest.mark.parametrize("K,N,G", [(64, 256, 64), (128, 8, 8), (192, 264, 32), (320, 288, 16), (448, 544, 64), (1152, 1000, 128),
+                                   (1600, 512, -1), (2304, 256, 192), (4096, 4112, 128)])
+def test_fused_tile_of_48_rows(sba, gpu, M, K, N, G):
+    """33 .. 48 rows run on a tile of 48, with a K split and (no workspace) without."""
+    from server_benchmark_amd import _lib
+    lib = _lib.load()
+    g = K if G <= 0 else G
+    sba.ops.get_workspace(gpu, 80 << 20)[65536:].fill_(255)
+    x, qw, s, qz = _np_case(M, K, N, g, seed=K + M)
+    y = _check_gemm(sba, gpu, x, qw, s, qz, g, 0, tag="tile 48")
+    assert lib.awqmi_dev_last_gemm_form() == _lib.FORM_FUSED
+    xd, qwd, sd, qzd = _dev(gpu, x, qw, s, qz)
+    y1 = torch.full((M, N), float("nan"), dtype=torch.float16, device=gpu)
+    assert lib.awqmi_gemm_f16(xd.data_ptr(), qwd.data_ptr(), sd.data_ptr(), qzd.data_ptr(), y1.data_ptr(), 0, 0, M, K, N, g, 0,
+                              torch.cuda.current_stream().cuda_stream) == 0
+    assert awq_ref.rel_frobenius(y1.cpu().numpy(), y) <= TOL
+
+
 @pytest.mark.parametrize("M,K,N", [(512, 1024, 1280), (300, 2048, 520), (2048, 512, 5120), (768, 1536, 8192 + 256)])
 def test_gemm_prefill_partial_rounds(sba, gpu, M, K, N):
     """Tile counts that are not a multiple of the CU count, ragged last row / column tiles;
