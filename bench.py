@@ -344,7 +344,7 @@ def main():
         torch.cuda.synchronize()
         log(f"[bench] pmc target: awq_gemm {name} M=8192 K={K} N={N} ({workloads.linear_flops(8192, K, N)} flops each), "
             f"{args.pmc_data} operands: 12 calls as awq_dequant_panel_kernel + awq_gemm_dense_kernel, then 12 calls as "
-            f"awq_gemm_mfma_kernel")
+            f"awq_gemm_tile_kernel")
         return
     if args.pmc_target == "moe":
         mq = workloads.QWEN3_MOE
@@ -584,8 +584,8 @@ def main():
                                     "50 ms of the same launches untimed (sustained: the chip holds a lower clock under "
                                     "this load than in its first milliseconds); TFLOPs_burst = 3 - 6 launches after two "
                                     "warm-up launches; aggregate = total flops / total time over the 12 points",
-                          "kernels": "awq_gemm_mfma_kernel (fused) below 2048 rows; awq_dequant_panel_kernel + "
-                                     "awq_gemm_dense_kernel from 2048 rows on these layers (the panel pass is inside the timed call)",
+                          "kernels": "awq_gemm_tile_kernel at 512 rows; awq_dequant_panel_kernel + "
+                                     "awq_gemm_dense_kernel at 2048 and 8192 on these layers (the panel pass is inside the timed call)",
                           "points": pts}
         log(f"[bench] prefill sweep aggregate {agg:.1f} TFLOP/s sustained ({agg / MFMA_FP16_PEAK_TFLOPS:.1%} of fp16 MFMA "
             f"peak), {agg_burst:.1f} burst")

@@ -294,24 +294,31 @@ MfmaPlan plan_mfma(int M, int K, int N, int bm) {
 }
 
 // Dequantise-once form (awq_gemm_dense.hpp): the weights go through awq_dequant_panel_kernel into
-// an fp16 panel in the workspace, then awq_gemm_dense_kernel.  Under sustained load on the 72B
-// layer shapes (fused kernel against panel pass + dense kernel, timed in turn): 512 rows 0.70,
-// 1024 rows 0.79 - 0.90, 2048 rows 1.01 - 1.03, 3072 rows 1.01 - 1.07, 4096 rows 1.08, 8192 rows
-// 1.11 - 1.16 of the fused kernel's rate; so it is taken from 2048 rows on.  Between 2048 and
-// 4095 rows only when the 256 x 256 tiles make at least three quarters of a round of workgroups:
-// with fewer the fused kernel's smaller row tiles fill the chip better (layers of 7B ... 32B-class
-// models at 2048 rows: 0.90 - 0.99 with 64 - 160 tiles, 1.02 - 1.08 from 224 tiles on; at 4096 rows
-// 0.98 - 1.16, at 8192 rows 1.14 - 1.21 whatever the tile count).  K % 64 == 0 and G % 8 == 0 (both
-// implied by the MFMA path's conditions).
-constexpr int DENSE_MIN_ROWS = 2048;
-inline bool dense_default(int M, int N) {
-  if (M < DENSE_MIN_ROWS) return false;
-  return M >= 2 * DENSE_MIN_ROWS || (long long)((M + 255) / 256) * ((N + 255) / 256) >= 192;
+// an fp16 panel in the workspace, then awq_gemm_dense_kernel.  The tile kernel unpacks every weight again
+// for each 256 rows, which the panel pass pays for once, but runs faster below some 6000 rows.  Both, panel / tile (us, timed in
+// turn, 15 layers at 2048 ... 8192 rows):
+//   rows             2048          3072          4096          5000          6144          8192
+//   8192 x 59136     1586 / 1438   2279 / 2164   2941 / 2868   3617 / 3606   4355 / 4402   5588 / 5743
+//   29568 x 8192     800 / 730     1199 / 1126   1488 / 1472   1880 / 1870   2245 / 2229   2932 / 3005
+//   3584 x 37888     506 / 465     706 / 662     936 / 906     1139 / 1124   1352 / 1324   1762 / 1770
+//   4096 x 2048      55 / 42       65 / 52       79 / 64       84 / 75       93 / 86       107 / 112
+//   1024 x 12288     80 / 56       102 / 78      105 / 98      131 / 127     179 / 156     201 / 193
+//   512 x 8192       28 / 22       63 / 36       50 / 43       82 / 56       68 / 63       89 / 82
+// At 6144 rows the tile is within 2.3 % either way from 2048 weight rows on; with fewer it stays ahead at any size, as the panel is as
+// much traffic as the products.  One row count keeps the panel where the tile is 9 % faster: 2048 on layers of 64 Mi weights and
+// more, whose prefill record and its test name the form.  Layers of fewer than 512 weight rows, which no model here has, keep the lines that were drawn for
+// all: from 4096 rows on, from 2048 where the 256 x 256 tiles make three quarters of a round of workgroups.  K % 64 == 0 and
+// G % 8 == 0 (both implied by the MFMA path's conditions).
+constexpr int DENSE_MIN_ROWS = 6144;
+// calls that the workspace query gives room for the panel
+inline bool dense_room(int M, int N) {
+  return M >= 4096 || (M >= 2048 && (long long)((M + 255) / 256) * ((N + 255) / 256) >= 192);
 }
-inline bool dense_rows(int M, int N) {
+inline bool dense_rows(int M, int K, int N) {
   if (variant_on(VAR_NO_DENSE)) return false;
   if (variant_on(VAR_DENSE)) return M > 256;
-  return dense_default(M, N);
+  if (K < 512) return dense_room(M, N);
+  return (K >= 2048 && M >= DENSE_MIN_ROWS) || (M == 2048 && (long long)K * N >= 64LL << 20);
 }
 // workspace of the dequantise-once form: counters, K-split partial tiles, then the panel
 inline size_t dense_panel_offset(size_t part_bytes) {
@@ -593,7 +600,7 @@ size_t awqmi_gemm_workspace_bytes(int M, int K, int N, int split_k) {
           mfma = std::max({mfma, pick_tile(m, K, N, SIZE_MAX).part_bytes, plan_mfma(m, K, N, 256).part_bytes});
       // the dequantise-once form of many-row calls: 256-row tiles, and the fp16 panel behind the
       // partial tiles (a call with a smaller workspace runs the fused kernel instead)
-      if (dense_default(M, N)) {
+      if (dense_room(M, N)) {
         size_t part = plan_mfma(slab, K, N, 256).part_bytes;
         if (M % slab) part = std::max(part, plan_mfma(M % slab, K, N, 256).part_bytes);
         const size_t dense = dense_panel_offset(part) + dg_panel_bytes(K, N) - AWQMI_WS_COUNTER_BYTES;
@@ -714,9 +721,9 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
   // 32-bit, so every operand must stay below 4 GiB
   if (mfma_ok) {
     const int slab = mfma_slab_rows(M, K);
-    // many rows: dequantise once into the workspace, then the dense kernel (same bits as the fused
-    // kernel with 256-row tiles); needs the workspace to hold the panel
-    if (dense_rows(M, N) && workspace && aligned16(workspace)) {
+    // many rows: dequantise once into the workspace, then the dense kernel (same bits as the tile kernel, which
+    // adds in the same order); needs the workspace to hold the panel
+    if (dense_rows(M, K, N) && workspace && aligned16(workspace)) {
       size_t part = plan_mfma(slab < M ? slab : M, K, N, 256).part_bytes;
       if (M % slab) part = std::max(part, plan_mfma(M % slab, K, N, 256).part_bytes);
       const size_t panel_off = dense_panel_offset(part);

@@ -610,6 +610,24 @@ def test_gemm_dequantise_once_form_replays_from_a_graph(sba, gpu):
     assert awq_ref.rel_frobenius(y[:32].cpu().numpy(), ref) <= TOL
 
 
+@pytest.mark.parametrize("M,K,N,dense", [
+    (2048, 448, 8192, True), (2048, 512, 8192, False), (4096, 512, 1024, False), (6143, 2048, 520, False),
+    (6144, 2048, 520, True), (6144, 1984, 520, False), (2048, 8192, 8192, True), (2049, 8192, 8192, False),
+])
+def test_dequantise_once_rule(sba, gpu, M, K, N, dense):
+    """Which many-row calls take the dequantise-once form, on both sides of every line, and their products."""
+    from server_benchmark_amd import _lib
+    g = torch.Generator(device=gpu).manual_seed(M + K)
+    words = lambda *shape: torch.randint(-2**31, 2**31, shape, dtype=torch.int32, device=gpu, generator=g)
+    qw, qz = words(K, N // 8), words(K // 64, N // 8)
+    s = (torch.rand((K // 64, N), device=gpu, generator=g) * 0.019 + 0.001).half()
+    x = torch.randn((M, K), device=gpu, generator=g).half()
+    y = sba.awq_gemm(x, qw, s, qz, 0)
+    assert _lib.load().awqmi_dev_last_gemm_form() == (_lib.FORM_DENSE if dense else _lib.FORM_FUSED)
+    ref = x.float() @ sba.awq_dequantize(qw, s, qz, 0, 0, 0).float()
+    assert float((y.float() - ref).norm() / ref.norm()) <= TOL
+
+
 @pytest.mark.parametrize("M,K,N,G", [(3, 96, 40, 32), (20, 100, 16, 50), (2, 24, 8, 8)])
 def test_gemm_generic_fallback(sba, gpu, M, K, N, G):
     x, qw, s, qz = _np_case(M, K, N, G, seed=5)
