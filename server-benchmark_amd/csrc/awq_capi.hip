@@ -342,6 +342,21 @@ TilePlan tile_plan(int M, int K, int N, int rt, int split) {
 // every height of 64 rows and more, up to five splits each): 0.6 % behind the best of them on average, 15 % at worst.  The same
 // price on 56 layers at 40, 48 and 64 rows with tiles of 48 as well: 1 % behind the best split of either height.  A price with
 // terms for two workgroups on a CU (and splits over 512) is no better: 1.3 % behind on average, 11 % slower than this pick at worst.
+double tile_price(const TilePlan& pl, int KT) {
+  const double stage = 0.28 + 0.0746 * pl.rt;
+  double t = 0.0;
+  if (pl.dp_tiles > 0) {
+    const double part = (pl.dp_tiles % 256) / 256.0;
+    const double rounds = pl.dp_tiles < 256 ? 0.79 + 0.21 * part : pl.dp_tiles / 256 + (part > 0 ? std::max(part, 0.88) : 0.0);
+    t += rounds * (KT + 3.8) * stage;
+  }
+  if (pl.sk_tiles > 0) {
+    const int wgs = pl.sk_tiles * pl.sk_split;
+    t += ((KT + pl.sk_split - 1) / pl.sk_split + 3.8) * stage * (0.79 + 0.21 * wgs / 256.0) + 4.3 +
+         0.22 * pl.sk_split + 0.003 * wgs * pl.rt;
+  }
+  return t;
+}
 TilePlan pick_tile(int M, int K, int N, size_t room) {
   const int KT = K / 64;
   TilePlan best{};
@@ -349,23 +364,8 @@ TilePlan pick_tile(int M, int K, int N, size_t room) {
   for (const int rt : TILE_RT) {
     const TilePlan one = tile_plan(M, K, N, rt, 1);
     const int tiles = one.dp_tiles, rem = tiles % 256;
-    const double stage = 0.28 + 0.0746 * rt;
-    auto price = [&](const TilePlan& pl) {
-      double t = 0.0;
-      if (pl.dp_tiles > 0) {
-        const double part = (pl.dp_tiles % 256) / 256.0;
-        const double rounds = pl.dp_tiles < 256 ? 0.79 + 0.21 * part : pl.dp_tiles / 256 + (part > 0 ? std::max(part, 0.88) : 0.0);
-        t += rounds * (KT + 3.8) * stage;
-      }
-      if (pl.sk_tiles > 0) {
-        const int wgs = pl.sk_tiles * pl.sk_split;
-        t += ((KT + pl.sk_split - 1) / pl.sk_split + 3.8) * stage * (0.79 + 0.21 * wgs / 256.0) + 4.3 +
-             0.22 * pl.sk_split + 0.003 * wgs * rt;
-      }
-      return t;
-    };
     auto take = [&](const TilePlan& pl) {
-      const double t = price(pl);
+      const double t = tile_price(pl, KT);
       if (t < best_t) { best_t = t; best = pl; }
     };
     take(one);
@@ -374,6 +374,29 @@ TilePlan pick_tile(int M, int K, int N, size_t room) {
       if (pl.part_bytes <= room) take(pl);
     }
     if (16 * rt >= M) break;        // one tile holds every row: a higher one multiplies more padding
+  }
+  return best;
+}
+// 17 .. 32 rows on a tile of 32 whose weights are the integers w - z and whose group sums are scaled in fp32 (SCALE32): as
+// exact as the skinny kernel, which multiplies a lane's weights by two row blocks in turn.  Both, skinny / tile, at 17 and 32 rows (us,
+// weights from HBM, rows as the layer method keeps them): 2048 x 2048 13.1, 16.2 / 10.0, 10.0; 5120 x 5120 17.8, 23.1 / 14.4, 14.3;
+// 4096 x 12288, G = 64, 21.8, 25.1 / 16.7, 16.7; 8192 x 10240 21.2, 25.0 / 20.4, 20.3; 13824 x 5120 24.0, 29.7 / 19.1, 19.1; 5120 x
+// 20480 27.3, 31.6 / 21.8, 21.8; 28672 x 4096 28.3, 33.8 / 26.9, 26.6.  Below 128 Mi weights no point of 35 layers is slower; from there
+// on the unsplit skinny launch streams better and only 25 rows and more, or groups of 64, gain (16384 x 8192 25.5, 29.1 / 26.0, 25.8;
+// 29568 x 8192 37.5, 41.0 / 38.9, 38.9, G = 64 41.6, 45.1 / 41.6, 41.4), and above 256 Mi neither (8192 x 59136 64, 60 / 68, 69).
+bool low_tile_pays(int M, int K, int N, int G) {
+  return M > 16 && M <= 32 && (G == 64 || G == 128) && N % 32 == 0 && K % 128 == 0 && 
+         (long long)K * N < (M > 24 || G == 64 ? 256LL << 20 : 128LL << 20);
+}
+// its K split, in whole pairs of stages
+TilePlan pick_low_tile(int K, int N) {
+  const int KT = K / 64, rem = (N + TG_COLS - 1) / TG_COLS % 256;
+  TilePlan best = tile_plan(32, K, N, 2, 1);
+  double best_t = tile_price(best, KT);
+  for (int c = 2; rem > 0 && c <= 16 && c * rem <= 256 && KT / c >= 4; ++c) {
+    const TilePlan pl = tile_plan(32, K, N, 2, c);
+    const double t = tile_price(pl, 2 * ((KT / 2 + c - 1) / c) * c);
+    if (t < best_t) { best_t = t; best = pl; }
   }
   return best;
 }
@@ -387,6 +410,13 @@ void launch_tile(const TileGemmParams& p, hipStream_t st) {
 }
 void launch_tile(int rt, const TileGemmParams& p, hipStream_t st) {
   switch (rt) {
+    case 2: {
+      const dim3 grid(p.per_xcd * 8 + p.sk_tiles * p.sk_split);
+      if (p.G == 64) hipLaunchKernelGGL((awq_gemm_tile_kernel<2, false, 1>), grid, dim3(256), 0, st, p);
+      else hipLaunchKernelGGL((awq_gemm_tile_kernel<2, false, 2>), grid, dim3(256), 0, st, p);
+      if (p.sk_tiles > 0) hipLaunchKernelGGL((awq_gemm_tile_reduce_kernel<2>), dim3(p.sk_tiles * 2), dim3(256), 0, st, p);
+      return;
+    }
     case 3: return launch_tile<3>(p, st);
     case 4: return launch_tile<4>(p, st);
     case 5: return launch_tile<5>(p, st);
@@ -650,6 +680,21 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
   const bool mfma_ok = K % DG_BK == 0 && (((G & (G - 1)) == 0 && G >= 8) || G % 64 == 0) &&
                        mfma_slab_rows(M, K) > 0 && (size_t)K * ldw * 4 < (1ull << 32) &&
                        (size_t)(K / G) * N * 2 < (1ull << 32);
+  // room for the partial tiles of a K split; without a workspace every tile runs on one workgroup
+  const size_t room = workspace && aligned16(workspace) && workspace_bytes > AWQMI_WS_COUNTER_BYTES
+                          ? workspace_bytes - AWQMI_WS_COUNTER_BYTES : 0;
+  // rows r0 .. r0 + Ms - 1 on the tile kernel
+  auto run_tile = [&](const TilePlan& pl, int r0, int Ms) {
+    TileGemmParams p{};
+    p.x = xx + (size_t)r0 * K; p.qw = qw; p.sc = sc; p.qz = qz; p.y = yy + (size_t)r0 * N;
+    p.M = Ms; p.K = K; p.N = N; p.NW = NW; p.ldw = ldw; p.G = G;
+    while ((2 << p.gshift) <= G) ++p.gshift;
+    p.mt = (Ms + 16 * pl.rt - 1) / (16 * pl.rt); p.nt = (N + TG_COLS - 1) / TG_COLS;
+    p.dp_tiles = pl.dp_tiles; p.sk_tiles = pl.sk_tiles; p.sk_split = pl.sk_split;
+    p.per_xcd = (pl.dp_tiles + 7) / 8;
+    p.sk_part = room ? reinterpret_cast<float*>(static_cast<char*>(workspace) + AWQMI_WS_COUNTER_BYTES) : nullptr;
+    launch_tile(pl.rt, p, st);
+  };
   const bool mid = mid_rows(M, K, N, G, ldw);
   if (mid && (variant_on(VAR_MID) || mid_beats_tile(K, N))) {
     t_last_gemm_form = AWQMI_FORM_MID;
@@ -687,6 +732,14 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
       if ((size_t)ncb * sizeof(int) > AWQMI_WS_COUNTER_BYTES) return AWQMI_BAD_SHAPE;
       if (workspace_bytes < AWQMI_WS_COUNTER_BYTES + gemv_partial_bytes(N, split, 1, M > 16 ? 32 : 16))
         return AWQMI_WORKSPACE_TOO_SMALL;
+    }
+    if (split_k == 0 && mfma_ok && !t_trace && !variant_on(VAR_MID_M_SKINNY) && low_tile_pays(M, K, N, G)) {
+      const TilePlan pl = pick_low_tile(K, N);
+      if (pl.part_bytes <= room) {
+        t_last_gemm_form = AWQMI_FORM_FUSED;
+        run_tile(pl, 0, M);
+        return launch_status();
+      }
     }
     t_last_gemm_form = AWQMI_FORM_SKINNY;
     GemvParams p{};
@@ -751,9 +804,6 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
       }
     }
     t_last_gemm_form = mid ? AWQMI_FORM_MID : AWQMI_FORM_FUSED;
-    // room for the partial tiles of a K split; without a workspace every tile runs on one workgroup
-    const size_t room = workspace && aligned16(workspace) && workspace_bytes > AWQMI_WS_COUNTER_BYTES
-                            ? workspace_bytes - AWQMI_WS_COUNTER_BYTES : 0;
     const int forced = forced_tile();
     for (int r0 = 0; r0 < M; r0 += slab) {
       const int Ms = M - r0 < slab ? M - r0 : slab;
@@ -765,15 +815,7 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
       } else {
         pl = pick_tile(Ms, K, N, room);
       }
-      TileGemmParams p{};
-      p.x = xx + (size_t)r0 * K; p.qw = qw; p.sc = sc; p.qz = qz; p.y = yy + (size_t)r0 * N;
-      p.M = Ms; p.K = K; p.N = N; p.NW = NW; p.ldw = ldw; p.G = G;
-      while ((2 << p.gshift) <= G) ++p.gshift;
-      p.mt = (Ms + 16 * pl.rt - 1) / (16 * pl.rt); p.nt = (N + TG_COLS - 1) / TG_COLS;
-      p.dp_tiles = pl.dp_tiles; p.sk_tiles = pl.sk_tiles; p.sk_split = pl.sk_split;
-      p.per_xcd = (pl.dp_tiles + 7) / 8;
-      p.sk_part = room ? reinterpret_cast<float*>(static_cast<char*>(workspace) + AWQMI_WS_COUNTER_BYTES) : nullptr;
-      launch_tile(pl.rt, p, st);
+      run_tile(pl, r0, Ms);
     }
     return launch_status();
   }

@@ -511,7 +511,7 @@ __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, 
 }
 #endif  // __HIP_DEVICE_COMPILE__
 
-template <int RT, bool ANY>
+template <int RT, bool ANY, int SCALE32 = 0>
 __global__ __launch_bounds__(256, tg_occupancy(RT, ANY)) void awq_gemm_tile_kernel(const TileGemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int D = tg_depth(RT, ANY, tg_lds_bytes(RT, tg_occupancy(RT, ANY)));
@@ -527,8 +527,9 @@ __global__ __launch_bounds__(256, tg_occupancy(RT, ANY)) void awq_gemm_tile_kern
     const int j = id - 8 * p.per_xcd;
     const int tl = j % p.sk_tiles, pt = j / p.sk_tiles;
     nid = p.dp_tiles + tl;
-    kb = (int)((long long)KT * pt / p.sk_split);
-    ke = (int)((long long)KT * (pt + 1) / p.sk_split);
+    constexpr int U = SCALE32 ? 2 : 1;      // stages that stay together
+    kb = (int)((long long)(KT / U) * pt / p.sk_split) * U;
+    ke = (int)((long long)(KT / U) * (pt + 1) / p.sk_split) * U;
     part = p.sk_part + (size_t)(tl * p.sk_split + pt) * tg_part_floats(RT);
   }
   const int gsize = PF_GROUP_M * p.nt;
@@ -536,7 +537,7 @@ __global__ __launch_bounds__(256, tg_occupancy(RT, ANY)) void awq_gemm_tile_kern
   const int gm = min(p.mt - first_m, PF_GROUP_M);
   const int mt_i = first_m + (nid % gsize) % gm;
   const int nt_i = (nid % gsize) / gm;
-  awq_tile<RT, D, ANY, false, false>(p, mt_i * (16 * RT), nt_i * 256, kb, ke, part, 0, (uint32_t)(uintptr_t)(lds_byte*)smem,
+  awq_tile<RT, D, ANY, false, false, SCALE32>(p, mt_i * (16 * RT), nt_i * 256, kb, ke, part, 0, (uint32_t)(uintptr_t)(lds_byte*)smem,
                                      nullptr, nullptr);
 #endif
 }

@@ -509,6 +509,46 @@ def test_fused_tile_of_48_rows(sba, gpu, M, K, N, G):
     assert awq_ref.rel_frobenius(y1.cpu().numpy(), y) <= TOL
 
 
+@pytest.mark.parametrize("M", [17, 31, 32])
+@pytest.mark.parametrize("K,N,G", [(128, 32, 64), (128, 256, 128), (384, 288, 64), (640, 544, 128), (1152, 1024, 128), (1920, 800, 64),
+                                   (4096, 4128, 128), (16384, 256, 128)])
+def test_fused_tile_of_32_rows(sba, gpu, M, K, N, G):
+    """17 .. 32 rows on the tile whose group sums are scaled in fp32: full and ragged column tiles, odd numbers of pairs of
+    stages, K splits; as near to the 64-bit product as the skinny kernel, whose launch a set split_k still takes."""
+    from server_benchmark_amd import _lib
+    lib = _lib.load()
+    sba.ops.get_workspace(gpu, 80 << 20)[65536:].fill_(255)
+    x, qw, s, qz = _np_case(M, K, N, G, seed=K + M)
+    y = _check_gemm(sba, gpu, x, qw, s, qz, G, 0, tag="tile 32")
+    assert lib.awqmi_dev_last_gemm_form() == _lib.FORM_FUSED
+    skinny = _check_gemm(sba, gpu, x, qw, s, qz, G, 1, tag="skinny")
+    assert lib.awqmi_dev_last_gemm_form() == _lib.FORM_SKINNY
+    W = (awq_ref.unpack_awq(qw).astype(np.float64) - awq_ref.unpack_awq(qz).astype(np.float64).repeat(G, 0)) \
+        * s.astype(np.float64).repeat(G, 0)
+    exact = x.astype(np.float64) @ W
+    # both round once, to fp16: 2 % for the noise of that rounding over the fewest outputs here (17 x 32)
+    assert awq_ref.rel_frobenius(y, exact) <= 1.02 * awq_ref.rel_frobenius(skinny, exact)
+
+
+@pytest.mark.parametrize("M,K,N,G,tile", [
+    (16, 1024, 1024, 128, False), (17, 1024, 1024, 128, True), (33, 1024, 1024, 128, True), (24, 1024, 1024, 32, False),
+    (24, 1024, 1040, 128, False), (24, 1024, 1024, 256, False), (24, 8192, 16352, 128, True), (24, 8192, 16384, 128, False),
+    (24, 8192, 16384, 64, True), (25, 8192, 16384, 128, True), (32, 16384, 16384, 64, False),
+])
+def test_tile_rule_up_to_32_rows(sba, gpu, M, K, N, G, tile):
+    """Which calls of up to 32 rows take the tile, on both sides of every line, and their products."""
+    from server_benchmark_amd import _lib
+    g = torch.Generator(device=gpu).manual_seed(M + K)
+    words = lambda *shape: torch.randint(-2**31, 2**31, shape, dtype=torch.int32, device=gpu, generator=g)
+    qw, qz = words(K, N // 8), words(K // G, N // 8)
+    s = (torch.rand((K // G, N), device=gpu, generator=g) * 0.019 + 0.001).half()
+    x = torch.randn((M, K), device=gpu, generator=g).half()
+    y = sba.awq_gemm(x, qw, s, qz, 0)
+    assert _lib.load().awqmi_dev_last_gemm_form() == (_lib.FORM_FUSED if tile else _lib.FORM_SKINNY)
+    ref = x.float() @ sba.awq_dequantize(qw, s, qz, 0, 0, 0).float()
+    assert float((y.float() - ref).norm() / ref.norm()) <= TOL
+
+
 @pytest.mark.parametrize("M,K,N", [(512, 1024, 1280), (300, 2048, 520), (2048, 512, 5120), (768, 1536, 8192 + 256)])
 def test_gemm_prefill_partial_rounds(sba, gpu, M, K, N):
     """Tile counts that are not a multiple of the CU count, ragged last row / column tiles;
