@@ -83,9 +83,9 @@ size_t awqmi_gemm_workspace_bytes(int M, int K, int N, int split_k);
  * Stands in for vLLM's `awq_gemm` op (every AWQ Linear at decode and prefill); reached
  * from the server started at reference utils/generate_compose.py:85-93.
  * fp32 accumulation, one final rounding to fp16.  M >= 1; K % group == 0; N % 8 == 0.
- * M <= 32 takes the HBM-bound skinny kernel (split_k honoured, 0 = auto).  More rows ignore
- * split_k: 33 .. 64 rows on large layers take a one-pass kernel, any other call the LDS-dequant
- * MFMA kernel (64- / 128- / 192- / 256-row tiles) and, from 2048 rows on, a dequantise-once form.
+ * M <= 16, and any M <= 32 with split_k set, takes the HBM-bound skinny kernel (split_k honoured, 0 = auto).
+ * More rows ignore split_k: they take an MFMA kernel that unpacks in registers (tiles of 32 .. 256 rows; 33 .. 64
+ * rows of the largest layers a one-pass kernel, 17 .. 32 the skinny kernel) and, from 6144 rows on, a dequantise-once form.
  * With a workspace of awqmi_gemm_workspace_bytes() these split K as the shape asks for and a
  * second short kernel sums the partial tiles; with less, every tile runs on one workgroup (and
  * the dequantise-once form is not taken).  Shapes outside the fast kernels' tiling (K % 128 != 0, group
@@ -169,7 +169,7 @@ size_t awqmi_moe_gemm_workspace_bytes(int n_slots, int E, int K, int N, int spli
 
 /* Expert-grouped AWQ GEMM over sorted-token blocks of tile_m rows; the ids must come from
  * awqmi_moe_align with the same tile_m.  tile_m 16 or 32: the skinny kernel (decode-sized
- * batches).  tile_m 64, 128 or 256: the MFMA kernel, for many slots per expert; it takes no
+ * batches).  tile_m 64, 128 or 256: the tile kernel, for many slots per expert; it takes no
  * split_k or workspace and needs x and each expert's tensors under 4 GiB.
  * For every non-pad entry s = sorted_token_ids[i] in a block owned by expert e:
  *     y[s, :] = (x[s / a_row_div, :] @ W_e) * (topk_weights ? topk_weights[s] : 1)
@@ -205,7 +205,7 @@ int awqmi_moe_sum_f16(const void* in_f16, void* out_f16, int T, int topk, int H,
  * graph.  H and inter must be multiples of 128 with group in {32, 64, 128 * i}. */
 size_t awqmi_fused_moe_workspace_bytes(int T, int H, int inter, int E, int topk);
 /* Sorted-token block rows awqmi_fused_moe_f16 uses for these shapes: 16 (skinny kernel) or
- * 64 / 128 / 256 (MFMA kernel, prefill-sized batches).  A query like awqmi_gemm_auto_split_k;
+ * 64 / 128 / 256 (tile kernel, prefill-sized batches).  A query like awqmi_gemm_auto_split_k;
  * 0 for shapes the call would refuse. */
 int awqmi_fused_moe_block_rows(int T, int H, int inter, int E, int topk, int group);
 int awqmi_fused_moe_f16(const void* hidden_f16, const float* router_logits, const int32_t* w13_qweight,

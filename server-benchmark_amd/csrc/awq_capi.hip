@@ -62,7 +62,7 @@ enum : int {
   VAR_ALIGN_ONE_WG = 16384,   // align always in one workgroup
   VAR_MOE_TILE_SHIFT = 16,    // bits 16..17 = v: the one-call MoE block uses 64 / 128 / 256-row blocks (v = 1 / 2 / 3)
   VAR_MID_M_SKINNY = 1 << 18, // awq_gemm with 17..64 rows: skinny passes wherever they can run
-  VAR_MID_M_MFMA = 1 << 19,   // awq_gemm with 17..64 rows: the MFMA kernel wherever it can run
+  VAR_MID_M_MFMA = 1 << 19,   // awq_gemm with 17..64 rows: the tile kernel wherever it can run
   VAR_MFMA_ROWS_SHIFT = 20,   // bits 20..22 = v: fused tiles of 64 v rows (v = 1..4) or 16 v rows (v = 5..7) whatever M is
   VAR_NO_TAIL_STEP = 1 << 23, // dense skinny launches never share left-over chunks step by step
   VAR_NO_FOLDED_ROUTE = 1 << 24, // the one-call MoE block always routes in a launch of its own
@@ -204,10 +204,9 @@ void launch_gemv(const GemvParams& p, dim3 grid, hipStream_t st) {
 // rows the skinny kernel takes in one awq_gemm call (passes of up to 32 rows)
 constexpr int SKINNY_MAX_M = 64;
 
-// Up to 32 rows one skinny pass (two row blocks share every unpacked operand); from 33 rows on
-// the 64-row MFMA tile beats two skinny passes on every layer shape measured (nine shapes from
-// 2048 x 5120 to 8192 x 59136, weights read from HBM: equal at worst, up to 2 x on small layers), and
-// on large layers the one-pass kernel below beats both.
+// Up to 32 rows one skinny pass (two row blocks share every unpacked operand; see low_tile_pays for the calls of more
+// than 16 rows that take a tile instead); from 33 rows on a tile or the one-pass kernel, which two skinny passes
+// never beat (nine shapes from 2048 x 5120 to 8192 x 59136, weights read from HBM).
 inline bool skinny_rows(int M, int /*N*/) { return M <= 32; }
 
 inline size_t mid_partial_bytes(int N, int split) {
@@ -264,10 +263,10 @@ inline bool mid_rows(int M, int K, int N, int G, int ldw) {
          !variant_on(VAR_MID_M_SKINNY) && !variant_on(VAR_MID_M_MFMA);
 }
 
-// Work split of the MFMA kernel: whole rounds of 256 tiles run one workgroup per tile; a
+// Work split of the dense kernel (and of a forced height of the tile kernel): whole rounds of 256 tiles run one workgroup per tile; a
 // last round of fewer than 129 tiles (and any launch that small) is split in K over
 // floor(256 / tiles) workgroups per tile (at most 8, at least 4 k-tiles each).
-// The MFMA kernel addresses X through 32-bit buffer offsets: calls with more than 4 GiB of
+// The MFMA kernels address X through 32-bit buffer offsets: calls with more than 4 GiB of
 // activations run as consecutive row slabs (multiples of 256 rows).
 inline int mfma_slab_rows(int M, int K) {
   const long long fit = ((1LL << 32) - 1) / ((long long)K * 2);
@@ -383,7 +382,9 @@ TilePlan pick_tile(int M, int K, int N, size_t room) {
 // 4096 x 12288, G = 64, 21.8, 25.1 / 16.7, 16.7; 8192 x 10240 21.2, 25.0 / 20.4, 20.3; 13824 x 5120 24.0, 29.7 / 19.1, 19.1; 5120 x
 // 20480 27.3, 31.6 / 21.8, 21.8; 28672 x 4096 28.3, 33.8 / 26.9, 26.6.  Below 128 Mi weights no point of 35 layers is slower; from there
 // on the unsplit skinny launch streams better and only 25 rows and more, or groups of 64, gain (16384 x 8192 25.5, 29.1 / 26.0, 25.8;
-// 29568 x 8192 37.5, 41.0 / 38.9, 38.9, G = 64 41.6, 45.1 / 41.6, 41.4), and above 256 Mi neither (8192 x 59136 64, 60 / 68, 69).
+// 29568 x 8192 37.5, 41.0 / 38.9, 38.9, G = 64 41.6, 45.1 / 41.6, 41.4), and above 256 Mi neither (8192 x 59136 64, 60 / 68, 69).  Up to 16 rows the
+// skinny kernel stays: at 16 it is 5 - 29 % faster on 12 of 16 layers, 7 % slower at worst (1024 x 12288 10.8 / 10.0), at 4 rows 15 - 49 %
+// faster.
 bool low_tile_pays(int M, int K, int N, int G) {
   return M > 16 && M <= 32 && (G == 64 || G == 128) && N % 32 == 0 && K % 128 == 0 && 
          (long long)K * N < (M > 24 || G == 64 ? 256LL << 20 : 128LL << 20);

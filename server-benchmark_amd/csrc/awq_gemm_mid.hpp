@@ -6,7 +6,7 @@
 // 8-row slabs of a 32-row step) and a contiguous range of 128-row chunks of K; a workgroup is four
 // waves on the same columns and different K ranges, one per SIMD.  Weights stay in registers, three
 // to four steps ahead; activations go through the wave's own piece of LDS by direct-to-LDS loads, two
-// steps a slot.  The multiply side is the MFMA kernel's: a lane's 8 x 8 nibble block becomes exact
+// steps a slot.  The multiply side: a lane's 8 x 8 nibble block becomes exact
 // fp16 (w - z) * s, as awq_dequantize rounds it, and is the A operand of v_mfma_f32_16x16x32_f16
 // against four 16-row blocks of X.  No dequantised weight goes through LDS and there is no barrier in
 // the loop.
@@ -14,10 +14,9 @@
 // What bounds it: the wave's own issue.  A 32-row step is 64 MFMAs and 224 unpack instructions and
 // takes 1.0 us (62 us for 64 steps with 32 workgroups on the chip), against 0.7 us in which HBM
 // delivers the 16 KiB of a CU (counters on 8192 x 59136: 63 % of a wave's cycles issue, 23 % are ready and do not,
-// 14 % wait for memory or LDS; on 8192 x 10240 and 8192 x 8192 it is 49, 27 - 30 and 21 - 24 %).  The 64-row tile of awq_gemm_mfma_kernel, which these calls took
-// before, sends every dequantised weight through LDS (32 KiB written and 64 KiB read back per 64 x 256
-// k-tile, beside 40 KiB of X) with 16 KiB of weights in flight per CU: 8192 x 59136 at 64 rows 111 - 115
-// us, here 79 (3.2 TB/s of packed weights).  Measured and dropped: two waves per SIMD with 128 columns each
+// 14 % wait for memory or LDS; on 8192 x 10240 and 8192 x 8192 it is 49, 27 - 30 and 21 - 24 %).  8192 x 59136 at 64 rows
+// takes 79 us (3.2 TB/s of packed weights), the tile kernel 85; the tile is ahead on layers of fewer than 320 Mi weights
+// (see mid_beats_tile).  Measured and dropped: two waves per SIMD with 128 columns each
 // (64-byte pieces of a row per load, X read twice: 105 us), 32 x 32 x 16 MFMAs with one word per lane
 // (twice the load instructions: 94 us), X in 64-byte pieces (84 us).
 //

@@ -25,6 +25,9 @@
 // taken out 59 of 90 us).  Against the kernel before it (weights dequantised into LDS by all waves, 32 x 32 x 16 MFMAs,
 // tiles of 64 rows' steps), us: 8192 x 59136 at 80 / 128 / 400 / 1000 / 2047 rows 145 / 149 / 430 / 889 / 1701 -> 95 / 125 / 325 /
 // 757 / 1500; 29568 x 8192 at 96 / 400 / 1000 81 / 226 / 433 -> 58 / 171 / 383; 3584 x 4608 at 64 / 1000 18.1 / 51 -> 15.7 / 42.
+// Tiles of up to 128 rows share a CU in pairs (us, one / two workgroups: 8192 x 59136 at 256 rows in 128-row tiles 234 / 216, 3584 x
+// 37888 100 / 85, 1024 x 12288 at 2047 60 / 53; a single round is even, 123 / 126).  32- and 48-row tiles against the skinny and the
+// one-pass kernel stand at low_tile_pays and mid_pays.
 // Measured and dropped: eight waves on two K halves of a tile, two per SIMD (8192 x 59136 at 64 rows 80 against 84 us, split
 // layers slower); a ring of distinct LDS objects with the compiler's own waits (even, four times the code).
 #pragma once
@@ -162,7 +165,7 @@ __device__ __forceinline__ void tg_wait_and_barrier() {
 // writes silu(gate) * up.
 // SCALE32 = stages of a group (1 or 2, 0: off): weights enter the product as the integers w - z, and a group's sum is
 // scaled in fp32 when the group ends -- the skinny kernel's precision, for tiles that take its place.  The group's sum and the
-// total are both in vector registers, so that tiles are at most 64 rows high; the scaling is dealt out over the next
+// total are both in vector registers, so that tiles are at most 64 rows high, and stages go in pairs (ke - kb is even); the scaling is dealt out over the next
 // group's first k-step.
 template <int RT, int D, bool ANY, bool GROUPED, bool ACT, int SCALE32 = 0>
 __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, const int n0, const int kb, const int ke,

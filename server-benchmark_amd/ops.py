@@ -325,7 +325,7 @@ def moe_awq_gemm(a: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor, q
                  out: torch.Tensor | None = None, block_size: int = MOE_TILE_M,
                  _dev_variant: int | None = None) -> torch.Tensor:
     """Expert-grouped AWQ GEMM over blocks of `block_size` sorted slots (16 or 32: the skinny
-    kernel; 64, 128 or 256: the MFMA kernel in its expert-grouped form, for many rows per expert):
+    kernel; 64, 128 or 256: the tile kernel in its expert-grouped form, for many rows per expert):
     out[s] = a[s // a_row_div] @ W[expert(s)] (* topk_weights[s]).  The ids must come from
     moe_align_block_size with the same block size."""
     _need(a, "a", torch.float16, 2)
