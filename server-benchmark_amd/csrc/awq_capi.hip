@@ -1299,8 +1299,9 @@ bool moe_runs(int T, int n_slots, int E, int H, int inter, int group) {
       (size_t)inter * (H / 8) * 4 >= (1ull << 32))
     return false;
   if (variant_on(VAR_MOE_RUNS)) return true;
-  const double avg = (double)n_slots / E, b16 = E * moe_expected_blocks(avg, 16), tiles = E * moe_expected_blocks(avg, 16 * TG_RUN);
+  const double avg = (double)n_slots / E;
   if (avg <= 32.0 || H < 1024 || inter < 384) return false;
+  const double b16 = E * moe_expected_blocks(avg, 16), tiles = E * moe_expected_blocks(avg, 16 * TG_RUN);
   const double stage = 2.0 * (0.344 + 0.09 * std::max(b16 / tiles, 2.0));
   auto gemm = [&](int K, int col_tiles) {
     const double r = tiles * col_tiles / 512.0, whole = std::floor(r), part = r - whole;
