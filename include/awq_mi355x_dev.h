@@ -15,8 +15,8 @@
  *   4|8|16   v = bits 2..4: runs of 1 << (v - 1) sorted-token blocks per XCD
  *   64       never two column blocks per workgroup
  *   512      the one-call MoE block takes its 16-slot blocks in tiles of up to four, whatever the shape
- *            (more than 16 tokens)
- *   1024     the one-call MoE block always runs the separate activation kernel
+ *            (more than 16 tokens, not with 1024)
+ *   1024     the one-call MoE block always runs the separate activation kernel, 16-slot blocks then one by one
  *   2048     the one-call MoE block always uses the skinny kernel's 16-row blocks
  *   4096     every launch keeps the weight ring in registers (no LDS ring)
  *   16384    the align step always runs in one workgroup
@@ -116,6 +116,9 @@ int awqmi_dev_fused_moe_routed_f16(const void* hidden_f16, const float* router_l
                                    int variant);
 
 int awqmi_dev_fused_moe_block_rows(int T, int H, int inter, int E, int topk, int group, int variant);
+
+/* 1 if the one-call MoE block takes its 16-slot blocks in tiles of up to four for these shapes, else 0. */
+int awqmi_dev_fused_moe_tiles(int T, int H, int inter, int E, int topk, int group, int variant);
 
 #ifdef __cplusplus
 }

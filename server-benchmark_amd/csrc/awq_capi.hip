@@ -1038,6 +1038,9 @@ static int moe_gemm_impl(const void* x, const int32_t* qweight, const void* scal
       p.n_live = runs;
       p.runs = runs + 1;
       tiles = moe_most_runs(n_slots, E);
+      // workgroups still read the list while others store their rows
+      const uintptr_t list = reinterpret_cast<uintptr_t>(runs), rows = reinterpret_cast<uintptr_t>(y);
+      if (rows < list + (1 + (size_t)tiles) * sizeof(int32_t) && list < rows + (size_t)n_slots * cols * 2) return AWQMI_BAD_ARGUMENT;
     }
     p.total = (int)(tiles * p.nt);
     // ranges per XCD are uneven in rows with few experts (see the kernel)
@@ -1313,6 +1316,23 @@ bool moe_runs(int T, int n_slots, int E, int H, int inter, int group) {
   return runs < (E < 16 ? 0.76 : 0.86) * skinny;
 }
 
+// How a one-call block runs: slots of its blocks, whether those of 16 go in tiles (moe_runs), and whether the first expert GEMM
+// writes silu(gate) * up itself: in a tile of gate columns and their up columns; in one workgroup per gate / up block pair;
+// or, with few blocks (the launch is split in K), in the last arrivers of such a pair.
+// The list of tiles lies where the gate / up sums go otherwise, so there are no tiles without the fused activation.
+struct MoeForm { int tile; bool runs, act; };
+MoeForm moe_form(int T, int H, int inter, int E, int topk, int group) {
+  const int n_slots = T * topk, G = norm_group(H, group);
+  MoeForm f{moe_pick_tile(n_slots, E, H, inter, group), false, false};
+  if (variant_on(VAR_NO_FUSED_ACT)) return f;
+  const bool tile_act = moe_tile_act_ok(inter, G);
+  f.runs = f.tile == 16 && tile_act && moe_runs(T, n_slots, E, H, inter, group);
+  f.act = f.tile >= 64 || f.runs ? tile_act
+                                 : gemv_tiled_ok(H, G) && (moe_can_fuse_act(n_slots, E, H, 2 * inter) ||
+                                                           moe_can_fuse_act_split(n_slots, E, H, 2 * inter));
+  return f;
+}
+
 // workspace carve-up of the fused MoE block; every piece starts 256-byte aligned
 struct FusedMoeLayout {
   size_t gemm_ws, ids, wts, sorted, experts, npp, h13, act, o, total;
@@ -1382,7 +1402,8 @@ int awqmi_fused_moe_routed_f16(const void* hidden, const float* router_logits, c
     return AWQMI_BAD_ARGUMENT;
   if ((scoring != 0 && scoring != 1) || (scoring == 0 && score_bias)) return AWQMI_BAD_ARGUMENT;
   if (!aligned16(workspace)) return AWQMI_BAD_ALIGN;
-  const int tile = moe_pick_tile(T * topk, E, H, inter, group);
+  const MoeForm form = moe_form(T, H, inter, E, topk, group);
+  const int tile = form.tile;
   const FusedMoeLayout L = fused_moe_layout(T, H, inter, E, topk, tile);
   if (workspace_bytes < L.total) return AWQMI_WORKSPACE_TOO_SMALL;
   char* ws = static_cast<char*>(workspace);
@@ -1395,8 +1416,7 @@ int awqmi_fused_moe_routed_f16(const void* hidden, const float* router_logits, c
   void* act_out = ws + L.act;
   void* o = ws + L.o;
   int st;
-  // tiles of several 16-slot blocks write silu(gate) * up themselves: their list is where the gate / up sums would be
-  int32_t* const runs = tile == 16 && moe_runs(T, L.n_slots, E, H, inter, group) ? reinterpret_cast<int32_t*>(h13) : nullptr;
+  int32_t* const runs = form.runs ? reinterpret_cast<int32_t*>(h13) : nullptr;
   const MoeRoute route{router_logits, score_bias, T, E, topk, scoring, renormalize, routed_scale,
                        ids, wts, sorted, experts, npp, runs};
   // a handful of tokens: the first expert GEMM takes the routing along (one launch less)
@@ -1428,15 +1448,7 @@ int awqmi_fused_moe_routed_f16(const void* hidden, const float* router_logits, c
     st = launch_status();
     if (st) return st;
   }
-  const int Gn = norm_group(H, group);
-  const bool tiles = tile >= 64 || runs;
-  const bool act = tiles ? moe_tile_act_ok(inter, Gn)
-                         : gemv_tiled_ok(H, Gn) && (moe_can_fuse_act(L.n_slots, E, H, 2 * inter) ||
-                                                    moe_can_fuse_act_split(L.n_slots, E, H, 2 * inter));
-  if (act && !variant_on(VAR_NO_FUSED_ACT)) {
-    // the w13 GEMM writes silu(gate) * up itself: in a tile of gate columns and their up columns; in one
-    // workgroup per gate / up block pair; or, with few blocks (the launch is split in K), in the last arrivers of
-    // such a pair
+  if (form.act) {
     st = moe_gemm_impl(hidden, w13_q, w13_s, w13_z, act_out, sorted, experts, npp, nullptr, L.n_slots, topk, tile, E, H,
                        2 * inter, group, 0, ws + L.gemm_ws, L.gemm_ws_bytes, stream, true, pending, runs);
     if (st) return st;
@@ -1567,6 +1579,12 @@ int awqmi_dev_fused_moe_routed_f16(const void* hidden, const float* router_logit
 int awqmi_dev_fused_moe_block_rows(int T, int H, int inter, int E, int topk, int group, int variant) {
   VariantScope scope(variant);
   return awqmi_fused_moe_block_rows(T, H, inter, E, topk, group);
+}
+
+int awqmi_dev_fused_moe_tiles(int T, int H, int inter, int E, int topk, int group, int variant) {
+  if (!awqmi_fused_moe_block_rows(T, H, inter, E, topk, group)) return 0;
+  VariantScope scope(variant);
+  return moe_form(T, H, inter, E, topk, group).runs;
 }
 
 }  // extern "C"

@@ -305,7 +305,8 @@ def test_moe_grouped_gemm_at_the_tile_edges(sba, gpu, bs, K, N, G, E):
             assert awq_ref.rel_frobenius(y[tok], ref) <= TOL, e
 
 
-@pytest.mark.parametrize("variant", [512, 1 << 16, 2 << 16, 3 << 16])    # 16-slot blocks in tiles of up to four; 64, 128, 256
+# 16-slot blocks in tiles of up to four; 64, 128, 256; the same with a separate activation kernel (no tiles then)
+@pytest.mark.parametrize("variant", [512, 1 << 16, 2 << 16, 3 << 16, 512 | 1024, 2 << 16 | 1024])
 @pytest.mark.parametrize("H,I,G,E", [(256, 128, 128, 22), (384, 384, 64, 22), (1152, 256, 128, 13), (128, 640, 64, 13)])
 def test_fused_call_on_the_grouped_kernel_at_the_tile_edges(sba, gpu, variant, H, I, G, E):
     """The one-call block with both expert GEMMs on the grouped kernel, the first writing silu(gate) * up itself, over
