@@ -304,20 +304,23 @@ MfmaPlan plan_mfma(int M, int K, int N, int bm) {
 //   1024 x 12288     80 / 56       102 / 78      105 / 98      131 / 127     179 / 156     201 / 193
 //   512 x 8192       28 / 22       63 / 36       50 / 43       82 / 56       68 / 63       89 / 82
 // At 6144 rows the tile is within 2.3 % either way from 2048 weight rows on; with fewer it stays ahead at any size, as the panel is as
-// much traffic as the products.  One row count keeps the panel where the tile is 9 % faster: 2048 on layers of 64 Mi weights and
-// more, whose prefill record and its test name the form.  Layers of fewer than 512 weight rows, which no model here has, keep the lines that were drawn for
-// all: from 4096 rows on, from 2048 where the 256 x 256 tiles make three quarters of a round of workgroups.  K % 64 == 0 and
-// G % 8 == 0 (both implied by the MFMA path's conditions).
+// much traffic as the products.  One row count keeps the panel where the tile is 8 - 11 % faster: 2048 on layers of 64 Mi weights and
+// more with three quarters of a round of 256 x 256 tiles, whose prefill record and its test name the form.  Narrower ones run the tile
+// there (18944 x 3584 260 / 229, 13824 x 5120, G = 32, 283 / 261).  Layers of fewer than 512 weight rows, which no model here has, keep the
+// lines that were drawn for all: from 4096 rows on, from 2048 with those three quarters of a round.  K % 64 == 0 and G % 8 == 0 (both
+// implied by the MFMA path's conditions).
 constexpr int DENSE_MIN_ROWS = 6144;
-// calls that the workspace query gives room for the panel
-inline bool dense_room(int M, int N) {
-  return M >= 4096 || (M >= 2048 && (long long)((M + 255) / 256) * ((N + 255) / 256) >= 192);
+// One rule for the call and for the workspace query: a call never takes the panel in room that another one's query asked for, and no
+// room is asked for that the call leaves unused.
+inline bool dense_default(int M, int K, int N) {
+  const bool wide = M >= 2048 && (long long)((M + 255) / 256) * ((N + 255) / 256) >= 192;
+  if (K < 512) return M >= 4096 || wide;
+  return (K >= 2048 && M >= DENSE_MIN_ROWS) || (M == 2048 && wide && (long long)K * N >= 64LL << 20);
 }
 inline bool dense_rows(int M, int K, int N) {
   if (variant_on(VAR_NO_DENSE)) return false;
   if (variant_on(VAR_DENSE)) return M > 256;
-  if (K < 512) return dense_room(M, N);
-  return (K >= 2048 && M >= DENSE_MIN_ROWS) || (M == 2048 && (long long)K * N >= 64LL << 20);
+  return dense_default(M, K, N);
 }
 // workspace of the dequantise-once form: counters, K-split partial tiles, then the panel
 inline size_t dense_panel_offset(size_t part_bytes) {
@@ -631,7 +634,7 @@ size_t awqmi_gemm_workspace_bytes(int M, int K, int N, int split_k) {
           mfma = std::max({mfma, pick_tile(m, K, N, SIZE_MAX).part_bytes, plan_mfma(m, K, N, 256).part_bytes});
       // the dequantise-once form of many-row calls: 256-row tiles, and the fp16 panel behind the
       // partial tiles (a call with a smaller workspace runs the fused kernel instead)
-      if (dense_room(M, N)) {
+      if (dense_default(M, K, N)) {
         size_t part = plan_mfma(slab, K, N, 256).part_bytes;
         if (M % slab) part = std::max(part, plan_mfma(M % slab, K, N, 256).part_bytes);
         const size_t dense = dense_panel_offset(part) + dg_panel_bytes(K, N) - AWQMI_WS_COUNTER_BYTES;

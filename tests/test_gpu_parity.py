@@ -668,6 +668,31 @@ def test_dequantise_once_rule(sba, gpu, M, K, N, dense):
     assert float((y.float() - ref).norm() / ref.norm()) <= TOL
 
 
+@pytest.mark.parametrize("M,K,N", [(2048, 13824, 5120), (2048, 16384, 4096), (2048, 8192, 8192), (2048, 448, 2048), (4096, 448, 1024),
+                                   (6143, 2048, 520), (6144, 2048, 520), (6144, 1984, 520),
+                                   (17, 8192, 5120), (32, 384, 32), (300, 2048, 520), (64, 8192, 1024)])
+def test_spare_workspace_changes_nothing(sba, gpu, M, K, N):
+    """The workspace of a stream only grows: a call runs the same kernel, bit for bit, in exactly the room that the query
+    asks for and in room for any form."""
+    from server_benchmark_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device=gpu).manual_seed(M + K)
+    words = lambda *shape: torch.randint(-2**31, 2**31, shape, dtype=torch.int32, device=gpu, generator=g)
+    qw, qz = words(K, N // 8), words(K // 64, N // 8)
+    s = (torch.rand((K // 64, N), device=gpu, generator=g) * 0.019 + 0.001).half()
+    x = torch.randn((M, K), device=gpu, generator=g).half()
+    got = []
+    need = lib.awqmi_gemm_workspace_bytes(M, K, N, 0)
+    for nbytes in (need, max(need, lib.awqmi_dev_gemm_dense_workspace_bytes(M, K, N)) + (64 << 20)):
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device=gpu)
+        y = torch.empty((M, N), dtype=torch.float16, device=gpu)
+        assert lib.awqmi_gemm_f16(x.data_ptr(), qw.data_ptr(), s.data_ptr(), qz.data_ptr(), y.data_ptr(), ws.data_ptr(), ws.numel(),
+                                  M, K, N, 64, 0, torch.cuda.current_stream().cuda_stream) == 0
+        got.append((lib.awqmi_dev_last_gemm_form(), y))
+    assert got[0][0] == got[1][0]
+    assert torch.equal(got[0][1].view(torch.int16), got[1][1].view(torch.int16))
+
+
 @pytest.mark.parametrize("M,K,N,G", [(3, 96, 40, 32), (20, 100, 16, 50), (2, 24, 8, 8)])
 def test_gemm_generic_fallback(sba, gpu, M, K, N, G):
     x, qw, s, qz = _np_case(M, K, N, G, seed=5)
