@@ -36,7 +36,7 @@
  *            split: one word per lane, two 128-column blocks per workgroup, weight ring in LDS, two
  *            workgroups per CU; with 4096 its ring stays in registers)
  *   1 << 28  awq_gemm with 33 .. 64 rows takes the one-pass kernel on layers of any size (by default
- *            on large layers only) and split_k forces its K split; without room for the split's
+ *            from 320 Mi weights on) and split_k forces its K split; without room for the split's
  *            partial tiles it runs unsplit
  * The workspace must be large enough for the form that is forced: the sizes the public queries
  * return cover every variant except a forced MFMA tile size, which silently runs without its K
@@ -62,8 +62,7 @@ enum {
   AWQMI_FORM_FUSED = 2,   /* awq_gemm_tile_kernel: weights unpacked per tile in registers */
   AWQMI_FORM_DENSE = 3,   /* awq_dequant_panel_kernel + awq_gemm_dense_kernel */
   AWQMI_FORM_GENERIC = 4, /* any-shape fallback */
-  AWQMI_FORM_MID = 5      /* 33 .. 64 rows of a large layer in one pass: awq_gemm_mid_kernel on the largest, else one
-                           * row of awq_gemm_tile_kernel's tiles */
+  AWQMI_FORM_MID = 5      /* awq_gemm_mid_kernel: 33 .. 64 rows of the largest layers in one pass */
 };
 int awqmi_dev_last_gemm_form(void);
 

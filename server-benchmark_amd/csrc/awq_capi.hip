@@ -226,39 +226,21 @@ int mid_pick_split(int K, int N) {
   return best;
 }
 
-// From 33 to 64 rows: the layers that count as the one-pass form, and the kernel they run on.
-// The lines of mid_pays were drawn where awq_gemm_mid_kernel beat the 64-row tile of the kernel that dequantised into
-// LDS (1700 points: 19 values of K from 512 to 40960, N from 1024 to 79000; from 40 Mi weights on 2048 rows, always from 13312 weight
-// rows on, elsewhere by size, by how even its K ranges are, and later where rows of qweight are no whole 128-byte lines).
-// Against awq_gemm_tile_kernel, whose tiles of 48 and 64 rows hold all rows of the call too, the mid kernel is faster on the
-// largest of them only: mid_beats_tile.  Both, mid / tile, at 40, 48 and 64 rows (us, weights from HBM, rows as the layer
+// From 33 to 64 rows: awq_gemm_mid_kernel on the largest layers, where it beats awq_gemm_tile_kernel, whose tiles of 48 and 64 rows hold
+// all rows of the call too.  Both, mid / tile, at 40, 48 and 64 rows (us, weights from HBM, rows as the layer
 // method keeps them): 16512 x 43904 (691 Mi weights, G = 32) 148, 149, 152 / 150, 149, 215; 8192 x 59136 (462 Mi) 81, 78, 80 / 79, 78,
 // 85; 15360 x 22848 (334 Mi) 78, 76, 77 / 75, 76, 79; 7936 x 41792 (316 Mi) 75, 74, 75 / 67, 67, 70; 29568 x 8192 49, 48, 49 / 44,
 // 44, 49; 8192 x 10240 26.4, 26.1, 27.6 / 22, 22, 23; 8320 x 5120 23, 23, 24 / 17.9, 17.8, 18.4; 13312 x 5632 28, 27, 28 / 22, 22, 23.
-// On 34 layers of mid_pays below the line the tile is 14 % faster on average and 0.3 % slower at worst.
-constexpr long long MID_MIN_WEIGHTS = 40LL << 20;
+// On 34 layers of 40 Mi weights and more below the line the tile is 14 % faster on average and 0.3 % slower at worst.  Its column
+// blocks run in whole rounds of workgroups: above 256 of them only multiples of 256.
+constexpr long long MID_MIN_WEIGHTS = 320LL << 20;
 inline bool mid_shape(int M, int K, int N) {
   const int ncb = (N + 255) / 256;
   return M > 32 && M <= MID_MAX_ROWS && K % 128 == 0 && N % 16 == 0 && K >= 2048 &&
          (long long)K * N >= MID_MIN_WEIGHTS && (ncb <= 256 || ncb % 256 == 0);
 }
-inline bool mid_pays(int M, int K, int N, int G, int ldw) {
-  if (!mid_shape(M, K, N)) return false;
-  const bool lines = ldw % 32 == 0;
-  const int ncb = (N + 255) / 256;
-  if (K >= (lines ? 13312 : 16384)) return true;
-  if (ncb <= 20) return K >= (lines ? 8192 : 11008);
-  const int nchunks = K / 128, parts = 4 * mid_pick_split(K, N);
-  const bool even = (nchunks + parts - 1) / parts * parts * 8 <= nchunks * 9;
-  const int heavy = (M > 48) + (G == 32);
-  const long long mi = (long long)K * N >> 20;
-  if (N % 2048 == 0 && K >= 3072 && even) return mi >= (heavy == 2 ? 80 : 40);
-  return mi >= (ncb > 128 ? 72 : 88) + (lines ? 0 : 24) + 8 * heavy + (even ? 0 : 16);
-}
-constexpr long long MID_KERNEL_WEIGHTS = 320LL << 20;
-inline bool mid_beats_tile(int K, int N) { return (long long)K * N >= MID_KERNEL_WEIGHTS; }
 inline bool mid_rows(int M, int K, int N, int G, int ldw) {
-  return (mid_pays(M, K, N, G, ldw) || (variant_on(VAR_MID) && M > 32 && M <= MID_MAX_ROWS && N % 16 == 0)) &&
+  return (mid_shape(M, K, N) || (variant_on(VAR_MID) && M > 32 && M <= MID_MAX_ROWS && N % 16 == 0)) &&
          gemv_tiled_ok(K, G) && (size_t)M * K * 2 < (1ull << 31) && (size_t)K * ldw * 4 < (1ull << 31) &&
          !variant_on(VAR_MID_M_SKINNY) && !variant_on(VAR_MID_M_MFMA);
 }
@@ -699,8 +681,7 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
     p.sk_part = room ? reinterpret_cast<float*>(static_cast<char*>(workspace) + AWQMI_WS_COUNTER_BYTES) : nullptr;
     launch_tile(pl.rt, p, st);
   };
-  const bool mid = mid_rows(M, K, N, G, ldw);
-  if (mid && (variant_on(VAR_MID) || mid_beats_tile(K, N))) {
+  if (mid_rows(M, K, N, G, ldw)) {
     t_last_gemm_form = AWQMI_FORM_MID;
     MidGemmParams p{};
     p.x = xx; p.qw = qw; p.sc = sc; p.qz = qz; p.y = yy;
@@ -807,7 +788,7 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
         return launch_status();
       }
     }
-    t_last_gemm_form = mid ? AWQMI_FORM_MID : AWQMI_FORM_FUSED;
+    t_last_gemm_form = AWQMI_FORM_FUSED;
     const int forced = forced_tile();
     for (int r0 = 0; r0 < M; r0 += slab) {
       const int Ms = M - r0 < slab ? M - r0 : slab;

@@ -16,7 +16,7 @@
 // delivers the 16 KiB of a CU (counters on 8192 x 59136: 63 % of a wave's cycles issue, 23 % are ready and do not,
 // 14 % wait for memory or LDS; on 8192 x 10240 and 8192 x 8192 it is 49, 27 - 30 and 21 - 24 %).  8192 x 59136 at 64 rows
 // takes 79 us (3.2 TB/s of packed weights), the tile kernel 85; the tile is ahead on layers of fewer than 320 Mi weights
-// (see mid_beats_tile).  Measured and dropped: two waves per SIMD with 128 columns each
+// (see mid_shape).  Measured and dropped: two waves per SIMD with 128 columns each
 // (64-byte pieces of a row per load, X read twice: 105 us), 32 x 32 x 16 MFMAs with one word per lane
 // (twice the load instructions: 94 us), X in 64-byte pieces (84 us).
 //

@@ -27,7 +27,7 @@
 // 757 / 1500; 29568 x 8192 at 96 / 400 / 1000 81 / 226 / 433 -> 58 / 171 / 383; 3584 x 4608 at 64 / 1000 18.1 / 51 -> 15.7 / 42.
 // Tiles of up to 128 rows share a CU in pairs (us, one / two workgroups: 8192 x 59136 at 256 rows in 128-row tiles 234 / 216, 3584 x
 // 37888 100 / 85, 1024 x 12288 at 2047 60 / 53; a single round is even, 123 / 126).  32- and 48-row tiles against the skinny and the
-// one-pass kernel stand at low_tile_pays and mid_pays.
+// one-pass kernel stand at low_tile_pays and mid_shape.
 // Measured and dropped: eight waves on two K halves of a tile, two per SIMD (8192 x 59136 at 64 rows 80 against 84 us, split
 // layers slower); a ring of distinct LDS objects with the compiler's own waits (even, four times the code).
 #pragma once

@@ -187,58 +187,76 @@ def test_mid_kernel_split_writes_its_partial_tiles(sba, gpu, M, K, N, G, split):
     assert torch.isnan(part[:split, :, mb:]).all() and torch.isnan(part[split]).all()
 
 
-@pytest.mark.parametrize("M,K,N,pad", [(64, 5120, 8192, True), (33, 5120, 8192, False), (48, 16384, 2560, False)])
-def test_mid_kernel_by_default_on_large_layers(sba, gpu, M, K, N, pad):
-    """Large layers take the one-pass kernel at 33 .. 64 rows, with padded rows of qweight too; without room
-    for the partial tiles of a K split it runs unsplit."""
+@pytest.mark.parametrize("M,K,N,pad,mid", [(64, 5120, 8192, True, False), (33, 5120, 8192, False, False), (48, 16384, 2560, False, False),
+                                           (64, 8192, 40960, True, True), (33, 32768, 10240, False, True)])
+def test_mid_kernel_by_default_on_large_layers(sba, gpu, M, K, N, pad, mid):
+    """The largest layers take the one-pass kernel at 33 .. 64 rows, others one row of tiles, with padded rows of qweight too;
+    without room for the partial tiles of a K split both run unsplit."""
     from server_benchmark_amd import _lib
     lib = _lib.load()
-    c = sba.workloads.make_linear_case(M, K, N, 128, seed=M).to(gpu)
-    qw = sba.ops.pad_qweight_rows(c.qweight) if pad else c.qweight
-    y = sba.awq_gemm(c.x, qw, c.scales, c.qzeros, 0)
-    assert lib.awqmi_dev_last_gemm_form() == _lib.FORM_MID
-    w = sba.awq_dequantize(c.qweight, c.scales, c.qzeros, 0, 0, 0)
-    ref = c.x.float() @ w.float()
+    form = _lib.FORM_MID if mid else _lib.FORM_FUSED
+    g = torch.Generator(device=gpu).manual_seed(M)
+    words = lambda *shape: torch.randint(-2**31, 2**31, shape, dtype=torch.int32, device=gpu, generator=g)
+    q, qz = words(K, N // 8), words(K // 128, N // 8)
+    s = (torch.rand((K // 128, N), device=gpu, generator=g) * 0.019 + 0.001).half()
+    x = torch.randn((M, K), device=gpu, generator=g).half()
+    qw = sba.ops.pad_qweight_rows(q) if pad else q
+    y = sba.awq_gemm(x, qw, s, qz, 0)
+    assert lib.awqmi_dev_last_gemm_form() == form
+    ref = x.float() @ sba.awq_dequantize(q, s, qz, 0, 0, 0).float()
     assert float((y.float() - ref).norm() / ref.norm()) <= TOL
     small = torch.zeros(65536, dtype=torch.uint8, device=gpu)
     y1 = torch.empty_like(y)
-    st = lib.awqmi_gemm_f16(c.x.data_ptr(), c.qweight.data_ptr(), c.scales.data_ptr(), c.qzeros.data_ptr(), y1.data_ptr(),
+    st = lib.awqmi_gemm_f16(x.data_ptr(), q.data_ptr(), s.data_ptr(), qz.data_ptr(), y1.data_ptr(),
                             small.data_ptr(), small.numel(), M, K, N, 128, 0, torch.cuda.current_stream().cuda_stream)
-    assert st == 0 and lib.awqmi_dev_last_gemm_form() == _lib.FORM_MID
+    assert st == 0 and lib.awqmi_dev_last_gemm_form() == form
     assert float((y1.float() - ref).norm() / ref.norm()) <= TOL
 
 
 @pytest.mark.parametrize("M,K,N,G,mid", [
     (64, 768, 58368, 128, False),
     (33, 1920, 24576, 64, False),
-    (64, 4096, 12288, 128, True),
-    (64, 4096, 12288, 64, True),
+    (64, 4096, 12288, 128, False),
+    (64, 4096, 12288, 64, False),
     (64, 4096, 12288, 32, False),
-    (33, 4096, 12288, 32, True),
-    (64, 4096, 20480, 32, True),
+    (33, 4096, 12288, 32, False),
+    (64, 4096, 20480, 32, False),
     (64, 3584, 12288, 128, False),
     (64, 4096, 11776, 128, False),
     (40, 4096, 22272, 64, False),
-    (40, 4096, 22784, 64, True),
+    (40, 4096, 22784, 64, False),
     (64, 4096, 22784, 64, False),
-    (64, 4096, 24832, 64, True),
+    (64, 4096, 24832, 64, False),
     (40, 4096, 28432, 128, False),
-    (40, 4096, 28944, 128, True),
+    (40, 4096, 28944, 128, False),
     (40, 5120, 20736, 128, False),
     (40, 2560, 29184, 128, False),
-    (40, 2560, 33024, 128, True),
+    (40, 2560, 33024, 128, False),
     (48, 10880, 4112, 32, False),
-    (48, 11008, 4112, 32, True),
+    (48, 11008, 4112, 32, False),
     (64, 8064, 5376, 128, False),
-    (64, 8320, 5120, 128, True),
+    (64, 8320, 5120, 128, False),
     (64, 13184, 5632, 128, False),
-    (64, 13312, 5632, 128, True),
+    (64, 13312, 5632, 128, False),
     (64, 13312, 5648, 128, False),
-    (64, 16384, 5648, 128, True),
+    (64, 16384, 5648, 128, False),
+    # both sides of 320 Mi weights, of whole 16 columns and 128 rows, of 256 column blocks and their multiples
+    (33, 8192, 40960, 128, True),
+    (64, 8192, 40960, 64, True),
+    (49, 8192, 40960, 32, True),
+    (64, 8192, 40944, 128, False),
+    (65, 8192, 40960, 128, False),
+    (48, 65536, 5120, 32, True),
+    (40, 2560, 131072, 64, True),
+    (40, 1920, 196608, 128, False),
+    (40, 4096, 82176, 128, False),
+    (64, 8192, 40968, 128, False),
+    (40, 8256, 40960, 64, False),
 ])
 def test_one_pass_kernel_rule(sba, gpu, M, K, N, G, mid):
-    """Which layers take the one-pass kernel at 33 .. 64 rows, on both sides of every line of the rule,
-    and their products against the dequantised weights."""
+    """Which layers take the one-pass kernel at 33 .. 64 rows, on both sides of every line of the rule (the first ones, of up to
+    113 Mi weights, are on both sides of where it stopped beating an earlier tile kernel), and their products against the
+    dequantised weights."""
     from server_benchmark_amd import _lib
     g = torch.Generator(device=gpu).manual_seed(K + N)
     words = lambda *shape: torch.randint(-2**31, 2**31, shape, dtype=torch.int32, device=gpu, generator=g)
@@ -252,19 +270,24 @@ def test_one_pass_kernel_rule(sba, gpu, M, K, N, G, mid):
 
 
 @pytest.mark.parametrize("split", [1, 8, 64])
-def test_one_pass_kernel_ignores_split_k(sba, gpu, split):
+@pytest.mark.parametrize("M,K,N,mid", [(64, 5120, 8192, False), (64, 8192, 40960, True), (64, 32768, 10240, True)])
+def test_one_pass_kernel_ignores_split_k(sba, gpu, M, K, N, mid, split):
     """More than 32 rows ignore split_k, with a workspace and without one of the caller's: the same bits
     from the same kernel as the library's own choice (64 partial tiles a column block would not fit the
     static scratch array, and a split of 1 would leave most of the chip idle)."""
     from server_benchmark_amd import _lib
     lib = _lib.load()
-    M, K, N, G = 64, 5120, 8192, 128
-    c = sba.workloads.make_linear_case(M, K, N, G, seed=1).to(gpu)
-    y = sba.awq_gemm(c.x, c.qweight, c.scales, c.qzeros, 0)
-    assert lib.awqmi_dev_last_gemm_form() == _lib.FORM_MID
-    y1 = sba.awq_gemm(c.x, c.qweight, c.scales, c.qzeros, 0, force_split_k=split)
-    y2 = sba.ops.awq_gemm_noalloc(c.x, c.qweight, c.scales, c.qzeros, torch.empty_like(y), force_split_k=split)
-    assert lib.awqmi_dev_last_gemm_form() == _lib.FORM_MID
+    form = _lib.FORM_MID if mid else _lib.FORM_FUSED
+    g = torch.Generator(device=gpu).manual_seed(1)
+    words = lambda *shape: torch.randint(-2**31, 2**31, shape, dtype=torch.int32, device=gpu, generator=g)
+    qw, qz = words(K, N // 8), words(K // 128, N // 8)
+    s = (torch.rand((K // 128, N), device=gpu, generator=g) * 0.019 + 0.001).half()
+    x = torch.randn((M, K), device=gpu, generator=g).half()
+    y = sba.awq_gemm(x, qw, s, qz, 0)
+    assert lib.awqmi_dev_last_gemm_form() == form
+    y1 = sba.awq_gemm(x, qw, s, qz, 0, force_split_k=split)
+    y2 = sba.ops.awq_gemm_noalloc(x, qw, s, qz, torch.empty_like(y), force_split_k=split)
+    assert lib.awqmi_dev_last_gemm_form() == form
     assert torch.equal(y, y1) and torch.equal(y, y2)
 
 
