@@ -185,7 +185,7 @@ def test_moe_grouped_gemm_32_row_forms(sba, gpu, T, E, topk, K, N, G, variant):
     (128, 700, 3, 3, 640, 1024, 128),   # several blocks per expert
 ])
 def test_moe_grouped_gemm_mfma_blocks(sba, gpu, bs, T, E, topk, K, N, G):
-    """The grouped GEMM over 64 / 128 / 256-row blocks (the MFMA kernel's expert-grouped form)
+    """The grouped GEMM over 64 / 128 / 256-row blocks (the tile kernel's expert-grouped form)
     against per-slot oracle products, with routing weights."""
     rng = np.random.default_rng(bs + T + K)
     w = rng.integers(0, 16, (E, K, N))
@@ -223,8 +223,8 @@ def test_moe_grouped_gemm_mfma_blocks(sba, gpu, bs, T, E, topk, K, N, G):
 
 @pytest.mark.parametrize("bs", [64, 128, 256])
 def test_moe_grouped_gemm_partly_filled_blocks(sba, gpu, bs):
-    """Blocks of the grouped MFMA kernel take a tile of as many rows as they hold real slots, in steps
-    of 64: experts with row counts on both sides of every step, one expert without rows, one with
+    """Blocks of the grouped tile kernel run on tiles of as many rows as they hold real slots:
+    experts with row counts on both sides of every 64 rows, one expert without rows, one with
     several blocks, against per-expert oracle products."""
     counts = [1, 64, 65, 128, 0, 129, 192, 193, 256, 257, 3 * 256 + 66]
     E, K, N, G = len(counts), 256, 264, 64
@@ -329,16 +329,40 @@ def test_fused_call_on_the_grouped_kernel_at_the_tile_edges(sba, gpu, variant, H
             assert float((y[r].float() - plain[r]).norm() / plain[r].norm()) <= TOL, e
 
 
+@pytest.mark.parametrize("G", [64, 128])
+def test_tiles_of_16_slot_blocks_are_as_near_to_64_bits_as_single_blocks(sba, gpu, G):
+    """16-slot blocks in tiles add their group sums in another order than one by one, and subtract the zero points before the
+    product instead of behind it: the result moves by some 2e-4 (the roundings of gate / up, activation and slot row on the way),
+    not further from the product in 64 bits."""
+    T, H, I, E = 1000, 1024, 512, 16
+    c = sba.workloads.make_moe_case(T, H, E, 1, I, G, seed=G).to(gpu)
+    own = torch.arange(T, device=gpu) % E
+    c.logits.zero_()
+    c.logits[torch.arange(T, device=gpu), own] = 8.0
+    def exact(q, s, z):
+        w = awq_ref.unpack_awq(q.cpu().numpy()).astype(np.float64) - awq_ref.unpack_awq(z.cpu().numpy()).astype(np.float64).repeat(G, 0)
+        return torch.from_numpy(w * s.cpu().numpy().astype(np.float64).repeat(G, 0)).to(gpu)
+    ref = torch.empty((T, H), dtype=torch.float64, device=gpu)
+    for e in range(E):
+        gate, up = (c.x[own == e].double() @ exact(*(t[e] for t in c.w13))).chunk(2, dim=-1)
+        ref[own == e] = (torch.nn.functional.silu(gate) * up) @ exact(*(t[e] for t in c.w2))
+    tiles, single = (sba.fused_moe_awq(c.x, c.w13, c.w2, c.logits, 1, True, _dev_variant=v).double() for v in (512, 2048))
+    assert not torch.equal(tiles, single)
+    # 1 %: what the two do not share, about half of either error, moves the norm of a million values' error by 0.1 %
+    assert float((tiles - ref).norm()) <= 1.01 * float((single - ref).norm())
+
+
 @pytest.mark.parametrize("T,H,E,topk,I,mfma", [(2048, 2048, 128, 8, 768, False), (1024, 1024, 8, 2, 2048, False),
                                                (4096, 512, 4, 2, 384, False),     # many rows per expert
                                                (640, 256, 4, 1, 1152, False),     # top-1
                                                (8192, 2048, 128, 8, 768, True), (4096, 2048, 64, 6, 1408, True)])
 def test_fused_call_on_prefill_batches(sba, gpu, T, H, E, topk, I, mfma):
-    """Batches with many slots per expert, where the one-call path takes 16-row blocks with the
-    weight ring in LDS or (mfma) the MFMA kernel's 64 / 128 / 256-row blocks: against the dense
-    expert path and against the step-by-step path over 16-row blocks."""
+    """Batches with many slots per expert, where the one-call path takes 16-row blocks, one by one with the
+    weight ring in LDS or (first case) in tiles of up to four, or (mfma) 64 / 128 / 256-row blocks of the tile kernel:
+    against the dense expert path and against the step-by-step path over 16-row blocks."""
     from server_benchmark_amd import _lib
     assert (_lib.load().awqmi_fused_moe_block_rows(T, H, I, E, topk, 128) >= 64) == mfma
+    assert _lib.load().awqmi_dev_fused_moe_tiles(T, H, I, E, topk, 128, -1) == (T == 2048)
     c = sba.workloads.make_moe_case(T, H, E, topk, I, 128, seed=T + I).to(gpu)
     one = sba.fused_moe_awq(c.x, c.w13, c.w2, c.logits, topk, True)
     ref = _dense_expert_reference(sba, c, gpu, T, H, E, topk, I)
@@ -554,7 +578,7 @@ def test_moe_block_sigmoid_routing(sba, gpu):
 @pytest.mark.parametrize("T", [64, 3000])
 def test_moe_block_sigmoid_routing_larger_batches(sba, gpu, T):
     """Sigmoid-routed block at batch sizes that take the separate routing kernel and, at 3000
-    tokens, the multi-workgroup align and the MFMA blocks: against the dense expert path with the
+    tokens, the multi-workgroup align and larger blocks: against the dense expert path with the
     routing kernel's own ids and weights."""
     H, E, topk, I = 512, 32, 6, 256
     c = sba.workloads.make_moe_case(T, H, E, topk, I, 128, seed=T).to(gpu)

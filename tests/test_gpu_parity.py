@@ -129,23 +129,35 @@ def test_gemm_decode_left_over_chunks_step_by_step(sba, gpu, K, N, split, M):
 
 @pytest.mark.parametrize("M", [17, 24, 32, 33, 48, 64])
 def test_gemm_mid_m_skinny_passes(sba, gpu, M):
-    """17 <= M <= 64 runs the skinny kernel in passes of up to 32 rows (two row blocks share
-    every unpacked weight)."""
+    """17 .. 32 rows with a set K split run one pass of the skinny kernel (two row blocks share every unpacked weight),
+    without one a tile of 32 rows; more rows ignore the split and run tiles; the skinny kernel's passes of up to 32 rows over
+    all of them by development variant bit 1 << 18."""
+    from server_benchmark_amd import _lib
+    form = _lib.load().awqmi_dev_last_gemm_form
     x, qw, s, qz = _np_case(M, 1024, 512, 128, seed=200 + M)
     for split in (0, 1, 4):
         _check_gemm(sba, gpu, x, qw, s, qz, 128, split, tag="mid-M")
+        assert form() == (_lib.FORM_SKINNY if split and M <= 32 else _lib.FORM_FUSED)
+        _check_gemm(sba, gpu, x, qw, s, qz, 128, split, tag="mid-M skinny", variant=1 << 18)
+        assert form() == _lib.FORM_SKINNY
     x, qw, s, qz = _np_case(M, 512, 264, 64, seed=300 + M)      # ragged N, G = 64
     _check_gemm(sba, gpu, x, qw, s, qz, 64, 0, tag="mid-M")
 
 
-@pytest.mark.parametrize("M,K,N,G,split", [(17, 4096, 264, 128, 1), (32, 3072, 2048, 64, 1), (24, 12288, 512, 128, 0),
-                                           (32, 8192, 256, 1024, 2)])
+@pytest.mark.parametrize("M,K,N,G,split", [(17, 4096, 272, 128, 1), (32, 3072, 2048, 64, 1), (24, 12288, 512, 128, 4),
+                                           (32, 8192, 256, 1024, 2), (24, 3072, 33280, 32, 0)])
 def test_gemm_32_row_pass_with_lds_weight_ring(sba, gpu, M, K, N, G, split):
-    """17 .. 32 rows over long wave ranges keep the weight ring in LDS; the register-ring form
-    (development variant bit 4096) must give the same bits."""
+    """17 .. 32 rows over long wave ranges (24 chunks of 128 rows a part and more) keep the weight ring in LDS; the
+    register-ring form (development variant bit 4096) must give the same bits.  Every case runs the skinny kernel: two words a
+    lane, and a set split or groups that no tile takes."""
+    from server_benchmark_amd import _lib
+    lib = _lib.load()
     x, qw, s, qz = _np_case(M, K, N, G, seed=M + K)
+    assert K // 128 >= 24 * (split or lib.awqmi_gemm_auto_split_k(M, K, N, G))
     y = _check_gemm(sba, gpu, x, qw, s, qz, G, split, tag="32-row lds ring")
+    assert lib.awqmi_dev_last_gemm_form() == _lib.FORM_SKINNY
     y_reg = sba.awq_gemm(*_dev(gpu, x, qw, s, qz), force_split_k=split, _dev_variant=4096).cpu().numpy()
+    assert lib.awqmi_dev_last_gemm_form() == _lib.FORM_SKINNY
     assert np.array_equal(y.view(np.uint16), y_reg.view(np.uint16))
 
 
@@ -293,8 +305,7 @@ def test_one_pass_kernel_ignores_split_k(sba, gpu, M, K, N, mid, split):
 
 @pytest.mark.parametrize("M", [32, 33, 48, 64])
 def test_gemm_wide_layer_mid_m(sba, gpu, M):
-    """More than 128 column tiles: 32 rows run as one skinny pass, 33 .. 64 rows on the 64-row
-    MFMA tile, whose tiles alone exceed one round of workgroups here."""
+    """More than 128 column tiles: 32, 48 and 64 rows run as one row of tiles of their height, unsplit."""
     x, qw, s, qz = _np_case(M, 256, 32768 + 512, 128, seed=M)
     _check_gemm(sba, gpu, x, qw, s, qz, 128, 0, tag="wide-mid-M")
 
@@ -321,7 +332,7 @@ def test_gemm_one_hot_is_exact_and_zero_weights(sba, gpu):
     bound = np.abs(xr.astype(np.float64)).sum(axis=1, keepdims=True) * 15 * float(s.max()) * 2.0 ** -18
     print(f"[w == z] max |y| = {np.abs(y).max():.3e}, bound {bound.min():.3e}", flush=True)
     assert np.all(np.abs(y.astype(np.float64)) <= bound)
-    # the MFMA path (M > 64) dequantises to exact fp16 zeros first: exact zeros there
+    # the tile kernel unpacks to exact fp16 zeros first: exact zeros there
     xl = np.random.default_rng(1).normal(0, 1, (80, K)).astype(np.float16)
     assert not sba.awq_gemm(*_dev(gpu, xl, awq_ref.pack_awq(zfull), s, qz), 0).cpu().numpy().any()
 
@@ -453,7 +464,7 @@ def test_gemm_prefill(sba, gpu, M, K, N, G):
                                      (129, 512, 512, 128), (160, 1024, 520, 64), (192, 2048, 1024, 128),
                                      (190, 512, 8192 + 256, 128)])
 def test_gemm_half_tile(sba, gpu, M, K, N, G):
-    """65 .. 192 rows run the 128- / 192-row workgroup tile (ragged rows / columns, K split included);
+    """65 .. 192 rows on the tiles that the library picks (ragged rows / columns, K split included);
     two runs agree bit for bit."""
     x, qw, s, qz = _np_case(M, K, N, G, seed=M + K + 1)
     g = K if G <= 0 else G
@@ -468,9 +479,9 @@ def test_gemm_half_tile(sba, gpu, M, K, N, G):
                                           (300, 1024, 1032, 128, 64), (300, 1024, 1032, 128, 128),
                                           (500, 1024, 1032, 128, 192), (100, 1024, 1032, 128, 256)])
 def test_gemm_several_row_tiles_of_every_size(sba, gpu, M, K, N, G, rows):
-    """Mid-sized batches: the library picks 64-, 128-, 192- or 256-row tiles per launch and runs
-    several row tiles of the size (ragged last tile, ragged columns, K split of the last round);
-    rows forces a size through the development entry point so that each one is covered."""
+    """Mid-sized batches: the library picks the height of the tiles per launch and runs
+    several row tiles of it (ragged last tile, ragged columns, K split of the last round);
+    rows forces a height through the development entry point."""
     x, qw, s, qz = _np_case(M, K, N, G, seed=M + N)
     variant = None if rows is None else (rows // 64) << 20
     y1 = _check_gemm(sba, gpu, x, qw, s, qz, G, 0, tag=f"row-tiles {rows}", variant=variant)
@@ -605,9 +616,9 @@ def test_gemm_dequantise_once_form(sba, gpu, M, K, N, G):
 
 
 def test_gemm_dequantise_once_default_rule_and_small_workspace(sba, gpu):
-    """From 2048 rows on the public entry point takes the dequantise-once form when the workspace
-    holds the panel (a row-padded qweight included) and the fused kernel when it does not; both
-    return the same bits."""
+    """Fewer than 512 weight rows, from 2048 rows on a wide layer and from 4096 on a narrow one: the public entry point takes the
+    dequantise-once form when the workspace holds the panel (a row-padded qweight included) and the tile kernel when it does
+    not; the same bits here, where neither splits K."""
     from server_benchmark_amd import _lib, ops
     lib = _lib.load()
     M, K, N, G = 2048, 256, 1024 * 8, 128
@@ -630,8 +641,7 @@ def test_gemm_dequantise_once_default_rule_and_small_workspace(sba, gpu):
     assert torch.equal(y, y_small)
     ref = awq_ref.gemm_wide(x[:64], qw, s, qz, G)
     assert awq_ref.rel_frobenius(y[:64].cpu().numpy(), ref) <= TOL
-    # the same row count on a narrow layer (64 tiles of 256 x 256): the fused kernel's smaller row tiles
-    # fill the chip better, so the default stays with it; from 4096 rows on the form is taken again
+    # the same row count on a narrow layer (64 tiles of 256 x 256): the tile kernel; from 4096 rows on the form is taken again
     for rows, form in ((2048, _lib.FORM_FUSED), (4096, _lib.FORM_DENSE)):
         xn, qwn, sn, qzn = _np_case(rows, K, 2048, G, seed=12)
         xnd, qwnd, snd, qznd = _dev(gpu, xn, qwn, sn, qzn)
@@ -797,8 +807,9 @@ def _with_pitch(qw_dev, extra_words):
 @pytest.mark.parametrize("M,K,N,G,pitch,split", [
     (1, 1024, 2048, 128, 32, 0), (16, 1024, 2048, 128, 32, 0), (5, 4096, 2048, 128, 32, 3),     # skinny, tail form
     (16, 2048, 264, 64, 4, 0), (3, 512, 136, 256, 12, 2), (7, 256, 8, 32, 36, 0),                 # other groups, one word per lane
-    (24, 12288, 512, 128, 32, 0), (32, 3072, 2048, 64, 32, 1), (48, 1024, 2048, 128, 32, 0),    # 32-row passes, LDS ring
-    (64, 512, 2048, 128, 32, 0), (100, 1024, 520, 128, 8, 0), (300, 2048, 2048, 128, 32, 0),    # MFMA tiles
+    (24, 12288, 512, 128, 32, 4), (32, 3072, 2048, 64, 32, 1),                                   # 32-row passes, LDS ring
+    (24, 12288, 512, 128, 32, 0), (48, 1024, 2048, 128, 32, 0),                                  # one row of tiles
+    (64, 512, 2048, 128, 32, 0), (100, 1024, 520, 128, 8, 0), (300, 2048, 2048, 128, 32, 0),
     (700, 1024, 2064, 32, 4, 0), (512, 1024, 4096, 128, 32, 0),
     (3, 96, 40, 32, 4, 0), (20, 100, 16, 50, 8, 0)])                                              # generic kernel
 def test_qweight_with_a_row_pitch(sba, gpu, M, K, N, G, pitch, split):

@@ -61,10 +61,10 @@ def test_noalloc_gemm_matches_workspace_gemm_on_calls_in_a_row(gpu):
     lib = _lib.load()
     # decode-sized calls whose split-K sums go through the static array (8 parts, then 6 of a
     # ragged width, then a forced split on a small layer), each smaller than the one before;
-    # then the MFMA kernel with a K split that fits the array (partial tiles of 256 KiB) and one
-    # that does not (every tile on one workgroup), and a call with no split at all
+    # then the tile kernel with two K splits that fit the array (48-row tiles, 3.4 and 5.3 MiB of parts) and one
+    # that does not (64 MiB: the best plan without it), and a call with no split at all
     calls = [(16, 8192, 8192, 128, 0, 1), (4, 8192, 2048 + 264, 128, 0, 2), (3, 1024, 512, 128, 4, 3),
-             (1, 1024, 512, 128, 4, 4), (100, 2048, 520, 128, 0, 5), (300, 2048, 1024, 128, 0, 5),
+             (1, 1024, 512, 128, 4, 4), (100, 2048, 520, 128, 0, 5), (300, 2048, 1024, 128, 0, 5), (500, 8192, 8192, 128, 0, 5),
              (16, 512, 59136, 128, 0, 6), (5, 256, 264, 64, 2, 7)]
     for M, K, N, G, split, seed in calls:
         y_na, y_ws = _both(lib, gpu, M, K, N, G, split, seed)
