@@ -386,20 +386,21 @@ TilePlan pick_low_tile(int K, int N) {
   }
   return best;
 }
-// Launch of a tile height with the larger of two kernels where the layer needs it (see awq_tile).
+// Launch of a tile height with the least of three kernels that holds the layer's groups and columns (see awq_tile).
 template <int RT>
 void launch_tile(const TileGemmParams& p, hipStream_t st) {
   const dim3 grid(p.per_xcd * 8 + p.sk_tiles * p.sk_split);
-  if (p.G % 64 == 0 && p.N % 32 == 0) hipLaunchKernelGGL((awq_gemm_tile_kernel<RT, false>), grid, dim3(256), 0, st, p);
-  else hipLaunchKernelGGL((awq_gemm_tile_kernel<RT, true>), grid, dim3(256), 0, st, p);
+  if (p.G % 64 == 0 && p.N % 32 == 0) hipLaunchKernelGGL((awq_gemm_tile_kernel<RT, 0>), grid, dim3(256), 0, st, p);
+  else if (p.G >= 32) hipLaunchKernelGGL((awq_gemm_tile_kernel<RT, 2>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((awq_gemm_tile_kernel<RT, 8>), grid, dim3(256), 0, st, p);
   if (p.sk_tiles > 0) hipLaunchKernelGGL((awq_gemm_tile_reduce_kernel<RT>), dim3(p.sk_tiles * RT), dim3(256), 0, st, p);
 }
 void launch_tile(int rt, const TileGemmParams& p, hipStream_t st) {
   switch (rt) {
     case 2: {
       const dim3 grid(p.per_xcd * 8 + p.sk_tiles * p.sk_split);
-      if (p.G == 64) hipLaunchKernelGGL((awq_gemm_tile_kernel<2, false, 1>), grid, dim3(256), 0, st, p);
-      else hipLaunchKernelGGL((awq_gemm_tile_kernel<2, false, 2>), grid, dim3(256), 0, st, p);
+      if (p.G == 64) hipLaunchKernelGGL((awq_gemm_tile_kernel<2, 0, 1>), grid, dim3(256), 0, st, p);
+      else hipLaunchKernelGGL((awq_gemm_tile_kernel<2, 0, 2>), grid, dim3(256), 0, st, p);
       if (p.sk_tiles > 0) hipLaunchKernelGGL((awq_gemm_tile_reduce_kernel<2>), dim3(p.sk_tiles * 2), dim3(256), 0, st, p);
       return;
     }
@@ -1033,17 +1034,17 @@ static int moe_gemm_impl(const void* x, const int32_t* qweight, const void* scal
     hipStream_t st = (hipStream_t)stream;
 #define AWQMI_GROUPED(...) hipLaunchKernelGGL((awq_gemm_tile_grouped_kernel<__VA_ARGS__>), grid, dim3(256), 0, st, p)
     if (runs && G == 64) {
-      if (fuse_act) AWQMI_GROUPED(false, true, 1);
-      else AWQMI_GROUPED(false, false, 1);
+      if (fuse_act) AWQMI_GROUPED(0, true, 1);
+      else AWQMI_GROUPED(0, false, 1);
     } else if (runs) {
-      if (fuse_act) AWQMI_GROUPED(false, true, 2);
-      else AWQMI_GROUPED(false, false, 2);
+      if (fuse_act) AWQMI_GROUPED(0, true, 2);
+      else AWQMI_GROUPED(0, false, 2);
     } else if (any) {
-      AWQMI_GROUPED(true, false, 0);
+      AWQMI_GROUPED(2, false, 0);
     } else if (fuse_act) {
-      AWQMI_GROUPED(false, true, 0);
+      AWQMI_GROUPED(0, true, 0);
     } else {
-      AWQMI_GROUPED(false, false, 0);
+      AWQMI_GROUPED(0, false, 0);
     }
 #undef AWQMI_GROUPED
     return launch_status();

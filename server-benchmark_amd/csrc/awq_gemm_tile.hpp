@@ -74,15 +74,16 @@ constexpr int TG_W_BYTES = 64 * 128;     // packed weights of a stage: 64 k x 25
 
 // LDS of one stage: X rows, packed weights, then each wave's group parameters
 __host__ __device__ constexpr int tg_x_bytes(int rt) { return rt * 16 * 128; }
-__host__ __device__ constexpr int tg_param_bytes(bool any) { return any ? 1280 : 256; }
-__host__ __device__ constexpr int tg_slot_bytes(int rt, bool any) { return tg_x_bytes(rt) + TG_W_BYTES + 4 * tg_param_bytes(any); }
+__host__ __device__ constexpr int tg_param_bytes(int any) { return any ? 160 * any : 256; }
+__host__ __device__ constexpr int tg_slot_bytes(int rt, int any) { return tg_x_bytes(rt) + TG_W_BYTES + 4 * tg_param_bytes(any); }
 // workgroups of a CU, LDS of each for the ring (the rest holds the slot lists of a grouped launch), and its stages
-__host__ __device__ constexpr int tg_occupancy(int rt, bool any) { return rt <= (any ? 5 : 8) ? 2 : 1; }
+__host__ __device__ constexpr int tg_occupancy(int rt, int any) { return rt <= (any ? 5 : 8) ? 2 : 1; }
 __host__ __device__ constexpr int tg_lds_bytes(int most, int occ) { return (160 * 1024 / occ - 128 * most - 256) / 1024 * 1024; }
-__host__ __device__ constexpr int tg_depth(int rt, bool any, int lds) {
+__host__ __device__ constexpr int tg_depth(int rt, int any, int lds) {
   const int fit = lds / tg_slot_bytes(rt, any);
   return fit < 7 ? fit : 7;
 }
+static_assert(tg_depth(4, 2, tg_lds_bytes(4, tg_occupancy(4, 2))) >= 4, "a tile of 64 rows keeps three stages on their way");
 // floats of a K split's partial tile
 __host__ __device__ constexpr size_t tg_part_floats(int rt) { return (size_t)rt * 16 * 256; }
 // X fragments in flight: a divisor of the 2 RT fragments of a stage
@@ -158,8 +159,10 @@ __device__ __forceinline__ void tg_wait_and_barrier() {
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(VM) : "memory");
 }
 
-// RT: 16-row tiles of the workgroup tile.  ANY = false: G a multiple of 64 (a stage lies in one group) and N of 32;
-// ANY = true: also G a power of two from 8 on, and any N.
+// RT: 16-row tiles of the workgroup tile.  ANY = 0: G a multiple of 64 (a stage lies in one group) and N of 32.
+// ANY = groups of a stage that there is room for, 2 or 8: also G a power of two from 64 / ANY on, and any N.  Room for 8 leaves a
+// tile of 64 rows three stages of the ring, which do not cover HBM; groups of 32 and ragged columns, which take 2, have four (us, 8 / 2:
+// 3840 x 36736, G = 32, at 54 rows 64 / 45; 2048 x 50512, G = 32, at 50 39 / 29; 2048 x 37272, G = 64, at 57 37 / 28).
 // GROUPED: rows are slots of one expert e, s_sid the slot of each row (n_slots or more: none), s_tw its output weight.
 // ACT (grouped): the matrix is [gate | up]; the tile is 128 gate columns from n0 on and their up columns, and
 // writes silu(gate) * up.
@@ -167,12 +170,12 @@ __device__ __forceinline__ void tg_wait_and_barrier() {
 // scaled in fp32 when the group ends -- the skinny kernel's precision, for tiles that take its place.  The group's sum and the
 // total are both in vector registers, so that tiles are at most 64 rows high, and stages go in pairs (ke - kb is even); the scaling is dealt out over the next
 // group's first k-step.
-template <int RT, int D, bool ANY, bool GROUPED, bool ACT, int SCALE32 = 0>
+template <int RT, int D, int ANY, bool GROUPED, bool ACT, int SCALE32 = 0>
 __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, const int n0, const int kb, const int ke,
                                          float* const part, const int e, const uint32_t smem, const int* const s_sid,
                                          const float* const s_tw) {
   constexpr int XB = tg_x_bytes(RT), SLOT = tg_slot_bytes(RT, ANY), PW = tg_param_bytes(ANY);
-  constexpr int ZO = ANY ? 1024 : 128;        // zero points behind the scales
+  constexpr int ZO = ANY ? 128 * ANY : 128;   // zero points behind the scales
   constexpr int XL = (RT + 1) / 2;            // X loads of a wave and stage
   constexpr int NL = XL + (ANY ? 4 : 3);      // all loads: weights (2), group parameters, X
   constexpr int XF = tg_ring(RT);
@@ -514,7 +517,7 @@ __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, 
 }
 #endif  // __HIP_DEVICE_COMPILE__
 
-template <int RT, bool ANY, int SCALE32 = 0>
+template <int RT, int ANY, int SCALE32 = 0>
 __global__ __launch_bounds__(256, tg_occupancy(RT, ANY)) void awq_gemm_tile_kernel(const TileGemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int D = tg_depth(RT, ANY, tg_lds_bytes(RT, tg_occupancy(RT, ANY)));
@@ -563,10 +566,11 @@ __global__ __launch_bounds__(256, tg_occupancy(RT, ANY)) void awq_gemm_tile_kern
 // few experts the ranges are uneven in rows and launch order is better.
 constexpr int TG_ROWS = 128;   // slots of a tile at most
 constexpr int TG_RUN = 4;      // 16-slot blocks of a SCALE32 tile at most
-template <bool ANY, bool ACT, int SCALE32>
-__global__ __launch_bounds__(256, tg_occupancy(TG_ROWS / 16, ANY)) void awq_gemm_tile_grouped_kernel(const TileGemmParams p) {
+constexpr int TG_GROUPED_WGS = 2;   // workgroups of a CU (groups of 32, 3000 tokens on 128 experts of 2048 x 768: one 422 us, two 345)
+template <int ANY, bool ACT, int SCALE32>
+__global__ __launch_bounds__(256, TG_GROUPED_WGS) void awq_gemm_tile_grouped_kernel(const TileGemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  constexpr int ROWS = SCALE32 ? 16 * TG_RUN : TG_ROWS, LDS = tg_lds_bytes(TG_ROWS / 16, tg_occupancy(TG_ROWS / 16, ANY));
+  constexpr int ROWS = SCALE32 ? 16 * TG_RUN : TG_ROWS, LDS = tg_lds_bytes(TG_ROWS / 16, TG_GROUPED_WGS);
   __shared__ __align__(1024) unsigned char smem[LDS];
   __shared__ int s_sid[ROWS];
   __shared__ float s_tw[ROWS];

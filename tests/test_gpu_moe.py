@@ -279,6 +279,7 @@ TILE_EDGES = [1, 16, 17, 32, 33, 48, 0, 49, 64, 65, 80, 81, 96, 97, 112, 113, 12
 @pytest.mark.parametrize("bs,K,N,G", [
     (64, 128, 256, 128), (128, 256, 264, 64), (256, 640, 512, 128), (256, 1280, 288, 128),   # 2 ... 20 stages of 64 k
     (128, 256, 72, 32), (256, 384, 520, 384), (64, 256, 40, 64),      # groups and columns of the general form
+    (128, 1280, 264, 32), (256, 1152, 512, 32),                       # ... over more stages than the ring holds
 ])
 def test_moe_grouped_gemm_at_the_tile_edges(sba, gpu, bs, K, N, G, E):
     """The grouped kernel takes the lowest tile, in steps of 16 rows, that holds a block's slots (a block of 256 runs as

@@ -543,6 +543,26 @@ def test_fused_tile_of_48_rows(sba, gpu, M, K, N, G):
     assert awq_ref.rel_frobenius(y1.cpu().numpy(), y) <= TOL
 
 
+@pytest.mark.parametrize("M", [33, 64, 65, 80, 81, 128, 257])
+@pytest.mark.parametrize("N,G", [(264, 8), (264, 16), (264, 32), (256, 32), (264, 64), (264, 128)])
+def test_fused_tile_groups_of_a_stage(sba, gpu, N, G, M):
+    """The tile kernel's three forms by the groups of a 64-row stage (eight; two, which ragged columns take too) over more stages
+    than its ring holds, on tiles of every ring depth: against the oracle, and on one-hot rows the dequantised weights themselves."""
+    from server_benchmark_amd import _lib
+    lib = _lib.load()
+    K = 1152
+    x, qw, s, qz = _np_case(M, K, N, G, seed=M + G)
+    _check_gemm(sba, gpu, x, qw, s, qz, G, 0, tag="groups of a stage")
+    assert lib.awqmi_dev_last_gemm_form() == _lib.FORM_FUSED
+    W = awq_ref.dequantize(qw, s, qz, G)
+    for k0 in range(0, K, M):                     # every row of W comes out once: a group misplaced shows
+        rows = min(M, K - k0)
+        one = np.zeros((M, K), np.float16)
+        one[np.arange(rows), k0 + np.arange(rows)] = 1
+        y = sba.awq_gemm(*_dev(gpu, one, qw, s, qz), 0).cpu().numpy()
+        assert np.array_equal(y[:rows], W[k0:k0 + rows])
+
+
 @pytest.mark.parametrize("M", [17, 31, 32])
 @pytest.mark.parametrize("K,N,G", [(128, 32, 64), (128, 256, 128), (384, 288, 64), (640, 544, 128), (1152, 1024, 128), (1920, 800, 64),
                                    (4096, 4128, 128), (16384, 256, 128)])
