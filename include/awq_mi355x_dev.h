@@ -22,7 +22,7 @@
  *   16384    the align step always runs in one workgroup
  *   1 << 16  v = bits 16..17: the one-call MoE block uses 64 / 128 / 256-row blocks (v = 1 / 2 / 3)
  *   1 << 18  awq_gemm with 17..64 rows: skinny passes wherever they can run
- *   1 << 19  awq_gemm with 17..64 rows: the MFMA kernel wherever it can run
+ *   1 << 19  awq_gemm with 17..64 rows: the tile kernel wherever it can run
  *   1 << 20  v = bits 20..22: fused tiles of 64 v rows (v = 1..4) or 16 v rows (v = 5..7) whatever M is
  *   1 << 29  v = bits 29..30: fused tiles of 160 / 208 / 224 rows (v = 1 / 2 / 3) whatever M is
  *   1 << 23  dense skinny launches never share left-over chunks step by step
@@ -39,7 +39,7 @@
  *            from 320 Mi weights on) and split_k forces its K split; without room for the split's
  *            partial tiles it runs unsplit
  * The workspace must be large enough for the form that is forced: the sizes the public queries
- * return cover every variant except a forced MFMA tile size, which silently runs without its K
+ * return cover every variant except a forced tile height, which silently runs without its K
  * split when the workspace is too small for it.
  */
 #ifndef AWQ_MI355X_DEV_H

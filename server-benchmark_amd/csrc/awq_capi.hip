@@ -290,7 +290,7 @@ MfmaPlan plan_mfma(int M, int K, int N, int bm) {
 // more with three quarters of a round of 256 x 256 tiles, whose prefill record and its test name the form.  Narrower ones run the tile
 // there (18944 x 3584 260 / 229, 13824 x 5120, G = 32, 283 / 261).  Layers of fewer than 512 weight rows, which no model here has, keep the
 // lines that were drawn for all: from 4096 rows on, from 2048 with those three quarters of a round.  K % 64 == 0 and G % 8 == 0 (both
-// implied by the MFMA path's conditions).
+// implied by mfma_ok).
 constexpr int DENSE_MIN_ROWS = 6144;
 // One rule for the call and for the workspace query: a call never takes the panel in room that another one's query asked for, and no
 // room is asked for that the call leaves unused.
@@ -370,8 +370,10 @@ TilePlan pick_tile(int M, int K, int N, size_t room) {
 // 29568 x 8192 37.5, 41.0 / 38.9, 38.9, G = 64 41.6, 45.1 / 41.6, 41.4), and above 256 Mi neither (8192 x 59136 64, 60 / 68, 69).  Up to 16 rows the
 // skinny kernel stays: at 16 it is 5 - 29 % faster on 12 of 16 layers, 7 % slower at worst (1024 x 12288 10.8 / 10.0), at 4 rows 15 - 49 %
 // faster.
+// Groups of 32 and of more than 128, and ragged columns, stay too: a tile scales its sums after one or two whole stages of 64 k, and
+// with weights rounded to fp16 as on higher tiles it would be less exact than the skinny kernel.
 bool low_tile_pays(int M, int K, int N, int G) {
-  return M > 16 && M <= 32 && (G == 64 || G == 128) && N % 32 == 0 && K % 128 == 0 && 
+  return M > 16 && M <= 32 && (G == 64 || G == 128) && N % 32 == 0 && K % 128 == 0 &&
          (long long)K * N < (M > 24 || G == 64 ? 256LL << 20 : 128LL << 20);
 }
 // its K split, in whole pairs of stages
@@ -760,8 +762,8 @@ int awqmi_gemm_ld_f16(const void* x, const int32_t* qweight, int ldw, const void
   // 32-bit, so every operand must stay below 4 GiB
   if (mfma_ok) {
     const int slab = mfma_slab_rows(M, K);
-    // many rows: dequantise once into the workspace, then the dense kernel (same bits as the tile kernel, which
-    // adds in the same order); needs the workspace to hold the panel
+    // many rows: dequantise once into the workspace, then the dense kernel (the tile kernel's products, added in the
+    // same order where both split K alike); needs the workspace to hold the panel
     if (dense_rows(M, K, N) && workspace && aligned16(workspace)) {
       size_t part = plan_mfma(slab < M ? slab : M, K, N, 256).part_bytes;
       if (M % slab) part = std::max(part, plan_mfma(M % slab, K, N, 256).part_bytes);
@@ -917,7 +919,7 @@ size_t awqmi_moe_gemm_workspace_bytes(int n_slots, int E, int K, int N, int spli
   if (n_slots <= 0 || E <= 0 || K <= 0 || N <= 0 || N % 8 != 0 ||
       (tile_m != 16 && tile_m != 32 && tile_m != 64 && tile_m != 128 && tile_m != 256))
     return 0;
-  if (tile_m >= 64) return AWQMI_WS_COUNTER_BYTES;    // the grouped MFMA form needs no partials
+  if (tile_m >= 64) return AWQMI_WS_COUNTER_BYTES;    // the grouped tile kernel needs no partials
   const MoePlan pl = moe_plan(n_slots, E, K, N, tile_m, split_k);
   return AWQMI_WS_COUNTER_BYTES + gemv_partial_bytes(N, pl.split, pl.nblk, tile_m);
 }
@@ -1193,16 +1195,16 @@ double moe_expected_blocks(double avg, int rows) {
 }
 
 // Rows per block for the two expert GEMMs of one MoE block: 16 (the skinny kernel) or 64 /
-// 128 / 256 (the MFMA kernel's expert-grouped form), by price:
+// 128 / 256 (the tile kernel's expert-grouped form), by price:
 //   skinny: flops / (540 TFLOP/s * avg / (avg + 26)), avg = slots per expert;
-//   MFMA:   per GEMM blocks * column tiles / 256 CUs rounds (a partial last round counts as
+//   larger: per GEMM blocks * column tiles / 256 CUs rounds (a partial last round counts as
 //           at least half) of (K / 64 + overhead) k-tiles at 5.4 ns * (rows + 112) each, plus the separate
 //           SiLU pass at 4 TB/s; blocks is the expected block count after padding each expert's run to whole
 //           blocks (slots spread evenly over the experts).
-// A second look at the larger blocks counts a partly filled block by its rows in steps of 64, as the grouped
-// kernel runs it (at 5.4 / 5.65 / 5.9 ns for 64 / 128 / 256 rows), and only goes upwards, to blocks that are fewer
-// (as many blocks run the same tiles, those of 256 rows with four waves instead of eight).
-// Every size forced in turn on 640 points (53 shapes: hidden 384 ... 7168, intermediate 384 ... 14336, 4 ... 512
+// A second look at the larger blocks counts a partly filled block by its rows in steps of 64, as that
+// kernel ran it (at 5.4 / 5.65 / 5.9 ns for 64 / 128 / 256 rows), and only goes upwards, to blocks that are fewer
+// (as many blocks run the same tiles).
+// Every size forced, with the grouped kernel before the present one, in turn on 640 points (53 shapes: hidden 384 ... 7168, intermediate 384 ... 14336, 4 ... 512
 // experts, top-1 ... 10, 32 ... 1400 slots per expert):
 //   - the choice is 1.7 % behind the best size on average, 48 % at worst (4919 tokens on 128 experts of 2048 x
 //     384: 16 rows 508 us, 256 rows 344; the first look chooses 16 rows there too);
@@ -1216,10 +1218,9 @@ double moe_expected_blocks(double avg, int rows) {
 // blocks of 16 slots end, which callers of the step-by-step path have in their own calls too.  With the present kernel, which is
 // faster for every size, and moe_runs beside it the choice is 4 % behind the best of 16, 16 in tiles and 128 on average of 129
 // points, 30 % at worst (896 tokens on 256 experts of 2048 x 384, top-8: 156 us, in tiles 120; see moe_runs for its line at 32).
-// Three sizes that the tests fix measure slower than another: 2048 tokens on 128 experts of 2048 x 768 (16 rows
-// 327 us, 256 rows 279), 1024 on 160 of 6144 x 2560 (64 rows 1775, 16 rows 1684), 2102 on 4 of 512 x 384 (16 rows
-// 52, 64 rows 43).
-// The MFMA form also needs every operand under 4 GiB (32-bit buffer offsets).
+// Two sizes that the tests fix measure slower than another: 2048 tokens on 128 experts of 2048 x 768 (16 rows in tiles
+// 254 us, 128 rows 248), 2102 on 4 of 512 x 384 (16 rows 51, in tiles 38, 64 rows 36).
+// Larger blocks also need every operand under 4 GiB (32-bit buffer offsets).
 int moe_pick_tile(int n_slots, int E, int H, int inter, int group) {
   if (variant_on(VAR_MOE_TILE16)) return 16;
   if (!gemv_tiled_ok(H, norm_group(H, group)) || !gemv_tiled_ok(inter, norm_group(inter, group))) return 16;
@@ -1272,8 +1273,8 @@ int moe_pick_tile(int n_slots, int E, int H, int inter, int group) {
 // Fitted on 129 points (ten expert shapes, 6 ... 400 slots per expert), the whole block timed both ways.  The tiles have to
 // look 14 % cheaper (24 % below 16 experts, whose few long tiles the price underestimates): then no point of them is slower
 // than with the skinny kernel, and they are 8 % faster on average over all.  Up to 32 slots per expert a tile is two blocks at
-// most on average: within 5 % either way up to 25 slots, 15 % at 32 (128 experts of 2048 x 768, top-8, 400 / 512 tokens:
-// both GEMMs 97 / 121 us by blocks, 102 / 100 by tiles).  There the block keeps the kernel that the separate calls on
+// most on average: within 5 % either way up to 25 slots, 13 - 14 % faster at 28 and 32 (whole block, blocks / tiles: 400 and 512 tokens
+// on 128 experts of 2048 x 768, top-8, 105 / 103 and 125 / 110 us; 560 on 160 of 6144 x 2560 1168 / 1001).  There the block keeps the kernel that the separate calls on
 // 16-slot blocks take, so that both add in one order; so do experts below the smallest measured (1024 x 512, 2048 x 384),
 // where the routing and the sum outweigh both GEMMs.  Both sides above, blocks / tiles (us): 576 / 768 / 1024 tokens on those
 // experts 143 / 164 / 192 and 116 / 130 / 163; 384 / 512 on 64 of 2048 x 1408 136 / 158 and 102 / 114; 560 on 160 of 6144 x
