@@ -77,7 +77,7 @@ __host__ __device__ constexpr int tg_x_bytes(int rt) { return rt * 16 * 128; }
 __host__ __device__ constexpr int tg_param_bytes(int any) { return any ? 160 * any : 256; }
 __host__ __device__ constexpr int tg_slot_bytes(int rt, int any) { return tg_x_bytes(rt) + TG_W_BYTES + 4 * tg_param_bytes(any); }
 // workgroups of a CU, LDS of each for the ring (the rest holds the slot lists of a grouped launch), and its stages
-__host__ __device__ constexpr int tg_occupancy(int rt, int any) { return rt <= (any ? 5 : 8) ? 2 : 1; }
+__host__ __device__ constexpr int tg_occupancy(int rt, int any) { return rt <= (any > 2 ? 3 : any ? 5 : 8) ? 2 : 1; }
 __host__ __device__ constexpr int tg_lds_bytes(int most, int occ) { return (160 * 1024 / occ - 128 * most - 256) / 1024 * 1024; }
 __host__ __device__ constexpr int tg_depth(int rt, int any, int lds) {
   const int fit = lds / tg_slot_bytes(rt, any);
@@ -161,8 +161,9 @@ __device__ __forceinline__ void tg_wait_and_barrier() {
 
 // RT: 16-row tiles of the workgroup tile.  ANY = 0: G a multiple of 64 (a stage lies in one group) and N of 32.
 // ANY = groups of a stage that there is room for, 2 or 8: also G a power of two from 64 / ANY on, and any N.  Room for 8 leaves a
-// tile of 64 rows three stages of the ring, which do not cover HBM; groups of 32 and ragged columns, which take 2, have four (us, 8 / 2:
-// 3840 x 36736, G = 32, at 54 rows 64 / 45; 2048 x 50512, G = 32, at 50 39 / 29; 2048 x 37272, G = 64, at 57 37 / 28).
+// tile of 64 rows three stages of the ring if two share a CU, which do not cover HBM; groups of 32 and ragged columns, which take 2, have four (us, 8 / 2:
+// 3840 x 36736, G = 32, at 54 rows 64 / 45; 2048 x 50512, G = 32, at 50 39 / 29; 2048 x 37272, G = 64, at 57 37 / 28).  With room for 8,
+// tiles of 64 and 80 rows have a CU each and six or seven stages: 5 % faster on 31 layers in groups of 8 and 16 at 49 - 64 rows, even above.
 // GROUPED: rows are slots of one expert e, s_sid the slot of each row (n_slots or more: none), s_tw its output weight.
 // ACT (grouped): the matrix is [gate | up]; the tile is 128 gate columns from n0 on and their up columns, and
 // writes silu(gate) * up.
