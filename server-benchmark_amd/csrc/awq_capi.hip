@@ -59,7 +59,7 @@ enum : int {
   VAR_NO_FUSED_ACT = 1024,    // the one-call MoE block always runs the separate activation kernel
   VAR_MOE_TILE16 = 2048,      // the one-call MoE block always uses the skinny kernel's 16-row blocks
   VAR_NO_LDS_RING = 4096,     // every launch keeps the weight ring in registers
-  VAR_ALIGN_ONE_WG = 16384,   // align always in one workgroup
+  VAR_ALIGN_ONE_WG = 16384,   // the one-call MoE block aligns batches of more than one routing launch in one workgroup
   VAR_MOE_TILE_SHIFT = 16,    // bits 16..17 = v: the one-call MoE block uses 64 / 128 / 256-row blocks (v = 1 / 2 / 3)
   VAR_MID_M_SKINNY = 1 << 18, // awq_gemm with 17..64 rows: skinny passes wherever they can run
   VAR_MID_M_MFMA = 1 << 19,   // awq_gemm with 17..64 rows: the tile kernel wherever it can run
@@ -422,6 +422,36 @@ void launch_tile(int rt, const TileGemmParams& p, hipStream_t st) {
 
 }  // namespace
 
+// The routing kernels come for 16 or 64 lanes per token, 4, 8 or 16 resp. 1 to 16 experts per lane, and both scorings:
+// f(lanes, experts per lane, sigmoid) for all of them ...
+template <class F>
+static void moe_topk_forms(F&& f) {
+  using std::integral_constant;
+  auto both = [&](auto L, auto P) {
+    f(L, P, std::false_type{});
+    f(L, P, std::true_type{});
+  };
+  both(integral_constant<int, 16>{}, integral_constant<int, 4>{});
+  both(integral_constant<int, 16>{}, integral_constant<int, 8>{});
+  both(integral_constant<int, 16>{}, integral_constant<int, 16>{});
+  both(integral_constant<int, 64>{}, integral_constant<int, 1>{});
+  both(integral_constant<int, 64>{}, integral_constant<int, 2>{});
+  both(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+  both(integral_constant<int, 64>{}, integral_constant<int, 8>{});
+  both(integral_constant<int, 64>{}, integral_constant<int, 16>{});
+}
+// ... and for the one that E experts, topk of them a token, take: a row of 16 lanes holds 16 picks and 16 keys a lane.
+static int moe_topk_lanes(int E, int topk) { return E <= 256 && topk <= 16 ? 16 : 64; }
+template <class F>
+static void moe_topk_form(int E, int topk, int scoring, F&& f) {
+  const int lanes = moe_topk_lanes(E, topk);
+  int per = lanes == 16 ? 4 : 1;
+  while (lanes * per < E) per *= 2;
+  moe_topk_forms([&](auto L, auto P, auto S) {
+    if (decltype(L)::value == lanes && decltype(P)::value == per && decltype(S)::value == (scoring == 1)) f(L, P, S);
+  });
+}
+
 // Kernels that use more dynamic LDS than the default limit need a function attribute; it is
 // set once per device for all of them (by awqmi_init, or by the first call on that device that
 // needs one).
@@ -432,54 +462,20 @@ static int ensure_kernel_attributes() {
   if (ge != hipSuccess) { t_last_hip_error = (int)ge; return AWQMI_LAUNCH_FAILED; }
   if (dev < 0 || dev >= MAX_DEVICES) return AWQMI_BAD_ARGUMENT;
   if (done[dev].load(std::memory_order_acquire)) return AWQMI_OK;
-  const void* align[] = {
-      reinterpret_cast<const void*>(moe_align_kernel),
-      reinterpret_cast<const void*>(moe_align_count_kernel), reinterpret_cast<const void*>(moe_align_place_kernel),
-      reinterpret_cast<const void*>(moe_route_align_kernel<1, false>), reinterpret_cast<const void*>(moe_route_align_kernel<2, false>),
-      reinterpret_cast<const void*>(moe_route_align_kernel<4, false>), reinterpret_cast<const void*>(moe_route_align_kernel<8, false>),
-      reinterpret_cast<const void*>(moe_route_align_kernel<16, false>),
-      reinterpret_cast<const void*>(moe_route_align_kernel<1, true>), reinterpret_cast<const void*>(moe_route_align_kernel<2, true>),
-      reinterpret_cast<const void*>(moe_route_align_kernel<4, true>), reinterpret_cast<const void*>(moe_route_align_kernel<8, true>),
-      reinterpret_cast<const void*>(moe_route_align_kernel<16, true>)};
-  for (const void* fn : align) {
-    const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             (MOE_ALIGN_WAVES + 2) * AWQMI_MAX_EXPERTS * (int)sizeof(int));
-    if (e != hipSuccess) { t_last_hip_error = (int)e; return AWQMI_LAUNCH_FAILED; }
-  }
+  auto allow = [](const void* fn, int bytes) {
+    const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e != hipSuccess) t_last_hip_error = (int)e;
+    return e == hipSuccess;
+  };
+  constexpr int align_lds = (MOE_ALIGN_WAVES + 2) * AWQMI_MAX_EXPERTS * (int)sizeof(int);
+  bool ok = allow(reinterpret_cast<const void*>(moe_align_kernel), align_lds) &&
+            allow(reinterpret_cast<const void*>(moe_align_parts_kernel), moe_parts_lds(AWQMI_MAX_EXPERTS));
+  moe_topk_forms([&](auto L, auto P, auto S) {
+    ok = ok && allow(reinterpret_cast<const void*>(moe_route_align_kernel<decltype(L)::value, decltype(P)::value, decltype(S)::value>), align_lds);
+  });
+  if (!ok) return AWQMI_LAUNCH_FAILED;
   done[dev].store(true, std::memory_order_release);
   return AWQMI_OK;
-}
-
-// routing and align in one launch (at most 16 tokens); same results as the two calls
-template <int P>
-static int moe_route_align_launch(const float* logits, const float* bias, int T, int E, int topk, int scoring,
-                                  int renormalize, float scale, int32_t* ids, float* wts, int tile_m, int cap,
-                                  int32_t* sorted, int32_t* experts, int32_t* npp, hipStream_t st) {
-  if (const int rc = ensure_kernel_attributes()) return rc;
-  const size_t lds = (size_t)(MOE_ALIGN_WAVES + 2) * E * sizeof(int);
-  if (scoring == 1)
-    hipLaunchKernelGGL((moe_route_align_kernel<P, true>), dim3(1), dim3(1024), lds, st, logits, bias, T, E, topk,
-                       renormalize, scale, ids, wts, tile_m, cap, sorted, experts, npp);
-  else
-    hipLaunchKernelGGL((moe_route_align_kernel<P, false>), dim3(1), dim3(1024), lds, st, logits, (const float*)nullptr,
-                       T, E, topk, renormalize, scale, ids, wts, tile_m, cap, sorted, experts, npp);
-  return launch_status();
-}
-
-static int moe_route_align_small(const float* logits, const float* bias, int T, int E, int topk, int scoring,
-                                 int renormalize, float scale, int32_t* ids, float* wts, int tile_m,
-                                 int32_t* sorted, int32_t* experts, int32_t* npp, void* stream) {
-  const int cap = (int)awqmi_moe_align_capacity(T * topk, E, tile_m);
-  hipStream_t st = (hipStream_t)stream;
-#define AWQMI_RA(P) \
-  return moe_route_align_launch<P>(logits, bias, T, E, topk, scoring, renormalize, scale, ids, wts, tile_m, cap, \
-                                   sorted, experts, npp, st)
-  if (E <= 64) AWQMI_RA(1);
-  if (E <= 128) AWQMI_RA(2);
-  if (E <= 256) AWQMI_RA(4);
-  if (E <= 512) AWQMI_RA(8);
-  AWQMI_RA(16);
-#undef AWQMI_RA
 }
 
 // Routing of one MoE block: inputs and the five lists it produces.
@@ -493,11 +489,10 @@ struct MoeRoute {
   int32_t* sorted;
   int32_t* experts;
   int32_t* npp;
-  int32_t* runs;     // tiles of several 16-slot blocks (more than 16 tokens only)
+  int32_t* runs;     // tiles of several 16-slot blocks, or null
+  int32_t* tab;      // expert counts of the parts of a longer batch, [MOE_PARTS_MAX][E]
 };
 
-// Routing + align of a short slot list as launches of their own (one launch for up to 16
-// tokens, else top-k and align apart).
 static int moe_align_launch(const int32_t* topk_ids, int n_slots, int E, int tile_m, int32_t* sorted, int32_t* experts,
                             int32_t* npp, int32_t* runs, void* stream) {
   const int cap = (int)awqmi_moe_align_capacity(n_slots, E, tile_m);
@@ -506,22 +501,45 @@ static int moe_align_launch(const int32_t* topk_ids, int n_slots, int E, int til
                      (hipStream_t)stream, topk_ids, n_slots, E, tile_m, cap, sorted, experts, npp, runs);
   return launch_status();
 }
+// Routing + align of a block as launches of their own.  Up to 32 tokens (16 with a token a wave): one launch of one workgroup.  Up to 2048
+// slots: top-k over many, then one workgroup for the align.  More: two launches over up to MOE_PARTS_MAX workgroups, each with at least
+// sixteen tokens.  Whole block, 128 experts of 2048 x 768, top-8, us, as it was before / one launch / top-k and one workgroup / two
+// launches of parts: 16 tokens 62.2 / 59.3 / - / -; 32 72.2 / 70.5 / - / -; 48 73.3 / 72.9 / 72.5 / -; 64 75.3 / 75.3 / 74.5 / -; 128 80.6 / - /
+// 80.1 / 81.2; 256 98 / - / 97.5 / 97.3; 1500 172 / - / - / 166; 8192 696 / - / - / 688.
+constexpr int MOE_ONE_WG_SLOTS = 2048;
 static int moe_route_launches(const MoeRoute& r, int tile, void* stream) {
-  if (r.T <= MOE_ALIGN_WAVES)
-    return moe_route_align_small(r.logits, r.bias, r.T, r.E, r.topk, r.scoring, r.renorm, r.scale, r.ids, r.wts, tile,
-                                 r.sorted, r.experts, r.npp, stream);
-  if (const int st = awqmi_moe_topk_f32(r.logits, r.bias, r.T, r.E, r.topk, r.scoring, r.renorm, r.scale, r.ids, r.wts,
-                                        stream))
-    return st;
-  return moe_align_launch(r.ids, r.T * r.topk, r.E, tile, r.sorted, r.experts, r.npp, r.runs, stream);
+  if (const int rc = ensure_kernel_attributes()) return rc;
+  const int n_slots = r.T * r.topk, cap = (int)awqmi_moe_align_capacity(n_slots, r.E, tile);
+  hipStream_t st = (hipStream_t)stream;
+  const int wave_tokens = 64 / moe_topk_lanes(r.E, r.topk);
+  if (r.T <= MOE_ALIGN_WAVES * std::min(wave_tokens, 2)) {
+    moe_topk_form(r.E, r.topk, r.scoring, [&](auto L, auto P, auto S) {
+      hipLaunchKernelGGL((moe_route_align_kernel<decltype(L)::value, decltype(P)::value, decltype(S)::value>), dim3(1), dim3(1024),
+                         (size_t)(MOE_ALIGN_WAVES + 2) * r.E * sizeof(int), st, r.logits, r.bias, r.T, r.E, r.topk, r.renorm,
+                         r.scale, r.ids, r.wts, tile, cap, r.sorted, r.experts, r.npp, r.runs);
+    });
+    return launch_status();
+  }
+  if (n_slots <= MOE_ONE_WG_SLOTS || variant_on(VAR_ALIGN_ONE_WG)) {
+    if (const int rc = awqmi_moe_topk_f32(r.logits, r.bias, r.T, r.E, r.topk, r.scoring, r.renorm, r.scale, r.ids, r.wts, stream))
+      return rc;
+    return moe_align_launch(r.ids, n_slots, r.E, tile, r.sorted, r.experts, r.npp, r.runs, stream);
+  }
+  const int part = (r.T + 16 * MOE_PARTS_MAX - 1) / (16 * MOE_PARTS_MAX) * 16, parts = (r.T + part - 1) / part;
+  const int waves = std::min(16, part / wave_tokens);
+  moe_topk_form(r.E, r.topk, r.scoring, [&](auto L, auto P, auto S) {
+    hipLaunchKernelGGL((moe_route_count_kernel<decltype(L)::value, decltype(P)::value, decltype(S)::value>), dim3(parts),
+                       dim3(64 * waves), 0, st, r.logits, r.bias, r.T, r.E, r.topk, r.renorm, r.scale, r.ids, r.wts, part, r.tab);
+  });
+  hipLaunchKernelGGL(moe_align_parts_kernel, dim3(parts), dim3(1024), (size_t)moe_parts_lds(r.E), st, r.ids, n_slots, r.E,
+                     part * r.topk, tile, cap, r.tab, r.sorted, r.experts, r.npp, r.runs);
+  return launch_status();
 }
 
-// Folded routing: at most four tokens (one per wave of a workgroup; the kernel would take up to
-// eight in turn, but from five tokens on every workgroup spends on the second round what the
-// saved launch gains: 128 experts, top-8, weights from HBM: 3.5 us of 29 - 38 faster at 1 - 4
-// tokens, 0.9 us at 5, nothing at 6 - 8), 64 slots (one lane each), 256 experts (four per lane).
+// Folded routing: at most four tokens, which one wave of a workgroup picks for at once (128 experts, top-8, weights from HBM:
+// 3.5 us of 29 - 38 faster at 1 - 4 tokens; from five on, a second round in every workgroup cost what the saved launch gains).
 static bool moe_route_foldable(int T, int E, int topk, int tile) {
-  return T <= 4 && T * topk <= 64 && E <= 256 && tile == 16 && !variant_on(VAR_NO_FOLDED_ROUTE);
+  return T <= 4 && moe_topk_lanes(E, topk) == 16 && tile == 16 && !variant_on(VAR_NO_FOLDED_ROUTE);
 }
 
 extern "C" {
@@ -838,23 +856,11 @@ int awqmi_moe_topk_f32(const float* logits, const float* score_bias, int T, int 
   if (E > AWQMI_MAX_EXPERTS || topk <= 0 || topk > E || topk > 64 || (scoring != 0 && scoring != 1))
     return AWQMI_BAD_ARGUMENT;
   if (scoring == 0 && score_bias) return AWQMI_BAD_ARGUMENT;   // the bias belongs to sigmoid scoring
-  const dim3 grid((T + 3) / 4);
-  hipStream_t st = (hipStream_t)stream;
-#define AWQMI_TOPK(P)                                                                              \
-  do {                                                                                             \
-    if (scoring == 1)                                                                              \
-      hipLaunchKernelGGL((moe_topk_kernel<P, true>), grid, dim3(256), 0, st, logits, score_bias, T, E, topk, \
-                         renormalize, scale, topk_ids, topk_weights);                              \
-    else                                                                                           \
-      hipLaunchKernelGGL((moe_topk_kernel<P, false>), grid, dim3(256), 0, st, logits, score_bias, T, E, topk, \
-                         renormalize, scale, topk_ids, topk_weights);                              \
-  } while (0)
-  if (E <= 64) AWQMI_TOPK(1);
-  else if (E <= 128) AWQMI_TOPK(2);
-  else if (E <= 256) AWQMI_TOPK(4);
-  else if (E <= 512) AWQMI_TOPK(8);
-  else AWQMI_TOPK(16);
-#undef AWQMI_TOPK
+  const int tokens = 4 * 64 / moe_topk_lanes(E, topk);      // of a workgroup
+  moe_topk_form(E, topk, scoring, [&](auto L, auto P, auto S) {
+    hipLaunchKernelGGL((moe_topk_kernel<decltype(L)::value, decltype(P)::value, decltype(S)::value>), dim3((T + tokens - 1) / tokens),
+                       dim3(256), 0, (hipStream_t)stream, logits, score_bias, T, E, topk, renormalize, scale, topk_ids, topk_weights);
+  });
   return launch_status();
 }
 
@@ -1136,9 +1142,9 @@ static int moe_gemm_impl(const void* x, const int32_t* qweight, const void* scal
     if (sig) hipLaunchKernelGGL((awq_gemv_route_kernel<2, PERV, true>), grid, dim3(256), 0, st, p);        \
     else hipLaunchKernelGGL((awq_gemv_route_kernel<2, PERV, false>), grid, dim3(256), 0, st, p);           \
   } while (0)
-      if (route->E <= 64) AWQMI_ROUTE(1);
-      else if (route->E <= 128) AWQMI_ROUTE(2);
-      else AWQMI_ROUTE(4);
+      if (route->E <= 64) AWQMI_ROUTE(4);
+      else if (route->E <= 128) AWQMI_ROUTE(8);
+      else AWQMI_ROUTE(16);
 #undef AWQMI_ROUTE
       return launch_status();
     }
@@ -1182,9 +1188,6 @@ int awqmi_moe_sum_f16(const void* in, void* out, int T, int topk, int H, void* s
 }
 
 namespace {
-constexpr int MOE_ALIGN_PARTS_MAX = 64;      // workgroups of the multi-workgroup align
-constexpr int MOE_ALIGN_SPLIT_MIN = 16384;   // slots from which it is used (4096 per workgroup)
-
 // Expected blocks of `rows` slots of an expert's run when its slot count is Poisson(avg) (normal tail past the
 // first block): sum_j P(count > j * rows)
 double moe_expected_blocks(double avg, int rows) {
@@ -1342,7 +1345,7 @@ FusedMoeLayout fused_moe_layout(int T, int H, int inter, int E, int topk, int ti
   L.sorted = off;  off += up((size_t)L.cap * 4);
   L.experts = off; off += up((size_t)(L.cap / L.tile) * 4);
   L.npp = off;     off += 256;
-  L.tab = off;     off += up((size_t)MOE_ALIGN_PARTS_MAX * E * 4);
+  L.tab = off;     off += up((size_t)MOE_PARTS_MAX * E * 4);
   L.h13 = off;     off += up((size_t)L.n_slots * 2 * inter * 2);
   L.act = off;     off += up((size_t)L.n_slots * inter * 2);
   L.o = off;       off += up((size_t)L.n_slots * H * 2);
@@ -1404,34 +1407,12 @@ int awqmi_fused_moe_routed_f16(const void* hidden, const float* router_logits, c
   int st;
   int32_t* const runs = form.runs ? reinterpret_cast<int32_t*>(h13) : nullptr;
   const MoeRoute route{router_logits, score_bias, T, E, topk, scoring, renormalize, routed_scale,
-                       ids, wts, sorted, experts, npp, runs};
+                       ids, wts, sorted, experts, npp, runs, reinterpret_cast<int32_t*>(ws + L.tab)};
   // a handful of tokens: the first expert GEMM takes the routing along (one launch less)
   const bool fold = moe_route_foldable(T, E, topk, tile);
   const MoeRoute* pending = fold ? &route : nullptr;
-  if (fold) {
-    // nothing to launch here
-  } else if (L.n_slots < MOE_ALIGN_SPLIT_MIN || variant_on(VAR_ALIGN_ONE_WG)) {
+  if (!fold) {
     st = moe_route_launches(route, tile, stream);
-    if (st) return st;
-  } else {
-    st = awqmi_moe_topk_f32(router_logits, score_bias, T, E, topk, scoring, renormalize, routed_scale, ids, wts,
-                            stream);
-    if (st) return st;
-    // long slot lists: count per part, scan, place per part (three launches, many workgroups)
-    if (const int rc = ensure_kernel_attributes()) return rc;
-    int parts = (L.n_slots + 4095) / 4096;
-    if (parts > MOE_ALIGN_PARTS_MAX) parts = MOE_ALIGN_PARTS_MAX;
-    const int part = ((L.n_slots + parts - 1) / parts + 63) / 64 * 64;
-    parts = (L.n_slots + part - 1) / part;
-    int32_t* tab = reinterpret_cast<int32_t*>(ws + L.tab);
-    const size_t lds = (size_t)(MOE_ALIGN_WAVES + 2) * E * sizeof(int);
-    hipStream_t hs = (hipStream_t)stream;
-    hipLaunchKernelGGL(moe_align_count_kernel, dim3(parts), dim3(1024), lds, hs, ids, L.n_slots, E, part, tab);
-    hipLaunchKernelGGL(moe_align_scan_kernel, dim3(1), dim3(1024), (size_t)2 * E * sizeof(int), hs, L.n_slots, E,
-                       tile, L.cap, parts, tab, sorted, experts, npp, runs);
-    hipLaunchKernelGGL(moe_align_place_kernel, dim3(parts), dim3(1024), lds, hs, ids, L.n_slots, E, part, tab,
-                       sorted);
-    st = launch_status();
     if (st) return st;
   }
   if (form.act) {

@@ -29,18 +29,19 @@ __device__ __forceinline__ float wave_reduce_f32(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
-// One wave per token.  PER = experts per lane (E <= 64 * PER).
+// Top-k of one token by LANES lanes of a wave, PER experts per lane (E <= LANES * PER); pick k ends up in lane k of the
+// token's lanes (id, w; topk <= LANES).
 // SIGMOID = false: softmax scores; selection runs on the raw logits (softmax is monotonic).
 // SIGMOID = true: score = sigmoid(logit); selection runs on score + bias[e] (bias may be
-// null), the weight is the score itself.  Ties go to the lowest expert id.  Weights are
-// optionally renormalised over the selected experts and multiplied by `scale`.
-// Each pick is one wave-wide max of the remaining keys, then a ballot of the lanes that hold
+// null), the weight is the score itself.  Ties go to the lowest expert id; NaN keys lose against every number and are
+// then taken in expert order, so that every id stays inside [0, E) (the weight is NaN and carries the bad logit forward).
+// Weights are optionally renormalised over the selected experts and multiplied by `scale`.
+//
+// LANES = 64 (one token a wave): each pick is one wave-wide max of the remaining keys, then a ballot of the lanes that hold
 // it (lowest expert id first); the winner's id and key are wave-uniform from there on.
 template <int PER, bool SIGMOID>
-__device__ __forceinline__ void moe_topk_token(const float* __restrict__ logits,
-                                               const float* __restrict__ bias, int t, int E, int topk,
-                                               int renorm, float scale, int* __restrict__ ids,
-                                               float* __restrict__ wts) {
+__device__ __forceinline__ void moe_pick_wave(const float* __restrict__ row, const float* __restrict__ bias, int E,
+                                              int topk, int renorm, float scale, int& id, float& w) {
   const int lane = threadIdx.x & 63;
   float v[PER];      // selection key
   float sc[PER];     // score (SIGMOID only)
@@ -50,7 +51,7 @@ __device__ __forceinline__ void moe_topk_token(const float* __restrict__ logits,
   for (int i = 0; i < PER; ++i) {
     const int e = lane + 64 * i;
     open[i] = e < E;
-    const float x = e < E ? logits[(size_t)t * E + e] : -INFINITY;
+    const float x = e < E ? row[e] : -INFINITY;
     if (SIGMOID) {
       sc[i] = 1.f / (1.f + __expf(-x));
       v[i] = e < E ? sc[i] + (bias ? bias[e] : 0.f) : -INFINITY;
@@ -86,9 +87,7 @@ __device__ __forceinline__ void moe_topk_token(const float* __restrict__ logits,
       if (b) bidx = 64 * i + __builtin_ctzll(b);
     }
     if (bidx == E) {
-      // only NaN keys are left (fmaxf skipped them, nothing equals `best`): take the lowest
-      // expert that is still open, so that every id stays inside [0, E) and every slot gets its
-      // rows written; the weight computed below is NaN and carries the bad logit forward
+      // only NaN keys are left (fmaxf skipped them, nothing equals `best`): the lowest expert that is still open
 #pragma unroll
       for (int i = PER - 1; i >= 0; --i) {
         const unsigned long long b = __ballot(open[i]);
@@ -116,25 +115,139 @@ __device__ __forceinline__ void moe_topk_token(const float* __restrict__ logits,
     for (int i = 0; i < PER; ++i)
       if (lane + 64 * i == bidx) open[i] = false;
   }
-  if (lane < topk) {
-    ids[(size_t)t * topk + lane] = my_id;
-    wts[(size_t)t * topk + lane] = (renorm ? my_w / sel_sum : my_w) * scale;
-  }
+  id = my_id;
+  w = (renorm ? my_w / sel_sum : my_w) * scale;
 }
 
+// All 16 lanes of a row get op over the row (DPP row rotations).
+template <class T, class OP>
+__device__ __forceinline__ T row_reduce(T v, OP op) {
+  auto step = [&](auto CTRL) {
+    v = op(v, __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), decltype(CTRL)::value, 0xf, 0xf, true)));
+  };
+  using std::integral_constant;
+  step(integral_constant<int, 0x128>{});   // row_ror:8
+  step(integral_constant<int, 0x124>{});
+  step(integral_constant<int, 0x122>{});
+  step(integral_constant<int, 0x121>{});
+  return v;
+}
+
+// LANES = 16 (four tokens a wave): lane l of a token holds experts PER l .. PER l + PER - 1.  The keys are integers that
+// order as the floats do (-0 as 0, NaN below -inf, a picked or absent expert below that).  A pick is a max over the
+// lane's keys and over the row, the lowest id that holds it, likewise a minimum over the row, and one select per key
+// to close it: some 50 vector instructions for four tokens, where the wave-wide form spends as many on one.  Weights are worked out once, by the lane that holds the pick.
 template <int PER, bool SIGMOID>
+__device__ __forceinline__ void moe_pick_row(const float* __restrict__ row, const float* __restrict__ bias, int E,
+                                             int topk, int renorm, float scale, int& id, float& w) {
+  constexpr int GONE = (int)0x80000000u, NOT_A_NUMBER = GONE + 1;
+  const int l = threadIdx.x & 15, e0 = PER * l;
+  // (absent experts read one that is there: no load and no select sits behind a branch)
+  float x[PER];
+  if ((E & 3) == 0 && (reinterpret_cast<uintptr_t>(row) & 15) == 0) {
+#pragma unroll
+    for (int i = 0; i < PER; i += 4) {
+      const f4 q = *reinterpret_cast<const f4*>(row + min(e0 + i, E - 4));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[i + j] = q[j];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) x[i] = row[min(e0 + i, E - 1)];
+  }
+  if (SIGMOID) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) x[i] = 1.f / (1.f + __expf(-x[i]));
+    if (bias)
+#pragma unroll
+      for (int i = 0; i < PER; ++i) x[i] += bias[min(e0 + i, E - 1)];
+  }
+  int key[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int b = __builtin_bit_cast(int, x[i] + 0.f);
+    const int k = x[i] == x[i] ? b ^ ((b >> 31) & 0x7fffffff) : NOT_A_NUMBER;
+    key[i] = e0 + i < E ? k : GONE;
+  }
+  auto value = [](int k) { return k == NOT_A_NUMBER ? NAN : __builtin_bit_cast(float, k ^ ((k >> 31) & 0x7fffffff)); };
+  int my_id = 0, my_key = 0, top = 0;
+  for (int it = 0; it < topk; ++it) {
+    int loc = key[0];
+#pragma unroll
+    for (int i = 1; i < PER; ++i) loc = max(loc, key[i]);
+    const int best = row_reduce(loc, [](int a, int b) { return max(a, b); });
+    if (it == 0) top = best;
+    int first = 0x7fffffff;                // the lane's first expert that holds the best key
+#pragma unroll
+    for (int i = PER - 1; i >= 0; --i) first = key[i] == best ? i : first;
+    const int win = row_reduce(first < PER ? e0 + first : first, [](int a, int b) { return min(a, b); });
+    my_id = l == it ? win : my_id;
+    my_key = l == it ? best : my_key;
+    const int own = win - e0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) key[i] = own == i ? GONE : key[i];
+  }
+  float pw;
+  if (SIGMOID) {
+    pw = 1.f / (1.f + __expf(-row[my_id]));
+  } else {
+    const float mx = value(top);           // NaN if every key is
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) sum += e0 + i < E ? __expf(x[i] - mx) : 0.f;
+    pw = __expf(value(my_key) - mx) / row_reduce(sum, [](float a, float b) { return a + b; });
+  }
+  const float sel_sum = row_reduce(l < topk ? pw : 0.f, [](float a, float b) { return a + b; });
+  id = my_id;
+  w = (renorm ? pw / sel_sum : pw) * scale;
+}
+
+// Tokens t0 .. t0 + 64 / LANES - 1 (t0 < T) by one wave: ids and weights to memory.  Returns the expert of this lane's
+// pick, -1 where the lane has none.
+template <int LANES, int PER, bool SIGMOID>
+__device__ __forceinline__ int moe_topk_tokens(const float* __restrict__ logits, const float* __restrict__ bias, int t0,
+                                               int T, int E, int topk, int renorm, float scale, int* __restrict__ ids,
+                                               float* __restrict__ wts) {
+  const int lane = threadIdx.x & 63, l = lane % LANES, t = t0 + lane / LANES;
+  const float* const row = logits + (size_t)min(t, T - 1) * E;
+  int id;
+  float w;
+  if constexpr (LANES == 16) moe_pick_row<PER, SIGMOID>(row, bias, E, topk, renorm, scale, id, w);
+  else moe_pick_wave<PER, SIGMOID>(row, bias, E, topk, renorm, scale, id, w);
+  if (t >= T || l >= topk) return -1;
+  ids[(size_t)t * topk + l] = id;
+  wts[(size_t)t * topk + l] = w;
+  return id;
+}
+
+template <int LANES, int PER, bool SIGMOID>
 __global__ __launch_bounds__(256) void moe_topk_kernel(const float* __restrict__ logits,
                                                        const float* __restrict__ bias, int T, int E,
                                                        int topk, int renorm, float scale,
                                                        int* __restrict__ ids, float* __restrict__ wts) {
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= T) return;
-  moe_topk_token<PER, SIGMOID>(logits, bias, t, E, topk, renorm, scale, ids, wts);
+  const int t0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / LANES);
+  if (t0 >= T) return;
+  moe_topk_tokens<LANES, PER, SIGMOID>(logits, bias, t0, T, E, topk, renorm, scale, ids, wts);
 }
 
 // Tiles of the expert GEMMs made of up to MOE_RUN consecutive 16-slot blocks of one expert: runs[0] tiles, then
 // first block * 32 + blocks of each (runs null: none wanted).
 constexpr int MOE_RUN = 4;
+
+// Inclusive prefix sum over the wave by DPP row shifts and row broadcasts.
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+  auto step = [&](auto CTRL, auto ROWS) {
+    v += __builtin_amdgcn_update_dpp(0, v, decltype(CTRL)::value, decltype(ROWS)::value, 0xf, false);
+  };
+  using std::integral_constant;
+  step(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});   // row_shr:1
+  step(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});   // row_shr:2
+  step(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});   // row_shr:4
+  step(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});   // row_shr:8
+  step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});   // row_bcast:15 into rows 1, 3
+  step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});   // row_bcast:31 into rows 2, 3
+  return v;
+}
 
 // Exclusive prefix sum of padded[] by one wave, a lane owning a contiguous range of experts; and the tiles of
 // each expert's run, as even as whole blocks allow.
@@ -149,12 +262,7 @@ __device__ __forceinline__ void moe_starts(const int* padded, int* start, int E,
       if (runs) tiles += (padded[e] / 16 + MOE_RUN - 1) / MOE_RUN;
     }
   }
-  int incl = local, tincl = tiles;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int v = __shfl_up(incl, o), w = __shfl_up(tincl, o);
-    if (lane >= o) { incl += v; tincl += w; }
-  }
+  const int incl = wave_prefix_sum(local), tincl = runs ? wave_prefix_sum(tiles) : 0;
   int pos = incl - local, tpos = tincl - tiles;
   for (int k = 0; k < per; ++k) {
     const int e = lane * per + k;
@@ -171,7 +279,7 @@ __device__ __forceinline__ void moe_starts(const int* padded, int* start, int E,
   }
   if (lane == 63) {
     *s_total = incl;
-    npp[0] = incl;
+    if (npp) npp[0] = incl;
     if (runs) runs[0] = tincl;
   }
 }
@@ -184,25 +292,22 @@ __device__ __forceinline__ void moe_starts(const int* padded, int* start, int E,
 // position per (wave, expert) lives in LDS and is bumped by one LDS atomic per slot after all
 // lanes of the batch have read it.
 constexpr int MOE_ALIGN_WAVES = 16;
-// MODE 0: the whole job in one workgroup.  For long slot lists the job is split over the
-// workgroups of three launches (one workgroup scatters about one slot per clock, whatever it
-// does): MODE 1 = count the experts of this workgroup's part [s0, s1) into block_cnt[block][E];
-// (moe_align_scan_kernel turns the counts into each part's first position per expert and writes
-// the padding;) MODE 2 = place this part's slots from block_start[block][E].
-template <int MODE>
+// PART = false: the whole job in one workgroup.  One workgroup scatters about one slot per clock, whatever it does, so
+// that longer lists are split over the workgroups of a launch: PART = true places slots [s0, s1) only, from first[e] (LDS) on,
+// see moe_align_parts_kernel.
+template <bool PART>
 __device__ __forceinline__ void moe_align_block(const int* __restrict__ ids, int n, int E, int tile_m,
                                                 int cap, int* __restrict__ sorted,
                                                 int* __restrict__ expert_ids, int* __restrict__ npp,
-                                                int* sm, int s0 = 0, int s1 = 0,
-                                                int* __restrict__ block_tab = nullptr,
-                                                int* __restrict__ runs = nullptr) {
+                                                int* __restrict__ runs, int* sm, int s0 = 0, int s1 = 0,
+                                                const int* first = nullptr) {
   constexpr int NWV = MOE_ALIGN_WAVES;
   int* cnt = sm;               // [NWV][E], later the running write position
   int* padded = sm + NWV * E;  // [E]
   int* start = padded + E;     // [E]
   __shared__ int s_total;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  if (MODE == 0) { s0 = 0; s1 = n; }
+  if (!PART) { s0 = 0; s1 = n; }
 
   for (int i = tid; i < NWV * E; i += 1024) cnt[i] = 0;
   __syncthreads();
@@ -212,15 +317,15 @@ __device__ __forceinline__ void moe_align_block(const int* __restrict__ ids, int
   // ids are read eight batches of 64 at a time (eight loads in flight instead of one
   // dependent load per batch); the first eight batches stay in registers for the second pass
   constexpr int NB = 8;
-  int first[NB];
+  int head[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
     const int i = sb + 64 * b + lane;
-    first[b] = i < se ? ids[i] : -1;
+    head[b] = i < se ? ids[i] : -1;
   }
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    const int e = first[b];
+    const int e = head[b];
     if (e >= 0 && e < E) atomicAdd(&cnt[wave * E + e], 1);
   }
   for (int c0 = sb + 64 * NB; c0 < se; c0 += 64 * NB) {
@@ -238,22 +343,13 @@ __device__ __forceinline__ void moe_align_block(const int* __restrict__ ids, int
   }
   __syncthreads();
 
-  if (MODE == 1) {
+  if constexpr (PART) {
     for (int e = tid; e < E; e += 1024) {
-      int tot = 0;
-      for (int w = 0; w < NWV; ++w) tot += cnt[w * E + e];
-      block_tab[(size_t)blockIdx.x * E + e] = tot;
-    }
-    return;
-  }
-  if (MODE == 2) {
-    for (int e = tid; e < E; e += 1024) {
-      int pos = block_tab[(size_t)blockIdx.x * E + e];
+      int pos = first[e];
       for (int w = 0; w < NWV; ++w) { const int c = cnt[w * E + e]; cnt[w * E + e] = pos; pos += c; }
     }
     __syncthreads();
-  }
-  if constexpr (MODE == 0) {
+  } else {
   for (int e = tid; e < E; e += 1024) {
     int tot = 0;
     for (int w = 0; w < NWV; ++w) tot += cnt[w * E + e];
@@ -273,7 +369,7 @@ __device__ __forceinline__ void moe_align_block(const int* __restrict__ ids, int
   for (int i = total + tid; i < cap; i += 1024) sorted[i] = n;           // unused tail
   for (int i = total / tile_m + tid; i < cap / tile_m; i += 1024) expert_ids[i] = -1;
   __syncthreads();
-  }   // MODE == 0
+  }   // !PART
 
   const int nbits = 32 - __builtin_clz(max(E - 1, 1));
   auto place = [&](int i, int e) {
@@ -296,7 +392,7 @@ __device__ __forceinline__ void moe_align_block(const int* __restrict__ ids, int
   };
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    if (sb + 64 * b < se) place(sb + 64 * b + lane, first[b]);     // wave-uniform condition
+    if (sb + 64 * b < se) place(sb + 64 * b + lane, head[b]);     // wave-uniform condition
   }
   for (int c0 = sb + 64 * NB; c0 < se; c0 += 64 * NB) {
     int more[NB];
@@ -318,97 +414,110 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
                                                          int* __restrict__ expert_ids,
                                                          int* __restrict__ npp, int* __restrict__ runs) {
   extern __shared__ int sm[];
-  moe_align_block<0>(ids, n, E, tile_m, cap, sorted, expert_ids, npp, sm, 0, 0, nullptr, runs);
+  moe_align_block<false>(ids, n, E, tile_m, cap, sorted, expert_ids, npp, runs, sm);
 }
 
-// Long slot lists: part b of gridDim.x parts covers slots [b * part, (b + 1) * part).
-__global__ __launch_bounds__(1024) void moe_align_count_kernel(const int* __restrict__ ids, int n, int E,
-                                                               int part, int* __restrict__ block_cnt) {
-  extern __shared__ int sm[];
-  const int s0 = min(n, (int)blockIdx.x * part), s1 = min(n, s0 + part);
-  moe_align_block<1>(ids, n, E, 1, 0, nullptr, nullptr, nullptr, sm, s0, s1, block_cnt);
-}
-
-// One workgroup: per expert the padded length and first position, then every part's first
-// position per expert (in place: counts in, positions out), the padding entries, the block
-// owners and the unused tails.
-__global__ __launch_bounds__(1024) void moe_align_scan_kernel(int n, int E, int tile_m, int cap, int parts,
-                                                              int* __restrict__ block_tab,
-                                                              int* __restrict__ sorted,
-                                                              int* __restrict__ expert_ids,
-                                                              int* __restrict__ npp, int* __restrict__ runs) {
-  extern __shared__ int sm[];
-  int* padded = sm;        // [E]
-  int* start = sm + E;     // [E]
-  __shared__ int s_total;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // thread e keeps its expert's counts of all parts in registers (one memory round trip;
-  // E <= 1024 = the workgroup size, parts <= 64)
-  constexpr int PMAX = 64;
-  int c[PMAX];
-  const int my_e = tid < E ? tid : 0;
-#pragma unroll
-  for (int b = 0; b < PMAX; ++b) c[b] = block_tab[(size_t)min(b, parts - 1) * E + my_e];
-  if (tid < E) {
-    int tot = 0;
-#pragma unroll
-    for (int b = 0; b < PMAX; ++b) tot += b < parts ? c[b] : 0;
-    padded[tid] = (tot + tile_m - 1) / tile_m * tile_m;
+// Longer batches in two launches, part b of each one's workgroups being tokens [b * part, (b + 1) * part):
+// the first picks the experts and counts its part's picks, the second places them.
+//
+// (Four launches before from 16384 slots on: top-k, count, scan in one workgroup, place; 12.6 + 4.9 + 12.0 + 7.8 us for 8192 tokens,
+// 128 experts, top-8, against 8.7 + 9.2.)
+constexpr int MOE_PARTS_MAX = 128;
+template <int LANES, int PER, bool SIGMOID>
+__global__ __launch_bounds__(1024) void moe_route_count_kernel(const float* __restrict__ logits, const float* __restrict__ bias,
+                                                               int T, int E, int topk, int renorm, float scale,
+                                                               int* __restrict__ ids, float* __restrict__ wts, int part,
+                                                               int* __restrict__ part_cnt) {
+  __shared__ int cnt[1024];      // E <= 1024
+  const int tid = threadIdx.x, threads = blockDim.x;
+  for (int e = tid; e < E; e += threads) cnt[e] = 0;
+  __syncthreads();
+  const int begin = (int)blockIdx.x * part, end = min(T, begin + part);
+  constexpr int TOK = 64 / LANES;      // tokens of a wave
+  for (int t0 = begin + (tid >> 6) * TOK; t0 < end; t0 += (threads >> 6) * TOK) {
+    const int e = moe_topk_tokens<LANES, PER, SIGMOID>(logits, bias, t0, end, E, topk, renorm, scale, ids, wts);
+    if (e >= 0) atomicAdd(&cnt[e], 1);
   }
   __syncthreads();
-  if (wave == 0) moe_starts(padded, start, E, lane, &s_total, npp, runs);
+  for (int e = tid; e < E; e += threads) part_cnt[(size_t)blockIdx.x * E + e] = cnt[e];
+}
+
+// Every workgroup adds up the table of counts (parts x E) by itself: each expert's slots in all and those of the parts before
+// its own.  With the expert's start that is where its slots go; the padding, the block owners and the unused tails
+// are shared out over the workgroups.  Dynamic LDS: moe_parts_lds(E).
+__host__ __device__ constexpr int moe_parts_lds(int E) { return ((MOE_ALIGN_WAVES * E > 2048 ? MOE_ALIGN_WAVES * E : 2048) + 4 * E) * 4; }
+__global__ __launch_bounds__(1024) void moe_align_parts_kernel(const int* __restrict__ ids, int n, int E, int part,
+                                                               int tile_m, int cap, const int* __restrict__ part_cnt,
+                                                               int* __restrict__ sorted, int* __restrict__ expert_ids,
+                                                               int* __restrict__ npp, int* __restrict__ runs) {
+  extern __shared__ int sm[];
+  __shared__ int s_total;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, b = blockIdx.x, parts = gridDim.x;
+  int* const padded = sm + max(MOE_ALIGN_WAVES * E, 2048);
+  int* const start = padded + E;
+  int* const count = start + E;
+  int* const first = count + E;
+  // threads (slice, expert): a slice takes every slices-th part; the sums of the slices meet in LDS
+  const int slices = 1024 / E;
+  if (tid < slices * E) {
+    const int e = tid % E, s = tid / E;
+    int all = 0, before = 0;
+#pragma unroll 16
+    for (int q = s; q < parts; q += slices) {
+      const int c = part_cnt[(size_t)q * E + e];
+      all += c;
+      before += q < b ? c : 0;
+    }
+    sm[tid] = all;
+    sm[1024 + tid] = before;
+  }
+  __syncthreads();
+  if (tid < E) {
+    int all = 0, before = 0;
+    for (int s = 0; s < slices; ++s) {
+      all += sm[s * E + tid];
+      before += sm[1024 + s * E + tid];
+    }
+    count[tid] = all;
+    first[tid] = before;
+    padded[tid] = (all + tile_m - 1) / tile_m * tile_m;
+  }
+  __syncthreads();
+  if (wave == 0) moe_starts(padded, start, E, lane, &s_total, b == 0 ? npp : nullptr, b == 0 ? runs : nullptr);
   __syncthreads();
   const int total = s_total;
-  if (tid < E) {
-    const int e = tid;
-    int pos = start[e];
-    const int e0 = pos;
-#pragma unroll
-    for (int b = 0; b < PMAX; ++b) {
-      if (b < parts) {
-        block_tab[(size_t)b * E + e] = pos;
-        pos += c[b];
-      }
-    }
-    padded[e] = pos;          // from here on: first padding position of the expert's run
-    (void)e0;
+  if (tid < E) first[tid] += start[tid];
+  for (int e = b + wave * parts; e < E; e += MOE_ALIGN_WAVES * parts) {
+    const int e0 = start[e], e1 = e0 + padded[e];
+    for (int i = e0 + count[e] + lane; i < e1; i += 64) sorted[i] = n;
+    for (int k = e0 / tile_m + lane; k < e1 / tile_m; k += 64) expert_ids[k] = e;
   }
-  __syncthreads();
-  // padding entries and block owners, one wave per expert at a time (coalesced stores)
-  for (int e = wave; e < E; e += 16) {
-    const int e0 = start[e];
-    const int e1 = e + 1 < E ? start[e + 1] : total;
-    for (int i = padded[e] + lane; i < e1; i += 64) sorted[i] = n;
-    for (int b = e0 / tile_m + lane; b < e1 / tile_m; b += 64) expert_ids[b] = e;
-  }
-  for (int i = total + tid; i < cap; i += 1024) sorted[i] = n;
-  for (int i = total / tile_m + tid; i < cap / tile_m; i += 1024) expert_ids[i] = -1;
+  const int at = b * 1024 + tid, step = parts * 1024;
+  for (int i = total + at; i < cap; i += step) sorted[i] = n;
+  for (int i = total / tile_m + at; i < cap / tile_m; i += step) expert_ids[i] = -1;
+  const int s0 = min(n, b * part), s1 = min(n, s0 + part);
+  moe_align_block<true>(ids, n, E, tile_m, cap, sorted, nullptr, nullptr, nullptr, sm, s0, s1, first);
 }
 
-__global__ __launch_bounds__(1024) void moe_align_place_kernel(const int* __restrict__ ids, int n, int E,
-                                                               int part, int* __restrict__ block_start,
-                                                               int* __restrict__ sorted) {
-  extern __shared__ int sm[];
-  const int s0 = min(n, (int)blockIdx.x * part), s1 = min(n, s0 + part);
-  moe_align_block<2>(ids, n, E, 1, 0, sorted, nullptr, nullptr, sm, s0, s1, block_start);
-}
-
-// Routing and align in one launch for batches of at most 16 tokens (one wave per token, the
-// same single workgroup then sorts the T * topk slots): a decode step of a few sequences
-// spends more on the second launch than on either kernel's work.
-template <int PER, bool SIGMOID>
+// Routing and align in one launch for up to MOE_ALIGN_WAVES * 64 / LANES tokens (the same single workgroup then sorts the
+// T * topk slots): a decode step of a few sequences spends more on the second launch than on either kernel's work.
+template <int LANES, int PER, bool SIGMOID>
 __global__ __launch_bounds__(1024) void moe_route_align_kernel(const float* __restrict__ logits,
                                                                const float* __restrict__ bias, int T,
                                                                int E, int topk, int renorm, float scale,
                                                                int* ids, float* __restrict__ wts, int tile_m,
                                                                int cap, int* __restrict__ sorted,
                                                                int* __restrict__ expert_ids,
-                                                               int* __restrict__ npp) {
+                                                               int* __restrict__ npp, int* __restrict__ runs) {
   extern __shared__ int sm[];
-  const int wave = threadIdx.x >> 6;
-  if (wave < T) moe_topk_token<PER, SIGMOID>(logits, bias, wave, E, topk, renorm, scale, ids, wts);
-  __syncthreads();   // the ids written above are read back by the same workgroup
-  moe_align_block<0>(ids, T * topk, E, tile_m, cap, sorted, expert_ids, npp, sm);
+  __shared__ int s_ids[MOE_ALIGN_WAVES * 64];      // 16 waves of 64 / LANES tokens with up to LANES picks each
+  const int lane = threadIdx.x & 63, t0 = (int)(threadIdx.x >> 6) * (64 / LANES);
+  if (t0 < T) {
+    const int e = moe_topk_tokens<LANES, PER, SIGMOID>(logits, bias, t0, T, E, topk, renorm, scale, ids, wts);
+    if (e >= 0) s_ids[(t0 + lane / LANES) * topk + lane % LANES] = e;
+  }
+  __syncthreads();
+  moe_align_block<false>(s_ids, T * topk, E, tile_m, cap, sorted, expert_ids, npp, runs, sm);
 }
 
 __global__ __launch_bounds__(256) void silu_and_mul_kernel(const half_t* __restrict__ in,

@@ -29,6 +29,28 @@ def test_topk_softmax(sba, gpu, T, E, topk):
 
 
 @pytest.mark.parametrize("scoring", ["softmax", "sigmoid"])
+@pytest.mark.parametrize("T,E,topk", [(1, 16, 16), (3, 17, 16), (5, 60, 1), (4, 64, 8), (9, 65, 8), (17, 127, 6), (6, 128, 16),
+                                      (7, 129, 4), (2, 255, 16), (18, 256, 8), (5, 257, 16), (5, 128, 17), (1, 1, 1)])
+def test_topk_with_many_ties_at_the_edges_of_its_forms(sba, gpu, scoring, T, E, topk):
+    """Experts and picks on both sides of what sixteen lanes a token hold (256 and 16), tokens that leave part of a wave
+    empty, rows that are no multiple of 16 bytes; logits of few values, zeros of both signs among them, so that ties lie inside
+    a lane, across lanes and across the experts' whole range."""
+    g = torch.Generator().manual_seed(31 * T + E + topk)
+    logits = torch.randint(-2, 3, (T, E), generator=g).float()
+    logits[torch.rand((T, E), generator=g) < 0.3] *= -0.0
+    if scoring == "softmax":
+        w, ids = sba.topk_softmax(logits.to(gpu), topk, True)
+        rid, rw = awq_ref.topk_softmax(logits.numpy(), topk, True)
+    else:
+        # (of a few values too: the scores of equal logits are equal)
+        bias = torch.randint(0, 2, (E,), generator=g).float()
+        w, ids = sba.topk_route(logits.to(gpu), topk, True, "sigmoid", bias.to(gpu))
+        rid, rw = awq_ref.topk_sigmoid(logits.numpy(), topk, True, bias.numpy())
+    assert np.array_equal(ids.cpu().numpy(), rid)
+    assert np.allclose(w.cpu().numpy(), rw, rtol=2e-5, atol=1e-8)
+
+
+@pytest.mark.parametrize("scoring", ["softmax", "sigmoid"])
 def test_topk_with_nan_and_infinite_logits_keeps_ids_in_range(sba, gpu, scoring):
     """Rows with fewer than top-k usable logits: NaN keys lose against every number and are then
     taken in expert order (the oracle's stable argsort puts them last the same way), -inf keys
@@ -628,6 +650,24 @@ def test_fused_call_with_long_slot_lists(sba, gpu, T, E, topk):
     step = sba.fused_moe_awq(c.x, c.w13, c.w2, c.logits, topk, True, block_size=bs)
     assert torch.equal(one, step)
     assert torch.equal(one, sba.fused_moe_awq(c.x, c.w13, c.w2, c.logits, topk, True))
+
+
+@pytest.mark.parametrize("scoring", ["softmax", "sigmoid"])
+@pytest.mark.parametrize("T,E,topk", [(32, 128, 8), (33, 128, 8), (16, 64, 17), (17, 64, 17), (256, 128, 8), (257, 128, 8),
+                                      (2049, 4, 2), (2050, 5, 1), (300, 1024, 17), (2100, 256, 16), (130, 257, 16)])
+def test_routing_in_one_two_and_several_workgroups(sba, gpu, scoring, T, E, topk):
+    """Both sides of the rule for the block's routing launches (32 tokens, 16 with a token a wave, 2048 slots; a last part of
+    one token): the block must equal the step-by-step path, whose top-k and align are checked against the oracle above."""
+    c = sba.workloads.make_moe_case(T, 256, E, topk, 128, 128, seed=T + E).to(gpu)
+    kw = {}
+    if scoring == "sigmoid":
+        kw = dict(scoring_func="sigmoid", e_score_correction_bias=torch.linspace(0, 0.1, E, device=gpu))
+    from server_benchmark_amd import _lib
+    bs = _lib.load().awqmi_fused_moe_block_rows(T, 256, 128, E, topk, 128)
+    for _ in range(2):
+        one = sba.fused_moe_awq(c.x, c.w13, c.w2, c.logits, topk, True, **kw)
+        step = sba.fused_moe_awq(c.x, c.w13, c.w2, c.logits, topk, True, block_size=bs, **kw)
+        assert torch.equal(one, step)
 
 
 @pytest.mark.parametrize("scoring", ["softmax", "sigmoid"])
