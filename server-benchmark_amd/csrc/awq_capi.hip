@@ -490,7 +490,7 @@ struct MoeRoute {
   int32_t* experts;
   int32_t* npp;
   int32_t* runs;     // tiles of several 16-slot blocks, or null
-  int32_t* tab;      // expert counts of the parts of a longer batch, [MOE_PARTS_MAX][E]
+  int32_t* tab;      // expert counts of the parts of a longer batch, [moe_parts(T).parts][E]
 };
 
 static int moe_align_launch(const int32_t* topk_ids, int n_slots, int E, int tile_m, int32_t* sorted, int32_t* experts,
@@ -507,6 +507,11 @@ static int moe_align_launch(const int32_t* topk_ids, int n_slots, int E, int til
 // launches of parts: 16 tokens 62.2 / 59.3 / - / -; 32 72.2 / 70.5 / - / -; 48 73.3 / 72.9 / 72.5 / -; 64 75.3 / 75.3 / 74.5 / -; 128 80.6 / - /
 // 80.1 / 81.2; 256 98 / - / 97.5 / 97.3; 1500 172 / - / - / 166; 8192 696 / - / - / 688.
 constexpr int MOE_ONE_WG_SLOTS = 2048;
+struct MoeParts { int part, parts; };     // tokens of a part, parts
+static MoeParts moe_parts(int T) {
+  const int part = (T + 16 * MOE_PARTS_MAX - 1) / (16 * MOE_PARTS_MAX) * 16;
+  return {part, (T + part - 1) / part};
+}
 static int moe_route_launches(const MoeRoute& r, int tile, void* stream) {
   if (const int rc = ensure_kernel_attributes()) return rc;
   const int n_slots = r.T * r.topk, cap = (int)awqmi_moe_align_capacity(n_slots, r.E, tile);
@@ -525,14 +530,14 @@ static int moe_route_launches(const MoeRoute& r, int tile, void* stream) {
       return rc;
     return moe_align_launch(r.ids, n_slots, r.E, tile, r.sorted, r.experts, r.npp, r.runs, stream);
   }
-  const int part = (r.T + 16 * MOE_PARTS_MAX - 1) / (16 * MOE_PARTS_MAX) * 16, parts = (r.T + part - 1) / part;
-  const int waves = std::min(16, part / wave_tokens);
+  const MoeParts pt = moe_parts(r.T);
+  const int waves = std::min(16, pt.part / wave_tokens);
   moe_topk_form(r.E, r.topk, r.scoring, [&](auto L, auto P, auto S) {
-    hipLaunchKernelGGL((moe_route_count_kernel<decltype(L)::value, decltype(P)::value, decltype(S)::value>), dim3(parts),
-                       dim3(64 * waves), 0, st, r.logits, r.bias, r.T, r.E, r.topk, r.renorm, r.scale, r.ids, r.wts, part, r.tab);
+    hipLaunchKernelGGL((moe_route_count_kernel<decltype(L)::value, decltype(P)::value, decltype(S)::value>), dim3(pt.parts),
+                       dim3(64 * waves), 0, st, r.logits, r.bias, r.T, r.E, r.topk, r.renorm, r.scale, r.ids, r.wts, pt.part, r.tab);
   });
-  hipLaunchKernelGGL(moe_align_parts_kernel, dim3(parts), dim3(1024), (size_t)moe_parts_lds(r.E), st, r.ids, n_slots, r.E,
-                     part * r.topk, tile, cap, r.tab, r.sorted, r.experts, r.npp, r.runs);
+  hipLaunchKernelGGL(moe_align_parts_kernel, dim3(pt.parts), dim3(1024), (size_t)moe_parts_lds(r.E), st, r.ids, n_slots, r.E,
+                     pt.part * r.topk, tile, cap, r.tab, r.sorted, r.experts, r.npp, r.runs);
   return launch_status();
 }
 
@@ -1327,7 +1332,7 @@ struct FusedMoeLayout {
   size_t gemm_ws, ids, wts, sorted, experts, npp, h13, act, o, total;
   size_t gemm_ws_bytes;
   int n_slots, cap, tile;
-  size_t tab;      // per-part expert counts / first positions of the multi-workgroup align
+  size_t tab;      // expert counts of the parts of a longer batch (room for 64 parts at least)
 };
 FusedMoeLayout fused_moe_layout(int T, int H, int inter, int E, int topk, int tile) {
   FusedMoeLayout L{};
@@ -1345,7 +1350,7 @@ FusedMoeLayout fused_moe_layout(int T, int H, int inter, int E, int topk, int ti
   L.sorted = off;  off += up((size_t)L.cap * 4);
   L.experts = off; off += up((size_t)(L.cap / L.tile) * 4);
   L.npp = off;     off += 256;
-  L.tab = off;     off += up((size_t)MOE_PARTS_MAX * E * 4);
+  L.tab = off;     off += up((size_t)std::max(64, moe_parts(T).parts) * E * 4);
   L.h13 = off;     off += up((size_t)L.n_slots * 2 * inter * 2);
   L.act = off;     off += up((size_t)L.n_slots * inter * 2);
   L.o = off;       off += up((size_t)L.n_slots * H * 2);
