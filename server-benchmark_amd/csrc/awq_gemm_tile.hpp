@@ -70,6 +70,10 @@ struct TileGemmParams {
 };
 
 constexpr int TG_COLS = 256;             // columns of a workgroup tile
+// Offset of an X row that is not there: past the range of the buffer (below 4 GiB), so that the load brings zeros without traffic.
+// (The range check takes the row's part that lies in the scalar offset into account; in the last 256 bytes below 4 GiB it
+// would be a piece of X, for rows that nobody stores.)
+constexpr uint32_t X_NOWHERE = 0xFFFFFF00u;
 constexpr int TG_W_BYTES = 64 * 128;     // packed weights of a stage: 64 k x 256 columns
 
 // LDS of one stage: X rows, packed weights, then each wave's group parameters
@@ -185,7 +189,19 @@ __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, 
   // at the loop's edges, where it does not know when an asm statement's result is ready
   constexpr int AG = SCALE32 ? 0 : RT < 14 ? RT : 14;
   static_assert(!SCALE32 || (!ANY && SCALE32 <= 2), "");
-  static_assert(D >= 3 && (D - 2) * NL < 64 && (D == 3 ? NP - 2 : 2 * NP - 4) >= NL, "every load has an MFMA of its own");
+  // loads of a stage are dealt out over it (over its first k-step with a ring of three)
+  constexpr int LP = D == 3 ? NP - 2 : 2 * NP - 4;
+  static_assert(D >= 3 && (D - 2) * NL < 64 && LP >= NL, "every load has an MFMA of its own");
+  // MID: the next stage is waited for in the middle of a stage, ahead of the first read of it, instead of at the stage's start, and a
+  // barrier of its own at the start frees the slot of the last stage.  A load then has half a stage more to arrive: with a ring of
+  // three, 1.25 stages instead of 0.75.  With the pad rows' loads out of range (X_NOWHERE), four layers, us before / after: 72B at 100
+  // rows 253 / 234, 7B (groups of 64) 122 / 111, 5120-wide 119 / 110, at 200 rows 173 / 158; at 400 and more 0 - 2.5 %; blocks of 1500
+  // and 8192 tokens on 128 experts of 2048 x 768, top-8, 172 / 165 and 704 / 695 (the wait alone gives a third of it at 100 rows).
+  // NL0: loads of the first k-step.
+  constexpr bool MID = RT >= 5;
+  constexpr int NL0 = ((NP - 1) * NL + LP - 1) / LP < NL ? ((NP - 1) * NL + LP - 1) / LP : NL;
+  constexpr int UF = 6;                       // MFMAs of the second k-step ahead of its unpacking
+  static_assert(!MID || XF <= RT, "fragments of the next stage are read in the second k-step");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -203,14 +219,14 @@ __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, 
     int idx = 4 * i + wave;
     if ((RT & 1) && idx >= 2 * RT) idx -= 2;
     const int r = 8 * idx + (lane >> 3);
-    int gr;
+    int gr = m0 + r;
+    bool real = gr < p.M;
     if (GROUPED) {
       const int sid = s_sid[r];
-      gr = sid < p.n_slots ? sid / p.a_row_div : 0;
-    } else {
-      gr = min(m0 + r, p.M - 1);
+      real = sid < p.n_slots;
+      gr = sid / p.a_row_div;
     }
-    x_voff[i] = (uint32_t)(((size_t)gr * p.K + 8 * ((lane & 7) ^ dg_swz(r))) * 2);
+    x_voff[i] = real ? (uint32_t)(((size_t)gr * p.K + 8 * ((lane & 7) ^ dg_swz(r))) * 2) : X_NOWHERE;
   }
   auto x_lds = [&](int i) __attribute__((always_inline)) -> uint32_t {
     int idx = 4 * i + wave;
@@ -355,11 +371,10 @@ __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, 
         if (first) flush(j, im);
         const u4v& w = wf[ks][j];
         const h8& x = xf[(ks * RT + im) % XF];
-        // loads of a stage: dealt out over it (over its first k-step with a ring of three)
         int ld = -1;
 #pragma unroll
         for (int i = 0; i < NL; ++i)
-          if ((D == 3 ? 1 + i * (NP - 2) / NL : 1 + i * (2 * NP - 4) / NL) == ks * NP + m) ld = i;
+          if (1 + i * LP / NL == ks * NP + m) ld = i;
         if (ld < 0) tg_mfma<ACC>(a, w, x);
         else if (ld < 2) tg_mfma_load<ACC>(a, w, x, fill + w_lds + ld * 4096, rw, w_addr(ld), 0);
         else if (!ANY && ld == 2) tg_mfma_load_at<ACC>(a, w, x, fill + p_lds, p_addr, 0x3ffull);
@@ -367,13 +382,25 @@ __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, 
         else if (ANY && ld == 3) tg_mfma_load_some<ACC>(a, w, x, fill + p_lds + ZO, rz, z_addr(), z_mask);
         else tg_mfma_load<ACC>(a, w, x, fill + x_lds(ld - (NL - XL)), rx, x_voff[ld < NL - XL ? 0 : ld - (NL - XL)], (uint32_t)kl * 128u);
         __builtin_amdgcn_sched_barrier(0);
-        // parameters of the next stage; SCALE32: of the next group, and the scales of the one that ends
-        if (last && m == 0 && (ANY || ks == 1)) expand();
-        if (last && m == 1 && (ANY || ks == 0)) read_params(nxt, ks);
-        if (SCALE32 && last && ks == 1 && (m == 1 || m == 2)) gs[m - 1] = lds_read<u4v>(cur + p_lds + 32 * fq + 16 * (m - 1));
+        if constexpr (MID) {
+          // second k-step: parameters and words of the next stage, and what the parameters are for
+          if (ANY && ks == 0 && m == 0) expand();
+          if (ks == 1 && m == 0) read_params(nxt, 0);
+          if (ks == 1 && m < 8) read_words(m >> 2, fwn, m >> 2, m & 3);
+          if (ks == 1 && m == UF - 1) expand();
+          if (ANY && ks == 1 && m == UF) read_params(nxt, 1);
+          constexpr int U = ks ? UF : 0;
 #pragma unroll
-        for (int i = 18 * m / NP; i < 18 * (m + 1) / NP; ++i) unpack(i, ks ^ 1, ks ^ 1);
-        if (m < 4) read_words(ks, fwn, ks, m);
+          for (int i = m < U ? 0 : 18 * (m - U) / (NP - U); i < (m < U ? 0 : 18 * (m - U + 1) / (NP - U)); ++i) unpack(i, ks ^ 1, ks ^ 1);
+        } else {
+          // parameters of the next stage; SCALE32: of the next group, and the scales of the one that ends
+          if (last && m == 0 && (ANY || ks == 1)) expand();
+          if (last && m == 1 && (ANY || ks == 0)) read_params(nxt, ks);
+          if (SCALE32 && last && ks == 1 && (m == 1 || m == 2)) gs[m - 1] = lds_read<u4v>(cur + p_lds + 32 * fq + 16 * (m - 1));
+#pragma unroll
+          for (int i = 18 * m / NP; i < 18 * (m + 1) / NP; ++i) unpack(i, ks ^ 1, ks ^ 1);
+          if (m < 4) read_words(ks, fwn, ks, m);
+        }
         if (jj == 3) {
           const int f = ks * RT + im + XF;
           if (f < 2 * RT) xf[f % XF] = lds_read<h8>(xc[f / RT] + (f % RT) * 2048);
@@ -435,9 +462,10 @@ __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, 
   pin(0);
 
   auto stage = [&](auto FIRST, auto LAST) __attribute__((always_inline)) {
-    // the next stage has landed (own loads; the barrier extends that to every wave's) and every wave has read
-    // the last one, whose slot takes the stage D - 1 ahead
-    tg_wait_and_barrier<(D - 3) * NL>();
+    // every wave has read the last stage, whose slot takes the stage D - 1 ahead; and, here or in the middle, the next stage
+    // has landed (own loads; the barrier extends that to every wave's)
+    if constexpr (MID) asm volatile("s_barrier" ::: "memory");
+    else tg_wait_and_barrier<(D - 3) * NL>();
     __builtin_amdgcn_sched_barrier(0);
     uint32_t nxt = cur + SLOT;
     if (nxt == smem + D * SLOT) nxt = smem;
@@ -446,6 +474,10 @@ __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, 
     // (opaque: the reads' offsets stay in their offset fields)
     asm volatile("" : "+v"(xn[0]), "+v"(xn[1]), "+v"(fwn));
     kstep(I0{}, FIRST, LAST, xc, xn, fwn, nxt);
+    if constexpr (MID) {
+      tg_wait_and_barrier<(D - 3) * NL + NL0>();
+      __builtin_amdgcn_sched_barrier(0);
+    }
     kstep(I1{}, FIRST, LAST, xc, xn, fwn, nxt);
     next_load();
     cur = nxt;
