@@ -193,12 +193,13 @@ __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, 
   constexpr int LP = D == 3 ? NP - 2 : 2 * NP - 4;
   static_assert(D >= 3 && (D - 2) * NL < 64 && LP >= NL, "every load has an MFMA of its own");
   // MID: the next stage is waited for in the middle of a stage, ahead of the first read of it, instead of at the stage's start, and a
-  // barrier of its own at the start frees the slot of the last stage.  A load then has half a stage more to arrive: with a ring of
-  // three, 1.25 stages instead of 0.75.  With the pad rows' loads out of range (X_NOWHERE), four layers, us before / after: 72B at 100
-  // rows 253 / 234, 7B (groups of 64) 122 / 111, 5120-wide 119 / 110, at 200 rows 173 / 158; at 400 and more 0 - 2.5 %; blocks of 1500
-  // and 8192 tokens on 128 experts of 2048 x 768, top-8, 172 / 165 and 704 / 695 (the wait alone gives a third of it at 100 rows).
+  // barrier of its own at the start frees the slot of the last stage.  With a ring of three a load then has 1.25 stages to arrive
+  // instead of 0.75; longer rings leave it time enough (80 rows, ring of four, 209 us without and 213 with it).  With the pad rows'
+  // loads out of range (X_NOWHERE), four layers, us before / after: 72B at 100 rows 258 / 246, 7B (groups of 64) 123.5 / 113.5, at 128
+  // rows 128 / 122, 5120-wide at 100 rows 121.6 / 116, at 200 176 / 164, at 256 189 / 181; others within 1 %; blocks of 1500 and
+  // 3000 tokens on 128 experts of 2048 x 768, top-8, 183 / 172 and 316 / 304.
   // NL0: loads of the first k-step.
-  constexpr bool MID = RT >= 5;
+  constexpr bool MID = D == 3;
   constexpr int NL0 = ((NP - 1) * NL + LP - 1) / LP < NL ? ((NP - 1) * NL + LP - 1) / LP : NL;
   constexpr int UF = 6;                       // MFMAs of the second k-step ahead of its unpacking
   static_assert(!MID || XF <= RT, "fragments of the next stage are read in the second k-step");
