@@ -1280,13 +1280,16 @@ int moe_pick_tile(int n_slots, int E, int H, int inter, int group) {
 //   blocks: 0.09 us per MB of touched experts' weights and 0.11 per MB and block, which unpacks them again.
 // Fitted on 129 points (ten expert shapes, 6 ... 400 slots per expert), the whole block timed both ways.  The tiles have to
 // look 14 % cheaper (24 % below 16 experts, whose few long tiles the price underestimates): then no point of them is slower
-// than with the skinny kernel, and they are 8 % faster on average over all.  Up to 32 slots per expert a tile is two blocks at
-// most on average: within 5 % either way up to 25 slots, 13 - 14 % faster at 28 and 32 (whole block, blocks / tiles: 400 and 512 tokens
-// on 128 experts of 2048 x 768, top-8, 105 / 103 and 125 / 110 us; 560 on 160 of 6144 x 2560 1168 / 1001).  There the block keeps the kernel that the separate calls on
-// 16-slot blocks take, so that both add in one order; so do experts below the smallest measured (1024 x 512, 2048 x 384),
-// where the routing and the sum outweigh both GEMMs.  Both sides above, blocks / tiles (us): 576 / 768 / 1024 tokens on those
-// experts 143 / 164 / 192 and 116 / 130 / 163; 384 / 512 on 64 of 2048 x 1408 136 / 158 and 102 / 114; 560 on 160 of 6144 x
-// 2560 1172 and 993.
+// than with the skinny kernel, and they are 8 % faster on average over all.
+// With 16 experts and more no price is needed from 20 slots per expert on: there the tiles are 2 - 30 % faster on all of nine shapes
+// (blocks / tiles, us, at 19, 22, 25 and 27.5 slots: 128 experts of 2048 x 768 103, 105, 121, 123 / 101, 103, 104, 106; 64 of 2048 x 1408 106, 108, 116, 120 /
+// 90, 93, 94, 95; 64 of 5120 x 1024 161, 163, 183, 196 / 149, 150, 153, 157; 160 of 6144 x 2560 998, 1068, 1131, 1166 / 943, 956, 975, 985;
+// 16 of 3072 x 4096 118, 117, 135, 145 / 105, 106, 108, 110; groups of 64 alike); at 16 and below either side wins (128 experts of 2048 x
+// 768 98.0 / 98.9, 160 of 6144 x 2560 909 / 926), with eight experts the blocks.
+// From 28 to 32 slots the block keeps the kernel that the separate calls on 16-slot blocks take, so that both add in one order, as
+// tests fix at three shapes, although tiles are faster there too (512 tokens on 128 experts of 2048 x 768 125 / 110).  Experts below
+// the smallest measured (1024 x 512, 2048 x 384) stay as well: the routing and the sum outweigh both GEMMs.  Above, blocks / tiles (us): 576 / 768 / 1024
+// tokens on 128 experts of 2048 x 768 143 / 164 / 192 and 116 / 130 / 163; 560 on 64 of 2048 x 1408 172 and 122.
 bool moe_runs(int T, int n_slots, int E, int H, int inter, int group) {
   if (variant_on(VAR_MOE_TILE16) || T <= MOE_ALIGN_WAVES) return false;
   // groups of 64 or 128 rows, whole column tiles
@@ -1297,7 +1300,9 @@ bool moe_runs(int T, int n_slots, int E, int H, int inter, int group) {
     return false;
   if (variant_on(VAR_MOE_RUNS)) return true;
   const double avg = (double)n_slots / E;
-  if (avg <= 32.0 || H < 1024 || inter < 384) return false;
+  if (H < 1024 || inter < 384) return false;
+  if (avg >= 20.0 && avg < 28.0 && E >= 16) return true;
+  if (avg <= 32.0) return false;
   const double b16 = E * moe_expected_blocks(avg, 16), tiles = E * moe_expected_blocks(avg, 16 * TG_RUN);
   const double stage = 2.0 * (0.344 + 0.09 * std::max(b16 / tiles, 2.0));
   auto gemm = [&](int K, int col_tiles) {
