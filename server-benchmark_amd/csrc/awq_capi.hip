@@ -395,7 +395,7 @@ void launch_tile(const TileGemmParams& p, hipStream_t st) {
   if (p.G % 64 == 0 && p.N % 32 == 0) hipLaunchKernelGGL((awq_gemm_tile_kernel<RT, 0>), grid, dim3(256), 0, st, p);
   else if (p.G >= 32) hipLaunchKernelGGL((awq_gemm_tile_kernel<RT, 2>), grid, dim3(256), 0, st, p);
   else hipLaunchKernelGGL((awq_gemm_tile_kernel<RT, 8>), grid, dim3(256), 0, st, p);
-  if (p.sk_tiles > 0) hipLaunchKernelGGL((awq_gemm_tile_reduce_kernel<RT>), dim3(p.sk_tiles * RT), dim3(256), 0, st, p);
+  if (p.sk_tiles > 0) hipLaunchKernelGGL((awq_gemm_tile_reduce_kernel<RT>), dim3(p.sk_tiles * RT), dim3(1024), 0, st, p);
 }
 void launch_tile(int rt, const TileGemmParams& p, hipStream_t st) {
   switch (rt) {
@@ -403,7 +403,7 @@ void launch_tile(int rt, const TileGemmParams& p, hipStream_t st) {
       const dim3 grid(p.per_xcd * 8 + p.sk_tiles * p.sk_split);
       if (p.G == 64) hipLaunchKernelGGL((awq_gemm_tile_kernel<2, 0, 1>), grid, dim3(256), 0, st, p);
       else hipLaunchKernelGGL((awq_gemm_tile_kernel<2, 0, 2>), grid, dim3(256), 0, st, p);
-      if (p.sk_tiles > 0) hipLaunchKernelGGL((awq_gemm_tile_reduce_kernel<2>), dim3(p.sk_tiles * 2), dim3(256), 0, st, p);
+      if (p.sk_tiles > 0) hipLaunchKernelGGL((awq_gemm_tile_reduce_kernel<2>), dim3(p.sk_tiles * 2), dim3(1024), 0, st, p);
       return;
     }
     case 3: return launch_tile<3>(p, st);

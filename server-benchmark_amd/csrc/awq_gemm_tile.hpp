@@ -659,32 +659,51 @@ __global__ __launch_bounds__(256, TG_GROUPED_WGS) void awq_gemm_tile_grouped_ker
 #endif
 }
 
+// Sum of a split tile's parts, in part order: a workgroup per row tile, a thread per four columns of a row.  All parts of
+// a thread are on their way at once (a loop of four paid a trip to memory for every part behind the fourth).  Launch and all, us a launch
+// less at splits of 4 - 8: 0.35 on 2048 x 5120 and 4096 x 2048 (both at 20 / 64 rows 22.9 / 27.8 -> 22.1 / 27.1), 1 on 3584 .. 18944 weight rows (four
+// layers in groups of 64 at 20 / 64 rows 82.4 / 92.8 -> 79.4 / 90.5); level from some 128 rows on, where it is the bytes.
 template <int RT>
-__global__ __launch_bounds__(256) void awq_gemm_tile_reduce_kernel(const TileGemmParams p) {
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, fi = lane & 15, fq = lane >> 4;
+__global__ __launch_bounds__(1024) void awq_gemm_tile_reduce_kernel(const TileGemmParams p) {
+  __shared__ __align__(16) h2 out[256][8];      // [thread of the tile kernel][its 16 columns]
+  const int tid = threadIdx.x, j = tid >> 8, t = tid & 255;
   const int tl = blockIdx.x / RT, im = blockIdx.x % RT;
   const int nid = p.dp_tiles + tl;
   const int gsize = PF_GROUP_M * p.nt;
   const int first_m = (nid / gsize) * PF_GROUP_M;
   const int gm = min(p.mt - first_m, PF_GROUP_M);
-  const int row = (first_m + (nid % gsize) % gm) * (16 * RT) + 16 * im + fi;
-  const int col = (nid % gsize) / gm * 256 + 64 * wave + 16 * fq;
-  const float* base = p.sk_part + (size_t)tl * p.sk_split * tg_part_floats(RT) + ((size_t)im * 4 * 256 + tid) * 4;
-  f4 v[4];
+  const int row0 = (first_m + (nid % gsize) % gm) * (16 * RT) + 16 * im, col0 = (nid % gsize) / gm * 256;
+  const float* base = p.sk_part + (size_t)tl * p.sk_split * tg_part_floats(RT) + ((size_t)(im * 4 + j) * 256 + t) * 4;
+  f4 v = {0.f, 0.f, 0.f, 0.f};
+  auto sum = [&](auto N) {
+    constexpr int n = decltype(N)::value;
+    f4 q[n];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) v[j] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int s = 0; s < p.sk_split; ++s)
+    for (int s = 0; s < n; ++s) q[s] = *reinterpret_cast<const f4*>(base + (size_t)s * tg_part_floats(RT));
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] += *reinterpret_cast<const f4*>(base + (size_t)s * tg_part_floats(RT) + j * 1024);
-  if (row >= p.M) return;
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
-    h8 o;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) o[t] = (half_t)v[t >> 1][2 * hf + (t & 1)];
-    if (col + 8 * hf < p.N) *reinterpret_cast<h8*>(p.y + (size_t)row * p.N + col + 8 * hf) = o;
+    for (int s = 0; s < n; ++s) v += q[s];
+    base += n * tg_part_floats(RT);
+  };
+  int left = p.sk_split;
+  for (; left >= 8; left -= 8) sum(std::integral_constant<int, 8>{});
+  switch (left) {
+    case 7: sum(std::integral_constant<int, 7>{}); break;
+    case 6: sum(std::integral_constant<int, 6>{}); break;
+    case 5: sum(std::integral_constant<int, 5>{}); break;
+    case 4: sum(std::integral_constant<int, 4>{}); break;
+    case 3: sum(std::integral_constant<int, 3>{}); break;
+    case 2: sum(std::integral_constant<int, 2>{}); break;
+    case 1: sum(std::integral_constant<int, 1>{}); break;
   }
+  out[t][j] = h2{(half_t)v[0], (half_t)v[1]};
+  out[t][4 + j] = h2{(half_t)v[2], (half_t)v[3]};
+  __syncthreads();
+  if (tid >= 512) return;
+  // eight columns a thread, a row's one after the other
+  const int fi = tid >> 5, wave = (tid >> 3) & 3, fq = (tid >> 1) & 3, hf = tid & 1;
+  const int row = row0 + fi, col = col0 + 8 * (tid & 31);
+  if (row < p.M && col < p.N)
+    *reinterpret_cast<h8*>(p.y + (size_t)row * p.N + col) = *reinterpret_cast<const h8*>(&out[64 * wave + 16 * fq + fi][4 * hf]);
 }
 
 }  // namespace awqmi
