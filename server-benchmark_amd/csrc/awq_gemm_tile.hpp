@@ -152,6 +152,15 @@ __device__ __forceinline__ void tg_load_at(uint32_t lds, uint64_t addr, uint64_t
   asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b64 exec, -1"
                :: "s"(lds), "v"(addr), "s"(mask) : "memory");
 }
+// 4 bytes a lane of the lanes in `mask` into LDS at lds + 4 * lane (every lane is active around it)
+__device__ __forceinline__ void tg_load_word(uint32_t lds, const void* addr, uint64_t mask) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %2\n\tglobal_load_lds_dword %1, off\n\ts_mov_b64 exec, -1"
+               :: "s"(lds), "v"(addr), "s"(mask) : "memory");
+}
+// Scalar load of what no kernel in flight writes
+__device__ __forceinline__ int tg_scalar(const int* p) {
+  return __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(4))) int*)(uintptr_t)p);
+}
 __device__ __forceinline__ u4v tg_rsrc(const void* base, size_t bytes) {
   const uint64_t a = reinterpret_cast<uint64_t>(base);
   return u4v{(uint32_t)a, (uint32_t)(a >> 32) & 0xFFFFu, bytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)bytes, 0x00020000u};
@@ -608,11 +617,10 @@ __global__ __launch_bounds__(256, TG_GROUPED_WGS) void awq_gemm_tile_grouped_ker
   __shared__ __align__(1024) unsigned char smem[LDS];
   __shared__ int s_sid[ROWS];
   __shared__ float s_tw[ROWS];
-  __shared__ int s_rows[2];
   const int tid = threadIdx.x;
   constexpr bool runs = SCALE32 != 0;
   const int tile_rows = min(p.block, ROWS);
-  const int live = min((runs ? *p.n_live : *p.n_live / tile_rows) * p.nt, p.total);
+  const int live = min((runs ? tg_scalar(p.n_live) : tg_scalar(p.n_live) / tile_rows) * p.nt, p.total);
   int nid = blockIdx.x;
   if (!p.in_order) {
     const int per = (live + 7) >> 3;
@@ -620,27 +628,33 @@ __global__ __launch_bounds__(256, TG_GROUPED_WGS) void awq_gemm_tile_grouped_ker
     if ((int)(blockIdx.x >> 3) >= per) return;
   }
   if (nid >= live) return;
-  const int t = nid / p.nt;
+  const int t = __builtin_amdgcn_readfirstlane(nid / p.nt);
   int first = t * tile_rows, most = tile_rows;
   if (runs) {
-    const int run = p.runs[t];
+    const int run = tg_scalar(p.runs + t);
     first = (run >> 5) * 16;
     most = (run & 31) * 16;
   }
   // the expert id is on its way while the slots are staged: its weights' addresses wait for it
-  const int e = p.expert_ids[first / p.block];
+  const int eu = tg_scalar(p.expert_ids + __builtin_amdgcn_readfirstlane(first / p.block));
+  const int lane = tid & 63;
   if (tid < ROWS) {
     const int sid = tid < most ? p.sorted_ids[first + tid] : p.n_slots;
-    const bool real = sid < p.n_slots;
     s_sid[tid] = sid;
-    s_tw[tid] = (real && p.topk_w) ? p.topk_w[sid] : 1.f;
-    const unsigned long long mask = __ballot(real);     // a wave's 64 slots
-    if ((tid & 63) == 0) s_rows[tid >> 6] = mask ? tid + 64 - __clzll(mask) : 0;
+    if (!p.topk_w) s_tw[tid] = 1.f;
   }
   __syncthreads();
-  // the last real slot's row + 1: rows behind it are padding
-  const int rows = __builtin_amdgcn_readfirstlane(ROWS > 64 ? max(s_rows[0], s_rows[1]) : s_rows[0]);
-  const int eu = __builtin_amdgcn_readfirstlane(e);
+  // the last real slot's row + 1: rows behind it are padding.  Every wave looks at all of them; the output weights, which nothing
+  // needs before the tile's end, go to LDS by themselves
+  int last = 0;
+#pragma unroll
+  for (int i = 0; i < ROWS; i += 64) {
+    const int sid = s_sid[i + lane];
+    const unsigned long long real = __ballot(sid < p.n_slots);
+    if (real) last = i + 64 - __clzll(real);
+    if (p.topk_w && __builtin_amdgcn_readfirstlane(tid >> 6) == i / 64) tg_load_word((uint32_t)(uintptr_t)(lds_byte*)(s_tw + i), p.topk_w + sid, real);
+  }
+  const int rows = __builtin_amdgcn_readfirstlane(last);
   const int n0 = (nid % p.nt) * (ACT ? TG_COLS / 2 : TG_COLS);
   const uint32_t lds = (uint32_t)(uintptr_t)(lds_byte*)smem;
   auto tile = [&](auto R) __attribute__((always_inline)) {
