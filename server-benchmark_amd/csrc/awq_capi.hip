@@ -541,10 +541,12 @@ static int moe_route_launches(const MoeRoute& r, int tile, void* stream) {
   return launch_status();
 }
 
-// Folded routing: at most four tokens, which one wave of a workgroup picks for at once (128 experts, top-8, weights from HBM:
-// 3.5 us of 29 - 38 faster at 1 - 4 tokens; from five on, a second round in every workgroup cost what the saved launch gains).
+// Folded routing: at most 16 tokens, which the four waves of a workgroup pick for at once, and 64 slots (one lane each).  Routed apart /
+// folded, us, weights from HBM: 128 experts of 2048 x 768, top-8, at 1, 4, 5, 6, 8 tokens 28.7, 36.7, 38.8, 40.5, 47.4 / 25.0, 31.9, 34.9, 36.6,
+// 43.5; 64 of 2048 x 1408, top-6, at 10 53.9 / 50.1; 64 of 5120 x 1024, top-4, at 8, 12, 16 62.2, 84.2, 88.8 / 58.3, 80.0, 84.7; 8 of 4096 x
+// 14336, top-2, at 8, 16 142.6, 151.4 / 138.5, 148.5; 256 of 3072 x 1536, top-4, at 16 89.2 / 89.0.
 static bool moe_route_foldable(int T, int E, int topk, int tile) {
-  return T <= 4 && moe_topk_lanes(E, topk) == 16 && tile == 16 && !variant_on(VAR_NO_FOLDED_ROUTE);
+  return T <= 16 && T * topk <= 64 && moe_topk_lanes(E, topk) == 16 && tile == 16 && !variant_on(VAR_NO_FOLDED_ROUTE);
 }
 
 extern "C" {

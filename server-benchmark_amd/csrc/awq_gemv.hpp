@@ -54,7 +54,7 @@ struct GemvParams {
   int act_split; // split-K launch over [gate | up] columns: the last arriver of a gate block and
                  // its up block writes silu(gate) * up (one 16-row block, four waves per column block)
   long long w_stride, s_stride, z_stride;  // elements per expert
-  // Routing folded into the launch (awq_gemv_route_kernel: at most four tokens, 16 picks each): every
+  // Routing folded into the launch (awq_gemv_route_kernel: at most 16 tokens and 64 slots): every
   // workgroup works the routing and the block list out by itself from the router logits, and
   // the first workgroup also leaves them in memory for the launches that follow.
   const float* r_logits;   // [r_T][r_E]
@@ -436,12 +436,12 @@ struct GemvWave {
 // LDSQ: weight ring of RING = 4 steps in LDS (see GemvWave), two workgroups per CU.
 // TAIL (dense launches, see GemvWave): every wave gets the same number of whole chunks and the
 // chunks left over are taken one 32-row step per wave.
-// RPER > 0 (MoE launches of up to four tokens, 16-row blocks): the launch does its
-// own routing.  The first wave of EVERY workgroup runs the top-k of the tokens (16 lanes each, RPER experts
+// RPER > 0 (MoE launches of up to 16 tokens and 64 slots, 16-row blocks): the launch does its
+// own routing.  The waves of EVERY workgroup run the top-k of four tokens each (16 lanes a token, RPER experts
 // per lane, RSIG = sigmoid scoring) into LDS; every wave then sorts the slots by expert in
 // registers (lane = slot: equal-expert mask from one ballot per id bit, block index = number of
 // distinct smaller experts) and so knows its block's expert and rows without a trip to memory.
-// A token picks distinct experts, so an expert holds at most T <= 4 slots and every block is one
+// A token picks distinct experts, so an expert holds at most T <= 16 slots and every block is one
 // expert's single block.  Workgroup 0 writes ids, weights, block list and padded count out for
 // the launches that follow (same layout as the align kernel's, entries past the last block that
 // runs left unwritten: nothing reads them).
@@ -505,9 +505,9 @@ __device__ __forceinline__ void awq_gemv_body(const GemvParams& p) {
       __shared__ int r_exp_s[64];
       const int n = p.n_slots;
       if (blk >= n) return;      // no more blocks than slots (workgroup 0 is block 0's)
-      if (wave == 0)
-        moe_topk_tokens<16, RPER, RSIG>(p.r_logits, p.r_bias, 0, p.r_T, p.r_E, p.r_topk, p.r_renorm, p.r_scale, r_ids_s,
-                                        r_wts_s);
+      if (4 * wave < p.r_T)
+        moe_topk_tokens<16, RPER, RSIG>(p.r_logits, p.r_bias, 4 * wave, p.r_T, p.r_E, p.r_topk, p.r_renorm, p.r_scale,
+                                        r_ids_s, r_wts_s);
       __syncthreads();
       const bool valid = lane < n;
       const int e_i = valid ? r_ids_s[lane] : 0x7fffffff;
@@ -521,9 +521,12 @@ __device__ __forceinline__ void awq_gemv_body(const GemvParams& p) {
       const int r_i = __popcll(same & ((1ull << lane) - 1ull));     // row inside the expert's block
       const unsigned long long firsts = __ballot(valid && r_i == 0);
       int b_i = 0;                                                  // block = distinct smaller experts
-      for (int jj = 0; jj < n; ++jj) {
-        const int ej = __builtin_amdgcn_readlane(e_i, jj);
-        if (((firsts >> jj) & 1ull) && ej < e_i) ++b_i;
+      // by a mask of the experts there are, 32 at a time (a loop over the slots, reading each one's expert, cost 0.04 us a slot)
+#pragma unroll
+      for (int w = 0; w < RPER / 2; ++w) {
+        const int at = e_i - 32 * w;
+        const unsigned there = wave_or(valid && (unsigned)at < 32u ? 1u << at : 0u);
+        b_i += __popc(at >= 32 ? there : at > 0 ? there & ((1u << at) - 1u) : 0u);
       }
       const int nb = __popcll(firsts);
       if (blockIdx.x == 0) {
@@ -546,15 +549,10 @@ __device__ __forceinline__ void awq_gemv_body(const GemvParams& p) {
       if (blk >= nb) return;
       const unsigned long long mine = __ballot(valid && b_i == blk);
       e = __builtin_amdgcn_readlane(e_i, __builtin_ctzll(mine));
-      // thread r takes the slot of row r: the r-th set lane of `mine` (at most four rows)
-      unsigned long long m = mine;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        if (m) {
-          if (tid == k) sid = __builtin_ctzll(m);
-          m &= m - 1ull;
-        }
-      }
+      // thread r takes the slot of row r: the r-th set lane of `mine` (at most a row per token)
+      int k = 0;
+      for (unsigned long long m = mine; m; m &= m - 1ull, ++k)
+        if (tid == k) sid = __builtin_ctzll(m);
     } else {
     // The block's padded count, expert and slot ids are read side by side (one trip to memory
     // instead of three in a row; blocks past the lists' end read the last block's entries and

@@ -234,6 +234,21 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const float* __restrict__
 // first block * 32 + blocks of each (runs null: none wanted).
 constexpr int MOE_RUN = 4;
 
+// OR over the wave, wave-uniform.
+__device__ __forceinline__ unsigned wave_or(unsigned v) {
+  auto step = [&](auto CTRL, auto ROWS) {
+    v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, decltype(CTRL)::value, decltype(ROWS)::value, 0xf, false);
+  };
+  using std::integral_constant;
+  step(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});   // row_shr:1
+  step(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});   // row_shr:2
+  step(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});   // row_shr:4
+  step(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});   // row_shr:8
+  step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});   // row_bcast:15 into rows 1, 3
+  step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});   // row_bcast:31 into rows 2, 3
+  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 // Inclusive prefix sum over the wave by DPP row shifts and row broadcasts.
 __device__ __forceinline__ int wave_prefix_sum(int v) {
   auto step = [&](auto CTRL, auto ROWS) {

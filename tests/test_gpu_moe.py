@@ -706,6 +706,21 @@ def test_routing_folded_into_the_first_expert_gemm(sba, gpu, scoring, T, H, E, t
         assert torch.equal(y1.view(torch.int16), y1_sep.view(torch.int16))
 
 
+@pytest.mark.parametrize("scoring", ["softmax", "sigmoid"])
+@pytest.mark.parametrize("T,E,topk", [(5, 128, 8), (8, 128, 8), (8, 4, 4), (7, 256, 9), (8, 33, 8), (5, 16, 12), (3, 64, 16), (9, 128, 7), (10, 128, 7),
+                                      (16, 4, 4), (16, 8, 2), (13, 256, 4), (17, 64, 2)])
+def test_routing_folded_for_five_to_sixteen_tokens(sba, gpu, scoring, T, E, topk):
+    """Up to four waves with four tokens each, up to 64 slots, blocks of up to 16 rows, experts in the first and the last word
+    of the mask; 70 slots and 17 tokens are past the lines.  The bits of the separately routed block."""
+    c = sba.workloads.make_moe_case(T, 512, E, topk, 256, 128, seed=5 * T + E).to(gpu)
+    kw = {}
+    if scoring == "sigmoid":
+        kw = dict(scoring_func="sigmoid", e_score_correction_bias=torch.linspace(0, 0.1, E, device=gpu), routed_scaling_factor=1.25)
+    y = sba.fused_moe_awq(c.x, c.w13, c.w2, c.logits, topk, True, **kw).clone()
+    y_sep = sba.fused_moe_awq(c.x, c.w13, c.w2, c.logits, topk, True, _dev_variant=1 << 24, **kw)
+    assert torch.equal(y.view(torch.int16), y_sep.view(torch.int16))
+
+
 def test_folded_routing_with_nan_logits(sba, gpu):
     """A NaN logit in a folded-routing block: ids stay in range (the block runs, every slot row is
     written) and the output equals the separately routed block's, NaNs included."""
