@@ -676,7 +676,7 @@ __global__ __launch_bounds__(256, TG_GROUPED_WGS) void awq_gemm_tile_grouped_ker
 // Sum of a split tile's parts, in part order: a workgroup per row tile, a thread per four columns of a row.  All parts of
 // a thread are on their way at once (a loop of four paid a trip to memory for every part behind the fourth).  Launch and all, us a launch
 // less at splits of 4 - 8: 0.35 on 2048 x 5120 and 4096 x 2048 (both at 20 / 64 rows 22.9 / 27.8 -> 22.1 / 27.1), 1 on 3584 .. 18944 weight rows (four
-// layers in groups of 64 at 20 / 64 rows 82.4 / 92.8 -> 79.4 / 90.5); level from some 128 rows on, where it is the bytes.
+// layers in groups of 64 at 20 / 64 rows 82.4 / 92.8 -> 79.4 / 90.5); level from some 128 rows on and on 8192 columns and more, where it is the bytes (4.9 us at 64 rows).
 template <int RT>
 __global__ __launch_bounds__(1024) void awq_gemm_tile_reduce_kernel(const TileGemmParams p) {
   __shared__ __align__(16) h2 out[256][8];      // [thread of the tile kernel][its 16 columns]
