@@ -26,8 +26,8 @@
  *   1 << 20  v = bits 20..22: fused tiles of 64 v rows (v = 1..4) or 16 v rows (v = 5..7) whatever M is
  *   1 << 29  v = bits 29..30: fused tiles of 160 / 208 / 224 rows (v = 1 / 2 / 3) whatever M is
  *   1 << 23  dense skinny launches never share left-over chunks step by step
- *   1 << 24  the one-call MoE block always routes in a launch of its own (blocks of at most four
- *            tokens otherwise fold the routing into the first expert GEMM)
+ *   1 << 24  the one-call MoE block always routes in a launch of its own (blocks of at most 16 tokens
+ *            and 64 slots otherwise fold the routing into the first expert GEMM)
  *   1 << 25  awq_gemm never takes the dequantise-once form (many-row calls run the fused kernel)
  *   1 << 26  awq_gemm takes the dequantise-once form from 257 rows on, when the workspace holds
  *            awqmi_dev_gemm_dense_workspace_bytes()
@@ -118,6 +118,9 @@ int awqmi_dev_fused_moe_block_rows(int T, int H, int inter, int E, int topk, int
 
 /* 1 if the one-call MoE block takes its 16-slot blocks in tiles of up to four for these shapes, else 0. */
 int awqmi_dev_fused_moe_tiles(int T, int H, int inter, int E, int topk, int group, int variant);
+
+/* 1 if the first expert GEMM of the one-call MoE block takes the routing along for these shapes, else 0. */
+int awqmi_dev_fused_moe_folds(int T, int H, int inter, int E, int topk, int group, int variant);
 
 #ifdef __cplusplus
 }

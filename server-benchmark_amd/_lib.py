@@ -53,7 +53,7 @@ for _name in ("awqmi_gemm_f16", "awqmi_moe_gemm_f16", "awqmi_fused_moe_routed_f1
     _res, _args = SIGNATURES[_name]
     SIGNATURES[_name.replace("awqmi_", "awqmi_dev_", 1)] = (_res, [*_args, c_int])
 
-SIGNATURES["awqmi_dev_fused_moe_tiles"] = SIGNATURES["awqmi_dev_fused_moe_block_rows"]
+SIGNATURES["awqmi_dev_fused_moe_tiles"] = SIGNATURES["awqmi_dev_fused_moe_folds"] = SIGNATURES["awqmi_dev_fused_moe_block_rows"]
 SIGNATURES["awqmi_dev_last_gemm_form"] = (c_int, [])
 SIGNATURES["awqmi_dev_gemm_dense_workspace_bytes"] = (c_size_t, [c_int, c_int, c_int])
 SIGNATURES["awqmi_dev_stream_probe"] = (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_size_t, c_void_p])

@@ -542,12 +542,15 @@ static int moe_route_launches(const MoeRoute& r, int tile, void* stream) {
   return launch_status();
 }
 
-// Folded routing: at most 16 tokens, which the four waves of a workgroup pick for at once, and 64 slots (one lane each).  Routed apart /
+// Folded routing: no more tokens than the four waves of a workgroup pick for at once (16, or 4 with a token a wave), 64 slots (one lane
+// each), 256 experts.  Routed apart /
 // folded, us, weights from HBM: 128 experts of 2048 x 768, top-8, at 1, 4, 5, 6, 8 tokens 28.7, 36.7, 38.8, 40.5, 47.4 / 25.0, 31.9, 34.9, 36.6,
 // 43.5; 64 of 2048 x 1408, top-6, at 10 53.9 / 50.1; 64 of 5120 x 1024, top-4, at 8, 12, 16 62.2, 84.2, 88.8 / 58.3, 80.0, 84.7; 8 of 4096 x
 // 14336, top-2, at 8, 16 142.6, 151.4 / 138.5, 148.5; 256 of 3072 x 1536, top-4, at 16 89.2 / 89.0.
+constexpr int MOE_FOLD_EXPERTS = 256;
 static bool moe_route_foldable(int T, int E, int topk, int tile) {
-  return T <= 16 && T * topk <= 64 && moe_topk_lanes(E, topk) == 16 && tile == 16 && !variant_on(VAR_NO_FOLDED_ROUTE);
+  return T <= 4 * (64 / moe_topk_lanes(E, topk)) && T * topk <= 64 && E <= MOE_FOLD_EXPERTS && tile == 16 &&
+         !variant_on(VAR_NO_FOLDED_ROUTE);
 }
 
 extern "C" {
@@ -970,6 +973,48 @@ static long long moe_most_runs(int n_slots, int E) {
 }
 static_assert(TG_RUN == MOE_RUN, "the tile lists are made for the grouped kernel");
 
+// Form of a grouped launch of 16-row blocks.
+struct MoeSkinnyForm {
+  bool pair_cols;      // two column blocks per workgroup, two waves each
+  bool act_split;      // fused activation by the last arrivers of a K split ...
+  bool act_pair;       // ... or in the workgroup that has the gate and the up block
+  bool ldsq;           // weight ring in LDS
+  bool plain;          // none of them but act_split, register ring of two: the form that can take the routing along
+};
+static MoeSkinnyForm moe_skinny_form(const MoePlan& pl, int n_slots, int E, int K, int N, int tile_m, bool fuse_act) {
+  MoeSkinnyForm f{};
+  // few chunks of K and no split across workgroups: two column blocks per workgroup, two
+  // waves each (three chunks per wave at K = 768 instead of 2 / 2 / 1 / 1)
+  // -- as long as the paired launch still fills the chip (blocks that will run: one per expert
+  // touched or per 16 slots, whichever is more)
+  const long long live_blocks = std::max<long long>((n_slots + 15) / 16, std::min(n_slots, E));
+  f.pair_cols = tile_m == 16 && pl.wpl == 2 && pl.split == 1 && K / 128 <= 8 && (K / 128) % 2 == 0 &&
+                live_blocks * ((pl.ncb + 1) / 2) >= 256 && !variant_on(VAR_NO_PAIR_COLS);
+  // fused activation: without a split the paired-column kernel (gate and up block in one
+  // workgroup); with a split the ordinary launch whose last arrivers pair the blocks up
+  f.act_split = fuse_act && pl.split > 1;
+  f.act_pair = fuse_act && pl.split == 1;
+  // weight ring of four steps in LDS instead of two in registers, from one full block per
+  // expert on (T = 256 ... 1024 of the 128-expert block: 6 - 10 % faster; with fewer rows per
+  // expert 1 - 4 % slower, and no gain for the few-block launches once their weights come from
+  // HBM rather than from a warm cache)
+  f.ldsq = pl.wpl == 2 && tile_m == 16 && (size_t)K * (N / 8) * 4 < (1ull << 31) && (long long)n_slots >= 16LL * E &&
+           !variant_on(VAR_NO_LDS_RING);
+  f.plain = !f.ldsq && !f.act_pair &&
+            (f.act_split || (tile_m == 16 && pl.wpl == 2 && !f.pair_cols && !variant_on(VAR_MOE_RING4)));
+  return f;
+}
+// Does a launch in that form take the routing along?  Every workgroup picks by itself, one pick after the other, and those that
+// start when others end are held up by it: with more than 16 picks the workgroups that are expected to run (a block more with several
+// tokens) have to fit the chip at once, two a CU.  Routed apart / folded, us: 20, 22, 24, 32 picks of 256 experts of 3072 x 1536, two
+// tokens (461, 505, 549, 720 workgroups) 74.9, 88.3, 94.3, 102.9 / 70.8, 91.9, 99.4, 111.4; 32 of 64 of 2048 x 2048, one and two tokens (512, 768)
+// 61.1, 86.2 / 57.4, 89.5.  Up to eight picks take less than the launch: 8 of 256 of 7168 x 2048, eight tokens (919) 245.3 / 240.5.
+static bool moe_launch_folds(const MoeSkinnyForm& f, const MoePlan& pl, int T, int E, int topk, int tile_m, int G) {
+  if (!f.plain || G != 128 || !moe_route_foldable(T, E, topk, tile_m)) return false;
+  const double blocks = E * (1.0 - std::pow(1.0 - (double)topk / E, T)) + (T > 1);
+  return topk <= 16 || blocks * pl.ncb * pl.split <= 512.0;
+}
+
 static int moe_gemm_impl(const void* x, const int32_t* qweight, const void* scales, const int32_t* qzeros,
                          void* y, const int32_t* sorted_token_ids, const int32_t* expert_ids,
                          const int32_t* num_tokens_post_padded, const float* topk_weights, int n_slots,
@@ -1106,21 +1151,12 @@ static int moe_gemm_impl(const void* x, const int32_t* qweight, const void* scal
   p.grp = (long long)n_slots * 2 >= 3LL * tile_m * E ? 32 : ((long long)n_slots * 4 >= 3LL * tile_m * E ? 8 : 1);
   if (E < 16) p.grp = 1;   // a handful of large experts: the plain order measured equal or up to 13 % faster
   if (variant >= 0 && ((variant >> VAR_XCD_RUN_SHIFT) & 7)) p.grp = 1 << (((variant >> VAR_XCD_RUN_SHIFT) & 7) - 1);
-  // few chunks of K and no split across workgroups: two column blocks per workgroup, two
-  // waves each (three chunks per wave at K = 768 instead of 2 / 2 / 1 / 1)
-  // -- as long as the paired launch still fills the chip (blocks that will run: one per expert
-  // touched or per 16 slots, whichever is more)
-  const long long live_blocks = std::max<long long>((n_slots + 15) / 16, std::min(n_slots, E));
-  const bool pair_cols = tile_m == 16 && wpl == 2 && split == 1 && K / 128 <= 8 && (K / 128) % 2 == 0 &&
-                         live_blocks * ((ncb + 1) / 2) >= 256 && !variant_on(VAR_NO_PAIR_COLS);
-  // fused activation: without a split the paired-column kernel (gate and up block in one
-  // workgroup); with a split the ordinary launch whose last arrivers pair the blocks up
+  const MoeSkinnyForm form = moe_skinny_form(pl, n_slots, E, K, N, tile_m, fuse_act);
+  const bool pair_cols = form.pair_cols, act_split = form.act_split, act_pair = form.act_pair, ldsq = form.ldsq;
   if (fuse_act && (wpl != 2 || tile_m != 16 || ncb % 2 != 0 || N % 512 != 0 ||
                    (split == 1 && (K / 128) % 2 != 0)))
     return AWQMI_BAD_ARGUMENT;
-  const bool act_split = fuse_act && split > 1;
   p.act_split = act_split ? 1 : 0;
-  const bool act_pair = fuse_act && split == 1;
   const int ncb1 = (NW + 15) / 16;       // column blocks of 128 (one word per lane)
   const bool t32_lds = t32_narrow && (size_t)K * NW * 4 < (1ull << 31) && !variant_on(VAR_NO_LDS_RING);
   const int ncg = t32_narrow ? (ncb1 + 1) / 2 : (act_pair ? ncb / 2 : (pair_cols ? (ncb + 1) / 2 : ncb));
@@ -1129,31 +1165,18 @@ static int moe_gemm_impl(const void* x, const int32_t* qweight, const void* scal
   const long long deals = (long long)(nblk / p.grp) * ncg * split;
   const dim3 grid((unsigned)((deals + 7) / 8 * 8 * p.grp));
   hipStream_t st = (hipStream_t)stream;
-  // weight ring of four steps in LDS instead of two in registers, from one full block per
-  // expert on (T = 256 ... 1024 of the 128-expert block: 6 - 10 % faster; with fewer rows per
-  // expert 1 - 4 % slower, and no gain for the few-block launches once their weights come from
-  // HBM rather than from a warm cache)
-  const bool ldsq = wpl == 2 && tile_m == 16 && (size_t)K * NW * 4 < (1ull << 31) &&
-                    (long long)n_slots >= 16LL * E && !variant_on(VAR_NO_LDS_RING);
-  const bool plain_form = !ldsq && !act_pair &&
-                          (act_split || (tile_m == 16 && wpl == 2 && !pair_cols && !variant_on(VAR_MOE_RING4)));
   if (route) {
-    if (plain_form && G == 128 && moe_route_foldable(route->T, route->E, route->topk, tile_m)) {
+    if (moe_launch_folds(form, pl, route->T, route->E, route->topk, tile_m, G)) {
       p.r_logits = route->logits; p.r_bias = route->bias;
       p.r_T = route->T; p.r_E = route->E; p.r_topk = route->topk; p.r_renorm = route->renorm;
       p.r_scale = route->scale;
       p.r_ids = route->ids; p.r_wts = route->wts; p.r_sorted = route->sorted; p.r_experts = route->experts;
       p.r_npp = route->npp;
-      const bool sig = route->scoring == 1;
-#define AWQMI_ROUTE(PERV)                                                                                   \
-  do {                                                                                                      \
-    if (sig) hipLaunchKernelGGL((awq_gemv_route_kernel<2, PERV, true>), grid, dim3(256), 0, st, p);        \
-    else hipLaunchKernelGGL((awq_gemv_route_kernel<2, PERV, false>), grid, dim3(256), 0, st, p);           \
-  } while (0)
-      if (route->E <= 64) AWQMI_ROUTE(4);
-      else if (route->E <= 128) AWQMI_ROUTE(8);
-      else AWQMI_ROUTE(16);
-#undef AWQMI_ROUTE
+      moe_topk_form(route->E, route->topk, route->scoring, [&](auto L, auto P, auto S) {
+        if constexpr (decltype(L)::value * decltype(P)::value <= MOE_FOLD_EXPERTS)
+          hipLaunchKernelGGL((awq_gemv_route_kernel<2, decltype(L)::value, decltype(P)::value, decltype(S)::value>), grid,
+                             dim3(256), 0, st, p);
+      });
       return launch_status();
     }
     if (const int rc = moe_route_launches(*route, tile_m, stream)) return rc;
@@ -1569,6 +1592,16 @@ int awqmi_dev_fused_moe_tiles(int T, int H, int inter, int E, int topk, int grou
   if (!awqmi_fused_moe_block_rows(T, H, inter, E, topk, group)) return 0;
   VariantScope scope(variant);
   return moe_form(T, H, inter, E, topk, group).runs;
+}
+
+int awqmi_dev_fused_moe_folds(int T, int H, int inter, int E, int topk, int group, int variant) {
+  if (!awqmi_fused_moe_block_rows(T, H, inter, E, topk, group)) return 0;
+  VariantScope scope(variant);
+  const MoeForm form = moe_form(T, H, inter, E, topk, group);
+  const int n_slots = T * topk, G = norm_group(H, group);
+  if (form.tile != 16 || form.runs || !gemv_tiled_ok(H, G)) return 0;
+  const MoePlan pl = moe_plan(n_slots, E, H, 2 * inter, 16, 0);
+  return moe_launch_folds(moe_skinny_form(pl, n_slots, E, H, 2 * inter, 16, form.act), pl, T, E, topk, 16, G);
 }
 
 }  // extern "C"

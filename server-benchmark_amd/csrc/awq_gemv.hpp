@@ -437,7 +437,7 @@ struct GemvWave {
 // TAIL (dense launches, see GemvWave): every wave gets the same number of whole chunks and the
 // chunks left over are taken one 32-row step per wave.
 // RPER > 0 (MoE launches of up to 16 tokens and 64 slots, 16-row blocks): the launch does its
-// own routing.  The waves of EVERY workgroup run the top-k of four tokens each (16 lanes a token, RPER experts
+// own routing.  The waves of EVERY workgroup run the top-k of 64 / RLANES tokens each (RLANES lanes a token, RPER experts
 // per lane, RSIG = sigmoid scoring) into LDS; every wave then sorts the slots by expert in
 // registers (lane = slot: equal-expert mask from one ballot per id bit, block index = number of
 // distinct smaller experts) and so knows its block's expert and rows without a trip to memory.
@@ -445,8 +445,8 @@ struct GemvWave {
 // expert's single block.  Workgroup 0 writes ids, weights, block list and padded count out for
 // the launches that follow (same layout as the align kernel's, entries past the last block that
 // runs left unwritten: nothing reads them).
-template <int WPL, int GMODE, int MB, bool MOE, int RING, int KW, bool ACT, bool LDSQ, bool TAIL, int RPER = 0,
-          bool RSIG = false>
+template <int WPL, int GMODE, int MB, bool MOE, int RING, int KW, bool ACT, bool LDSQ, bool TAIL, int RLANES = 16,
+          int RPER = 0, bool RSIG = false>
 __device__ __forceinline__ void awq_gemv_body(const GemvParams& p) {
   static_assert(RPER == 0 || (MOE && MB == 1 && !TAIL), "folded routing: expert-grouped launches of 16-row blocks");
   static_assert(!ACT || (KW == 2 && MB == 1), "fused activation pairs two column blocks");
@@ -505,9 +505,10 @@ __device__ __forceinline__ void awq_gemv_body(const GemvParams& p) {
       __shared__ int r_exp_s[64];
       const int n = p.n_slots;
       if (blk >= n) return;      // no more blocks than slots (workgroup 0 is block 0's)
-      if (4 * wave < p.r_T)
-        moe_topk_tokens<16, RPER, RSIG>(p.r_logits, p.r_bias, 4 * wave, p.r_T, p.r_E, p.r_topk, p.r_renorm, p.r_scale,
-                                        r_ids_s, r_wts_s);
+      constexpr int TOK = 64 / RLANES;      // tokens of a wave (the call has at most four waves' worth)
+      if (TOK * wave < p.r_T)
+        moe_topk_tokens<RLANES, RPER, RSIG>(p.r_logits, p.r_bias, TOK * wave, p.r_T, p.r_E, p.r_topk, p.r_renorm,
+                                            p.r_scale, r_ids_s, r_wts_s);
       __syncthreads();
       const bool valid = lane < n;
       const int e_i = valid ? r_ids_s[lane] : 0x7fffffff;
@@ -523,7 +524,7 @@ __device__ __forceinline__ void awq_gemv_body(const GemvParams& p) {
       int b_i = 0;                                                  // block = distinct smaller experts
       // by a mask of the experts there are, 32 at a time (a loop over the slots, reading each one's expert, cost 0.04 us a slot)
 #pragma unroll
-      for (int w = 0; w < RPER / 2; ++w) {
+      for (int w = 0; w < RLANES * RPER / 32; ++w) {
         const int at = e_i - 32 * w;
         const unsigned there = wave_or(valid && (unsigned)at < 32u ? 1u << at : 0u);
         b_i += __popc(at >= 32 ? there : at > 0 ? there & ((1u << at) - 1u) : 0u);
@@ -883,10 +884,10 @@ __global__ __launch_bounds__(256, ((RING == 4 && !LDSQ) || (MB == 2 && WPL == 2)
 }
 
 // the expert-grouped launch of 16-row blocks (two words per lane, register ring of two) with the
-// routing folded in: RPER experts per lane, RSIG = sigmoid scoring
-template <int GMODE, int RPER, bool RSIG>
+// routing folded in: RLANES lanes a token, RPER experts per lane, RSIG = sigmoid scoring
+template <int GMODE, int RLANES, int RPER, bool RSIG>
 __global__ __launch_bounds__(256, 2) void awq_gemv_route_kernel(const GemvParams p) {
-  awq_gemv_body<2, GMODE, 1, true, 2, 4, false, false, false, RPER, RSIG>(p);
+  awq_gemv_body<2, GMODE, 1, true, 2, 4, false, false, false, RLANES, RPER, RSIG>(p);
 }
 
 // the dense G = 128 launch in its TAIL form (left-over chunks step by step)

@@ -721,6 +721,28 @@ def test_routing_folded_for_five_to_sixteen_tokens(sba, gpu, scoring, T, E, topk
     assert torch.equal(y.view(torch.int16), y_sep.view(torch.int16))
 
 
+@pytest.mark.parametrize("scoring", ["softmax", "sigmoid"])
+@pytest.mark.parametrize("T,E,topk", [(1, 17, 17), (1, 64, 64), (2, 65, 32), (3, 128, 21), (2, 129, 17), (3, 256, 20)])
+def test_routing_folded_with_more_than_sixteen_picks(sba, gpu, scoring, T, E, topk):
+    """A token a wave, up to three tokens, experts on both sides of one, two and four a lane: the bits of the separately routed block,
+    and the oracle's result."""
+    from server_benchmark_amd import _lib
+    assert _lib.load().awqmi_dev_fused_moe_folds(T, 512, 256, E, topk, 128, -1) == 1
+    c = sba.workloads.make_moe_case(T, 512, E, topk, 256, 128, seed=5 * T + E)
+    d = c.to(gpu)
+    kw = {}
+    if scoring == "sigmoid":
+        kw = dict(scoring_func="sigmoid", e_score_correction_bias=torch.linspace(0, 0.1, E, device=gpu), routed_scaling_factor=1.25)
+        ids, tw = awq_ref.topk_sigmoid(c.logits.numpy(), topk, True, np.linspace(0, 0.1, E, dtype=np.float32), 1.25)
+    else:
+        ids, tw = awq_ref.topk_softmax(c.logits.numpy(), topk, True)
+    y = sba.fused_moe_awq(d.x, d.w13, d.w2, d.logits, topk, True, **kw).clone()
+    y_sep = sba.fused_moe_awq(d.x, d.w13, d.w2, d.logits, topk, True, _dev_variant=1 << 24, **kw)
+    assert torch.equal(y.view(torch.int16), y_sep.view(torch.int16))
+    ref = awq_ref.moe_forward(c.x.numpy(), tuple(a.numpy() for a in c.w13), tuple(a.numpy() for a in c.w2), ids, tw, 128)
+    assert awq_ref.rel_frobenius(y.cpu().numpy(), ref) <= TOL
+
+
 def test_folded_routing_with_nan_logits(sba, gpu):
     """A NaN logit in a folded-routing block: ids stay in range (the block runs, every slot row is
     written) and the output equals the separately routed block's, NaNs included."""
