@@ -1005,14 +1005,15 @@ static MoeSkinnyForm moe_skinny_form(const MoePlan& pl, int n_slots, int E, int 
   return f;
 }
 // Does a launch in that form take the routing along?  Every workgroup picks by itself, one pick after the other, and those that
-// start when others end are held up by it: with more than 16 picks the workgroups that are expected to run (a block more with several
+// start when others end are held up by it: with more than eight picks the workgroups that are expected to run (a block more with several
 // tokens) have to fit the chip at once, two a CU.  Routed apart / folded, us: 20, 22, 24, 32 picks of 256 experts of 3072 x 1536, two
 // tokens (461, 505, 549, 720 workgroups) 74.9, 88.3, 94.3, 102.9 / 70.8, 91.9, 99.4, 111.4; 32 of 64 of 2048 x 2048, one and two tokens (512, 768)
-// 61.1, 86.2 / 57.4, 89.5.  Up to eight picks take less than the launch: 8 of 256 of 7168 x 2048, eight tokens (919) 245.3 / 240.5.
+// 61.1, 86.2 / 57.4, 89.5; 16 of 128 of 2048 x 1408, three and four (465, 583) 57.7, 67.5 / 54.2, 68.7; 12 of 256 of 3072 x 1536, five (656)
+// 91.0 / 92.1.  Up to eight picks take less than the launch: 8 of 256 of 7168 x 2048, eight tokens (919) 245.3 / 240.5.
 static bool moe_launch_folds(const MoeSkinnyForm& f, const MoePlan& pl, int T, int E, int topk, int tile_m, int G) {
   if (!f.plain || G != 128 || !moe_route_foldable(T, E, topk, tile_m)) return false;
   const double blocks = E * (1.0 - std::pow(1.0 - (double)topk / E, T)) + (T > 1);
-  return topk <= 16 || blocks * pl.ncb * pl.split <= 512.0;
+  return topk <= 8 || blocks * pl.ncb * pl.split <= 512.0;
 }
 
 static int moe_gemm_impl(const void* x, const int32_t* qweight, const void* scales, const int32_t* qzeros,
