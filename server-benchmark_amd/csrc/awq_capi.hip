@@ -10,6 +10,7 @@
 #include <cmath>
 #include <cstdint>
 #include <type_traits>
+#include <utility>
 
 #include "../../include/awq_mi355x.h"
 #include "../../include/awq_mi355x_dev.h"
@@ -1433,6 +1434,13 @@ int awqmi_fused_moe_routed_f16(const void* hidden, const float* router_logits, c
   const int tile = form.tile;
   const FusedMoeLayout L = fused_moe_layout(T, H, inter, E, topk, tile);
   if (workspace_bytes < L.total) return AWQMI_WORKSPACE_TOO_SMALL;
+  // what the launches behind the first one would refuse, so that a call either runs whole or leaves nothing on the stream
+  for (const auto& [K, N] : {std::pair{H, 2 * inter}, std::pair{inter, H}}) {
+    if (const int rc = check_awq_shape(K, N, norm_group(K, group))) return rc;
+    if (!gemv_tiled_ok(K, norm_group(K, group))) return AWQMI_UNSUPPORTED_GROUP;
+  }
+  for (const void* p : {hidden, (const void*)w13_q, w13_s, (const void*)w13_z, (const void*)w2_q, w2_s, (const void*)w2_z, (const void*)out})
+    if (!aligned16(p)) return AWQMI_BAD_ALIGN;
   char* ws = static_cast<char*>(workspace);
   int32_t* ids = reinterpret_cast<int32_t*>(ws + L.ids);
   float* wts = reinterpret_cast<float*>(ws + L.wts);
