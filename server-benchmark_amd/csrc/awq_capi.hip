@@ -491,8 +491,7 @@ struct MoeRoute {
   int32_t* experts;
   int32_t* npp;
   int32_t* runs;     // tiles of several 16-slot blocks, or null
-  int32_t* tab;      // expert counts of the parts of a longer batch, [tab_parts][E]
-  int tab_parts;
+  int32_t* tab;      // expert counts of the parts of a longer batch, [MOE_PARTS_MAX][E]
 };
 
 static int moe_align_launch(const int32_t* topk_ids, int n_slots, int E, int tile_m, int32_t* sorted, int32_t* experts,
@@ -510,10 +509,16 @@ static int moe_align_launch(const int32_t* topk_ids, int n_slots, int E, int til
 // 80.1 / 81.2; 256 98 / - / 97.5 / 97.3; 1500 172 / - / - / 166; 8192 696 / - / - / 688.
 constexpr int MOE_ONE_WG_SLOTS = 2048;
 struct MoeParts { int part, parts; };     // tokens of a part, parts
-static MoeParts moe_parts(int T, int most) {
-  const int part = (T + 16 * most - 1) / (16 * most) * 16;
+static MoeParts moe_parts(int T) {
+  const int part = (T + 16 * MOE_PARTS_MAX - 1) / (16 * MOE_PARTS_MAX) * 16;
   return {part, (T + part - 1) / part};
 }
+// The table of counts has room of its own for 64 parts, the rest lies where the activation goes later: a block in parts has more
+// than MOE_ONE_WG_SLOTS rows of that, each of 128 columns or more (K of the second expert GEMM).
+constexpr int MOE_TAB_PARTS = 64;
+static_assert((MOE_ONE_WG_SLOTS + 1) * 128 * sizeof(half_t) >=
+                  (size_t)(MOE_PARTS_MAX - MOE_TAB_PARTS) * AWQMI_MAX_EXPERTS * sizeof(int32_t),
+              "every part's counts lie inside the workspace");
 static int moe_route_launches(const MoeRoute& r, int tile, void* stream) {
   if (const int rc = ensure_kernel_attributes()) return rc;
   const int n_slots = r.T * r.topk, cap = (int)awqmi_moe_align_capacity(n_slots, r.E, tile);
@@ -532,7 +537,7 @@ static int moe_route_launches(const MoeRoute& r, int tile, void* stream) {
       return rc;
     return moe_align_launch(r.ids, n_slots, r.E, tile, r.sorted, r.experts, r.npp, r.runs, stream);
   }
-  const MoeParts pt = moe_parts(r.T, r.tab_parts);
+  const MoeParts pt = moe_parts(r.T);
   const int waves = std::min(16, pt.part / wave_tokens);
   moe_topk_form(r.E, r.topk, r.scoring, [&](auto L, auto P, auto S) {
     hipLaunchKernelGGL((moe_route_count_kernel<decltype(L)::value, decltype(P)::value, decltype(S)::value>), dim3(pt.parts),
@@ -1365,9 +1370,8 @@ struct FusedMoeLayout {
   size_t gemm_ws, ids, wts, sorted, experts, npp, h13, act, o, total;
   size_t gemm_ws_bytes;
   int n_slots, cap, tile;
-  size_t tab;      // expert counts of the parts of a longer batch
+  size_t tab;      // expert counts of the parts of a longer batch; runs on into act
 };
-constexpr int MOE_TAB_PARTS = 64;
 FusedMoeLayout fused_moe_layout(int T, int H, int inter, int E, int topk, int tile) {
   FusedMoeLayout L{};
   auto up = [](size_t v) { return (v + 255) / 256 * 256; };
@@ -1384,8 +1388,8 @@ FusedMoeLayout fused_moe_layout(int T, int H, int inter, int E, int topk, int ti
   L.sorted = off;  off += up((size_t)L.cap * 4);
   L.experts = off; off += up((size_t)(L.cap / L.tile) * 4);
   L.npp = off;     off += 256;
-  L.tab = off;     off += up((size_t)MOE_TAB_PARTS * E * 4);
   L.h13 = off;     off += up((size_t)L.n_slots * 2 * inter * 2);
+  L.tab = off;     off += up((size_t)MOE_TAB_PARTS * E * 4);
   L.act = off;     off += up((size_t)L.n_slots * inter * 2);
   L.o = off;       off += up((size_t)L.n_slots * H * 2);
   L.total = off;
@@ -1452,11 +1456,8 @@ int awqmi_fused_moe_routed_f16(const void* hidden, const float* router_logits, c
   void* o = ws + L.o;
   int st;
   int32_t* const runs = form.runs ? reinterpret_cast<int32_t*>(h13) : nullptr;
-  // the table of more parts lies where the activation goes later
-  const bool more = (size_t)L.n_slots * inter * 2 >= (size_t)MOE_PARTS_MAX * E * 4;
   const MoeRoute route{router_logits, score_bias, T, E, topk, scoring, renormalize, routed_scale,
-                       ids, wts, sorted, experts, npp, runs, more ? static_cast<int32_t*>(act_out) : reinterpret_cast<int32_t*>(ws + L.tab),
-                       more ? MOE_PARTS_MAX : MOE_TAB_PARTS};
+                       ids, wts, sorted, experts, npp, runs, reinterpret_cast<int32_t*>(ws + L.tab)};
   // a handful of tokens: the first expert GEMM takes the routing along (one launch less)
   const bool fold = moe_route_foldable(T, E, topk, tile);
   const MoeRoute* pending = fold ? &route : nullptr;

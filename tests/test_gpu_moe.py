@@ -670,6 +670,47 @@ def test_routing_in_one_two_and_several_workgroups(sba, gpu, scoring, T, E, topk
         assert torch.equal(one, step)
 
 
+@pytest.mark.parametrize("T,E,topk", [(257, 128, 8), (2049, 4, 2), (2050, 5, 1), (300, 1024, 17), (2100, 256, 16), (8192, 128, 8),
+                                      (3001, 1024, 3)])
+def test_parts_leave_the_lists_of_one_workgroup(sba, gpu, T, E, topk):
+    """The one-call block with its routing in parts and with the align in one workgroup (development variant 16384): picks,
+    weights, sorted slots, block owners and padded count in the workspace are the same words, to the end of the lists, whatever the
+    workspace held, and the align's are the oracle's."""
+    from server_benchmark_amd import _lib
+    lib = _lib.load()
+    H, I, n = 256, 128, T * topk
+    assert n > 2048
+    c = sba.workloads.make_moe_case(T, H, E, topk, I, 128, seed=T + E).to(gpu)
+    bs = lib.awqmi_fused_moe_block_rows(T, H, I, E, topk, 128)
+    need = lib.awqmi_fused_moe_workspace_bytes(T, H, I, E, topk)
+    up = lambda v: (v + 255) // 256 * 256
+    cap = lib.awqmi_moe_align_capacity(n, E, bs)
+    start = up(max(lib.awqmi_moe_gemm_workspace_bytes(n, E, H, 2 * I, 0, bs), lib.awqmi_moe_gemm_workspace_bytes(n, E, I, H, 0, bs))) // 4
+    words = [n, n, cap, cap // bs, 1]                  # ids, weights, sorted slots, block owners, padded count
+    lists, outs = [], []
+    for variant, fill in ((-1, 0x55), (16384, 0x33)):
+        ws = torch.full((need,), fill, dtype=torch.uint8, device=gpu)
+        ws[:65536] = 0                                 # arrival counters
+        y = torch.empty((T, H), dtype=torch.float16, device=gpu)
+        st = lib.awqmi_dev_fused_moe_routed_f16(
+            c.x.data_ptr(), c.logits.data_ptr(), 0, *(t.data_ptr() for t in (*c.w13, *c.w2)), y.data_ptr(), T, H, I, E, topk, 128, 0, 1,
+            1.0, ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream, variant)
+        assert st == 0
+        w, at, got = ws[:need // 4 * 4].view(torch.int32), start, []
+        for k in words:
+            got.append(w[at:at + k].cpu())
+            at += up(4 * k) // 4
+        lists.append(got)
+        outs.append(y)
+    for a, b in zip(*lists):
+        assert torch.equal(a, b)
+    rs, re, rn = awq_ref.moe_align(lists[0][0].numpy().reshape(T, topk), E, bs)
+    s, e = lists[0][2].numpy(), lists[0][3].numpy()
+    assert int(lists[0][4]) == rn and np.array_equal(s[:rn], rs) and np.array_equal(e[:rn // bs], re)
+    assert np.all(s[rn:] == n) and np.all(e[rn // bs:] == -1)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
 @pytest.mark.parametrize("scoring", ["softmax", "sigmoid"])
 @pytest.mark.parametrize("T,H,E,topk,I", [(1, 2048, 128, 8, 768), (2, 2048, 128, 8, 768), (3, 2048, 128, 8, 768),
                                           (4, 2048, 128, 8, 768), (4, 512, 64, 6, 256), (1, 256, 8, 1, 128),
