@@ -375,6 +375,33 @@ def test_tiles_of_16_slot_blocks_are_as_near_to_64_bits_as_single_blocks(sba, gp
     assert float((tiles - ref).norm()) <= 1.01 * float((single - ref).norm())
 
 
+@pytest.mark.parametrize("T,H,E,topk,I,G", [(320, 1024, 64, 4, 512, 128), (440, 1024, 64, 4, 512, 64), (400, 2048, 128, 8, 768, 128)])
+def test_blocks_of_twenty_slots_per_expert_are_as_near_to_64_bits_in_tiles(sba, gpu, T, H, E, topk, I, G):
+    """From 20 to 28 slots per expert, where the call takes its 16-slot blocks in tiles by its own rule: several picks a token, the
+    block against exact weights and float64 sums, routed as the kernel routed it, beside the same block on single blocks."""
+    from server_benchmark_amd import _lib
+    assert _lib.load().awqmi_dev_fused_moe_tiles(T, H, I, E, topk, G, -1) == 1 and 20 <= T * topk / E < 28
+    c = sba.workloads.make_moe_case(T, H, E, topk, I, G, seed=T + G).to(gpu)
+    w, ids = sba.topk_softmax(c.logits, topk, True)
+    def exact(q, s, z):
+        v = awq_ref.unpack_awq(q.cpu().numpy()).astype(np.float64) - awq_ref.unpack_awq(z.cpu().numpy()).astype(np.float64).repeat(G, 0)
+        return torch.from_numpy(v * s.cpu().numpy().astype(np.float64).repeat(G, 0)).to(gpu)
+    ref = torch.zeros((T, H), dtype=torch.float64, device=gpu)
+    for e in range(E):
+        tok, slot = torch.nonzero(ids == e, as_tuple=True)
+        if tok.numel() == 0:
+            continue
+        gate, up = (c.x[tok].double() @ exact(*(t[e] for t in c.w13))).chunk(2, dim=-1)
+        o = (torch.nn.functional.silu(gate) * up) @ exact(*(t[e] for t in c.w2))
+        ref.index_add_(0, tok, o * w[tok, slot].double()[:, None])
+    tiles, single = (sba.fused_moe_awq(c.x, c.w13, c.w2, c.logits, topk, True, _dev_variant=v).double() for v in (-1, 2048))
+    assert not torch.equal(tiles, single)
+    err = [float((y - ref).norm() / ref.norm()) for y in (tiles, single)]
+    print(f"[moe tiles T={T} E={E} G={G}] to 64 bits {err[0]:.5e}, single blocks {err[1]:.5e}", flush=True)
+    # 1 %: half of either error is not shared (above); 300 thousand values' norm moves by 0.2 %
+    assert err[0] <= 1.01 * err[1]
+
+
 @pytest.mark.parametrize("T,H,E,topk,I,mfma", [(2048, 2048, 128, 8, 768, False), (1024, 1024, 8, 2, 2048, False),
                                                (4096, 512, 4, 2, 384, False),     # many rows per expert
                                                (640, 256, 4, 1, 1152, False),     # top-1
@@ -751,8 +778,10 @@ def test_routing_folded_into_the_first_expert_gemm(sba, gpu, scoring, T, H, E, t
 @pytest.mark.parametrize("T,E,topk", [(5, 128, 8), (8, 128, 8), (8, 4, 4), (7, 256, 9), (8, 33, 8), (5, 16, 12), (3, 64, 16), (9, 128, 7), (10, 128, 7),
                                       (16, 4, 4), (16, 8, 2), (13, 256, 4), (17, 64, 2)])
 def test_routing_folded_for_five_to_sixteen_tokens(sba, gpu, scoring, T, E, topk):
-    """Up to four waves with four tokens each, up to 64 slots, blocks of up to 16 rows, experts in the first and the last word
-    of the mask; 70 slots and 17 tokens are past the lines.  The bits of the separately routed block."""
+    """Up to four waves with four tokens each, up to 64 slots, experts in the first and the last word of the mask; 70 slots, 17
+    tokens and a full block for every expert (16 tokens on four) are past the lines.  The bits of the separately routed block."""
+    from server_benchmark_amd import _lib
+    assert _lib.load().awqmi_dev_fused_moe_folds(T, 512, 256, E, topk, 128, -1) == ((T, E, topk) not in ((10, 128, 7), (16, 4, 4), (17, 64, 2)))
     c = sba.workloads.make_moe_case(T, 512, E, topk, 256, 128, seed=5 * T + E).to(gpu)
     kw = {}
     if scoring == "sigmoid":
@@ -760,6 +789,31 @@ def test_routing_folded_for_five_to_sixteen_tokens(sba, gpu, scoring, T, E, topk
     y = sba.fused_moe_awq(c.x, c.w13, c.w2, c.logits, topk, True, **kw).clone()
     y_sep = sba.fused_moe_awq(c.x, c.w13, c.w2, c.logits, topk, True, _dev_variant=1 << 24, **kw)
     assert torch.equal(y.view(torch.int16), y_sep.view(torch.int16))
+
+
+@pytest.mark.parametrize("scoring", ["softmax", "sigmoid"])
+@pytest.mark.parametrize("T,E,topk,busy", [(16, 8, 4, 0), (16, 8, 4, 7), (9, 64, 2, 63), (16, 64, 2, 0), (13, 33, 4, 32), (16, 256, 4, 255),
+                                           (12, 128, 5, 31), (16, 16, 1, 15), (16, 64, 4, 40)])
+def test_folded_routing_fills_a_block_to_its_last_row(sba, gpu, scoring, T, E, topk, busy):
+    """One expert -- the first, the last, one at a word's edge of the mask -- is picked by all of 9 to 16 tokens, so that its block
+    has that many rows: the bits of the separately routed block, and the oracle's result."""
+    from server_benchmark_amd import _lib
+    assert _lib.load().awqmi_dev_fused_moe_folds(T, 512, 256, E, topk, 128, -1) == 1
+    c = sba.workloads.make_moe_case(T, 512, E, topk, 256, 128, seed=3 * T + E + busy)
+    c.logits[:, busy] = c.logits.max(dim=1).values + torch.linspace(-0.01, 0.4, T)       # first pick, or (first token) second
+    kw = {}
+    if scoring == "sigmoid":
+        kw = dict(scoring_func="sigmoid", routed_scaling_factor=1.25)
+        ids, tw = awq_ref.topk_sigmoid(c.logits.numpy(), topk, True, None, 1.25)
+    else:
+        ids, tw = awq_ref.topk_softmax(c.logits.numpy(), topk, True)
+    assert 9 <= (np.asarray(ids) == busy).sum() >= T - (topk == 1)
+    d = c.to(gpu)
+    y = sba.fused_moe_awq(d.x, d.w13, d.w2, d.logits, topk, True, **kw).clone()
+    y_sep = sba.fused_moe_awq(d.x, d.w13, d.w2, d.logits, topk, True, _dev_variant=1 << 24, **kw)
+    assert torch.equal(y.view(torch.int16), y_sep.view(torch.int16))
+    ref = awq_ref.moe_forward(c.x.numpy(), tuple(a.numpy() for a in c.w13), tuple(a.numpy() for a in c.w2), ids, tw, 128)
+    assert awq_ref.rel_frobenius(y.cpu().numpy(), ref) <= TOL
 
 
 @pytest.mark.parametrize("scoring", ["softmax", "sigmoid"])
