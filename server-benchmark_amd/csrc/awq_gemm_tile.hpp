@@ -207,11 +207,11 @@ __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, 
   // loads out of range (X_NOWHERE), four layers, us before / after: 72B at 100 rows 258 / 246, 7B (groups of 64) 123.5 / 113.5, at 128
   // rows 128 / 122, 5120-wide at 100 rows 121.6 / 116, at 200 176 / 164, at 256 189 / 181; others within 1 %; blocks of 1500 and
   // 3000 tokens on 128 experts of 2048 x 768, top-8, 183 / 172 and 316 / 304.
-  // NL0: loads of the first k-step.
   constexpr bool MID = D == 3;
-  constexpr int NL0 = ((NP - 1) * NL + LP - 1) / LP < NL ? ((NP - 1) * NL + LP - 1) / LP : NL;
   constexpr int UF = 6;                       // MFMAs of the second k-step ahead of its unpacking
   static_assert(!MID || XF <= RT, "fragments of the next stage are read in the second k-step");
+  static_assert(!MID || 1 + (NL - 1) * LP / NL < NP, "the wait in mid-stage counts on all loads of a stage being in its first k-step");
+  static_assert(!MID || !SCALE32, "the scales of a group's sum are read in the other form only");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -485,7 +485,7 @@ __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, 
     asm volatile("" : "+v"(xn[0]), "+v"(xn[1]), "+v"(fwn));
     kstep(I0{}, FIRST, LAST, xc, xn, fwn, nxt);
     if constexpr (MID) {
-      tg_wait_and_barrier<(D - 3) * NL + NL0>();
+      tg_wait_and_barrier<NL>();
       __builtin_amdgcn_sched_barrier(0);
     }
     kstep(I1{}, FIRST, LAST, xc, xn, fwn, nxt);
