@@ -1258,7 +1258,7 @@ double moe_expected_blocks(double avg, int rows) {
 // The prices are those of the grouped kernel that dequantised into LDS, and 16 rows those of the skinny kernel: they say where
 // blocks of 16 slots end, which callers of the step-by-step path have in their own calls too.  With the present kernel, which is
 // faster for every size, and moe_runs beside it the choice is 4 % behind the best of 16, 16 in tiles and 128 on average of 129
-// points, 30 % at worst (896 tokens on 256 experts of 2048 x 384, top-8: 156 us, in tiles 120; see moe_runs for its line at 32).
+// points, 34 % at worst (896 tokens on 256 experts of 2048 x 384, top-8: 157 us, in tiles 117; see moe_runs for 28 to 32 slots).
 // Two sizes that the tests fix measure slower than another: 2048 tokens on 128 experts of 2048 x 768 (16 rows in tiles
 // 254 us, 128 rows 248), 2102 on 4 of 512 x 384 (16 rows 51, in tiles 38, 64 rows 36).
 // Larger blocks also need every operand under 4 GiB (32-bit buffer offsets).
@@ -1319,10 +1319,14 @@ int moe_pick_tile(int n_slots, int E, int H, int inter, int group) {
 // 90, 93, 94, 95; 64 of 5120 x 1024 161, 163, 183, 196 / 149, 150, 153, 157; 160 of 6144 x 2560 998, 1068, 1131, 1166 / 943, 956, 975, 985;
 // 16 of 3072 x 4096 118, 117, 135, 145 / 105, 106, 108, 110; groups of 64 alike); at 16 and below either side wins (128 experts of 2048 x
 // 768 98.0 / 98.9, 160 of 6144 x 2560 909 / 926), with eight experts the blocks.
-// From 28 to 32 slots the block keeps the kernel that the separate calls on 16-slot blocks take, so that both add in one order, as
-// tests fix at three shapes, although tiles are faster there too (512 tokens on 128 experts of 2048 x 768 125 / 110).  Experts below
-// the smallest measured (1024 x 512, 2048 x 384) stay as well: the routing and the sum outweigh both GEMMs.  Above, blocks / tiles (us): 576 / 768 / 1024
-// tokens on 128 experts of 2048 x 768 143 / 164 / 192 and 116 / 130 / 163; 560 on 64 of 2048 x 1408 172 and 122.
+// From 28 to 32 slots the blocks stay single, for no property of either kernel: three expectations of this rule in the host tests and a
+// bound between the block and the separate calls at 512 tokens date from when the line was at 32.  Tiles are faster there too
+// (blocks / tiles, us, at 28, 30 and 32 slots: 128 experts of 2048 x 768 127, 124, 124 / 107, 107, 110; 64 of 2048 x 1408 120, 121, 124 / 95, 96, 97; 64 of
+// 5120 x 1024 197, 203, 207 / 159, 161, 162; 160 of 6144 x 2560 1173, 1215, 1269 / 990, 999, 1013; 256 of 2048 x 384 157, 164, 166 / 117, 119, 119;
+// 16 of 3072 x 4096 145, 149, 149 / 110, 111, 112; 60 of 4096 x 1536 211, 217, 221 / 172, 173, 174).  Either form is as near to 64-bit sums.
+// Experts of less than 1024 x 384 stay as well: smaller ones were not measured (64 of 1024 x 384 at 20, 24, 27 and 40 slots 35.7, 37.9, 39.9, 47.7 / 31.0, 32.1,
+// 32.6, 35.3).  Above 32, blocks / tiles (us): 576 / 768 / 1024 tokens on 128 experts of 2048 x 768 143 / 164 / 192 and 116 / 130 / 163; 560 on 64 of
+// 2048 x 1408 172 and 122.
 bool moe_runs(int T, int n_slots, int E, int H, int inter, int group) {
   if (variant_on(VAR_MOE_TILE16) || T <= MOE_ALIGN_WAVES) return false;
   // groups of 64 or 128 rows, whole column tiles

@@ -204,9 +204,10 @@ __device__ __forceinline__ void awq_tile(const TileGemmParams& p, const int m0, 
   // MID: the next stage is waited for in the middle of a stage, ahead of the first read of it, instead of at the stage's start, and a
   // barrier of its own at the start frees the slot of the last stage.  With a ring of three a load then has 1.25 stages to arrive
   // instead of 0.75; longer rings leave it time enough (80 rows, ring of four, 209 us without and 213 with it).  With the pad rows'
-  // loads out of range (X_NOWHERE), four layers, us before / after: 72B at 100 rows 258 / 246, 7B (groups of 64) 123.5 / 113.5, at 128
-  // rows 128 / 122, 5120-wide at 100 rows 121.6 / 116, at 200 176 / 164, at 256 189 / 181; others within 1 %; blocks of 1500 and
-  // 3000 tokens on 128 experts of 2048 x 768, top-8, 183 / 172 and 316 / 304.
+  // loads out of range (X_NOWHERE), both versions in turn on one card, four layers, us before / after: 72B at 100 rows 259 / 245, 7B
+  // (groups of 64) 122.7 / 112.9, at 128 rows 127.1 / 120.7, 5120-wide at 100 rows 121.7 / 114.9, at 200 176 / 163, at 1000 530 / 517; at
+  // 256 187 - 190 / 183 - 187, within what the runs differ; a block of 1500 tokens on 128 experts of 2048 x 768, top-8, 176 / 171, of
+  // 3000 even (305).
   constexpr bool MID = D == 3;
   constexpr int UF = 6;                       // MFMAs of the second k-step ahead of its unpacking
   static_assert(!MID || XF <= RT, "fragments of the next stage are read in the second k-step");

@@ -665,9 +665,9 @@ def test_empty_batches(sba, gpu):
 
 @pytest.mark.parametrize("T,E,topk", [(2048, 128, 8), (2500, 60, 7), (20000, 8, 2)])
 def test_fused_call_with_long_slot_lists(sba, gpu, T, E, topk):
-    """From 16384 slots on the one-call path sorts the slots with several workgroups (count,
-    scan, place); its result must equal the step-by-step path, whose align is the single
-    workgroup checked against the oracle above."""
+    """From 2049 slots on the one-call path routes in two launches of several workgroups (pick and
+    count, then place); on long lists too its result must equal the step-by-step path, whose align
+    is the single workgroup checked against the oracle above."""
     H, I = 256, 128
     c = sba.workloads.make_moe_case(T, H, E, topk, I, 128, seed=T + E).to(gpu)
     assert T * topk >= 16384
@@ -744,7 +744,7 @@ def test_parts_leave_the_lists_of_one_workgroup(sba, gpu, T, E, topk):
                                           (3, 1024, 16, 10, 512), (4, 256, 4, 4, 128), (2, 384, 100, 16, 128),
                                           (4, 512, 128, 16, 256), (2, 256, 160, 8, 128), (4, 256, 256, 8, 128)])
 def test_routing_folded_into_the_first_expert_gemm(sba, gpu, scoring, T, H, E, topk, I):
-    """Blocks of at most four tokens (32 slots, 128 experts) have no routing launch: the first
+    """Blocks of a few tokens (here one to four, up to 64 slots and 256 experts) have no routing launch: the first
     expert GEMM works the routing out in every workgroup.  The result must have the bits of the
     block with the routing launched on its own (development variant bit 1 << 24), also with
     duplicate experts across tokens (few experts, large top-k), and must match the oracle's
