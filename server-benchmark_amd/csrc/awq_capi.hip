@@ -503,11 +503,14 @@ static int moe_align_launch(const int32_t* topk_ids, int n_slots, int E, int til
   return launch_status();
 }
 // Routing + align of a block as launches of their own.  Up to 32 tokens (16 with a token a wave): one launch of one workgroup.  Up to 2048
-// slots: top-k over many, then one workgroup for the align.  More: two launches over up to MOE_PARTS_MAX workgroups, each with at least
-// sixteen tokens.  Whole block, 128 experts of 2048 x 768, top-8, us, as it was before / one launch / top-k and one workgroup / two
+// slots (11264 with a token a wave): top-k over many, then one workgroup for the align.  More: two launches over up to MOE_PARTS_MAX
+// workgroups, each with at least sixteen tokens; with a token a wave three, the picks having one of their own.  Whole block, 128 experts of 2048 x 768, top-8, us, as it was before / one launch / top-k and one workgroup / two
 // launches of parts: 16 tokens 62.2 / 59.3 / - / -; 32 72.2 / 70.5 / - / -; 48 73.3 / 72.9 / 72.5 / -; 64 75.3 / 75.3 / 74.5 / -; 128 80.6 / - /
 // 80.1 / 81.2; 256 98 / - / 97.5 / 97.3; 1500 172 / - / - / 166; 8192 696 / - / - / 688.
-constexpr int MOE_ONE_WG_SLOTS = 2048;
+// A token a wave, blocks of 256 x 128, us, align in one workgroup / in parts: 4096, 8192, 12000, 16000, 24000 slots of 512 experts, top-10 49.3,
+// 54.8, 62.4, 73.5, 94.2 / 51.9, 54.0, 58.8, 67.6, 82.0; of 257, top-8 38.2, 50.1, 58.5, 69.1, 89.7 / 40.8, 49.5, 56.9, 64.7, 80.2; of 1024, top-2 56.1, 69.1,
+// 76.8, 88.5, 116 / 60.2, 71.8, 78.7, 87.0, 107.7; of 64, top-17 35.1, 47.8, 53.8, 62.6, 76.7 / 35.8, 45.9, 50.9, 57.7, 66.1.
+constexpr int MOE_ONE_WG_SLOTS = 2048, MOE_ONE_WG_SLOTS_WAVE = 11264;
 struct MoeParts { int part, parts; };     // tokens of a part, parts
 static MoeParts moe_parts(int T) {
   const int part = (T + 16 * MOE_PARTS_MAX - 1) / (16 * MOE_PARTS_MAX) * 16;
@@ -532,17 +535,24 @@ static int moe_route_launches(const MoeRoute& r, int tile, void* stream) {
     });
     return launch_status();
   }
-  if (n_slots <= MOE_ONE_WG_SLOTS || variant_on(VAR_ALIGN_ONE_WG)) {
+  if (n_slots <= (wave_tokens > 1 ? MOE_ONE_WG_SLOTS : MOE_ONE_WG_SLOTS_WAVE) || variant_on(VAR_ALIGN_ONE_WG)) {
     if (const int rc = awqmi_moe_topk_f32(r.logits, r.bias, r.T, r.E, r.topk, r.scoring, r.renorm, r.scale, r.ids, r.wts, stream))
       return rc;
     return moe_align_launch(r.ids, n_slots, r.E, tile, r.sorted, r.experts, r.npp, r.runs, stream);
   }
   const MoeParts pt = moe_parts(r.T);
-  const int waves = std::min(16, pt.part / wave_tokens);
-  moe_topk_form(r.E, r.topk, r.scoring, [&](auto L, auto P, auto S) {
-    hipLaunchKernelGGL((moe_route_count_kernel<decltype(L)::value, decltype(P)::value, decltype(S)::value>), dim3(pt.parts),
-                       dim3(64 * waves), 0, st, r.logits, r.bias, r.T, r.E, r.topk, r.renorm, r.scale, r.ids, r.wts, pt.part, r.tab);
-  });
+  if (wave_tokens > 1) {
+    const int waves = std::min(16, pt.part / wave_tokens);
+    moe_topk_form(r.E, r.topk, r.scoring, [&](auto L, auto P, auto S) {
+      if constexpr (decltype(L)::value == 16)
+        hipLaunchKernelGGL((moe_route_count_kernel<decltype(P)::value, decltype(S)::value>), dim3(pt.parts), dim3(64 * waves), 0, st,
+                           r.logits, r.bias, r.T, r.E, r.topk, r.renorm, r.scale, r.ids, r.wts, pt.part, r.tab);
+    });
+  } else {
+    if (const int rc = awqmi_moe_topk_f32(r.logits, r.bias, r.T, r.E, r.topk, r.scoring, r.renorm, r.scale, r.ids, r.wts, stream))
+      return rc;
+    hipLaunchKernelGGL(moe_count_kernel, dim3(pt.parts), dim3(1024), 0, st, r.ids, n_slots, r.E, pt.part * r.topk, r.tab);
+  }
   hipLaunchKernelGGL(moe_align_parts_kernel, dim3(pt.parts), dim3(1024), (size_t)moe_parts_lds(r.E), st, r.ids, n_slots, r.E,
                      pt.part * r.topk, tile, cap, r.tab, r.sorted, r.experts, r.npp, r.runs);
   return launch_status();

@@ -433,12 +433,12 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
 }
 
 // Longer batches in two launches, part b of each one's workgroups being tokens [b * part, (b + 1) * part):
-// the first picks the experts and counts its part's picks, the second places them.
+// the first picks the experts (16 lanes a token) and counts its part's picks, the second places them.
 //
 // (Four launches before from 16384 slots on: top-k, count, scan in one workgroup, place; 12.6 + 4.9 + 12.0 + 7.8 us for 8192 tokens,
 // 128 experts, top-8, against 8.7 + 9.2.)
 constexpr int MOE_PARTS_MAX = 128;
-template <int LANES, int PER, bool SIGMOID>
+template <int PER, bool SIGMOID>
 __global__ __launch_bounds__(1024) void moe_route_count_kernel(const float* __restrict__ logits, const float* __restrict__ bias,
                                                                int T, int E, int topk, int renorm, float scale,
                                                                int* __restrict__ ids, float* __restrict__ wts, int part,
@@ -448,13 +448,27 @@ __global__ __launch_bounds__(1024) void moe_route_count_kernel(const float* __re
   for (int e = tid; e < E; e += threads) cnt[e] = 0;
   __syncthreads();
   const int begin = (int)blockIdx.x * part, end = min(T, begin + part);
-  constexpr int TOK = 64 / LANES;      // tokens of a wave
-  for (int t0 = begin + (tid >> 6) * TOK; t0 < end; t0 += (threads >> 6) * TOK) {
-    const int e = moe_topk_tokens<LANES, PER, SIGMOID>(logits, bias, t0, end, E, topk, renorm, scale, ids, wts);
+  for (int t0 = begin + (tid >> 6) * 4; t0 < end; t0 += (threads >> 6) * 4) {
+    const int e = moe_topk_tokens<16, PER, SIGMOID>(logits, bias, t0, end, E, topk, renorm, scale, ids, wts);
     if (e >= 0) atomicAdd(&cnt[e], 1);
   }
   __syncthreads();
   for (int e = tid; e < E; e += threads) part_cnt[(size_t)blockIdx.x * E + e] = cnt[e];
+}
+
+// With a token a wave the picks need the whole chip, and have a launch of their own; a part's are counted from memory.  Block of 256 x 128, us,
+// picked and counted by 128 workgroups / apart / top-k, count, scan and place: 2048, 8192, 16384 tokens, 8 of 1024 experts 89.5, 224, 402 / 86.9, 186,
+// 319 / 113, 214, 345; 8 of 257 67.2, 179, 323 / 65.5, 156, 271 / 74.0, 166, 281; 65536 tokens, 2 of 1024 447 / 336 / 363.
+__global__ __launch_bounds__(1024) void moe_count_kernel(const int* __restrict__ ids, int n, int E, int part,
+                                                         int* __restrict__ part_cnt) {
+  __shared__ int cnt[1024];      // E <= 1024
+  const int tid = threadIdx.x;
+  for (int e = tid; e < E; e += 1024) cnt[e] = 0;
+  __syncthreads();
+  const int s0 = min(n, (int)blockIdx.x * part), s1 = min(n, s0 + part);
+  for (int i = s0 + tid; i < s1; i += 1024) atomicAdd(&cnt[ids[i]], 1);
+  __syncthreads();
+  for (int e = tid; e < E; e += 1024) part_cnt[(size_t)blockIdx.x * E + e] = cnt[e];
 }
 
 // Every workgroup adds up the table of counts (parts x E) by itself: each expert's slots in all and those of the parts before

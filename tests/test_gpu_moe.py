@@ -665,8 +665,8 @@ def test_empty_batches(sba, gpu):
 
 @pytest.mark.parametrize("T,E,topk", [(2048, 128, 8), (2500, 60, 7), (20000, 8, 2)])
 def test_fused_call_with_long_slot_lists(sba, gpu, T, E, topk):
-    """From 2049 slots on the one-call path routes in two launches of several workgroups (pick and
-    count, then place); on long lists too its result must equal the step-by-step path, whose align
+    """On long slot lists the one-call path picks, counts and places with several workgroups;
+    there too its result must equal the step-by-step path, whose align
     is the single workgroup checked against the oracle above."""
     H, I = 256, 128
     c = sba.workloads.make_moe_case(T, H, E, topk, I, 128, seed=T + E).to(gpu)
@@ -681,10 +681,10 @@ def test_fused_call_with_long_slot_lists(sba, gpu, T, E, topk):
 
 @pytest.mark.parametrize("scoring", ["softmax", "sigmoid"])
 @pytest.mark.parametrize("T,E,topk", [(32, 128, 8), (33, 128, 8), (16, 64, 17), (17, 64, 17), (256, 128, 8), (257, 128, 8),
-                                      (2049, 4, 2), (2050, 5, 1), (300, 1024, 17), (2100, 256, 16), (130, 257, 16)])
+                                      (2049, 4, 2), (2050, 5, 1), (300, 1024, 17), (2100, 256, 16), (130, 257, 16), (662, 64, 17), (663, 64, 17)])
 def test_routing_in_one_two_and_several_workgroups(sba, gpu, scoring, T, E, topk):
-    """Both sides of the rule for the block's routing launches (32 tokens, 16 with a token a wave, 2048 slots; a last part of
-    one token): the block must equal the step-by-step path, whose top-k and align are checked against the oracle above."""
+    """Both sides of the rule for the block's routing launches (32 tokens, 16 with a token a wave; 2048 slots, 11264 with a token
+    a wave; a last part of one token): the block must equal the step-by-step path, whose top-k and align are checked against the oracle above."""
     c = sba.workloads.make_moe_case(T, 256, E, topk, 128, 128, seed=T + E).to(gpu)
     kw = {}
     if scoring == "sigmoid":
@@ -698,7 +698,7 @@ def test_routing_in_one_two_and_several_workgroups(sba, gpu, scoring, T, E, topk
 
 
 @pytest.mark.parametrize("T,E,topk", [(257, 128, 8), (2049, 4, 2), (2050, 5, 1), (300, 1024, 17), (2100, 256, 16), (8192, 128, 8),
-                                      (3001, 1024, 3)])
+                                      (700, 1024, 17), (3761, 1024, 3), (4097, 257, 4), (16385, 300, 1)])
 def test_parts_leave_the_lists_of_one_workgroup(sba, gpu, T, E, topk):
     """The one-call block with its routing in parts and with the align in one workgroup (development variant 16384): picks,
     weights, sorted slots, block owners and padded count in the workspace are the same words, to the end of the lists, whatever the
