@@ -19,7 +19,7 @@
  *   1024     the one-call MoE block always runs the separate activation kernel, 16-slot blocks then one by one
  *   2048     the one-call MoE block always uses the skinny kernel's 16-row blocks
  *   4096     every launch keeps the weight ring in registers (no LDS ring)
- *   16384    the one-call MoE block: top-k, then the align in one workgroup, also beyond 2048 slots
+ *   16384    the one-call MoE block: top-k, then the align in one workgroup, however many slots
  *   1 << 16  v = bits 16..17: the one-call MoE block uses 64 / 128 / 256-row blocks (v = 1 / 2 / 3)
  *   1 << 18  awq_gemm with 17..64 rows: skinny passes wherever they can run
  *   1 << 19  awq_gemm with 17..64 rows: the tile kernel wherever it can run

@@ -502,15 +502,18 @@ static int moe_align_launch(const int32_t* topk_ids, int n_slots, int E, int til
                      (hipStream_t)stream, topk_ids, n_slots, E, tile_m, cap, sorted, experts, npp, runs);
   return launch_status();
 }
-// Routing + align of a block as launches of their own.  Up to 32 tokens (16 with a token a wave): one launch of one workgroup.  Up to 2048
+// Routing + align of a block as launches of their own.  Up to 32 tokens (16 with a token a wave): one launch of one workgroup.  Up to 3584
 // slots (11264 with a token a wave): top-k over many, then one workgroup for the align.  More: two launches over up to MOE_PARTS_MAX
 // workgroups, each with at least sixteen tokens; with a token a wave three, the picks having one of their own.  Whole block, 128 experts of 2048 x 768, top-8, us, as it was before / one launch / top-k and one workgroup / two
 // launches of parts: 16 tokens 62.2 / 59.3 / - / -; 32 72.2 / 70.5 / - / -; 48 73.3 / 72.9 / 72.5 / -; 64 75.3 / 75.3 / 74.5 / -; 128 80.6 / - /
 // 80.1 / 81.2; 256 98 / - / 97.5 / 97.3; 1500 172 / - / - / 166; 8192 696 / - / - / 688.
-// A token a wave, blocks of 256 x 128, us, align in one workgroup / in parts: 4096, 8192, 12000, 16000, 24000 slots of 512 experts, top-10 49.3,
+// Four tokens a wave, blocks of 256 x 128, align in one workgroup / in parts at 2064, 3200, 4096, 6500 slots: 256 experts, top-8 31.9, 33.9, 34.8, 44.2 / 32.7,
+// 34.7, 35.2, 44.1; 256, top-2 30.0, 32.3, 33.2, 43.0 / 30.9, 34.6, 33.5, 43.2; 128, top-8 27.5, 29.5, 32.2, 35.8 / 28.0, 29.5, 31.7, 34.3; 128, top-2
+// 26.2, 28.6, 30.8, 34.8 / 28.1, 31.0, 30.7, 35.2; 64, top-6 26.6, 27.6, 30.9, 34.5 / 26.7, 27.3, 30.3, 32.8; 8, top-2 25.7, 27.3, 30.3, 35.5 / 26.5, 27.3, 29.6, 33.0.
+// A token a wave, the same block, us, align in one workgroup / in parts: 4096, 8192, 12000, 16000, 24000 slots of 512 experts, top-10 49.3,
 // 54.8, 62.4, 73.5, 94.2 / 51.9, 54.0, 58.8, 67.6, 82.0; of 257, top-8 38.2, 50.1, 58.5, 69.1, 89.7 / 40.8, 49.5, 56.9, 64.7, 80.2; of 1024, top-2 56.1, 69.1,
 // 76.8, 88.5, 116 / 60.2, 71.8, 78.7, 87.0, 107.7; of 64, top-17 35.1, 47.8, 53.8, 62.6, 76.7 / 35.8, 45.9, 50.9, 57.7, 66.1.
-constexpr int MOE_ONE_WG_SLOTS = 2048, MOE_ONE_WG_SLOTS_WAVE = 11264;
+constexpr int MOE_ONE_WG_SLOTS = 3584, MOE_ONE_WG_SLOTS_WAVE = 11264;
 struct MoeParts { int part, parts; };     // tokens of a part, parts
 static MoeParts moe_parts(int T) {
   const int part = (T + 16 * MOE_PARTS_MAX - 1) / (16 * MOE_PARTS_MAX) * 16;
